@@ -10,22 +10,134 @@
 namespace mxq {
 
 // ---------------------------------------------------------------- router logits
-// logit[t, e] = sum_h W_gate[e, h] * x[t, h]: one wave per (expert, token), fp32 weights,
-// 4 elements per lane per step (16-byte weight loads).
+// logit[t, e] = sum_h W_gate[e, h] * x[t, h], fp32 weights and sums.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Up to this many (expert, token) rows a workgroup per row is the faster form (128 experts, hidden 2048: 48 tokens 5.0 us against
+// 7.6 in tiles, 64 tokens about 6.2, 333 tokens 24 against 7.6).
+constexpr uint64_t kRouterRowGroups = 8192;
+// A few tokens: one workgroup per (expert, token), so that a row is two or three loads per thread, all of them in flight
+// at once (latency is all there is: 32 experts, hidden 2880, one token 3.0 -> 2.0 us against one wave per row).
 __global__ __launch_bounds__(256) void router_logits_kernel(const half_t* x, const float* W, float* logits, uint32_t hidden, uint32_t E) {
-    const uint32_t lane = threadIdx.x & 63u, e = blockIdx.x * 4u + (threadIdx.x >> 6), t = blockIdx.y;
+    __shared__ float red[4];
+    const uint32_t e = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
+    const float* wr = W + (size_t)e * hidden;
+    const half_t* xr = x + (size_t)t * hidden;
     float acc = 0.f;
-    if (e < E) {
-        const float* wr = W + (size_t)e * hidden;
-        const half_t* xr = x + (size_t)t * hidden;
-        for (uint32_t i = lane * 4; i < hidden; i += 256) {
-            const float4 w4 = *reinterpret_cast<const float4*>(wr + i);
-            const uint2 xu = *reinterpret_cast<const uint2*>(xr + i);
-            acc += w4.x * h2f(xu.x & 0xFFFFu) + w4.y * h2f(xu.x >> 16) + w4.z * h2f(xu.y & 0xFFFFu) + w4.w * h2f(xu.y >> 16);
-        }
+#pragma unroll 4
+    for (uint32_t i = tid * 4; i < hidden; i += 1024) {
+        const float4 w4 = *reinterpret_cast<const float4*>(wr + i);
+        const uint2 xu = *reinterpret_cast<const uint2*>(xr + i);
+        acc += w4.x * h2f(xu.x & 0xFFFFu) + w4.y * h2f(xu.x >> 16) + w4.z * h2f(xu.y & 0xFFFFu) + w4.w * h2f(xu.y >> 16);
     }
     acc = group_sum<64>(acc);
-    if (lane == 63 && e < E) logits[(size_t)t * E + e] = acc;
+    if ((tid & 63u) == 63u) red[tid >> 6] = acc;
+    __syncthreads();
+    if (tid == 0) logits[(size_t)t * E + e] = red[0] + red[1] + red[2] + red[3];
+}
+
+// Many tokens: 16 MI tokens x 16 NI experts per workgroup on v_mfma_f32_16x16x4_f32 (fp32 in, fp32 accumulate: the products
+// and sums of the scalar form in another order).  Lane (i, q) feeds elements 8 q .. 8 q + 7 of a 32-element piece of row i, so
+// four lanes read 64 consecutive bytes of x and 128 of W; the WV waves take the pieces of the row in turn and their sums meet in
+// LDS.  One workgroup per (expert, token), as above, reads W once per token (2048 tokens, 128 experts, hidden 2048: 2 GB through
+// the L2s, 134 us); a tile reads it once per 16 MI tokens: 17 us.  The matrix instructions alone are 6.8 us there.  With
+// 32x32x2 instructions (two lanes per row, 32-byte pieces) the loads run at half the rate and the same launch took 25.7 us with WV = 4.
+// MI = NI = 2 halves the traffic and is taken once its tiles fill half of the CUs; below that the smaller tiles spread the rows
+// over more CUs (a CU takes about 64 B a clock from its L2: 333 tokens 14.9 us with 32 x 32 tiles).
+template <int MI, int NI, int WV>
+__global__ __launch_bounds__(64 * WV) void router_logits_mfma_kernel(const half_t* __restrict__ x, const float* __restrict__ W, float* __restrict__ logits,
+                                                                     uint32_t T, uint32_t hidden, uint32_t E) {
+    constexpr int U = MI * NI == 1 ? 4 : 2;   // pieces requested together
+    __shared__ __align__(16) float red[(WV - 1) * MI * NI * 256];
+    const uint32_t lane = threadIdx.x & 63u, i = lane & 15u, q = lane >> 4;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t t0 = blockIdx.y * (16u * MI), e0 = blockIdx.x * (16u * NI);
+    const uint4* xr[MI];
+    const float4* wr[NI];
+#pragma unroll
+    for (int m = 0; m < MI; ++m) {
+        const uint32_t t = t0 + 16u * m + i;
+        xr[m] = reinterpret_cast<const uint4*>(x + (size_t)(t < T ? t : T - 1u) * hidden) + q;          // piece c: xr[4 c]
+    }
+#pragma unroll
+    for (int n = 0; n < NI; ++n) {
+        const uint32_t e = e0 + 16u * n + i;
+        wr[n] = reinterpret_cast<const float4*>(W + (size_t)(e < E ? e : E - 1u) * hidden) + 2u * q;    // piece c: wr[8 c], wr[8 c + 1]
+    }
+    const uint32_t n_pieces = hidden / 32u;
+    f32x4 acc[MI][NI];
+#pragma unroll
+    for (int m = 0; m < MI; ++m)
+#pragma unroll
+        for (int n = 0; n < NI; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Piece {
+        uint4 x[MI];
+        float4 w[NI][2];
+    };
+    auto load = [&](uint32_t c, Piece& p) {
+#pragma unroll
+        for (int m = 0; m < MI; ++m) p.x[m] = xr[m][4u * c];
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+            p.w[n][0] = wr[n][8u * c];
+            p.w[n][1] = wr[n][8u * c + 1u];
+        }
+    };
+    auto step = [&](const Piece& p) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            float a[MI], b[NI];
+#pragma unroll
+            for (int m = 0; m < MI; ++m) {
+                const uint32_t w = k < 2 ? p.x[m].x : k < 4 ? p.x[m].y : k < 6 ? p.x[m].z : p.x[m].w;
+                a[m] = h2f((k & 1) ? w >> 16 : w & 0xFFFFu);
+            }
+#pragma unroll
+            for (int n = 0; n < NI; ++n) {
+                const float4 w = p.w[n][k >> 2];
+                b[n] = (k & 3) == 0 ? w.x : (k & 3) == 1 ? w.y : (k & 3) == 2 ? w.z : w.w;
+            }
+#pragma unroll
+            for (int m = 0; m < MI; ++m)
+#pragma unroll
+                for (int n = 0; n < NI; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], b[n], acc[m][n], 0, 0, 0);
+        }
+    };
+    uint32_t c = wave;
+    for (; c + (U - 1) * WV < n_pieces; c += U * WV) {
+        Piece p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) load(c + u * WV, p[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) step(p[u]);
+    }
+    for (; c < n_pieces; c += WV) {
+        Piece p;
+        load(c, p);
+        step(p);
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int m = 0; m < MI; ++m)
+#pragma unroll
+            for (int n = 0; n < NI; ++n) *reinterpret_cast<f32x4*>(&red[(((wave - 1u) * MI + m) * NI + n) * 256u + lane * 4u]) = acc[m][n];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int m = 0; m < MI; ++m)
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+            f32x4 s = acc[m][n];
+#pragma unroll
+            for (int w = 0; w < WV - 1; ++w) s += *reinterpret_cast<const f32x4*>(&red[((w * MI + m) * NI + n) * 256 + lane * 4u]);
+            const uint32_t e = e0 + 16u * n + i;                                    // lane (i, q): column (expert) i, rows 4 q + v
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const uint32_t t = t0 + 16u * m + 4u * q + v;
+                if (t < T && e < E) logits[(size_t)t * E + e] = s[v];
+            }
+        }
 }
 
 // ---------------------------------------------------------------- softmax + top-k
@@ -36,74 +148,92 @@ __device__ __forceinline__ float wave_max_f(float v) {
     for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
     return v;
 }
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        const unsigned long long o = __shfl_xor(v, d);
-        v = o > v ? o : v;
-    }
-    return v;
+// maximum over the wave in a scalar register: DPP inside the rows, row broadcasts across them, lane 63 holds the result
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    auto step = [&](uint32_t o) { v = o > v ? o : v; };
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// One workgroup per token, one thread per expert (E <= 1024).  p = softmax(logits); K rounds of
-// a workgroup-wide maximum over the keys (bits(p) << 32 | e) — positive float bits are
-// monotonic, an exact tie goes to the higher expert id — then thread 0 renormalises the K
-// winners and orders them by ascending expert id.
-template <class LogitT>
-__global__ __launch_bounds__(1024) void topk_kernel(const LogitT* logits, int32_t* topk_idx, half_t* topk_w, uint32_t E, uint32_t K) {
-    __shared__ float red_f[16];
-    __shared__ unsigned long long red_k[16];
-    __shared__ int32_t idx_s[kMaxTopK];
-    __shared__ float w_s[kMaxTopK];
-    const uint32_t e = threadIdx.x, t = blockIdx.x, lane = e & 63u, wave = e >> 6, n_waves = (blockDim.x + 63) / 64;
-    const bool in = e < E;
-    const float logit = in ? load_act(logits + (size_t)t * E + e) : -INFINITY;
-    float m = wave_max_f(logit);
-    if (lane == 0) red_f[wave] = m;
-    __syncthreads();
-    m = red_f[0];
-    for (uint32_t w = 1; w < n_waves; ++w) m = fmaxf(m, red_f[w]);
-    __syncthreads();
-    const float ev = in ? __expf(logit - m) : 0.f;
-    float s = group_sum<64>(ev);
-    if (lane == 63) red_f[wave] = s;
-    __syncthreads();
-    s = 0.f;
-    for (uint32_t w = 0; w < n_waves; ++w) s += red_f[w];
-    const float p = ev / s;
-    bool live = in;
+// One wave per token, lane l holds the experts l, l + 64, .. (NJ of them).  p = softmax(logits); K rounds of a wave-wide
+// maximum over the float bits of p (monotonic for p >= 0; 1 is added so that 0 can mark an expert that is taken), the
+// highest id among exact ties; then every winner renormalises its own weight and finds its place by counting the winners
+// with a lower id.  No barrier, no LDS: 2048 tokens of 128 experts, k = 8, take 3.8 us where one workgroup per token with
+// two barriers per round and a serial sort took 11.8; one token of 32 experts 2.3 (4.4).
+template <class LogitT, int NJ>
+__global__ __launch_bounds__(256) void topk_kernel(const LogitT* logits, int32_t* topk_idx, half_t* topk_w, uint32_t E, uint32_t K, uint32_t n_tokens) {
+    const uint32_t lane = threadIdx.x & 63u, t = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (t >= n_tokens) return;
+    const LogitT* lg = logits + (size_t)t * E;
+    float p[NJ];
+    float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const uint32_t e = lane + 64u * j;
+        p[j] = e < E ? load_act(lg + e) : -INFINITY;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) m = fmaxf(m, p[j]);
+    m = wave_max_f(m);
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        p[j] = lane + 64u * j < E ? __expf(p[j] - m) : 0.f;
+        s += u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(group_sum<64>(p[j])), 63));
+    }
+    uint32_t key[NJ];
+    unsigned long long taken[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        p[j] = p[j] / s;
+        key[j] = lane + 64u * j < E ? f2u(p[j]) + 1u : 0u;
+        taken[j] = 0ull;
+    }
+    float ren = 0.f;
     for (uint32_t kk = 0; kk < K; ++kk) {
-        const unsigned long long key = live ? (((unsigned long long)f2u(p) << 32) | e) : 0ull;
-        const unsigned long long wm = wave_max_u64(key);
-        __syncthreads();
-        if (lane == 0) red_k[wave] = wm;
-        __syncthreads();
-        unsigned long long win = red_k[0];
-        for (uint32_t w = 1; w < n_waves; ++w) win = red_k[w] > win ? red_k[w] : win;
-        if (live && e == (uint32_t)(win & 0xFFFFFFFFull)) {
-            live = false;
-            idx_s[kk] = (int32_t)e;
-            w_s[kk] = u2f((uint32_t)(win >> 32));
+        uint32_t best = key[0];
+#pragma unroll
+        for (int j = 1; j < NJ; ++j) best = key[j] > best ? key[j] : best;
+        const uint32_t win = wave_max_u32(best);
+        ren += u2f(win - 1u);
+        bool open = true;
+#pragma unroll
+        for (int j = NJ - 1; j >= 0; --j) {
+            const unsigned long long hit = open ? __ballot(key[j] == win && key[j] != 0u) : 0ull;
+            if (hit) {
+                const uint32_t l = 63u - (uint32_t)__builtin_clzll(hit);
+                taken[j] |= 1ull << l;
+                if (lane == l) key[j] = 0u;
+                open = false;
+            }
         }
     }
-    __syncthreads();
-    if (e == 0) {
-        float ren = 0.f;
-        for (uint32_t kk = 0; kk < K; ++kk) ren += w_s[kk];
-        const float inv = 1.0f / ren;
-        for (uint32_t kk = 0; kk < K; ++kk) w_s[kk] *= inv;
-        for (uint32_t i = 0; i + 1 < K; ++i)
-            for (uint32_t j = 0; j + 1 + i < K; ++j)
-                if (idx_s[j] > idx_s[j + 1]) {
-                    const int32_t ti = idx_s[j]; idx_s[j] = idx_s[j + 1]; idx_s[j + 1] = ti;
-                    const float tw = w_s[j]; w_s[j] = w_s[j + 1]; w_s[j + 1] = tw;
-                }
+    const float inv = 1.0f / ren;
+    uint32_t below = 0;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        if ((taken[j] >> lane) & 1ull) {
+            const uint32_t at = below + (uint32_t)__builtin_popcountll(taken[j] & ((1ull << lane) - 1ull));
+            topk_idx[(size_t)t * K + at] = (int32_t)(lane + 64u * j);
+            topk_w[(size_t)t * K + at] = (half_t)(p[j] * inv);
+        }
+        below += (uint32_t)__builtin_popcountll(taken[j]);
     }
-    __syncthreads();
-    if (e < K) {
-        topk_idx[(size_t)t * K + e] = idx_s[e];
-        topk_w[(size_t)t * K + e] = (half_t)w_s[e];
-    }
+}
+
+template <class LogitT>
+static int launch_topk(hipStream_t st, const LogitT* logits, int32_t* topk_idx, half_t* topk_w, uint32_t E, uint32_t K, uint32_t n_tokens) {
+    const dim3 grid((n_tokens + 3) / 4), block(256);
+    if (E <= 64) hipLaunchKernelGGL((topk_kernel<LogitT, 1>), grid, block, 0, st, logits, topk_idx, topk_w, E, K, n_tokens);
+    else if (E <= 128) hipLaunchKernelGGL((topk_kernel<LogitT, 2>), grid, block, 0, st, logits, topk_idx, topk_w, E, K, n_tokens);
+    else if (E <= 256) hipLaunchKernelGGL((topk_kernel<LogitT, 4>), grid, block, 0, st, logits, topk_idx, topk_w, E, K, n_tokens);
+    else hipLaunchKernelGGL((topk_kernel<LogitT, 16>), grid, block, 0, st, logits, topk_idx, topk_w, E, K, n_tokens);
+    return launch_status();
 }
 
 // ---------------------------------------------------------------- packing
@@ -123,7 +253,120 @@ __global__ void pack_decode_kernel(const int32_t* topk_idx, const half_t* topk_w
     }
 }
 
-// T tokens: stable counting sort of the T*K slots by expert id, in three launches.
+// T tokens, up to kPackMaxExperts experts: stable counting sort of the T*K slots by expert id in one workgroup.  Wave w owns a
+// contiguous range of the slots.  Count: 64 slots at a time, the lanes of one expert are found with one ballot per id bit, a
+// slot's rank among its wave's slots of that expert is kept in tk_to_packed.  Scan: per expert over the waves, then over the
+// experts.  Place: every slot knows its position; the inverse (position -> slot) is built in LDS when it fits (`staged`: u16
+// slot and the weight of every position), so that every global store is coalesced, and scattered straight to memory else.
+// One CU does it because the work is small and serial in the experts' totals: 16384 slots, 128 experts 16.5 us (three
+// launches, in which every expert's workgroup read all slots, took 41), 128 slots of 32 experts 3.7 us (5.7).
+constexpr uint32_t kPackMaxExperts = 1024;
+constexpr uint32_t kPackLdsMax = 152u * 1024u;
+__global__ __launch_bounds__(1024) void pack_kernel(const int32_t* __restrict__ topk_idx, const uint16_t* __restrict__ topk_w, uint32_t n, uint32_t K, uint32_t E,
+                                                    uint32_t id_bits, uint32_t staged, uint32_t* __restrict__ expert_offsets, int32_t* __restrict__ sorted_idx,
+                                                    uint16_t* __restrict__ weights_packed, uint32_t* tk_to_packed) {
+    extern __shared__ __align__(16) uint32_t pack_lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, n_waves = blockDim.x / 64u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    uint32_t* hist = pack_lds;                       // [n_waves][E]: counts, then positions of the wave's first slot of an expert
+    uint32_t* base = hist + n_waves * E;             // [E + 1]
+    uint16_t* slot_s = reinterpret_cast<uint16_t*>(base + E + 1);   // staged: [n] slot and [n] weight of every position
+    uint16_t* w_s = slot_s + n;
+    for (uint32_t i = tid; i < n_waves * E; i += blockDim.x) hist[i] = 0u;
+    __syncthreads();
+    const uint32_t seg = (n + n_waves * 64u - 1u) / (n_waves * 64u) * 64u, lo = wave * seg < n ? wave * seg : n, hi = lo + seg < n ? lo + seg : n;
+    uint32_t* own = hist + wave * E;
+    constexpr int U = 4;
+    for (uint32_t c = lo; c < hi; c += 64u * U) {
+        uint32_t id[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = c + 64u * u + lane;
+            id[u] = i < hi ? (uint32_t)topk_idx[i] : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = c + 64u * u + lane;
+            const bool valid = id[u] < E;                                  // slots without an expert of the bank are left out
+            const unsigned long long ok = __ballot(valid);
+            uint32_t s_lo = (uint32_t)ok, s_hi = (uint32_t)(ok >> 32);     // lanes whose id agrees with this lane's in the bits seen so far
+            for (uint32_t b = 0; b < id_bits; ++b) {
+                const uint32_t t = (uint32_t)((int)(id[u] << (31u - b)) >> 31);   // all ones where the bit is set
+                const unsigned long long m = __ballot(t != 0u);
+                s_lo &= ~((uint32_t)m ^ t);
+                s_hi &= ~((uint32_t)(m >> 32) ^ t);
+            }
+            const uint32_t before = (uint32_t)__builtin_amdgcn_mbcnt_hi(s_hi, __builtin_amdgcn_mbcnt_lo(s_lo, 0u));
+            if (valid) {
+                const uint32_t first = own[id[u]];
+                if (before == 0u) own[id[u]] = first + (uint32_t)(__builtin_popcount(s_lo) + __builtin_popcount(s_hi));
+                tk_to_packed[i] = first + before;
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t e = tid; e < E; e += blockDim.x) {
+        uint32_t s = 0;
+#pragma unroll 4
+        for (uint32_t w = 0; w < n_waves; ++w) {
+            const uint32_t c = hist[w * E + e];
+            hist[w * E + e] = s;
+            s += c;
+        }
+        base[e + 1] = s;
+    }
+    if (tid == 0) base[0] = 0u;
+    __syncthreads();
+    if (wave == 0) {
+        uint32_t run = 0;
+        for (uint32_t e0 = 0; e0 < E; e0 += 64u) {
+            uint32_t v = e0 + lane < E ? base[e0 + lane + 1u] : 0u;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t o = (uint32_t)__shfl_up((int)v, d);
+                if (lane >= (uint32_t)d) v += o;
+            }
+            if (e0 + lane < E) base[e0 + lane + 1u] = run + v;
+            run += (uint32_t)__shfl((int)v, 63);
+        }
+    }
+    __syncthreads();
+    for (uint32_t e = tid; e <= E; e += blockDim.x) expert_offsets[e] = base[e];
+    for (uint32_t c = lo; c < hi; c += 64u * U) {
+        uint32_t id[U], rank[U];
+        uint16_t wt[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = c + 64u * u + lane;
+            id[u] = i < hi ? (uint32_t)topk_idx[i] : 0xFFFFFFFFu;
+            rank[u] = i < hi ? tk_to_packed[i] : 0u;
+            wt[u] = i < hi ? topk_w[i] : (uint16_t)0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = c + 64u * u + lane;
+            if (id[u] < E) {
+                const uint32_t p = base[id[u]] + own[id[u]] + rank[u];
+                tk_to_packed[i] = p;
+                if (staged) {
+                    slot_s[p] = (uint16_t)i;
+                    w_s[p] = wt[u];
+                } else {
+                    sorted_idx[p] = (int32_t)(i / K);
+                    weights_packed[p] = wt[u];
+                }
+            }
+        }
+    }
+    if (!staged) return;
+    __syncthreads();
+    for (uint32_t p = tid; p < base[E]; p += blockDim.x) {
+        sorted_idx[p] = (int32_t)((uint32_t)slot_s[p] / K);
+        weights_packed[p] = w_s[p];
+    }
+}
+
+// More experts than that: the same sort, in three launches.
 //   count : workgroup e counts its slots                      -> expert_offsets[e + 1]
 //   scan  : one workgroup turns the counts into offsets        (inclusive scan in place)
 //   place : workgroup e walks the slots in order and writes its own, keeping slot order
@@ -193,9 +436,7 @@ extern "C" {
 int mx_moe_topk_from_logits(mx_stream_t s, const uint16_t* logits, int32_t* topk_idx, uint16_t* topk_w, uint32_t E, uint32_t K, uint32_t n_tokens) {
     MX_REQUIRE_PTR(logits); MX_REQUIRE_PTR(topk_idx); MX_REQUIRE_PTR(topk_w);
     MX_REQUIRE_SHAPE(E > 0 && E <= 1024 && K > 0 && K <= E && K <= (uint32_t)kMaxTopK && n_tokens > 0);
-    hipLaunchKernelGGL((topk_kernel<half_t>), dim3(n_tokens), dim3((E + 63) / 64 * 64), 0, as_stream(s), reinterpret_cast<const half_t*>(logits), topk_idx,
-                       reinterpret_cast<half_t*>(topk_w), E, K);
-    return launch_status();
+    return launch_topk(as_stream(s), reinterpret_cast<const half_t*>(logits), topk_idx, reinterpret_cast<half_t*>(topk_w), E, K, n_tokens);
 }
 
 int mx_moe_router(mx_stream_t s, const uint16_t* x, const float* W_gate, int32_t* topk_idx, uint16_t* topk_w, uint32_t n_tokens, uint32_t hidden,
@@ -204,12 +445,18 @@ int mx_moe_router(mx_stream_t s, const uint16_t* x, const float* W_gate, int32_t
     MX_REQUIRE_SHAPE(n_tokens > 0 && n_tokens <= 65535 && hidden > 0 && hidden % 4 == 0 && n_experts > 0 && n_experts <= 1024 && k > 0 && k <= n_experts &&
                      k <= (uint32_t)kMaxTopK);
     MX_REQUIRE_ALIGN(x, 8); MX_REQUIRE_ALIGN(W_gate, 16);
-    hipLaunchKernelGGL(router_logits_kernel, dim3((n_experts + 3) / 4, n_tokens), dim3(256), 0, as_stream(s), reinterpret_cast<const half_t*>(x), W_gate,
-                       logits_ws, hidden, n_experts);
+    hipStream_t st = as_stream(s);
+    const half_t* xh = reinterpret_cast<const half_t*>(x);
+    if ((uint64_t)n_tokens * n_experts > kRouterRowGroups && hidden % 32 == 0 && aligned(x, 16)) {
+        const uint32_t te = (n_experts + 31) / 32, tt = (n_tokens + 31) / 32;
+        const dim3 small((n_experts + 15) / 16, (n_tokens + 15) / 16);
+        if (te * tt >= 128) hipLaunchKernelGGL((router_logits_mfma_kernel<2, 2, 8>), dim3(te, tt), dim3(512), 0, st, xh, W_gate, logits_ws, n_tokens, hidden, n_experts);
+        else hipLaunchKernelGGL((router_logits_mfma_kernel<1, 1, 16>), small, dim3(1024), 0, st, xh, W_gate, logits_ws, n_tokens, hidden, n_experts);
+    } else {
+        hipLaunchKernelGGL(router_logits_kernel, dim3(n_experts, n_tokens), dim3(256), 0, st, xh, W_gate, logits_ws, hidden, n_experts);
+    }
     if (int rc = launch_status()) return rc;
-    hipLaunchKernelGGL((topk_kernel<float>), dim3(n_tokens), dim3((n_experts + 63) / 64 * 64), 0, as_stream(s), (const float*)logits_ws, topk_idx,
-                       reinterpret_cast<half_t*>(topk_w), n_experts, k);
-    return launch_status();
+    return launch_topk(st, (const float*)logits_ws, topk_idx, reinterpret_cast<half_t*>(topk_w), n_experts, k, n_tokens);
 }
 
 int mx_moe_build_pack_decode(mx_stream_t s, const int32_t* topk_idx, const uint16_t* topk_w, uint32_t* expert_offsets, int32_t* sorted_idx,
@@ -229,6 +476,26 @@ int mx_moe_build_packing_device(mx_stream_t s, const int32_t* topk_idx, const ui
     MX_REQUIRE_SHAPE(E > 0 && E <= 65535 && K > 0 && T > 0 && (uint64_t)T * K <= 0x7FFFFFFFull);
     const uint32_t n = T * K;
     hipStream_t st = as_stream(s);
+    if (E <= kPackMaxExperts) {
+        const uint32_t waves = n <= 256 ? 4u : n <= 2048 ? 8u : 16u;
+        const uint32_t lds_min = (waves * E + E + 1) * 4u;
+        const uint32_t staged = n <= 65536u && lds_min + 4u * n <= kPackLdsMax ? 1u : 0u;
+        const uint32_t lds = lds_min + (staged ? 4u * n : 0u);
+        uint32_t id_bits = 0;
+        while ((1u << id_bits) < E) ++id_bits;
+        static std::atomic<bool> attr_set{false};   // dynamic LDS past 64 KB: opt in once
+        if (!attr_set.load(std::memory_order_acquire)) {
+            const hipError_t er = hipFuncSetAttribute(reinterpret_cast<const void*>(&pack_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPackLdsMax);
+            if (er != hipSuccess) {
+                g_last_hip_error = (int)er;
+                return MX_ERR_LAUNCH;
+            }
+            attr_set.store(true, std::memory_order_release);
+        }
+        hipLaunchKernelGGL(pack_kernel, dim3(1), dim3(64 * waves), lds, st, topk_idx, topk_w, n, K, E, id_bits, staged, expert_offsets, sorted_idx, weights_packed,
+                           reinterpret_cast<uint32_t*>(tk_to_packed));
+        return launch_status();
+    }
     hipLaunchKernelGGL(pack_count_kernel, dim3(E), dim3(256), 0, st, topk_idx, n, expert_offsets);
     if (int rc = launch_status()) return rc;
     hipLaunchKernelGGL(pack_scan_kernel, dim3(1), dim3(64), 0, st, expert_offsets, E);

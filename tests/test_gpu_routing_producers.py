@@ -69,6 +69,75 @@ def test_moe_packing_device_equals_host(mx, T, E, K):
         assert np.array_equal(host(wp).astype(np.float32), wp_r)
 
 
+@pytest.mark.parametrize("T,E,k,H", [(16, 33, 5, 1040), (40, 65, 4, 16), (300, 33, 5, 36), (250, 33, 5, 1056), (333, 128, 8, 2048), (1030, 257, 8, 288), (2050, 60, 6, 544)])
+def test_moe_router_token_tiles(mx, T, E, k, H):
+    """Token and expert counts off the 16 x 16 and 32 x 32 tiles and the one-row-per-workgroup form, hidden sizes that end inside
+    a wave's turn of 32-element pieces (and some that are no whole number of them).  The logits are fp32 sums of H <= 2048 products: a pick may
+    differ only where two probabilities are within H * 2^-24 of each other."""
+    x = f16(O.normal(9150 + T, (T, H)))
+    Wg = O.normal(9151 + E, (E, H), 0.0, 1.0 / np.sqrt(H)).astype(np.float32)
+    idx, w = mx.ops.moe_router(dev(x).half(), dev(Wg), E, k)
+    logits = (x.astype(np.float64) @ Wg.astype(np.float64).T).astype(np.float32)
+    ids_ref, w_ref = O.route_from_logits(logits, k)
+    idx_h = host(idx)
+    same = (idx_h == ids_ref).all(axis=1)
+    for t in np.where(~same)[0]:
+        a, b = sorted(set(idx_h[t]) - set(ids_ref[t])), sorted(set(ids_ref[t]) - set(idx_h[t]))
+        assert len(a) == len(b) == len(set(a)) and np.abs(logits[t, a] - logits[t, b]).max() <= 4 * H * 2.0 ** -24, "differs beyond a tie"
+    assert same.mean() >= 0.99
+    check(host(w).astype(np.float32)[same], w_ref[same], "router weights", max_rel=2e-3)
+
+
+@pytest.mark.parametrize("T,E,k", [(5, 64, 64), (3, 65, 2), (9, 129, 8), (2, 257, 8), (4, 1, 1), (6, 1000, 64)])
+def test_moe_topk_expert_counts(mx, T, E, k):
+    """Experts per lane 1, 2, 4 and 16, every expert picked, one expert only."""
+    logits = f16(O.normal(9250 + E, (T, E), 0.0, 2.0))
+    idx, w = mx.ops.moe_topk_from_logits(dev(logits).half(), k)
+    ids_ref, w_ref = O.route_from_logits(logits, k)
+    idx_h = host(idx)
+    for t in range(T):
+        a, b = set(idx_h[t]) - set(ids_ref[t]), set(ids_ref[t]) - set(idx_h[t])
+        assert len(a) == len(b) and sorted(logits[t, list(a)]) == sorted(logits[t, list(b)]), "differs beyond an exact tie"
+    assert (np.diff(idx_h, axis=1) > 0).all() if k > 1 else True
+    same = (idx_h == ids_ref).all(axis=1)
+    check(host(w).astype(np.float32)[same], w_ref[same], "topk weights", max_rel=2e-3)
+
+
+@pytest.mark.parametrize("T,E,K", [(1, 1, 1), (7, 3, 9), (64, 1024, 1), (65, 1000, 4), (513, 7, 4), (1025, 128, 2), (9000, 1024, 4), (20001, 60, 4), (300, 1100, 3)])
+def test_moe_packing_device_sizes(mx, T, E, K):
+    """Slot counts around the waves' 64-slot pieces, one expert, the most experts of the one-workgroup form and one more, positions
+    that fit in LDS and that do not; every id drawn freely (a token may name an expert twice)."""
+    rng = np.random.default_rng(T * E)
+    ids = np.minimum(rng.integers(0, E, (T, K)), rng.integers(0, E, (T, K))).astype(np.int32)
+    w = f16(rng.random((T, K)).astype(np.float32))
+    off_r, si_r, wp_r, t2p_r = O.build_moe_packing(ids, w, E)
+    off, si, wp, t2p = mx.ops.moe_build_packing_device(dev(ids), dev(w).half(), E)
+    assert np.array_equal(host(off).view(np.uint32), off_r)
+    assert np.array_equal(host(si), si_r)
+    assert np.array_equal(host(t2p), t2p_r)
+    assert np.array_equal(host(wp).astype(np.float32), wp_r)
+
+
+@pytest.mark.parametrize("T,K,H", [(1, 4, 2880), (3, 5, 8), (2, 9, 20), (33, 8, 1032)])
+def test_moe_reduce_columns(mx, T, K, H):
+    """Rows of whole 8-column pieces and not, slot counts around the four rows in flight: fp32 sums of the fp16 rows in slot order."""
+    rng = np.random.default_rng(H)
+    packed = f16(O.normal(9600, (T * K, H)))
+    rows = rng.permutation(T * K).astype(np.int32)
+    w = f16(rng.random(T * K).astype(np.float32))
+    y0 = f16(O.normal(9601, (T, H)))
+    s, a = np.zeros((T, H), np.float32), y0.astype(np.float32).copy()
+    for k in range(K):
+        r = rows.reshape(T, K)[:, k]
+        s += packed[r].astype(np.float32)
+        a = (a.astype(np.float64) + w[r, None].astype(np.float64) * packed[r].astype(np.float64)).astype(np.float32)   # one rounding per term (fma)
+    y = mx.ops.moe_prefill_reduce_sum(dev(packed).half(), dev(rows), T, K, H)
+    assert np.array_equal(host(y).astype(np.float32), f16(s))
+    ya = mx.ops.moe_prefill_reduce(dev(packed).half(), dev(rows), dev(w).half(), dev(y0).half(), T, K, H)
+    d = np.abs(host(ya).astype(np.float32) - f16(a))
+    assert (d <= np.maximum(np.abs(a), 2.0 ** -14) * 2.0 ** -10).all()   # one fp16 unit in the last place: fma or multiply and add
+
+
 def ref_q8_of(y_half):
     return O.quantize_q8_1(y_half.astype(np.float32))
 
