@@ -315,6 +315,47 @@ __global__ __launch_bounds__(256) void merge_f32_kernel(const float* y32, half_t
 // moe_reduce_q8 (src/ops/moe_q8.cpp:149-158): y[t] = sum_k y_packed[t*K+k]
 // moe_prefill_reduce_sum (:368-384): y[t] = sum_k out_packed[tk_to_packed[t*K+k]]
 // moe_prefill_reduce (src/ops/moe_fused.cpp:1927-1954): y[t] += sum_k w[row] * out_packed[row]
+// A thread owns 8 consecutive columns (16-byte loads) and requests four packed rows before it adds the first, in slot order:
+// 2048 tokens of hidden 2048, k = 8 (75 MB) take 12.5 us (6 TB/s); one column per thread, row after row, took 44.
+template <bool WEIGHTED, bool ACCUMULATE>
+__global__ __launch_bounds__(256) void moe_reduce8_kernel(const half_t* __restrict__ packed, const uint32_t* __restrict__ tk_to_packed, const half_t* __restrict__ w,
+                                                          half_t* __restrict__ y, uint32_t T, uint32_t Ktop, uint32_t H8) {
+    typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (uint64_t)T * H8) return;
+    const uint32_t t = (uint32_t)(i / H8), n = (uint32_t)(i % H8);
+    const h8_t* rows = reinterpret_cast<const h8_t*>(packed) + n;
+    h8_t* out = reinterpret_cast<h8_t*>(y) + i;
+    float s[8];
+    h8_t y0{};
+    if (ACCUMULATE) y0 = *out;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) s[c] = ACCUMULATE ? (float)y0[c] : 0.f;
+    for (uint32_t k0 = 0; k0 < Ktop; k0 += 4) {
+        h8_t v[4];
+        float wt[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k0 + u < Ktop) {
+                const uint32_t slot = t * Ktop + k0 + u, row = tk_to_packed ? tk_to_packed[slot] : slot;
+                v[u] = rows[(size_t)row * H8];
+                wt[u] = WEIGHTED ? (float)w[row] : 1.f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k0 + u < Ktop) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) s[c] += WEIGHTED ? wt[u] * (float)v[u][c] : (float)v[u][c];
+            }
+        }
+    }
+    h8_t o;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) o[c] = (half_t)s[c];
+    *out = o;
+}
+// any H, any alignment
 template <bool WEIGHTED, bool ACCUMULATE>
 __global__ __launch_bounds__(256) void moe_reduce_kernel(const half_t* packed, const uint32_t* tk_to_packed, const half_t* w, half_t* y,
                                                          uint32_t T, uint32_t Ktop, uint32_t H) {
@@ -328,6 +369,20 @@ __global__ __launch_bounds__(256) void moe_reduce_kernel(const half_t* packed, c
         s += WEIGHTED ? (float)w[row] * v : v;
     }
     y[i] = (half_t)s;
+}
+
+template <bool WEIGHTED, bool ACCUMULATE>
+static int launch_reduce(hipStream_t st, const uint16_t* packed, const uint32_t* tk_to_packed, const uint16_t* w, uint16_t* y, uint32_t T, uint32_t K, uint32_t H) {
+    const half_t *p = reinterpret_cast<const half_t*>(packed), *wh = reinterpret_cast<const half_t*>(w);
+    half_t* yh = reinterpret_cast<half_t*>(y);
+    if (H % 8 == 0 && aligned(packed, 16) && aligned(y, 16)) {
+        const uint64_t n = (uint64_t)T * (H / 8);
+        hipLaunchKernelGGL((moe_reduce8_kernel<WEIGHTED, ACCUMULATE>), dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, p, tk_to_packed, wh, yh, T, K, H / 8);
+    } else {
+        hipLaunchKernelGGL((moe_reduce_kernel<WEIGHTED, ACCUMULATE>), dim3((uint32_t)(((uint64_t)T * H + 255) / 256)), dim3(256), 0, st, p, tk_to_packed, wh, yh,
+                           T, K, H);
+    }
+    return launch_status();
 }
 
 // ---------------------------------------------------------------- host side
@@ -869,26 +924,19 @@ static int reduce_common(const void* packed, const void* y, uint32_t T, uint32_t
 }
 int mx_moe_reduce_q8(mx_stream_t s, const uint16_t* y_packed, uint16_t* y, uint32_t T, uint32_t K, uint32_t H) {
     if (int rc = reduce_common(y_packed, y, T, K, H)) return rc;
-    hipLaunchKernelGGL((moe_reduce_kernel<false, false>), dim3((uint32_t)(((uint64_t)T * H + 255) / 256)), dim3(256), 0, as_stream(s),
-                       reinterpret_cast<const half_t*>(y_packed), nullptr, nullptr, reinterpret_cast<half_t*>(y), T, K, H);
-    return launch_status();
+    return launch_reduce<false, false>(as_stream(s), y_packed, nullptr, nullptr, y, T, K, H);
 }
 int mx_moe_prefill_reduce_sum(mx_stream_t s, const uint16_t* out_packed, const uint32_t* tk_to_packed, uint16_t* y, uint32_t T, uint32_t K,
                               uint32_t H) {
     if (int rc = reduce_common(out_packed, y, T, K, H)) return rc;
     MX_REQUIRE_PTR(tk_to_packed);
-    hipLaunchKernelGGL((moe_reduce_kernel<false, false>), dim3((uint32_t)(((uint64_t)T * H + 255) / 256)), dim3(256), 0, as_stream(s),
-                       reinterpret_cast<const half_t*>(out_packed), tk_to_packed, nullptr, reinterpret_cast<half_t*>(y), T, K, H);
-    return launch_status();
+    return launch_reduce<false, false>(as_stream(s), out_packed, tk_to_packed, nullptr, y, T, K, H);
 }
 int mx_moe_prefill_reduce(mx_stream_t s, const uint16_t* out_packed, const uint32_t* tk_to_packed, const uint16_t* weights_packed, uint16_t* y,
                           uint32_t T, uint32_t K_top, uint32_t H) {
     if (int rc = reduce_common(out_packed, y, T, K_top, H)) return rc;
     MX_REQUIRE_PTR(tk_to_packed); MX_REQUIRE_PTR(weights_packed);
-    hipLaunchKernelGGL((moe_reduce_kernel<true, true>), dim3((uint32_t)(((uint64_t)T * H + 255) / 256)), dim3(256), 0, as_stream(s),
-                       reinterpret_cast<const half_t*>(out_packed), tk_to_packed, reinterpret_cast<const half_t*>(weights_packed),
-                       reinterpret_cast<half_t*>(y), T, K_top, H);
-    return launch_status();
+    return launch_reduce<true, true>(as_stream(s), out_packed, tk_to_packed, weights_packed, y, T, K_top, H);
 }
 
 // build_moe_packing (src/model/qwen3moe_pack.cpp:5-31), host pointers: stable counting sort of the
