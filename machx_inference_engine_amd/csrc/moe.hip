@@ -457,7 +457,7 @@ static int launch_mmq_grouped_cfg(hipStream_t st, const typename P::Bank& b0, co
         a.deal_rows = 1;
     }
     constexpr uint32_t TT = 2 * TV, gran = 256u * WK;
-    constexpr uint32_t red = (uint32_t)(NW * WR * WK) * TV * 64u * 4u;
+    constexpr uint32_t red = NW * WK > 1 ? (uint32_t)(NW * WR * WK) * TV * 64u * 4u : 0u;   // one wave per row block exchanges nothing
     const uint32_t per256 = TT * (NATIVE ? 512u : 256u) + 8u * TT * 4u * (P::HAS_MIN ? 2u : 1u);
     const uint32_t budget = (TV == 16 || (NATIVE && TV == 8)) ? kMmqMoeLdsBudgetBig : (NATIVE ? 64u * 1024u : kMmqMoeLdsBudget);
     const uint32_t need = ((m.K + 255u) / 256u + WK - 1u) / WK * WK * 256u;

@@ -99,15 +99,10 @@ struct MmqQ8Soa {
     }
     template <int S>
     __device__ static __forceinline__ v4i_t operand(const Raw& r, uint32_t) { return as_v4i(r.q[S]); }
-    struct Dec {
-        float c[8];
-    };
-    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t) {
-        Dec o;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) o.c[s] = h2f((s & 1) ? r.d[s >> 1] >> 16 : r.d[s >> 1] & 0xFFFFu);
-        return o;
-    }
+    struct Dec {};
+    __device__ static __forceinline__ Dec prepare(const Raw&, uint32_t) { return {}; }
+    template <int S>
+    __device__ static __forceinline__ float factor(const Raw& r, const Dec&) { return h2f((S & 1) ? r.d[S >> 1] >> 16 : r.d[S >> 1] & 0xFFFFu); }
 };
 
 // Q8_0 GGUF blocks (34 B: fp16 d, 32 int8; 2-byte aligned): lane half h reads the 16 quants at byte 2 + 16 h of each
@@ -154,7 +149,9 @@ struct MmqQ8Aos {
     }
     template <int S>
     __device__ static __forceinline__ v4i_t operand(const Raw& r, uint32_t) { return as_v4i(r.q[S]); }
-    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t h) { return MmqQ8Soa::prepare(r, h); }
+    __device__ static __forceinline__ Dec prepare(const Raw&, uint32_t) { return {}; }
+    template <int S>
+    __device__ static __forceinline__ float factor(const Raw& r, const Dec& o) { return MmqQ8Soa::factor<S>(r, o); }
 };
 
 // MXFP4 SoA planes: qs_plane[n*(K/2) + 16 b + j] (element j in the low, 16 + j in the high nibble), e_plane[n*(K/32) + b]
@@ -208,15 +205,10 @@ struct MmqMxfp4Soa {
         o.w = (int)mxfp4_lut4(w[3] & 0x07070707u, ((w[3] >> 1) & 0x04040404u) | 0x03020100u);
         return o;
     }
-    struct Dec {
-        float c[8];
-    };
-    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t) {
-        Dec o;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) o.c[s] = e8m0_half((r.e[s >> 2] >> (8 * (s & 3))) & 0xFFu);
-        return o;
-    }
+    struct Dec {};
+    __device__ static __forceinline__ Dec prepare(const Raw&, uint32_t) { return {}; }
+    template <int S>
+    __device__ static __forceinline__ float factor(const Raw& r, const Dec&) { return e8m0_half((r.e[S >> 2] >> (8 * (S & 3))) & 0xFFu); }
 };
 
 // MXFP4 planes fed to the matrix cores as they lie in memory: v_mfma_scale_f32_32x32x64_f8f6f4 takes E2M1 codes and one
@@ -306,22 +298,21 @@ struct MmqQ4K {
         return o;
     }
     struct Dec {
-        float c[8], m[8];
+        float d, dmin;
+        uint32_t sc[4], mn[4];   // scale and min bytes of blocks 2 i (bits 0..7) and 2 i + 1 (bits 8..15)
     };
     __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t) {
-        const float d = h2f(r.hdr.x & 0xFFFFu), dmin = h2f(r.hdr.x >> 16);
         Dec o;
+        o.d = h2f(r.hdr.x & 0xFFFFu);
+        o.dmin = h2f(r.hdr.x >> 16);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            uint32_t sc, mn;
-            q4k_scale_pair(r.hdr.y, r.hdr.z, r.hdr.w, g, sc, mn);
-            o.c[2 * g] = d * (float)(sc & 0xFFu);
-            o.c[2 * g + 1] = d * (float)(sc >> 8);
-            o.m[2 * g] = dmin * (float)(mn & 0xFFu);
-            o.m[2 * g + 1] = dmin * (float)(mn >> 8);
-        }
+        for (int g = 0; g < 4; ++g) q4k_scale_pair(r.hdr.y, r.hdr.z, r.hdr.w, g, o.sc[g], o.mn[g]);
         return o;
     }
+    template <int S>
+    __device__ static __forceinline__ float factor(const Raw&, const Dec& o) { return o.d * (float)((S & 1) ? o.sc[S >> 1] >> 8 : o.sc[S >> 1] & 0xFFu); }
+    template <int S>
+    __device__ static __forceinline__ float minimum(const Raw&, const Dec& o) { return o.dmin * (float)((S & 1) ? o.mn[S >> 1] >> 8 : o.mn[S >> 1] & 0xFFu); }
 };
 
 // Q4_0 (32-element blocks: fp16 d, 16 bytes with element j in the low and j + 16 in the high nibble of byte j;
@@ -371,18 +362,12 @@ struct MmqQ40Soa {
         o.z = (int)((r.q[S].z >> sh) & 0x0F0F0F0Fu); o.w = (int)((r.q[S].w >> sh) & 0x0F0F0F0Fu);
         return o;
     }
-    struct Dec {
-        float c[8], m[8];
-    };
-    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t) {
-        Dec o;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            o.c[s] = h2f((s & 1) ? r.d[s >> 1] >> 16 : r.d[s >> 1] & 0xFFFFu);
-            o.m[s] = 8.f * o.c[s];
-        }
-        return o;
-    }
+    struct Dec {};
+    __device__ static __forceinline__ Dec prepare(const Raw&, uint32_t) { return {}; }
+    template <int S>
+    __device__ static __forceinline__ float factor(const Raw& r, const Dec&) { return h2f((S & 1) ? r.d[S >> 1] >> 16 : r.d[S >> 1] & 0xFFFFu); }
+    template <int S>
+    __device__ static __forceinline__ float minimum(const Raw& r, const Dec& o) { return 8.f * factor<S>(r, o); }
 };
 struct MmqQ40Aos {
     using W = FmtQ40Aos::W;
@@ -422,7 +407,11 @@ struct MmqQ40Aos {
     }
     template <int S>
     __device__ static __forceinline__ v4i_t operand(const Raw& r, uint32_t h) { return MmqQ40Soa::operand<S>(r, h); }
-    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t h) { return MmqQ40Soa::prepare(r, h); }
+    __device__ static __forceinline__ Dec prepare(const Raw&, uint32_t) { return {}; }
+    template <int S>
+    __device__ static __forceinline__ float factor(const Raw& r, const Dec& o) { return MmqQ40Soa::factor<S>(r, o); }
+    template <int S>
+    __device__ static __forceinline__ float minimum(const Raw& r, const Dec& o) { return MmqQ40Soa::minimum<S>(r, o); }
 };
 
 // Q6_K AoS blocks (210 B, 2-byte aligned): element 128 hf + 32 sub + l has its low nibble in nibble (sub >> 1) of
@@ -466,15 +455,14 @@ struct MmqQ6K {
         return o;
     }
     struct Dec {
-        float c[16];   // c[2 S + half]
+        float d;
     };
-    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t) {
-        const float d = h2f(r.d);
-        const uint32_t s[4] = {r.sc.x, r.sc.y, r.sc.z, r.sc.w};
-        Dec o;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o.c[i] = d * (float)(int)(int8_t)(s[i >> 2] >> (8 * (i & 3)));
-        return o;
+    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t) { return {h2f(r.d)}; }
+    // scale of 16-element group I = 2 S + half of the super-block
+    template <int I>
+    __device__ static __forceinline__ int int_scale(const Raw& r) {
+        const uint32_t w = (I >> 2) == 0 ? r.sc.x : (I >> 2) == 1 ? r.sc.y : (I >> 2) == 2 ? r.sc.z : r.sc.w;
+        return (int)(int8_t)(w >> (8 * (I & 3)));
     }
 };
 
@@ -672,12 +660,6 @@ __device__ __forceinline__ MmqAct mmq_stage_f16(uint8_t* lds, RowFn hrow, uint32
 
 // ---------------------------------------------------------------- one group of 8 blocks
 template <int TV>
-__device__ __forceinline__ void mmq_fold(const v16i_t& I, const float (&dxv)[TV], float c, float (&acc)[TV]) {
-#pragma unroll
-    for (int v = 0; v < TV; ++v) acc[v] += c * (dxv[v] * (float)I[v]);
-}
-
-template <int TV>
 __device__ __forceinline__ void mmq_read4(const float* p, uint32_t h, float (&o)[TV]) {
     // token slots of lane half h: 8 q + 4 h + (0..3), q = 0 .. TV/4 - 1
 #pragma unroll
@@ -687,61 +669,82 @@ __device__ __forceinline__ void mmq_read4(const float* p, uint32_t h, float (&o)
     }
 }
 
+template <class P, int S>
+__device__ __forceinline__ void mmq_issue(const typename P::Raw& raw, const v4i_t& a, uint32_t h, v16i_t (&I)[P::SUBS]) {
+    const v4i_t b = P::template operand<S>(raw, h);
+    const v16i_t z = {};
+    if constexpr (P::SUBS == 1) {
+        I[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, z, 0, 0, 0);
+    } else {
+        const v4i_t zero = {};
+        I[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(h ? zero : a, b, z, 0, 0, 0);
+        I[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(h ? a : zero, b, z, 0, 0, 0);
+    }
+}
+
 // Block S of group `gl` (group index inside the staged range).  The matrix instruction of block S + 1 is issued
-// before the fold of block S, so the fold never waits on the instruction it depends on alone.
+// before the fold of block S, so the fold never waits on the instruction it depends on alone; the LDS words of the
+// next step (token codes of block S + 2, block scales of block S + 1) are requested a whole step ahead.  The barrier at
+// the end of a step keeps the scheduler from merging the eight steps of the unrolled group: left alone it reads every
+// step's scales first and holds the integer results of several blocks.
 template <class P, int TV, int S>
-__device__ __forceinline__ void mmq_block(const typename P::Raw& raw, const typename P::Dec& dec, const MmqAct& act, uint32_t a_off, uint32_t gl,
-                                          uint32_t h, float (&acc)[TV], v16i_t (&I)[2][P::SUBS]) {
+__device__ __forceinline__ void mmq_block(const typename P::Raw& raw, const typename P::Dec& dec, const MmqAct& act, const uint8_t* ap, const float* dp,
+                                          const float* sp, uint32_t h, const v4i_t& a, const float (&dxv)[TV], const float (&sxv)[P::HAS_MIN ? TV : 1],
+                                          float (&acc)[TV], v16i_t (&I)[2][P::SUBS]) {
     constexpr uint32_t TP = 2 * TV;
-    if constexpr (S < 8) {
-        constexpr int cur = S & 1, nxt = cur ^ 1;
-        if constexpr (S + 1 < 8) {
-            const v4i_t a = as_v4i(*reinterpret_cast<const uint4*>(act.plane + a_off + (8u * gl + S + 1) * 32u));
-            const v4i_t b = P::template operand<S + 1>(raw, h);
-            const v16i_t z = {};
-            if constexpr (P::SUBS == 1) {
-                I[nxt][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, z, 0, 0, 0);
-            } else {
-                const v4i_t zero = {};
-                I[nxt][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(h ? zero : a, b, z, 0, 0, 0);
-                I[nxt][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(h ? a : zero, b, z, 0, 0, 0);
-            }
-        }
-        float dxv[TV];
-        mmq_read4<TV>(act.dx + (size_t)(8u * gl + S) * TP, h, dxv);
-        if constexpr (P::SUBS == 1) {
-            mmq_fold<TV>(I[cur][0], dxv, dec.c[S], acc);
-        } else {
-            mmq_fold<TV>(I[cur][0], dxv, dec.c[2 * S], acc);
-            mmq_fold<TV>(I[cur][1], dxv, dec.c[2 * S + 1], acc);
-        }
-        if constexpr (P::HAS_MIN) {
-            float sxv[TV];
-            mmq_read4<TV>(act.sx + (size_t)(8u * gl + S) * TP, h, sxv);
+    constexpr int cur = S & 1, nxt = cur ^ 1;
+    v4i_t an = {};
+    float dn[TV], sn[P::HAS_MIN ? TV : 1];
+    if constexpr (S + 1 < 8) {
+        mmq_issue<P, S + 1>(raw, a, h, I[nxt]);
+        if constexpr (S + 2 < 8) an = as_v4i(*reinterpret_cast<const uint4*>(ap + (S + 2) * 32u));
+        mmq_read4<TV>(dp + (S + 1) * TP, h, dn);
+        if constexpr (P::HAS_MIN) mmq_read4<TV>(sp + (S + 1) * TP, h, sn);
+    }
+    if constexpr (P::SUBS == 1) {
+        const float c = P::template factor<S>(raw, dec);
 #pragma unroll
-            for (int v = 0; v < TV; ++v) acc[v] -= dec.m[S] * sxv[v];
-        }
-        mmq_block<P, TV, S + 1>(raw, dec, act, a_off, gl, h, acc, I);
+        for (int v = 0; v < TV; ++v) acc[v] += c * (dxv[v] * (float)I[cur][0][v]);
+    } else {
+        // int8 scale x integer dot of 16 elements: below 2^24 also summed over the two halves, so the integer sum and its
+        // conversion are exact and one fp32 multiply-add per block remains
+        const int s0 = P::template int_scale<2 * S>(raw), s1 = P::template int_scale<2 * S + 1>(raw);
+#pragma unroll
+        for (int v = 0; v < TV; ++v) acc[v] += dxv[v] * (float)(__mul24(I[cur][0][v], s0) + __mul24(I[cur][1][v], s1));
+    }
+    if constexpr (P::HAS_MIN) {
+        const float m = P::template minimum<S>(raw, dec);
+#pragma unroll
+        for (int v = 0; v < TV; ++v) acc[v] -= m * sxv[v];
+    }
+    if constexpr (S + 1 < 8) {
+        __builtin_amdgcn_sched_barrier(0);
+        mmq_block<P, TV, S + 1>(raw, dec, act, ap, dp, sp, h, an, dn, sn, acc, I);
     }
 }
 
 template <class P, int TV>
 __device__ __forceinline__ void mmq_group(const typename P::Raw& raw, const MmqAct& act, uint32_t a_off, uint32_t gl, uint32_t h, float (&acc)[TV]) {
+    constexpr uint32_t TP = 2 * TV;
+    const uint8_t* ap = act.plane + a_off + (8u * gl) * 32u;
+    const float *dp = act.dx + (size_t)(8u * gl) * TP, *sp = act.sx + (size_t)(8u * gl) * TP;
+    const v4i_t a0 = as_v4i(*reinterpret_cast<const uint4*>(ap)), a1 = as_v4i(*reinterpret_cast<const uint4*>(ap + 32));
+    float dxv[TV], sxv[P::HAS_MIN ? TV : 1];
+    mmq_read4<TV>(dp, h, dxv);
+    if constexpr (P::HAS_MIN) mmq_read4<TV>(sp, h, sxv);
     const typename P::Dec dec = P::prepare(raw, h);
     v16i_t I[2][P::SUBS];
-    {
-        const v4i_t a = as_v4i(*reinterpret_cast<const uint4*>(act.plane + a_off + (8u * gl) * 32u));
-        const v4i_t b = P::template operand<0>(raw, h);
-        const v16i_t z = {};
-        if constexpr (P::SUBS == 1) {
-            I[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, z, 0, 0, 0);
-        } else {
-            const v4i_t zero = {};
-            I[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(h ? zero : a, b, z, 0, 0, 0);
-            I[0][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(h ? a : zero, b, z, 0, 0, 0);
-        }
+    mmq_issue<P, 0>(raw, a0, h, I[0]);
+    if constexpr (P::SUBS == 1) {
+        mmq_block<P, TV, 0>(raw, dec, act, ap, dp, sp, h, a1, dxv, sxv, acc, I);
+    } else {
+        float part[TV];   // the group's sum before the super-block scale
+#pragma unroll
+        for (int v = 0; v < TV; ++v) part[v] = 0.f;
+        mmq_block<P, TV, 0>(raw, dec, act, ap, dp, sp, h, a1, dxv, sxv, part, I);
+#pragma unroll
+        for (int v = 0; v < TV; ++v) acc[v] += dec.d * part[v];
     }
-    mmq_block<P, TV, 0>(raw, dec, act, a_off, gl, h, acc, I);
 }
 
 // Groups [g_lo, g_hi) of weight row `n` (row-relative group numbers) against the staged range that starts at group
@@ -774,14 +777,10 @@ struct MmqWalk {
             mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
             g += 2;
         }
-        if (g + 1 < g_hi) {
-            raw[1] = P::load(w, n, g + 1, h, nb);
-            __builtin_amdgcn_sched_barrier(0);
-            mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
-            mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
-        } else {
-            mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
-        }
+        if (g + 1 < g_hi) raw[1] = P::load(w, n, g + 1, h, nb);
+        __builtin_amdgcn_sched_barrier(0);
+        mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
+        if (g + 1 < g_hi) mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
     }
 };
 
@@ -902,6 +901,9 @@ struct MmqArgs {
     uint32_t deal_rows;               // one matrix with many rows [0, M): gridDim.z deals the token tiles (no K ranges, no `part`)
 };
 
+// token row of result register v, without the lane half's 4 h
+__host__ __device__ constexpr uint32_t mmq_row(int v) { return 8u * (uint32_t)(v / 4) + (uint32_t)(v % 4); }
+
 __device__ __forceinline__ float mmq_silu_mul(float g, float u) { return (g / (1.f + __expf(-g))) * u; }
 __device__ __forceinline__ float mmq_swiglu_oai(float g, float u, float alpha, float limit) {
     const float x = fminf(g, limit), z = fmaxf(fminf(u, limit), -limit);
@@ -956,11 +958,13 @@ __global__ __launch_bounds__(64 * NW * WR * WK, 2) void mmq_kernel(MmqArgs<P> a)
         bool staged = false, requested = false;
         // what the epilogue reads from global memory is requested ahead of the weight walk: a load issued in the epilogue
         // would have to wait for the whole queue of weight words requested for the next row block before it
-        float rw[TV];
+        float rw[EPI == MMQ_DOWN_WEIGHTED ? TV : 1];
+        if constexpr (EPI == MMQ_DOWN_WEIGHTED) {
 #pragma unroll
-        for (int v = 0; v < TV; ++v) {
-            const uint32_t t = 8u * (v / 4) + 4u * h + (v % 4);
-            rw[v] = (EPI == MMQ_DOWN_WEIGHTED) ? (float)a.route_w[t0 + (t < nt ? t : nt - 1u)] : 0.f;
+            for (int v = 0; v < TV; ++v) {
+                const uint32_t t = mmq_row(v) + 4u * h;
+                rw[v] = (float)a.route_w[t0 + (t < nt ? t : nt - 1u)];
+            }
         }
         for (uint32_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x) {
             const uint32_t n0 = (rb * WR + wr) * 32u;
@@ -996,8 +1000,10 @@ __global__ __launch_bounds__(64 * NW * WR * WK, 2) void mmq_kernel(MmqArgs<P> a)
                 // the epilogue's operands are made to arrive here, while nothing else is outstanding: otherwise the wait for
                 // them would sit in the epilogue, behind the weight words requested just below
                 asm volatile("" : "+v"(bias_a));
+                if constexpr (EPI == MMQ_DOWN_WEIGHTED) {
 #pragma unroll
-                for (int v = 0; v < TV; ++v) asm volatile("" : "+v"(rw[v]));
+                    for (int v = 0; v < TV; ++v) asm volatile("" : "+v"(rw[v]));
+                }
                 if (EPI == MMQ_OAI && ge == G1 && wk == 0) {
 #pragma unroll
                     for (int v = 0; v < TV; ++v) acc[v] += bias_a;
@@ -1009,43 +1015,62 @@ __global__ __launch_bounds__(64 * NW * WR * WK, 2) void mmq_kernel(MmqArgs<P> a)
                     requested = true;
                 }
             }
-            // ---- partial sums of the WK waves (and the NW matrices) meet in LDS
-            mmq_lds_barrier();
+            // ---- partial sums of the WK waves (and the NW matrices) meet in LDS; a workgroup of row blocks only has none to meet
+            if constexpr (NW * WK > 1) {
+                mmq_lds_barrier();
 #pragma unroll
-            for (int v = 0; v < TV; ++v) red[((size_t)wave * TV + v) * 64u + lane] = acc[v];
-            mmq_lds_barrier();
+                for (int v = 0; v < TV; ++v) red[((size_t)wave * TV + v) * 64u + lane] = acc[v];
+                mmq_lds_barrier();
+            }
             if (wk == 0 && wm == 0) {
+                // Row v of a lane is t0 + 4 h + mmq_row(v): the lane's share of an address is one 32-bit offset and the rest is
+                // uniform.  The offset is made opaque here, once per row block: 2 TV addresses kept in registers across the
+                // weight walk were what made the walk spill (Q6_K, TV = 16: 256 registers and 46 more in scratch).
+                uint32_t lane_at = 4u * h * a.N + j;
+                asm volatile("" : "+v"(lane_at));
+                const bool col_ok = n0 + j < a.N;
+                if (a.part) {
+                    float* base = a.part + ((size_t)kzi * a.M + t0) * a.N + n0;
 #pragma unroll
-                for (int v = 0; v < TV; ++v) {
-                    const uint32_t t = 8u * (v / 4) + 4u * h + (v % 4);
-                    float s0 = 0.f, s1 = 0.f;
+                    for (int v = 0; v < TV; ++v) {
+                        float s0 = acc[v];
+                        if constexpr (NW * WK > 1) {
+                            s0 = 0.f;
 #pragma unroll
-                    for (int k = 0; k < WK; ++k) {
-                        s0 += red[((size_t)((0 * WR + wr) * WK + k) * TV + v) * 64u + lane];
-                        if (NW == 2) s1 += red[((size_t)((1 * WR + wr) * WK + k) * TV + v) * 64u + lane];
+                            for (int k = 0; k < WK; ++k) s0 += red[((size_t)(wr * WK + k) * TV + v) * 64u + lane];
+                        }
+                        if (mmq_row(v) + 4u * h < nt && col_ok) (base + (size_t)mmq_row(v) * a.N)[lane_at] = s0;
                     }
-                    if (t >= nt || n0 + j >= a.N) continue;
-                    const uint32_t row = t0 + t, col = n0 + j;
-                    if (a.part) {
-                        a.part[((size_t)kzi * a.M + row) * a.N + col] = s0;
-                        continue;
+                } else {
+                    half_t* base = a.out + (size_t)t0 * a.N + n0;
+#pragma unroll
+                    for (int v = 0; v < TV; ++v) {
+                        float s0 = acc[v], s1 = 0.f;
+                        if constexpr (NW * WK > 1) {
+                            s0 = 0.f;
+#pragma unroll
+                            for (int k = 0; k < WK; ++k) {
+                                s0 += red[((size_t)((0 * WR + wr) * WK + k) * TV + v) * 64u + lane];
+                                if (NW == 2) s1 += red[((size_t)((1 * WR + wr) * WK + k) * TV + v) * 64u + lane];
+                            }
+                        }
+                        float o;
+                        if constexpr (EPI == MMQ_SILU) {
+                            o = mmq_silu_mul(s0, s1);                                          // src/ops/moe_q8.cpp:94-97
+                        } else if constexpr (EPI == MMQ_OAI) {
+                            // rounding points of the reference chain: half(acc + bias) per projection, then the fp16 activation
+                            const float g = (float)(half_t)s0, u = (float)(half_t)s1;   // sums with their biases
+                            o = mmq_swiglu_oai(g, u, a.alpha, a.limit);
+                        } else if constexpr (EPI == MMQ_DOWN_WEIGHTED) {
+                            o = rw[v] * s0;                                                   // src/ops/moe_q8.cpp:143-144
+                        } else if constexpr (EPI == MMQ_DOWN_BIAS) {
+                            o = (float)(half_t)s0;                                            // gemv out, then add_bias (elementwise.cpp:782-793)
+                            if (a.bias0) o += bias_a;
+                        } else {
+                            o = s0;
+                        }
+                        if (mmq_row(v) + 4u * h < nt && col_ok) (base + (size_t)mmq_row(v) * a.N)[lane_at] = (half_t)o;
                     }
-                    float o;
-                    if (EPI == MMQ_SILU) {
-                        o = mmq_silu_mul(s0, s1);                                          // src/ops/moe_q8.cpp:94-97
-                    } else if (EPI == MMQ_OAI) {
-                        // rounding points of the reference chain: half(acc + bias) per projection, then the fp16 activation
-                        const float g = (float)(half_t)s0, u = (float)(half_t)s1;   // sums with their biases
-                        o = mmq_swiglu_oai(g, u, a.alpha, a.limit);
-                    } else if (EPI == MMQ_DOWN_WEIGHTED) {
-                        o = rw[v] * s0;                                                   // src/ops/moe_q8.cpp:143-144
-                    } else if (EPI == MMQ_DOWN_BIAS) {
-                        o = (float)(half_t)s0;                                            // gemv out, then add_bias (elementwise.cpp:782-793)
-                        if (a.bias0) o += bias_a;
-                    } else {
-                        o = s0;
-                    }
-                    a.out[(size_t)row * a.N + col] = (half_t)o;
                 }
             }
         }
