@@ -191,7 +191,8 @@ __global__ __launch_bounds__(256) void topk_kernel(const LogitT* logits, int32_t
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         p[j] = p[j] / s;
-        key[j] = lane + 64u * j < E ? f2u(p[j]) + 1u : 0u;
+        const uint32_t bits = f2u(p[j]) < 0xFFFFFFFEu ? f2u(p[j]) : 0xFFFFFFFEu;   // a NaN of all ones stays a key: every round has a winner
+        key[j] = lane + 64u * j < E ? bits + 1u : 0u;
         taken[j] = 0ull;
     }
     float ren = 0.f;
@@ -299,9 +300,11 @@ __global__ __launch_bounds__(1024) void pack_kernel(const int32_t* __restrict__ 
             const uint32_t before = (uint32_t)__builtin_amdgcn_mbcnt_hi(s_hi, __builtin_amdgcn_mbcnt_lo(s_lo, 0u));
             if (valid) {
                 const uint32_t first = own[id[u]];
+                __builtin_amdgcn_wave_barrier();   // every lane has read its count before one of them moves it
                 if (before == 0u) own[id[u]] = first + (uint32_t)(__builtin_popcount(s_lo) + __builtin_popcount(s_hi));
                 tk_to_packed[i] = first + before;
             }
+            __builtin_amdgcn_wave_barrier();
         }
     }
     __syncthreads();

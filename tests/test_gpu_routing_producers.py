@@ -53,6 +53,13 @@ def test_moe_topk_tie_goes_to_higher_id(mx):
     np.testing.assert_allclose(host(w).astype(np.float32), [[0.5, 0.5]], atol=1e-3)
 
 
+def test_moe_router_nan_payload_keeps_ids_in_range(mx):
+    """Every bit of a NaN set (the largest key there is): each token still gets k distinct ids of the bank."""
+    Wg = torch.full((8, 256), -1, dtype=torch.int32).view(torch.float32)
+    idx, _ = mx.ops.moe_router(dev(np.ones((2, 256), np.float32)).half(), Wg.cuda(), 8, 4)
+    assert host(idx).tolist() == [[4, 5, 6, 7]] * 2
+
+
 @pytest.mark.parametrize("T,E,K", [(1, 32, 4), (64, 8, 2), (300, 128, 8), (2048, 128, 8)])
 def test_moe_packing_device_equals_host(mx, T, E, K):
     rng = np.random.default_rng(T + E)
