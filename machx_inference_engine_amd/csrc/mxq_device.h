@@ -90,6 +90,14 @@ __device__ __forceinline__ int group_sum8_i(int v) {
     return v;
 }
 
+// (int)roundf(x), halves away from zero: adding the largest float below 1/2 with x's sign and truncating gives the same integer
+// for every float (compared for every x below 2^23 of both signs; above, the sum is x).  Three instructions where roundf and its
+// conversion take seven.  The sum must see the rounded product it is given, so it is not contracted into a multiply-add.
+__device__ __forceinline__ int round_away_i(float x) {
+#pragma clang fp contract(off)
+    return (int)(x + copysignf(0x1.fffffep-2f, x));
+}
+
 // ---------------------------------------------------------------- block_q8_1x emission
 // 8 lanes per 32-element block, 4 consecutive elements per lane (v), l8 = lane % 8.  All 8
 // lanes of a group must call.  d = amax/127, inv = 127/amax (0 for a zero block),
@@ -100,7 +108,7 @@ __device__ __forceinline__ void emit_q8_1x(const float (&v)[4], uint32_t l8, boo
     int q[4], sum = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        q[i] = (int)roundf(v[i] * inv);
+        q[i] = round_away_i(v[i] * inv);
         sum += q[i];
     }
     const uint32_t packed = (uint32_t)(q[0] & 0xFF) | ((uint32_t)(q[1] & 0xFF) << 8) | ((uint32_t)(q[2] & 0xFF) << 16) | ((uint32_t)(q[3] & 0xFF) << 24);
@@ -108,6 +116,34 @@ __device__ __forceinline__ void emit_q8_1x(const float (&v)[4], uint32_t l8, boo
     if (!live) return;
     reinterpret_cast<uint32_t*>(blk + 8)[l8] = packed;
     if (l8 == 0) *reinterpret_cast<float2*>(blk) = make_float2(d, d * (float)tot);
+}
+
+// The same block from four lanes of 8 consecutive elements each (l4 = lane % 4): 16-byte fp16 loads, and the two divisions and the
+// lane exchanges of a block are shared by twice the elements.  SPLIT = true writes block_q8_1s (sums per half, 48 bytes).
+template <bool SPLIT>
+__device__ __forceinline__ void emit_q8_wide(const float (&v)[8], uint32_t l4, bool live, uint8_t* blk) {
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    amax = fmaxf(amax, dpp_f<0xB1>(amax));
+    amax = fmaxf(amax, dpp_f<0x4E>(amax));
+    const float d = amax / 127.0f, inv = amax > 0.f ? 127.0f / amax : 0.f;
+    int q[8], sum = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        q[i] = round_away_i(v[i] * inv);
+        sum += q[i];
+    }
+    auto pack = [](int a, int b, int c, int e) {
+        return (uint32_t)(a & 0xFF) | ((uint32_t)(b & 0xFF) << 8) | ((uint32_t)(c & 0xFF) << 16) | ((uint32_t)(e & 0xFF) << 24);
+    };
+    const int half = sum + __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, true);       // 16 elements
+    const int other = __builtin_amdgcn_update_dpp(0, half, 0x4E, 0xF, 0xF, true);           // the other half of the block
+    if (!live) return;
+    reinterpret_cast<uint2*>(blk + (SPLIT ? 16 : 8))[l4] = make_uint2(pack(q[0], q[1], q[2], q[3]), pack(q[4], q[5], q[6], q[7]));
+    if (l4 != 0) return;
+    if (SPLIT) *reinterpret_cast<float4*>(blk) = make_float4(d, d * (float)half, d * (float)other, 0.f);
+    else *reinterpret_cast<float2*>(blk) = make_float2(d, d * (float)(half + other));
 }
 
 // ---------------------------------------------------------------- scales

@@ -208,7 +208,7 @@ __device__ __forceinline__ ActTile stage_act_f16(uint8_t* lds, RowFn hrow, uint3
             uint32_t pk = 0;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                const int qi = (int)roundf(v[4 * j + b] * inv);
+                const int qi = round_away_i(v[4 * j + b] * inv);
                 s16 += qi;
                 pk |= (uint32_t)(qi & 0xFF) << (8 * b);
             }

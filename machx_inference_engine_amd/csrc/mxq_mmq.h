@@ -643,7 +643,7 @@ __device__ __forceinline__ MmqAct mmq_stage_f16(uint8_t* lds, RowFn hrow, uint32
                 uint32_t pk = 0;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    const int qi = (int)roundf(v[4 * j + c] * inv);
+                    const int qi = round_away_i(v[4 * j + c] * inv);
                     sum += qi;
                     pk |= (uint32_t)(qi & 0xFF) << (8 * c);
                 }

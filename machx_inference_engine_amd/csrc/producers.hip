@@ -72,31 +72,37 @@ __global__ __launch_bounds__(kNormThreads) void norm_q8_kernel(const XT* x, cons
 // gpt-oss form x = min(gate, limit), z = clamp(up, -limit, limit), y = half(x * sigmoid(alpha x) * (z + 1))
 // (swiglu_oai, :469-492), written as fp16 (when y != NULL) and as the block_q8_1x stream of the rounded
 // values: the down projection's int-dot input without a quantize launch.  Thread = 4 elements.
-template <bool OAI>
+// E = 8 elements per thread where gate, up and y lie on 16-byte boundaries, else 4: 58.7 M elements 87.2 -> 77.3 us
+// (5.4 TB/s, memory-bound), 7.3 M 12.8 -> 11.4 us; below 1 M elements the launch is all there is.
+template <bool OAI, int E>
 __global__ __launch_bounds__(256) void act_q8_kernel(const half_t* gate, const half_t* up, half_t* y, uint8_t* q8, uint64_t n, float alpha, float limit) {
-    const uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    typedef _Float16 vec_t __attribute__((ext_vector_type(E)));
+    const uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * E;
     const bool live = i < n;
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
-    if (live) {
-        half_t g4[4], u4[4], h4[4];
-        *reinterpret_cast<uint2*>(g4) = *reinterpret_cast<const uint2*>(gate + i);
-        *reinterpret_cast<uint2*>(u4) = *reinterpret_cast<const uint2*>(up + i);
+    float v[E];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < E; ++j) v[j] = 0.f;
+    if (live) {
+        const vec_t gv = *reinterpret_cast<const vec_t*>(gate + i), uv = *reinterpret_cast<const vec_t*>(up + i);
+        vec_t hv;
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
             float o;
             if (OAI) {
-                const float x = fminf((float)g4[j], limit), z = fmaxf(fminf((float)u4[j], limit), -limit);
+                const float x = fminf((float)gv[j], limit), z = fmaxf(fminf((float)uv[j], limit), -limit);
                 o = (x / (1.f + __expf(alpha * (-x)))) * (z + 1.f);
             } else {
-                const float g = (float)g4[j];
-                o = (g / (1.f + __expf(-g))) * (float)u4[j];
+                const float g = (float)gv[j];
+                o = (g / (1.f + __expf(-g))) * (float)uv[j];
             }
-            h4[j] = (half_t)o;
-            v[j] = (float)h4[j];
+            hv[j] = (half_t)o;
+            v[j] = (float)hv[j];
         }
-        if (y) *reinterpret_cast<uint2*>(y + i) = *reinterpret_cast<const uint2*>(h4);
+        if (y) *reinterpret_cast<vec_t*>(y + i) = hv;
     }
-    emit_q8_1x(v, threadIdx.x & 7u, live, q8 + (i / 32) * kQ81xBytes);
+    uint8_t* blk = q8 + (i / 32) * kQ81xBytes;
+    if constexpr (E == 8) emit_q8_wide<false>(v, threadIdx.x & 3u, live, blk);
+    else emit_q8_1x(v, threadIdx.x & 7u, live, blk);
 }
 
 template <bool OAI>
@@ -104,8 +110,13 @@ static int act_q8(mx_stream_t s, const uint16_t* gate, const uint16_t* up, uint1
     MX_REQUIRE_PTR(gate); MX_REQUIRE_PTR(up); MX_REQUIRE_PTR(q8_out);
     MX_REQUIRE_SHAPE(n > 0 && n % 32 == 0 && (n / 4 + 255) / 256 <= 0x7FFFFFFFull);
     MX_REQUIRE_ALIGN(gate, 8); MX_REQUIRE_ALIGN(up, 8); MX_REQUIRE_ALIGN(y, 8); MX_REQUIRE_ALIGN(q8_out, 8);
-    hipLaunchKernelGGL((act_q8_kernel<OAI>), dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, as_stream(s), reinterpret_cast<const half_t*>(gate),
-                       reinterpret_cast<const half_t*>(up), reinterpret_cast<half_t*>(y), static_cast<uint8_t*>(q8_out), n, alpha, limit);
+    const half_t *g = reinterpret_cast<const half_t*>(gate), *u = reinterpret_cast<const half_t*>(up);
+    half_t* yh = reinterpret_cast<half_t*>(y);
+    uint8_t* q = static_cast<uint8_t*>(q8_out);
+    if (aligned(gate, 16) && aligned(up, 16) && aligned(y, 16))
+        hipLaunchKernelGGL((act_q8_kernel<OAI, 8>), dim3((uint32_t)((n / 8 + 255) / 256)), dim3(256), 0, as_stream(s), g, u, yh, q, n, alpha, limit);
+    else
+        hipLaunchKernelGGL((act_q8_kernel<OAI, 4>), dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, as_stream(s), g, u, yh, q, n, alpha, limit);
     return launch_status();
 }
 

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const ActT* x, uint8
     int q[4], sum = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        q[i] = (int)roundf(v[i] * inv);
+        q[i] = round_away_i(v[i] * inv);
         sum += q[i];
     }
     const uint32_t packed = (uint32_t)(q[0] & 0xFF) | ((uint32_t)(q[1] & 0xFF) << 8) | ((uint32_t)(q[2] & 0xFF) << 16) | ((uint32_t)(q[3] & 0xFF) << 24);
@@ -56,6 +56,20 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const ActT* x, uint8
     }
 }
 
+// fp16 rows on 16-byte boundaries: 8 elements per thread (33.6 M elements 26.7 -> 18.9 us, block_q8_1s 25.0 -> 19.5 us; small rows are
+// bound by the launch either way)
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void quantize_q8_wide_kernel(const half_t* __restrict__ x, uint8_t* __restrict__ out, uint64_t n_blocks) {
+    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t b = gid >> 2;
+    const bool live = b < n_blocks;
+    uint4 u = make_uint4(0u, 0u, 0u, 0u);
+    if (live) u = reinterpret_cast<const uint4*>(x)[gid];
+    const float v[8] = {h2f(u.x & 0xFFFFu), h2f(u.x >> 16), h2f(u.y & 0xFFFFu), h2f(u.y >> 16),
+                        h2f(u.z & 0xFFFFu), h2f(u.z >> 16), h2f(u.w & 0xFFFFu), h2f(u.w >> 16)};
+    emit_q8_wide<SPLIT>(v, (uint32_t)gid & 3u, live, out + b * (SPLIT ? kQ81sBytes : kQ81xBytes));
+}
+
 template <class ActT, bool SPLIT>
 static int quantize_launch(mx_stream_t s, const ActT* x, void* out, uint64_t n) {
     MX_REQUIRE_PTR(x);
@@ -66,6 +80,13 @@ static int quantize_launch(mx_stream_t s, const ActT* x, void* out, uint64_t n) 
     const uint64_t nb = n / 32, threads = nb * 8;
     const uint64_t blocks = (threads + 255) / 256;
     MX_REQUIRE_SHAPE(blocks <= 0x7FFFFFFFull);
+    if constexpr (std::is_same<ActT, half_t>::value) {
+        if (aligned(x, 16)) {
+            hipLaunchKernelGGL((quantize_q8_wide_kernel<SPLIT>), dim3((uint32_t)((nb * 4 + 255) / 256)), dim3(256), 0, as_stream(s), x,
+                               static_cast<uint8_t*>(out), nb);
+            return launch_status();
+        }
+    }
     hipLaunchKernelGGL((quantize_q8_1_kernel<ActT, SPLIT>), dim3((uint32_t)blocks), dim3(256), 0, as_stream(s), x, static_cast<uint8_t*>(out), nb);
     return launch_status();
 }

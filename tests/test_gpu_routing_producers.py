@@ -196,3 +196,27 @@ def test_swiglu_q8(mx, n, oai):
     assert np.array_equal(host(q8), ref_q8_of(y_h).reshape(-1)), "q8 stream == quantize_q8_1(y)"
     _, q8_only = mx.ops.swiglu_q8(dev(g).half(), dev(u).half(), oai=oai, want_y=False)
     assert torch.equal(q8_only, q8)
+
+
+@pytest.mark.parametrize("n", [32, 64, 1024, 2048 + 96, 32 * 1001])
+def test_q8_producers_on_8_and_16_byte_boundaries(mx, n):
+    """Eight elements per thread on 16-byte boundaries, four on 8-byte ones: the same fp16 values and q8 bytes (both evaluate one
+    element alike), at sizes that end inside a workgroup, against the quantizer of the oracle; halves, a signed zero and an infinity among them."""
+    g, u = f16(O.normal(9600 + n, (n + 4,), 0.0, 3.0)), f16(O.normal(9601 + n, (n + 4,)))
+    g[5:12] = [127.0, 0.5, -0.5, 2.5, -2.5, 1.5, -0.0]
+    tg, tu = dev(g).half(), dev(u).half()
+    x8, x16 = tg[4:], tg[4:].clone()
+    assert x8.data_ptr() % 16 == 8 and x16.data_ptr() % 16 == 0
+    for quantize, oracle in ((mx.ops.quantize_q8_1, O.quantize_q8_1), (mx.ops.quantize_q8_1s, O.quantize_q8_1s)):
+        ref = oracle(g[4:])
+        assert np.array_equal(host(quantize(x8)).reshape(-1), ref.reshape(-1)) and np.array_equal(host(quantize(x16)).reshape(-1), ref.reshape(-1))
+    for oai in (False, True):
+        y8, q8 = mx.ops.swiglu_q8(x8, tu[4:], oai=oai)
+        y16, q16 = mx.ops.swiglu_q8(x16, tu[4:].clone(), oai=oai)
+        assert torch.equal(y8, y16) and torch.equal(q8, q16)
+        assert np.array_equal(host(q16), ref_q8_of(host(y16)).reshape(-1))
+    inf = x16.clone()
+    inf[3] = float("inf")
+    off = torch.empty(n + 4, dtype=torch.float16, device=inf.device)[4:]
+    off.copy_(inf)
+    assert torch.equal(mx.ops.quantize_q8_1(inf), mx.ops.quantize_q8_1(off))
