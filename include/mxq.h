@@ -614,6 +614,8 @@ int mx_moe_down_q8_f16_n(mx_stream_t s, const uint16_t* h_f16, const int8_t* d_q
  *     logits = W_gate[E,H] (fp32) . x_t, softmax, top-k, renormalise, ascending expert id; any
  *     E <= 1024, k <= 64 (the reference handles E = 256, k = 8 only).  logits_ws: caller-owned
  *     workspace of n_tokens*n_experts floats (the reference keeps a static per-device buffer).
+ *     A token's logits, ids and weights are the same bits in every call: alone, in any batch, at any
+ *     alignment of x.
  *   moe_topk_from_logits   include/ie/ops.hpp:790-793, src/ops/moe.cpp:366-412   (fp16 logits, n_tokens rows)
  *   moe_build_pack_decode  include/ie/ops.hpp:797-802, src/ops/moe.cpp:423-446   (one token)
  *   mx_moe_build_packing_device: the arrays of build_moe_packing (src/model/qwen3moe_pack.cpp:5-31)

@@ -10,134 +10,128 @@
 namespace mxq {
 
 // ---------------------------------------------------------------- router logits
-// logit[t, e] = sum_h W_gate[e, h] * x[t, h], fp32 weights and sums.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Up to this many (expert, token) rows a workgroup per row is the faster form (128 experts, hidden 2048: 48 tokens 5.0 us against
-// 7.6 in tiles, 64 tokens about 6.2, 333 tokens 24 against 7.6).
-constexpr uint64_t kRouterRowGroups = 8192;
-// A few tokens: one workgroup per (expert, token), so that a row is two or three loads per thread, all of them in flight
-// at once (latency is all there is: 32 experts, hidden 2880, one token 3.0 -> 2.0 us against one wave per row).
-__global__ __launch_bounds__(256) void router_logits_kernel(const half_t* x, const float* W, float* logits, uint32_t hidden, uint32_t E) {
-    __shared__ float red[4];
-    const uint32_t e = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-    const float* wr = W + (size_t)e * hidden;
-    const half_t* xr = x + (size_t)t * hidden;
-    float acc = 0.f;
-#pragma unroll 4
-    for (uint32_t i = tid * 4; i < hidden; i += 1024) {
-        const float4 w4 = *reinterpret_cast<const float4*>(wr + i);
-        const uint2 xu = *reinterpret_cast<const uint2*>(xr + i);
-        acc += w4.x * h2f(xu.x & 0xFFFFu) + w4.y * h2f(xu.x >> 16) + w4.z * h2f(xu.y & 0xFFFFu) + w4.w * h2f(xu.y >> 16);
-    }
-    acc = group_sum<64>(acc);
-    if ((tid & 63u) == 63u) red[tid >> 6] = acc;
-    __syncthreads();
-    if (tid == 0) logits[(size_t)t * E + e] = red[0] + red[1] + red[2] + red[3];
+// logit[t, e] = sum_h W_gate[e, h] * x[t, h], fp32 weights and sums.  One summation order for every call, whatever its batch,
+// sizes and alignments, so that a token is routed alike alone, in a decode batch and in a prompt:
+//   lane l takes the elements 4 l .. 4 l + 3 of every 256-element piece, router_dot4 over the four, pieces added in order;
+//   the 64 lane sums meet in a balanced tree of neighbours.
+// (32 products a lane at hidden 2048, then six levels: rms error against 64-bit sums 9.6e-8, maximum 5.4e-7, logits of unit variance.
+// One fp32 MFMA accumulator per output, a chain of 128 or 256 products, takes 17 us where this takes 25 to 27 (2048 tokens, 128
+// experts) but has rms 2.2e-7 to 2.9e-7 and maximum 1.8e-6: near ties are routed otherwise.)
+__device__ __forceinline__ float router_dot4(const float4& w, const float (&x)[4]) {
+    return __builtin_fmaf(w.w, x[3], __builtin_fmaf(w.z, x[2], __builtin_fmaf(w.x, x[0], w.y * x[1])));
 }
 
-// Many tokens: 16 MI tokens x 16 NI experts per workgroup on v_mfma_f32_16x16x4_f32 (fp32 in, fp32 accumulate: the products
-// and sums of the scalar form in another order).  Lane (i, q) feeds elements 8 q .. 8 q + 7 of a 32-element piece of row i, so
-// four lanes read 64 consecutive bytes of x and 128 of W; the WV waves take the pieces of the row in turn and their sums meet in
-// LDS.  One workgroup per (expert, token), as above, reads W once per token (2048 tokens, 128 experts, hidden 2048: 2 GB through
-// the L2s, 134 us); a tile reads it once per 16 MI tokens: 17 us.  The matrix instructions alone are 6.8 us there.  With
-// 32x32x2 instructions (two lanes per row, 32-byte pieces) the loads run at half the rate and the same launch took 25.7 us with WV = 4.
-// MI = NI = 2 halves the traffic and is taken once its tiles fill half of the CUs; below that the smaller tiles spread the rows
-// over more CUs (a CU takes about 64 B a clock from its L2: 333 tokens 14.9 us with 32 x 32 tiles).
-template <int MI, int NI, int WV>
-__global__ __launch_bounds__(64 * WV) void router_logits_mfma_kernel(const half_t* __restrict__ x, const float* __restrict__ W, float* __restrict__ logits,
-                                                                     uint32_t T, uint32_t hidden, uint32_t E) {
-    constexpr int U = MI * NI == 1 ? 4 : 2;   // pieces requested together
-    __shared__ __align__(16) float red[(WV - 1) * MI * NI * 256];
-    const uint32_t lane = threadIdx.x & 63u, i = lane & 15u, q = lane >> 4;
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t t0 = blockIdx.y * (16u * MI), e0 = blockIdx.x * (16u * NI);
-    const uint4* xr[MI];
-    const float4* wr[NI];
+// Halves N values per lane: the lane keeps the odd or the even ones (sel) and adds its partner's, or, with one value left, adds
+// the partner's.  Level d pairs neighbouring groups of 2^d lanes.  DPP has no exchange at distance 4 or 8, but mirrors of 8 and 16
+// lanes; `sel` of the lower levels is chosen so that mirrored lanes hold the same values.
+template <int N, int D>
+__device__ __forceinline__ void router_level(float (&v)[N], float (&o)[N > 1 ? N / 2 : 1], uint32_t lane) {
+    auto partner = [](float x) {
+        if constexpr (D == 0) return dpp_f<0xB1>(x);
+        else if constexpr (D == 1) return dpp_f<0x4E>(x);
+        else if constexpr (D == 2) return dpp_f<0x141>(x);
+        else if constexpr (D == 3) return dpp_f<0x140>(x);
+        else return __shfl_xor(x, 1 << D);
+    };
+    if constexpr (N == 1) {
+        o[0] = v[0] + partner(v[0]);
+    } else {
+        const bool sel = ((D == 0 ? lane ^ (lane >> 2) : D == 1 ? (lane >> 1) ^ (lane >> 2) : D == 2 ? (lane >> 2) ^ (lane >> 3) : lane >> D) & 1u) != 0u;
 #pragma unroll
-    for (int m = 0; m < MI; ++m) {
-        const uint32_t t = t0 + 16u * m + i;
-        xr[m] = reinterpret_cast<const uint4*>(x + (size_t)(t < T ? t : T - 1u) * hidden) + q;          // piece c: xr[4 c]
+        for (int i = 0; i < N / 2; ++i) {
+            const float keep = sel ? v[2 * i + 1] : v[2 * i], send = sel ? v[2 * i] : v[2 * i + 1];
+            o[i] = keep + partner(send);
+        }
     }
+}
+template <int N, int D = 0>
+__device__ __forceinline__ float router_tree(float (&v)[N], uint32_t lane) {
+    float o[N > 1 ? N / 2 : 1];
+    router_level<N, D>(v, o, lane);
+    if constexpr (D == 5) return o[0];
+    else return router_tree<(N > 1 ? N / 2 : 1), D + 1>(o, lane);
+}
+
+// One wave = MT tokens x NE experts, MT NE accumulators per lane (a power of two up to 64).  U: pieces whose loads are requested
+// together.  The waves of a workgroup take neighbouring token tiles of the same experts.  Bound by: the load latency of a row at a
+// few tokens, five vector instructions per four products at many (2048 tokens, 128 experts, hidden 2048: 17 us of issue, 25 to
+// 27 measured; one wave per output, which reads W once per token: 140).
+template <int MT, int NE, int U>
+__global__ __launch_bounds__(256) void router_logits_kernel(const half_t* __restrict__ x, const float* __restrict__ W, float* __restrict__ logits, uint32_t T,
+                                                            uint32_t hidden, uint32_t E) {
+    constexpr int P = MT * NE;
+    static_assert((P & (P - 1)) == 0 && P <= 64, "one result per lane at most");
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t tile = blockIdx.x * (blockDim.x / 64u) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t t_tiles = (T + MT - 1u) / MT, e0 = tile / t_tiles * NE, t0 = tile % t_tiles * MT;
+    if (e0 >= E) return;
+    const uint2* xr[MT];
+    const float4* wr[NE];
 #pragma unroll
-    for (int n = 0; n < NI; ++n) {
-        const uint32_t e = e0 + 16u * n + i;
-        wr[n] = reinterpret_cast<const float4*>(W + (size_t)(e < E ? e : E - 1u) * hidden) + 2u * q;    // piece c: wr[8 c], wr[8 c + 1]
-    }
-    const uint32_t n_pieces = hidden / 32u;
-    f32x4 acc[MI][NI];
+    for (int m = 0; m < MT; ++m) xr[m] = reinterpret_cast<const uint2*>(x + (size_t)(t0 + m < T ? t0 + m : T - 1u) * hidden);   // uniform; piece c: xr[64 c + lane]
 #pragma unroll
-    for (int m = 0; m < MI; ++m)
+    for (int n = 0; n < NE; ++n) wr[n] = reinterpret_cast<const float4*>(W + (size_t)(e0 + n < E ? e0 + n : E - 1u) * hidden);
+    float acc[P];
 #pragma unroll
-        for (int n = 0; n < NI; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < P; ++p) acc[p] = 0.f;
     struct Piece {
-        uint4 x[MI];
-        float4 w[NI][2];
+        uint2 x[MT];
+        float4 w[NE];
     };
     auto load = [&](uint32_t c, Piece& p) {
 #pragma unroll
-        for (int m = 0; m < MI; ++m) p.x[m] = xr[m][4u * c];
+        for (int n = 0; n < NE; ++n) p.w[n] = wr[n][64u * c + lane];
 #pragma unroll
-        for (int n = 0; n < NI; ++n) {
-            p.w[n][0] = wr[n][8u * c];
-            p.w[n][1] = wr[n][8u * c + 1u];
+        for (int m = 0; m < MT; ++m) p.x[m] = xr[m][64u * c + lane];
+    };
+    auto add = [&](const Piece& p) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const float v[4] = {h2f(p.x[m].x & 0xFFFFu), h2f(p.x[m].x >> 16), h2f(p.x[m].y & 0xFFFFu), h2f(p.x[m].y >> 16)};
+#pragma unroll
+            for (int n = 0; n < NE; ++n) acc[m * NE + n] += router_dot4(p.w[n], v);
         }
     };
-    auto step = [&](const Piece& p) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            float a[MI], b[NI];
-#pragma unroll
-            for (int m = 0; m < MI; ++m) {
-                const uint32_t w = k < 2 ? p.x[m].x : k < 4 ? p.x[m].y : k < 6 ? p.x[m].z : p.x[m].w;
-                a[m] = h2f((k & 1) ? w >> 16 : w & 0xFFFFu);
-            }
-#pragma unroll
-            for (int n = 0; n < NI; ++n) {
-                const float4 w = p.w[n][k >> 2];
-                b[n] = (k & 3) == 0 ? w.x : (k & 3) == 1 ? w.y : (k & 3) == 2 ? w.z : w.w;
-            }
-#pragma unroll
-            for (int m = 0; m < MI; ++m)
-#pragma unroll
-                for (int n = 0; n < NI; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], b[n], acc[m][n], 0, 0, 0);
-        }
-    };
-    uint32_t c = wave;
-    for (; c + (U - 1) * WV < n_pieces; c += U * WV) {
+    const uint32_t n_full = hidden / 256u;
+    const bool last = n_full * 256u + lane * 4u < hidden;   // the lanes that take part in the last, partial piece
+    Piece end{};
+    if (P <= 4 && last) load(n_full, end);                  // few outputs: requested ahead of everything else
+    for (uint32_t c = 0; c < n_full; c += U) {
         Piece p[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) load(c + u * WV, p[u]);
+        for (int u = 0; u < U; ++u)
+            if (U == 1 || c + u < n_full) load(c + u, p[u]);
 #pragma unroll
-        for (int u = 0; u < U; ++u) step(p[u]);
+        for (int u = 0; u < U; ++u)
+            if (U == 1 || c + u < n_full) add(p[u]);
     }
-    for (; c < n_pieces; c += WV) {
-        Piece p;
-        load(c, p);
-        step(p);
+    if (last) {
+        if (P > 4) load(n_full, end);
+        add(end);
     }
-    if (wave > 0) {
-#pragma unroll
-        for (int m = 0; m < MI; ++m)
-#pragma unroll
-            for (int n = 0; n < NI; ++n) *reinterpret_cast<f32x4*>(&red[(((wave - 1u) * MI + m) * NI + n) * 256u + lane * 4u]) = acc[m][n];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-#pragma unroll
-    for (int m = 0; m < MI; ++m)
-#pragma unroll
-        for (int n = 0; n < NI; ++n) {
-            f32x4 s = acc[m][n];
-#pragma unroll
-            for (int w = 0; w < WV - 1; ++w) s += *reinterpret_cast<const f32x4*>(&red[((w * MI + m) * NI + n) * 256 + lane * 4u]);
-            const uint32_t e = e0 + 16u * n + i;                                    // lane (i, q): column (expert) i, rows 4 q + v
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t t = t0 + 16u * m + 4u * q + v;
-                if (t < T && e < E) logits[(size_t)t * E + e] = s[v];
-            }
-        }
+    const float sum = router_tree(acc, lane);
+    // which value this lane has kept: one bit per halving level, the level's `sel`
+    const uint32_t key = ((lane ^ (lane >> 2)) & 1u) | (((lane >> 1) ^ (lane >> 2)) & 1u) << 1 | (((lane >> 2) ^ (lane >> 3)) & 1u) << 2 | (lane & 56u);
+    const uint32_t k = key & (P - 1u), t = t0 + k / NE, e = e0 + k % NE;
+    if (lane < P && t < T && e < E) logits[(size_t)t * E + e] = sum;
+}
+
+template <int MT, int NE, int U, uint32_t WV>
+static int launch_router(hipStream_t st, const half_t* x, const float* W, float* logits, uint32_t T, uint32_t hidden, uint32_t E) {
+    const uint32_t tiles = ((T + MT - 1u) / MT) * ((E + NE - 1u) / NE);
+    hipLaunchKernelGGL((router_logits_kernel<MT, NE, U>), dim3((tiles + WV - 1u) / WV), dim3(64u * WV), 0, st, x, W, logits, T, hidden, E);
+    return launch_status();
+}
+// The tile by the number of outputs: small tiles spread few outputs over the CUs, large ones read the rows less often.  Times with
+// the top-k behind it, us, 1 x 1 (one wave per workgroup) / 2 x 2 / 4 x 4 / 8 x 8: 128 experts, hidden 2048: 16 tokens 6.8 / 6.9 / 7.9 /
+// 13, 64 tokens 9.7 / 8.0 / 8.1 / 13, 333 tokens 26 / 16 / 11.9 / 13, 1024 tokens 67 / 35 / 21.5 / 18; 32 experts, hidden 2880:
+// one token 4.8 / 6.2 / 7.5 / 14, 512 tokens 17 / 11 / 8.7 / 15, 2048 tokens 54 / 29 / 16.9 / 15.6.
+static int launch_router_logits(hipStream_t st, const half_t* x, const float* W, float* logits, uint32_t T, uint32_t hidden, uint32_t E) {
+    const uint32_t n = T * E;   // at most 65535 x 1024
+    if (n <= 2048u) return launch_router<1, 1, 8, 1>(st, x, W, logits, T, hidden, E);
+    if (n <= 8192u) return launch_router<2, 2, 4, 4>(st, x, W, logits, T, hidden, E);
+    if (n < 65536u) return launch_router<4, 4, 1, 4>(st, x, W, logits, T, hidden, E);
+    return launch_router<8, 8, 1, 4>(st, x, W, logits, T, hidden, E);
 }
 
 // ---------------------------------------------------------------- softmax + top-k
@@ -449,16 +443,7 @@ int mx_moe_router(mx_stream_t s, const uint16_t* x, const float* W_gate, int32_t
                      k <= (uint32_t)kMaxTopK);
     MX_REQUIRE_ALIGN(x, 8); MX_REQUIRE_ALIGN(W_gate, 16);
     hipStream_t st = as_stream(s);
-    const half_t* xh = reinterpret_cast<const half_t*>(x);
-    if ((uint64_t)n_tokens * n_experts > kRouterRowGroups && hidden % 32 == 0 && aligned(x, 16)) {
-        const uint32_t te = (n_experts + 31) / 32, tt = (n_tokens + 31) / 32;
-        const dim3 small((n_experts + 15) / 16, (n_tokens + 15) / 16);
-        if (te * tt >= 128) hipLaunchKernelGGL((router_logits_mfma_kernel<2, 2, 8>), dim3(te, tt), dim3(512), 0, st, xh, W_gate, logits_ws, n_tokens, hidden, n_experts);
-        else hipLaunchKernelGGL((router_logits_mfma_kernel<1, 1, 16>), small, dim3(1024), 0, st, xh, W_gate, logits_ws, n_tokens, hidden, n_experts);
-    } else {
-        hipLaunchKernelGGL(router_logits_kernel, dim3(n_experts, n_tokens), dim3(256), 0, st, xh, W_gate, logits_ws, hidden, n_experts);
-    }
-    if (int rc = launch_status()) return rc;
+    if (int rc = launch_router_logits(st, reinterpret_cast<const half_t*>(x), W_gate, logits_ws, n_tokens, hidden, n_experts)) return rc;
     return launch_topk(st, (const float*)logits_ws, topk_idx, reinterpret_cast<half_t*>(topk_w), n_experts, k, n_tokens);
 }
 

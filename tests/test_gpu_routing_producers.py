@@ -76,11 +76,68 @@ def test_moe_packing_device_equals_host(mx, T, E, K):
         assert np.array_equal(host(wp).astype(np.float32), wp_r)
 
 
+def _fma32(a, b, c):
+    """fp32 fused multiply-add of fp32 a, c and fp16-valued b: the product is exact in 64 bits, the sum is rounded to odd there (so
+    that rounding it again to fp32 is one correct rounding)."""
+    p, c = a.astype(np.float64) * b, c.astype(np.float64)
+    s = p + c
+    t = s - p
+    err = (p - (s - t)) + (c - t)
+    odd = (s.view(np.int64) & 1) == 1
+    s = np.where((err != 0) & ~odd, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s)
+    return s.astype(np.float32)
+
+
+def router_logits(x, W):
+    """The documented order of the router's sums: lane l takes elements 4 l .. 4 l + 3 of every 256, then a tree of neighbours."""
+    T, H = x.shape
+    acc = np.zeros((T, len(W), 64), np.float32)
+    for c in range(0, H, 256):
+        n = min(256, H - c) // 4
+        xs, ws = x[:, None, c:c + 4 * n].reshape(T, 1, n, 4), W[None, :, c:c + 4 * n].reshape(1, len(W), n, 4)
+        d = (ws[..., 1].astype(np.float64) * xs[..., 1]).astype(np.float32)
+        for i in (0, 2, 3):
+            d = _fma32(np.broadcast_to(ws[..., i], d.shape), xs[..., i], d)
+        acc[..., :n] += d
+    while acc.shape[-1] > 1:
+        acc = acc[..., 0::2] + acc[..., 1::2]
+    return acc[..., 0]
+
+
+@pytest.mark.parametrize("T,E,H", [(1, 33, 2880), (3, 32, 36), (60, 65, 264), (64, 128, 1028), (333, 60, 516), (65, 128, 256), (1030, 65, 260), (64, 1024, 256)])
+def test_moe_router_logits_do_not_depend_on_the_call(mx, T, E, H):
+    """Every tile size of the logits kernel (1 x 1, 2 x 2, 4 x 4, 8 x 8 by T * E), whole and partial pieces, ragged tiles: the bits of
+    the one summation order, also for a token alone and for rows on an 8-byte boundary."""
+    x = f16(O.normal(9170 + T, (T, H)))
+    Wg = O.normal(9171 + E, (E, H), 0.0, 1.0 / np.sqrt(H)).astype(np.float32)
+    flat = torch.zeros(T * H + 4, dtype=torch.float16, device="cuda")
+    flat[4:] = dev(x).half().reshape(-1)
+    k = min(4, E)
+
+    def logits(rows):
+        n = rows.shape[0]
+        ws = torch.full((n, E), float("nan"), device="cuda")
+        idx, w = torch.empty((n, k), dtype=torch.int32, device="cuda"), torch.empty((n, k), dtype=torch.float16, device="cuda")
+        mx.ops._call("mx_moe_router", rows.data_ptr(), Wt.data_ptr(), idx.data_ptr(), w.data_ptr(), n, H, E, k, ws.data_ptr())
+        return host(ws), host(idx), host(w)
+
+    Wt, xt = dev(Wg), dev(x).half()
+    got, ids, w = logits(xt)
+    ref = router_logits(x, Wg)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), "logits: %d of %d differ" % ((got != ref).sum(), ref.size)
+    shifted = flat[4:].reshape(T, H)
+    assert shifted.data_ptr() % 16 == 8
+    for a, b in zip(logits(shifted), (got, ids, w)):
+        assert np.array_equal(a, b)
+    for a, b in zip(logits(xt[T - 1:].clone()), (got, ids, w)):
+        assert np.array_equal(a[0], b[T - 1])
+
+
 @pytest.mark.parametrize("T,E,k,H", [(16, 33, 5, 1040), (40, 65, 4, 16), (300, 33, 5, 36), (250, 33, 5, 1056), (333, 128, 8, 2048), (1030, 257, 8, 288), (2050, 60, 6, 544)])
 def test_moe_router_token_tiles(mx, T, E, k, H):
-    """Token and expert counts off the 16 x 16 and 32 x 32 tiles and the one-row-per-workgroup form, hidden sizes that end inside
-    a wave's turn of 32-element pieces (and some that are no whole number of them).  The logits are fp32 sums of H <= 2048 products: a pick may
-    differ only where two probabilities are within H * 2^-24 of each other."""
+    """Picks against logits summed in 64 bits, over the tile sizes.  A pick may differ only where two logits are within 4e-6: the fp32 sums of up to 2048
+    products are off by 6e-7 each (weights of 1 / sqrt(H)), and a probability carries (max - logit) * 2^-23 of exp, below 2e-6 here.
+    Neighbours at the edge of the top k are about 0.05 apart, so fewer than one token in a thousand can differ."""
     x = f16(O.normal(9150 + T, (T, H)))
     Wg = O.normal(9151 + E, (E, H), 0.0, 1.0 / np.sqrt(H)).astype(np.float32)
     idx, w = mx.ops.moe_router(dev(x).half(), dev(Wg), E, k)
@@ -90,8 +147,8 @@ def test_moe_router_token_tiles(mx, T, E, k, H):
     same = (idx_h == ids_ref).all(axis=1)
     for t in np.where(~same)[0]:
         a, b = sorted(set(idx_h[t]) - set(ids_ref[t])), sorted(set(ids_ref[t]) - set(idx_h[t]))
-        assert len(a) == len(b) == len(set(a)) and np.abs(logits[t, a] - logits[t, b]).max() <= 4 * H * 2.0 ** -24, "differs beyond a tie"
-    assert same.mean() >= 0.99
+        assert len(a) == len(b) == len(set(a)) and np.abs(logits[t, a] - logits[t, b]).max() <= 4e-6, "differs beyond a tie"
+    assert (~same).sum() <= T // 1000
     check(host(w).astype(np.float32)[same], w_ref[same], "router weights", max_rel=2e-3)
 
 
