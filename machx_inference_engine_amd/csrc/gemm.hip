@@ -1325,15 +1325,9 @@ static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const type
     const uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.k_split;
     const uint64_t grid = (total + 7) / 8 * 8;
     if (grid > 0x7FFFFFFFull) return MX_ERR_SHAPE;
-    static bool attr_set = false;   // LDS at the 64 KB default limit: opt in once per kernel
-    if (!attr_set) {
-        const hipError_t er = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<QF, MODE, NI, KW>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (er != hipSuccess) {
-            g_last_hip_error = (int)er;
-            return MX_ERR_LAUNCH;
-        }
-        attr_set = true;
+    if constexpr (lds > kLdsDefaultLimit) {
+        static LdsLimit limit;
+        if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&gemm_kernel<QF, MODE, NI, KW>), limit, lds)) return rc;
     }
     hipLaunchKernelGGL((gemm_kernel<QF, MODE, NI, KW>), dim3((uint32_t)grid), dim3(kGemmThreads * KW), lds, as_stream(s), b0, b1, g);
     return launch_status();

@@ -477,17 +477,9 @@ static int launch_mmq_grouped_cfg(hipStream_t st, const typename P::Bank& b0, co
     const uint32_t lds = overlay ? (image > red ? image : red) : image + red;
     const uint32_t rgs = (m.N + 32u * WR - 1u) / (32u * WR);
     if (E > 65535u) return MX_ERR_SHAPE;
-    if (lds > 64u * 1024u) {
-        static bool attr_set = false;   // LDS above the 64 KB default limit: opt in once per kernel
-        if (!attr_set) {
-            const hipError_t er = hipFuncSetAttribute(reinterpret_cast<const void*>(&mmq_kernel<P, TV, NW, WR, WK, EPI>),
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMmqMoeLdsBudgetBig);
-            if (er != hipSuccess) {
-                g_last_hip_error = (int)er;
-                return MX_ERR_LAUNCH;
-            }
-            attr_set = true;
-        }
+    if (lds > kLdsDefaultLimit) {
+        static LdsLimit limit;
+        if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&mmq_kernel<P, TV, NW, WR, WK, EPI>), limit, kMmqMoeLdsBudgetBig)) return rc;
     }
     // token tiles of an expert are dealt over gridDim.z workgroups: the expert sizes live on the device and are skewed (a few
     // experts hold most rows), so the split is sized for experts several times the average; workgroups without a tile leave at once

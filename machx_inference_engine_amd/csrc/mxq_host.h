@@ -59,14 +59,37 @@ inline int scratch_address(const Sym& symbol, std::atomic<void*> (&slot)[kMaxDev
     return MX_OK;
 }
 
+// Dynamic LDS above the default limit is opted into per kernel AND per device (hipFuncSetAttribute acts on the current device's
+// copy of the kernel).  `done` belongs to one kernel, is indexed by device ordinal and remembers that its device took the limit;
+// every caller of one kernel passes the same `limit`.  A refusal leaves no error behind for the next launch_status().
+constexpr uint32_t kLdsDefaultLimit = 64u * 1024u;
+struct LdsLimit {
+    std::atomic<bool> done[kMaxDevices];
+};
+inline int raise_lds_limit(const void* kernel, LdsLimit& slot, uint32_t limit) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess && (dev < 0 || dev >= kMaxDevices)) e = hipErrorInvalidDevice;
+    if (e == hipSuccess && slot.done[dev].load(std::memory_order_acquire)) return MX_OK;
+    if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
+    if (e != hipSuccess) {
+        g_last_hip_error = (int)e;
+        (void)hipGetLastError();
+        return MX_ERR_LAUNCH;
+    }
+    slot.done[dev].store(true, std::memory_order_release);
+    return MX_OK;
+}
+
 // gemv_q6_planes.hip: one token against one or two (gate and up) Q6_K plane sets; MX_ERR_UNSUPPORTED for a shape it
 // does not take (K % 512, K > 16384, planes of 4 GB and more, misaligned scale planes)
 int launch_gemv_q6_planes(hipStream_t st, int nseg, const void* x_q8, const uint8_t* const* lo, const uint8_t* const* hi, const int8_t* const* sc,
                           const uint16_t* const* d, uint16_t* const* y, uint32_t K, uint32_t N);
 
-// per-device set-up of the translation units that own scratch arrays (mx_init)
+// per-device set-up of the translation units that own scratch arrays or raise an LDS limit (mx_init)
 int gemv_init_device();
 int gemm_init_device();
+int routing_init_device();
 
 }  // namespace mxq
 

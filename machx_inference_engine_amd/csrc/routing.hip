@@ -363,6 +363,15 @@ __global__ __launch_bounds__(1024) void pack_kernel(const int32_t* __restrict__ 
     }
 }
 
+static int raise_pack_lds() {
+    static LdsLimit limit;
+    return raise_lds_limit(reinterpret_cast<const void*>(&pack_kernel), limit, kPackLdsMax);
+}
+int routing_init_device() {
+    (void)raise_pack_lds();   // refused: the launches take the form that needs no more than the default
+    return MX_OK;
+}
+
 // More experts than that: the same sort, in three launches.
 //   count : workgroup e counts its slots                      -> expert_offsets[e + 1]
 //   scan  : one workgroup turns the counts into offsets        (inclusive scan in place)
@@ -465,21 +474,16 @@ int mx_moe_build_packing_device(mx_stream_t s, const int32_t* topk_idx, const ui
     const uint32_t n = T * K;
     hipStream_t st = as_stream(s);
     if (E <= kPackMaxExperts) {
-        const uint32_t waves = n <= 256 ? 4u : n <= 2048 ? 8u : 16u;
-        const uint32_t lds_min = (waves * E + E + 1) * 4u;
-        const uint32_t staged = n <= 65536u && lds_min + 4u * n <= kPackLdsMax ? 1u : 0u;
-        const uint32_t lds = lds_min + (staged ? 4u * n : 0u);
+        uint32_t waves = n <= 256 ? 4u : n <= 2048 ? 8u : 16u;
+        auto hist_bytes = [&] { return (waves * E + E + 1) * 4u; };
+        uint32_t staged = n <= 65536u && hist_bytes() + 4u * n <= kPackLdsMax ? 1u : 0u;
+        if (hist_bytes() + (staged ? 4u * n : 0u) > kLdsDefaultLimit && raise_pack_lds() != MX_OK) {   // the form that needs no more
+            staged = 0u;
+            while (hist_bytes() > kLdsDefaultLimit) waves /= 2u;
+        }
+        const uint32_t lds = hist_bytes() + (staged ? 4u * n : 0u);
         uint32_t id_bits = 0;
         while ((1u << id_bits) < E) ++id_bits;
-        static std::atomic<bool> attr_set{false};   // dynamic LDS past 64 KB: opt in once
-        if (!attr_set.load(std::memory_order_acquire)) {
-            const hipError_t er = hipFuncSetAttribute(reinterpret_cast<const void*>(&pack_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPackLdsMax);
-            if (er != hipSuccess) {
-                g_last_hip_error = (int)er;
-                return MX_ERR_LAUNCH;
-            }
-            attr_set.store(true, std::memory_order_release);
-        }
         hipLaunchKernelGGL(pack_kernel, dim3(1), dim3(64 * waves), lds, st, topk_idx, topk_w, n, K, E, id_bits, staged, expert_offsets, sorted_idx, weights_packed,
                            reinterpret_cast<uint32_t*>(tk_to_packed));
         return launch_status();
