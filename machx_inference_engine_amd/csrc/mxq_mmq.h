@@ -751,8 +751,8 @@ __device__ __forceinline__ void mmq_group(const typename P::Raw& raw, const MmqA
 // `g_base`.  One group of weight words is in flight while the previous one is multiplied (two register sets, never
 // copied, no load under a branch that a later iteration depends on).  Measured on this part: a wave streams best
 // with about eight 16-byte loads outstanding; deeper per-wave prefetch loses to more waves (a 58.7 MB read as 1792
-// walks of 32 rows x 1 KB: everything requested up front 13.0 us, one group ahead 11.7 us).
-template <class P, int TV>
+// walks of 32 rows x 1 KB: everything requested up front 13.0 us, one group ahead 11.7 us).  SEP: see mmq_two_tails.
+template <class P, int TV, bool SEP>
 struct MmqWalk {
     typename P::Raw raw[2];
     // the first group, requested by the caller before it stages the activations (it does not depend on them)
@@ -777,10 +777,21 @@ struct MmqWalk {
             mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
             g += 2;
         }
-        if (g + 1 < g_hi) raw[1] = P::load(w, n, g + 1, h, nb);
-        __builtin_amdgcn_sched_barrier(0);
-        mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
-        if (g + 1 < g_hi) mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
+        if constexpr (SEP) {
+            if (g + 1 < g_hi) {
+                raw[1] = P::load(w, n, g + 1, h, nb);
+                __builtin_amdgcn_sched_barrier(0);
+                mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
+                mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
+            } else {
+                mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
+            }
+        } else {
+            if (g + 1 < g_hi) raw[1] = P::load(w, n, g + 1, h, nb);
+            __builtin_amdgcn_sched_barrier(0);
+            mmq_group<P, TV>(raw[0], act, a_off, g - g_base, h, acc);
+            if (g + 1 < g_hi) mmq_group<P, TV>(raw[1], act, a_off, g + 1 - g_base, h, acc);
+        }
     }
 };
 
@@ -882,6 +893,23 @@ __device__ __forceinline__ void mmq_lds_barrier() { asm volatile("s_waitcnt lgkm
 // ---------------------------------------------------------------- kernel
 enum { MMQ_STORE = 0, MMQ_SILU = 1, MMQ_OAI = 2, MMQ_DOWN_WEIGHTED = 3, MMQ_DOWN_BIAS = 4 };
 
+// How a walk ends: SEP = true writes the last two groups and the last one out as two paths, where each group's arithmetic overlaps
+// the next one's; false shares the code, which keeps fewer registers.  Two paths: Q8_0 planes everywhere (also fewer registers
+// there) and dense products of one matrix, whose waves have few groups each: 4096 x 4096, us, shared / two paths: 5 tokens, Q8_0
+// planes 9.75 / 9.5, Q4_K 9.55 / 8.95, Q6_K 11.15 / 10.45; 16 tokens 11.45 / 10.8, 11.5 / 10.9, 12.95 / 12.25.  Shared: grouped K-quant
+// rows (Q4_K + Q6_K expert block, 128 experts, 20 tokens 94 / 102), passes of 32, GGUF Q8_0 blocks (14336 -> 4096, 12 tokens 31.2 /
+// 32.2) and 16-token passes of MXFP4 (4096 -> 14336, 12 tokens 20.6 / 21.6), which the registers of two paths cost more.
+template <class P, int TV, int EPI>
+constexpr bool mmq_two_tails() {
+    return std::is_same<P, MmqQ8Soa>::value || (EPI == MMQ_STORE && (TV == 4 || (TV == 8 && P::K_ALIGN == 256)));
+}
+// Three workgroups of four waves per CU instead of two where that costs no scratch: a dense launch of 512 to 768 workgroups is then one
+// round (4096 -> 14336, 12 tokens: Q4_K 19.6 -> 16.4 us, Q8_0 planes 23.4 -> 21.6).  Q6_K and MXFP4 would spill.
+template <class P, int TV, int NW, int EPI>
+constexpr int mmq_workgroups_per_cu() {
+    return TV == 8 && NW == 1 && (std::is_same<P, MmqQ8Soa>::value || (EPI == MMQ_STORE && std::is_same<P, MmqQ4K>::value)) ? 3 : 2;
+}
+
 template <class P>
 struct MmqArgs {
     typename P::Bank bank0, bank1;    // NW = 2: gate and up
@@ -918,7 +946,7 @@ __device__ __forceinline__ float mmq_swiglu_oai(float g, float u, float alpha, f
 // partial sums of the current one meet, so a workgroup with several row blocks streams without gaps.
 // LDS: the staged image, then `red` [waves][TV][64] floats where the partial sums of the WK waves (and the NW matrices) meet.
 template <class P, int TV, int NW, int WR, int WK, int EPI>
-__global__ __launch_bounds__(64 * NW * WR * WK, 2) void mmq_kernel(MmqArgs<P> a) {
+__global__ __launch_bounds__(64 * NW * WR * WK, (mmq_workgroups_per_cu<P, TV, NW, EPI>())) void mmq_kernel(MmqArgs<P> a) {
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr uint32_t TT = 2 * TV;   // token rows per pass
     constexpr bool NATIVE = mmq_native<P>::value;
@@ -953,7 +981,7 @@ __global__ __launch_bounds__(64 * NW * WR * WK, 2) void mmq_kernel(MmqArgs<P> a)
         auto hrow = [&](uint32_t t) { return a.act_f16 + (size_t)(t0 + t) * a.K; };
         // token rows past the tile re-read its last row (their results are dropped)
         const uint32_t jt = NATIVE ? (j & 15u) : j, row_a = jt < nt ? jt : nt - 1u;
-        typename std::conditional<NATIVE, MmqWalkNative<P, TV>, MmqWalk<P, TV>>::type walk;
+        typename std::conditional<NATIVE, MmqWalkNative<P, TV>, MmqWalk<P, TV, mmq_two_tails<P, TV, EPI>()>>::type walk;
         MmqAct act{};
         bool staged = false, requested = false;
         // what the epilogue reads from global memory is requested ahead of the weight walk: a load issued in the epilogue

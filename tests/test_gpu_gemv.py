@@ -68,6 +68,23 @@ def test_gemv_q8_batched(mx, fmt, T):
     check(one, ref[0], "row 0 alone")
 
 
+@pytest.mark.parametrize("fmt", (O.Q4_K, O.Q6_K, O.Q8_0, O.MXFP4))
+@pytest.mark.parametrize("T", (5, 12))
+@pytest.mark.parametrize("groups", (1, 2, 4, 6, 7, 11, 15))
+def test_gemv_q8_batched_groups_per_wave(mx, fmt, T, groups):
+    """Rows of a few 256-element groups, dealt to two (T > 8) or four waves: one, two, three and four groups a wave, uneven shares and
+    waves without any, both ends of the weight walk (Q8_0 as planes and as blocks)."""
+    K, N = 256 * groups, 40
+    W = weights(fmt, 320 + fmt, N, K)
+    xq = O.quantize_q8_1(acts(420 + groups, T, K))
+    ref = O.gemv_q8chain(fmt, W, xq, K, N)
+    check(run_q8(mx, fmt, W, xq, K, N, T), ref, "%s T=%d K=%d" % (O.FMT_NAMES[fmt], T, K))
+    if fmt == O.Q8_0:
+        qs, d = O.repack_q8_0_to_soa(W)
+        got = host(mx.ops.gemv_q8_0_soa_q8_batched(dev(xq), dev(qs), dev(d), K, N, T)).astype(np.float32)
+        check(got, ref, "Q8_0 planes T=%d K=%d" % (T, K))
+
+
 @pytest.mark.parametrize("fmt", (O.Q4_K, O.Q6_K, O.Q8_0))
 def test_gemv_q8_multi_tile_K(mx, fmt):
     """K large enough that the activation is staged in several LDS tiles (T=8, K=14336)."""
