@@ -71,9 +71,10 @@ __global__ __launch_bounds__(kNormThreads) void norm_q8_kernel(const XT* x, cons
 // y = half(silu(gate) * up) (swiglu, src/ops/elementwise.cpp:449-467) or, OAI = true, the clamped
 // gpt-oss form x = min(gate, limit), z = clamp(up, -limit, limit), y = half(x * sigmoid(alpha x) * (z + 1))
 // (swiglu_oai, :469-492), written as fp16 (when y != NULL) and as the block_q8_1x stream of the rounded
-// values: the down projection's int-dot input without a quantize launch.  Thread = 4 elements.
-// E = 8 elements per thread where gate, up and y lie on 16-byte boundaries, else 4: 58.7 M elements 87.2 -> 77.3 us
-// (5.4 TB/s, memory-bound), 7.3 M 12.8 -> 11.4 us; below 1 M elements the launch is all there is.
+// values: the down projection's int-dot input without a quantize launch.
+// E = 8 elements per thread, from kActWideFrom elements on and where gate, up and y lie on 16-byte boundaries: 58.7 M elements 87.2 ->
+// 77.3 us (5.4 TB/s, memory-bound), 7.3 M 12.8 -> 11.4 us, 524288 2.5 -> 2.4 us; fewer leave too few waves: 229376 2.12 -> 2.24 us.
+constexpr uint64_t kActWideFrom = 524288;
 template <bool OAI, int E>
 __global__ __launch_bounds__(256) void act_q8_kernel(const half_t* gate, const half_t* up, half_t* y, uint8_t* q8, uint64_t n, float alpha, float limit) {
     typedef _Float16 vec_t __attribute__((ext_vector_type(E)));
@@ -113,7 +114,7 @@ static int act_q8(mx_stream_t s, const uint16_t* gate, const uint16_t* up, uint1
     const half_t *g = reinterpret_cast<const half_t*>(gate), *u = reinterpret_cast<const half_t*>(up);
     half_t* yh = reinterpret_cast<half_t*>(y);
     uint8_t* q = static_cast<uint8_t*>(q8_out);
-    if (aligned(gate, 16) && aligned(up, 16) && aligned(y, 16))
+    if (n >= kActWideFrom && aligned(gate, 16) && aligned(up, 16) && aligned(y, 16))
         hipLaunchKernelGGL((act_q8_kernel<OAI, 8>), dim3((uint32_t)((n / 8 + 255) / 256)), dim3(256), 0, as_stream(s), g, u, yh, q, n, alpha, limit);
     else
         hipLaunchKernelGGL((act_q8_kernel<OAI, 4>), dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, as_stream(s), g, u, yh, q, n, alpha, limit);

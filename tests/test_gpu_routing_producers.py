@@ -255,9 +255,9 @@ def test_swiglu_q8(mx, n, oai):
     assert torch.equal(q8_only, q8)
 
 
-@pytest.mark.parametrize("n", [32, 64, 1024, 2048 + 96, 32 * 1001])
+@pytest.mark.parametrize("n", [32, 64, 1024, 2048 + 96, 32 * 1001, 524288 - 32, 524288, 524288 + 96])
 def test_q8_producers_on_8_and_16_byte_boundaries(mx, n):
-    """Eight elements per thread on 16-byte boundaries, four on 8-byte ones: the same fp16 values and q8 bytes (both evaluate one
+    """Eight elements per thread on 16-byte boundaries (SwiGLU: from 524288 elements on), four on 8-byte ones: the same fp16 values and q8 bytes (both evaluate one
     element alike), at sizes that end inside a workgroup, against the quantizer of the oracle; halves, a signed zero and an infinity among them."""
     g, u = f16(O.normal(9600 + n, (n + 4,), 0.0, 3.0)), f16(O.normal(9601 + n, (n + 4,)))
     g[5:12] = [127.0, 0.5, -0.5, 2.5, -2.5, 1.5, -0.0]
