@@ -486,6 +486,51 @@ def test_moe_grouped_kquant_int_dot(mx, T, E, Kt, H, EF):
         check(host(op).astype(np.float32), o_ref, "grouped down packed %s int-dot (q8_1s rows)" % fmt)
 
 
+@pytest.mark.parametrize("avg,K,N_gate,N_down", [(5, 1024, 2090, 2090), (12, 1024, 2090, 2090), (24, 512, 2090, 4170)])
+def test_moe_grouped_int_dot_streams_row_blocks(mx, avg, K, N_gate, N_down):
+    """So many row blocks that a workgroup takes several of them against one staged image (128 experts, more than 4096
+    workgroups otherwise), for passes of 8, 16 and 32 rows: ragged last row blocks, empty experts, experts of several passes.  The experts'
+    matrices are overlapping windows of one, expert e starting at row e, so that they differ and stay cheap to encode."""
+    ops = mx.ops
+    E = 128
+    rng = np.random.default_rng(avg)
+    counts = rng.multinomial(avg * E - 90, np.random.default_rng(1).permutation(1.0 / np.arange(1, E + 1) ** 0.5) / np.sum(1.0 / np.arange(1, E + 1) ** 0.5))
+    counts[rng.permutation(E)[:12]] = 0
+    counts[7] = 70
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    TK = int(off[-1])
+    assert (TK + E - 1) // E <= avg <= 32 and counts.max() > 32 and counts.min() == 0
+    x = f16(O.normal(8650 + avg, (TK, K)))
+    xq = ops.quantize_q8_1s(dev(x).half())
+    rows_s, rows_x = host(xq).reshape(TK, -1), O.quantize_q8_1(x).reshape(TK, -1)   # the same codes; Q4_0's oracle and MXFP4 read the 40-byte layout
+
+    def reference(F, W, N):
+        y = np.empty((TK, N), np.float64)
+        chain, rows = (O.gemv_q8chain, rows_x) if F in (O.Q4_0, O.MXFP4) else (O.gemv_q8schain, rows_s)
+        for e in range(E):
+            if counts[e]:
+                y[off[e]:off[e + 1]] = chain(F, W[e:e + N], rows[off[e]:off[e + 1]], K, N)
+        return y
+
+    for fmt, F in (("q4k", O.Q4_K), ("q6k", O.Q6_K)):
+        bank = lambda seed, N: O.quantize(F, O.normal(seed, (N + E, K), 0.0, 0.02))  # noqa: E731
+        Wg, Wu, Wd = bank(8660, N_gate), bank(8661, N_gate), bank(8662, N_down)
+        stride = Wg[0].size
+        hp = ops.moe_prefill_gate_up_silu_kquant_q8(fmt, xq, dev(Wg), dev(Wu), dev(off), TK, E, K, N_gate, stride)
+        check(host(hp).astype(np.float32), O.swiglu_np(reference(F, Wg, N_gate).astype(np.float32), reference(F, Wu, N_gate).astype(np.float32)),
+              "gate_up %s, %d rows an expert" % (fmt, avg))
+        out = ops.moe_prefill_down_packed_kquant_q8(fmt, xq, dev(Wd), dev(off), TK, E, N_down, K, stride)
+        check(host(out).astype(np.float32), reference(F, Wd, N_down), "down %s, %d rows an expert" % (fmt, avg))
+    W = O.quantize(O.Q4_0, O.normal(8663, (N_down + E, K), 0.0, 0.02))
+    out = ops.moe_prefill_proj_q4_0("q8", xq, dev(W), dev(off), TK, E, K, N_down, W[0].size)
+    check(host(out).astype(np.float32), reference(O.Q4_0, W, N_down), "proj q4_0, %d rows an expert" % avg)
+    W = O.quantize(O.MXFP4, O.normal(8664, (N_down + E, K), 0.0, 0.02))
+    qs, e8 = O.repack_mxfp4_to_soa(W)
+    bias = torch.zeros((E, N_down), device="cuda")
+    out = ops.moe_grouped_down_mxfp4(dev(rows_x.ravel()), dev(qs), dev(e8), K // 2, K // 32, bias, dev(off), TK, E, N_down, K)
+    check(host(out).astype(np.float32), reference(O.MXFP4, W, N_down), "down mxfp4, %d rows an expert" % avg)
+
+
 @pytest.mark.parametrize("n_tok,hidden", [(7, 2048), (5, 100), (1, 8)])
 def test_moe_scatter_add_bit_exact(mx, n_tok, hidden):
     """moe_scatter_add (src/ops/moe.cpp:284-313): y[idx[i]] = half(float(y[idx[i]]) + float(x[i]) * w[i]).
