@@ -215,7 +215,9 @@ __global__ __launch_bounds__(256) void topk_kernel(const LogitT* logits, int32_t
         if ((taken[j] >> lane) & 1ull) {
             const uint32_t at = below + (uint32_t)__builtin_popcountll(taken[j] & ((1ull << lane) - 1ull));
             topk_idx[(size_t)t * K + at] = (int32_t)(lane + 64u * j);
-            topk_w[(size_t)t * K + at] = (half_t)(p[j] * inv);
+            float w = p[j] * inv;
+            asm volatile("" : "+v"(w));   // an fp32 value first: the compiler would round the product to fp16 at once
+            topk_w[(size_t)t * K + at] = (half_t)w;
         }
         below += (uint32_t)__builtin_popcountll(taken[j]);
     }

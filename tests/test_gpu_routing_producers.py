@@ -60,6 +60,19 @@ def test_moe_router_nan_payload_keeps_ids_in_range(mx):
     assert host(idx).tolist() == [[4, 5, 6, 7]] * 2
 
 
+def test_moe_topk_weights_are_rounded_twice(mx):
+    """p * (1 / sum) is an fp32 value before it is an fp16 one: tokens whose fp32 product lies on the midpoint of
+    two halves while the unrounded product does not, so that one rounding would give the other half.  Bits pinned from the kernel that
+    kept the weights in fp32 in LDS."""
+    rows = [(0xB92C, 0x3B64, 0xB834, 0xBC45, 0x40A1, 0x377F), (0x3C55, 0xC098, 0x3FC0, 0xC2F2, 0x34D8, 0xC4B5), (0x411D, 0xBD95, 0x3773, 0x31CB, 0xC097, 0xC17E),
+            (0xA993, 0xBCF1, 0x3FF5, 0xC16A, 0xB558, 0xB86D), (0xBB45, 0x30CA, 0xC2C2, 0x3D73, 0xBE2E, 0xBBCA), (0x3D46, 0xC0CA, 0xBACC, 0x3E00, 0xB9FC, 0x4037)]
+    ids = [(1, 4, 5), (0, 2, 4), (0, 2, 3), (0, 2, 4), (0, 1, 3), (0, 3, 5)]
+    bits = [(0x31AA, 0x39B0, 0x2F2F), (0x3434, 0x38F0, 0x2FB4), (0x3A94, 0x2E80, 0x2CE4), (0x2ED2, 0x3A82, 0x2D1A), (0x2CB7, 0x32CC, 0x39B6), (0x3346, 0x345C, 0x3800)]
+    idx, w = mx.ops.moe_topk_from_logits(dev(np.array(rows, np.uint16).view(np.float16)), 3)
+    assert host(idx).tolist() == [list(r) for r in ids]
+    assert host(w).view(np.uint16).tolist() == [list(r) for r in bits]
+
+
 @pytest.mark.parametrize("T,E,K", [(1, 32, 4), (64, 8, 2), (300, 128, 8), (2048, 128, 8)])
 def test_moe_packing_device_equals_host(mx, T, E, K):
     rng = np.random.default_rng(T + E)
