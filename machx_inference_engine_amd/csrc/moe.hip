@@ -499,8 +499,8 @@ static int launch_mmq_grouped_cfg(hipStream_t st, const typename P::Bank& b0, co
     // its one image; otherwise one workgroup per row block.  How many in all: experts differ in size and some are empty, so a
     // launch of just the two workgroups per CU that launch_bounds asks for leaves CUs idle behind the large experts, and small
     // images let more than two reside.  Whole expert block over q8 rows, 2 / 4 / 8 / 16 / 64 per CU: Q4_K + Q6_K, 128 experts, k = 8,
-    // hidden 2048: 64 tokens 338 / 242 / 198 / 176 / 172 us, 128 tokens 621 / 389 / 306 / 252 / 242, 333 tokens 411 / 359 / 332 / 331 / 333;
-    // Q8_0 the same to 1 %.  The native MXFP4 image is twice as large per row and dearer to build: four per CU, but never fewer than
+    // hidden 2048: 64 tokens 334 / 236 / 195 / 172 / 169 us, 128 tokens 620 / 390 / 305 / 250 / 242, 333 tokens 405 / 361 / 328 / 326 / 325;
+    // The native MXFP4 image is twice as large per row and dearer to build: four per CU, but never fewer than
     // 32 for one expert, so that the largest is spread (2 / 4 / 8 / 16 per CU: 32 experts, k = 4, hidden 2880, 32 tokens 207 / 157 / 164 / 176
     // us, 16 experts of 4096 x 2048, 128 tokens 145 / 139 / 147 / 147; 64 experts of 2048 x 2048, 128 tokens 365 / 299 / 247 / 247; 128 experts
     // of 2048 x 768, k = 8, 128 tokens 558 / 381 / 305 / 265).
