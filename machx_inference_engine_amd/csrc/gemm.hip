@@ -8,9 +8,10 @@
 // weight matrix: every weight byte is read once per 128-token tile and
 // dequantized in registers straight into MFMA operand fragments.
 //
-// Tiling (wave64, v_mfma_f32_32x32x16_f16):
-//   workgroup = 4 waves, 128 tokens x (4 x 64) weight rows, K walked in chunks of 128;
-//   wave      = 128 tokens x 64 rows = 4 x 2 MFMA tiles (128 accumulator VGPRs);
+// Tiling (wave64, v_mfma_f32_32x32x16_f16), K walked in chunks of 128:
+//   workgroup = 4 waves, 128 tokens x (4 x 64) weight rows, two per CU; wave = 128 tokens x 64 rows = 4 x 2 MFMA tiles
+//               (128 accumulator VGPRs).  Dense launches that would not fill the chip so: 8 waves, one workgroup per CU, the
+//               two halves of K (or of a K slice) side by side, 32 .. 128 tokens x 128 or 256 weight rows (gemm_plan);
 //   tokens    : the fp16 A chunk [128 x 128] is staged in LDS (double buffered, unpadded
 //               256-byte rows whose 16-byte columns are XOR-swizzled by the row number, so a
 //               fragment read is bank-conflict free) and shared by the four waves;
@@ -36,7 +37,7 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kBK = 128;            // K chunk
-constexpr int kWaveN = 64;          // weight rows per wave (2 MFMA tiles)
+constexpr int kWaveN = 64;          // weight rows per wave of a grouped or four-wave tile (2 MFMA tiles)
 constexpr int kGemmThreads = 256;
 // One A chunk in LDS: BM rows x 256 B, unpadded, 16-byte columns XOR-swizzled by row.
 
@@ -679,12 +680,24 @@ int gemm_init_device() {
     return scratch_address(HIP_SYMBOL(g_gemm_splitk_acc), g_gemm_splitk_addr, &p);
 }
 
-__global__ __launch_bounds__(256) void gemm_splitk_store_kernel(half_t* y, const float* acc, uint32_t n, uint32_t k_split) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// V outputs per thread: four where the planes and y can be addressed that way, else one.
+template <int V>
+__global__ __launch_bounds__(256) void gemm_splitk_store_kernel(half_t* y, const float* acc, uint64_t n, uint32_t k_split) {
+    typedef float fv_t __attribute__((ext_vector_type(V)));
+    typedef half_t hv_t __attribute__((ext_vector_type(V)));
+    const uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (i >= n) return;
-    float v = acc[i];
-    for (uint32_t k = 1; k < k_split; ++k) v += acc[(size_t)k * n + i];
-    y[i] = (half_t)v;
+    fv_t v = *reinterpret_cast<const fv_t*>(acc + i);
+#pragma unroll 4
+    for (uint32_t k = 1; k < k_split; ++k) v += *reinterpret_cast<const fv_t*>(acc + (size_t)k * n + i);
+    *reinterpret_cast<hv_t*>(y + i) = __builtin_convertvector(v, hv_t);
+}
+static int launch_splitk_store(mx_stream_t s, half_t* y, const float* acc, uint64_t n, uint32_t k_split) {
+    if (n % 4 == 0 && aligned(y, 8))
+        hipLaunchKernelGGL(gemm_splitk_store_kernel<4>, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, as_stream(s), y, acc, n, k_split);
+    else
+        hipLaunchKernelGGL(gemm_splitk_store_kernel<1>, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, as_stream(s), y, acc, n, k_split);
+    return launch_status();
 }
 
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -705,82 +718,48 @@ __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_of
 // R * 256 + ((c ^ (R & 15)) << 4): the 16 lanes of a quarter wave then hit 16 different
 // columns, i.e. all 64 banks once.  For step S the column is QF::H_COL * h + QF::step_col(S),
 // so the address is the lane's step-0 address XOR-ed with step_col(S) << 4.
-// `mi` = number of live 32-token tiles of this workgroup tile (4 unless PARTIAL: expert-grouped
-// tiles are often mostly empty, and their dead token tiles skip both the LDS reads and the MFMAs).
-template <int S, class QF, bool PARTIAL, int NI>
-__device__ __forceinline__ void mma_step(const typename QF::Raw (&raw)[2], const typename QF::Dec (&dec)[2], const uint8_t* lds, uint32_t a_frag0,
-                                         float16_t (&acc)[NI][2], uint32_t mi) {
-    Frag af[NI], bf[2];
-    const uint32_t a_s = a_frag0 ^ (QF::step_col(S) << 4);
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-        if (!PARTIAL || (uint32_t)i < mi) af[i].q = *reinterpret_cast<const uint4*>(lds + a_s + i * 8192);
-    QF::template frag<S>(raw[0], dec[0], bf[0]);
-    QF::template frag<S>(raw[1], dec[1], bf[1]);
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-        if (!PARTIAL || (uint32_t)i < mi) {
-            acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i].v, bf[0].v, acc[i][0], 0, 0, 0);
-            acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i].v, bf[1].v, acc[i][1], 0, 0, 0);
-        }
-}
-
-// The chunk as one software pipeline over NI token tiles, all of them multiplied (no branch inside a chunk: a branch
+//
+// The chunk is one software pipeline over NI token tiles, all of them multiplied (no branch inside a chunk: a branch
 // per token tile ends the scheduling region, and each step then runs as LDS read, wait, dequantisation, MFMAs one after
-// the other).  A step is cut into NI segments, one per token tile: its 2 MFMAs, the LDS read that refills that A
-// fragment for step S+1, and 4 / NI of the four half-fragment dequantisations of the weight fragments of step S+1
-// into the other fragment pair.  The scheduling fences between segments keep that interleaving, so neither the VALU
-// work nor the LDS latency ends up between two clusters of MFMAs.
-template <int S, class QF, int NI>
-__device__ __forceinline__ void mma_pipe(const typename QF::Raw (&raw)[2], const typename QF::Dec (&dec)[2], const uint8_t* lds, uint32_t a_frag0,
-                                         float16_t (&acc)[NI][2], Frag (&af)[NI], Frag (&bf)[2][2]) {
-    static_assert(NI == 1 || NI == 2 || NI == 4, "token tiles per pipelined chunk");
+// the other).  A step is cut into NI segments, one per token tile: its NJ MFMAs (one per column tile), the LDS read that
+// refills that A fragment for step S+1, and its share of the 2 NJ half-fragment dequantisations of the weight fragments
+// of step S+1 into the other fragment set.  The scheduling fences between segments keep that interleaving, so neither the
+// VALU work nor the LDS latency ends up between two clusters of MFMAs.
+template <int S, class QF, int NI, int NJ>
+__device__ __forceinline__ void mma_pipe(const typename QF::Raw (&raw)[NJ], const typename QF::Dec (&dec)[NJ], const uint8_t* lds, uint32_t a_frag0,
+                                         float16_t (&acc)[NI][NJ], Frag (&af)[NI], Frag (&bf)[2][NJ]) {
     if constexpr (S < 8) {
         constexpr int cur = S & 1, nxt = cur ^ 1, SN = (S + 1) & 7;
         constexpr bool more = S + 1 < 8;
-        constexpr int per = 4 / NI;   // half fragments dequantized per segment
         const uint32_t a_n = a_frag0 ^ (QF::step_col(SN) << 4);
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i].v, bf[cur][0].v, acc[i][0], 0, 0, 0);
-            acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i].v, bf[cur][1].v, acc[i][1], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i].v, bf[cur][j].v, acc[i][j], 0, 0, 0);
             if (more) {
                 af[i].q = *reinterpret_cast<const uint4*>(lds + a_n + i * 8192);
 #pragma unroll
-                for (int q = i * per; q < (i + 1) * per; ++q) {
-                    if (q == 0) QF::template frag_half<SN, 0>(raw[0], dec[0], bf[nxt][0]);
-                    if (q == 1) QF::template frag_half<SN, 1>(raw[0], dec[0], bf[nxt][0]);
-                    if (q == 2) QF::template frag_half<SN, 0>(raw[1], dec[1], bf[nxt][1]);
-                    if (q == 3) QF::template frag_half<SN, 1>(raw[1], dec[1], bf[nxt][1]);
+                for (int q = 2 * NJ * i / NI; q < 2 * NJ * (i + 1) / NI; ++q) {
+                    if (q & 1) QF::template frag_half<SN, 1>(raw[q >> 1], dec[q >> 1], bf[nxt][q >> 1]);
+                    else QF::template frag_half<SN, 0>(raw[q >> 1], dec[q >> 1], bf[nxt][q >> 1]);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        mma_pipe<S + 1, QF, NI>(raw, dec, lds, a_frag0, acc, af, bf);
+        mma_pipe<S + 1, QF, NI, NJ>(raw, dec, lds, a_frag0, acc, af, bf);
     }
 }
 
-template <class QF, bool PIPE, bool PARTIAL, int NI>
-__device__ __forceinline__ void mma_chunk(const typename QF::Raw (&raw)[2], const typename QF::Dec (&dec)[2], const uint8_t* lds, uint32_t a_frag0,
-                                          float16_t (&acc)[NI][2], uint32_t mi) {
-    if constexpr (PIPE) {
-        Frag af[NI], bf[2][2];
+template <class QF, int NI, int NJ>
+__device__ __forceinline__ void mma_chunk(const typename QF::Raw (&raw)[NJ], const typename QF::Dec (&dec)[NJ], const uint8_t* lds, uint32_t a_frag0,
+                                          float16_t (&acc)[NI][NJ]) {
+    Frag af[NI], bf[2][NJ];
 #pragma unroll
-        for (int i = 0; i < NI; ++i) af[i].q = *reinterpret_cast<const uint4*>(lds + a_frag0 + i * 8192);
-        QF::template frag<0>(raw[0], dec[0], bf[0][0]);
-        QF::template frag<0>(raw[1], dec[1], bf[0][1]);
-        __builtin_amdgcn_sched_barrier(0);   // prologue stays ahead of the pipelined steps
-        mma_pipe<0, QF, NI>(raw, dec, lds, a_frag0, acc, af, bf);
-    } else {
-        mma_step<0, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<1, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<2, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<3, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<4, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<5, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<6, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-        mma_step<7, QF, PARTIAL, NI>(raw, dec, lds, a_frag0, acc, mi);
-    }
+    for (int i = 0; i < NI; ++i) af[i].q = *reinterpret_cast<const uint4*>(lds + a_frag0 + i * 8192);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) QF::template frag<0>(raw[j], dec[j], bf[0][j]);
+    __builtin_amdgcn_sched_barrier(0);   // prologue stays ahead of the pipelined steps
+    mma_pipe<0, QF, NI, NJ>(raw, dec, lds, a_frag0, acc, af, bf);
 }
 
 // vmcnt(N) with every other counter left alone
@@ -825,7 +804,7 @@ struct TileCtx {
     const uint8_t* a_glb;
     uint32_t a_dst;
     const uint8_t* lds_raw;
-    uint32_t frag0, n_chunks, mi;
+    uint32_t frag0, n_chunks;
     uint32_t c0;   // first chunk of this K slice (chunk numbers below are slice-local)
     uint32_t tail_chunk;   // row-relative number of the chunk whose upper 64 columns lie past K (0xFFFFFFFF: none)
     uint32_t row_step;     // (BM / 4) * wave, for the A column of a lane
@@ -850,29 +829,33 @@ __device__ __forceinline__ void a_rows_to_lds(const TileCtx<QF, NA>& t, const ui
     }
 }
 
+// The weight words of chunk `kc` of the lane's NJ weight rows.
+template <class QF, int NA, int NJ>
+__device__ __forceinline__ void load_weights(const TileCtx<QF, NA>& t, uint32_t kc, typename QF::Raw (&raw)[NJ]) {
+    raw[0] = QF::load(t.w0, t.wrow0, kc, t.h);
+    if constexpr (NJ == 2) raw[1] = QF::load(t.w1, t.wrow1, kc, t.h);
+}
+
 // Chunk c out of register set P; meanwhile (`more`) the A rows of chunk c+1 and the weights of chunk c+DEPTH are requested.
 // TAIL = one of the last chunks of the K loop, where chunk c+DEPTH may lie past the end: then no weight loads are issued
 // (loads nobody reads may be dropped by the compiler, and the wait below counts on them) and the A rows are waited for
 // with vmcnt(0).
-template <class QF, bool PIPE, bool PARTIAL, int NA, int DEPTH, int P, bool TAIL>
-__device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA>& t, const uint32_t (&a_off)[2 * NA], typename QF::Raw (&raw)[DEPTH + 1][2],
-                                           const typename GemmWin<QF>::type (&win)[2], float16_t (&acc)[NA][2], uint32_t c, bool more) {
+template <class QF, int NA, int NJ, int DEPTH, int P, bool TAIL>
+__device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA>& t, const uint32_t (&a_off)[2 * NA], typename QF::Raw (&raw)[DEPTH + 1][NJ],
+                                           const typename GemmWin<QF>::type (&win)[2], float16_t (&acc)[NA][NJ], uint32_t c, bool more) {
     constexpr int NSET = DEPTH + 1, PN = (P + DEPTH) % NSET;
     constexpr uint32_t ABUF = 32u * NA * kBK * 2u;
-    constexpr int W_LOADS_MIN = 2 * (int)((sizeof(typename QF::Raw) + 15) / 16);
+    constexpr int W_LOADS_MIN = NJ * (int)((sizeof(typename QF::Raw) + 15) / 16);
     const bool w_next = !TAIL || c + DEPTH < t.n_chunks;   // the weights of chunk c+DEPTH exist
     if (more) {
         a_rows_to_lds<QF, NA>(t, a_off, c + 1, t.a_dst + ((c + 1) & 1u) * ABUF);
-        if (w_next) {
-            raw[PN][0] = QF::load(t.w0, t.wrow0, t.c0 + c + DEPTH, t.h);
-            raw[PN][1] = QF::load(t.w1, t.wrow1, t.c0 + c + DEPTH, t.h);
-        }
+        if (w_next) load_weights<QF, NA, NJ>(t, t.c0 + c + DEPTH, raw[PN]);
         __builtin_amdgcn_sched_barrier(0);   // the scheduler must not sink these loads towards their uses
     }
-    typename QF::Dec dec[2];
-    dec[0] = gemm_prepare<QF>(raw[P][0], win[0], t.c0 + c, t.h);
-    dec[1] = gemm_prepare<QF>(raw[P][1], win[1], t.c0 + c, t.h);
-    mma_chunk<QF, PIPE, PARTIAL, NA>(raw[P], dec, t.lds_raw, (c & 1u) * ABUF + t.frag0, acc, t.mi);
+    typename QF::Dec dec[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) dec[j] = gemm_prepare<QF>(raw[P][j], win[j], t.c0 + c, t.h);
+    mma_chunk<QF, NA, NJ>(raw[P], dec, t.lds_raw, (c & 1u) * ABUF + t.frag0, acc);
     if (more) {
         // A rows of chunk c+1 are in LDS.  DEPTH > 1: the weight loads issued behind them in this chunk stay in flight
         // (memory returns in order, so at most that many outstanding loads means the A rows have landed).
@@ -885,8 +868,8 @@ __device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA>& t, const uint3
 }
 
 // One output tile: accumulators, A staging, the K loop and the epilogue.  NA = 32-token tiles this instance
-// keeps accumulators for and stages (the tile's live rows fit in 32 NA rows); PIPE = the hand-pipelined chunk
-// (needs NA = 4 and a full tile); DEPTH = how many K chunks ahead the weight words are requested.
+// keeps accumulators for and stages (the tile's live rows fit in 32 NA rows); NJ = 32-row column tiles per wave;
+// DEPTH = how many K chunks ahead the weight words are requested.
 //
 // Software pipeline over K chunks: at the top of chunk c the A rows of chunk c+1 start their way into the
 // other LDS buffer, then the weight words of chunk c+DEPTH into registers.  Memory returns in order, the A
@@ -899,16 +882,17 @@ __device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA>& t, const uint3
 // whatever the compiler made of QF::load.
 // KW = 2: a workgroup of eight waves, waves 4 - 7 walking the second half of K over A buffers of their own (`lds_raw` is
 // then this half's buffer pair, `lds_red` the start of the workgroup's LDS); their sums meet the first half's in LDS
-// before the epilogue.  Both halves run the same number of chunks, so their barriers pair up.
-template <class QF, int MODE, bool PIPE, int NA, int DEPTH, int KW = 1>
+// before the epilogue.  The first half runs `n_chunks_max` chunks, the second as many or one fewer; every chunk ends in one
+// barrier of the workgroup, and a half that is a chunk short adds one, so the barriers pair up.
+template <class QF, int MODE, int NA, int DEPTH, int KW = 1, int NJ = 2>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::W& w0, const typename QF::W& w1, const uint32_t (&wrow)[2],
                                           uint32_t row_lo, uint32_t row_hi, uint32_t n_base, uint8_t* lds_raw, uint32_t c0 = 0,
-                                          uint32_t n_chunks_slice = 0, uint32_t ks = 0, uint32_t e = 0, uint8_t* lds_red = nullptr) {
+                                          uint32_t n_chunks_slice = 0, uint32_t ks = 0, uint32_t e = 0, uint8_t* lds_red = nullptr,
+                                          uint32_t n_chunks_max = 0) {
     static_assert(DEPTH == 1 || DEPTH == 2, "prefetch depth");
-    static_assert(KW == 1 || (KW == 2 && MODE == GEMM_DENSE && NA == 4), "K halves inside a workgroup: dense full tiles only");
-    static_assert(!PIPE || NA == 1 || NA == 2 || NA == 4, "the pipelined chunk is written for one, two or four token tiles");
+    static_assert(KW == 1 || (KW == 2 && MODE == GEMM_DENSE), "K halves inside a workgroup: dense launches only");
     constexpr bool GATE_UP = MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI;
-    constexpr bool PARTIAL = MODE != GEMM_DENSE && !PIPE;
+    static_assert(NJ == 2 || (NJ == 1 && MODE == GEMM_DENSE), "gate and up are the two column tiles of a wave");
     constexpr uint32_t BM = 32u * NA;
     constexpr int NL = 2 * NA;   // 1 KB loads per wave per chunk
     const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 31u, h = lane >> 5;
@@ -916,7 +900,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
     const uint32_t n_all = (g.K + kBK - 1) / kBK;                             // a row that ends half way through its last chunk counts it
     const uint32_t n_chunks = n_chunks_slice ? n_chunks_slice : n_all;       // chunks of this K slice (all of K unless split)
     const uint32_t live_rows = (row_hi - row_lo) >= BM ? BM : row_hi - row_lo;
-    const uint32_t mi = (live_rows + 31u) / 32u;
 
     // A staging: wave w brings rows (BM/4) w .. of the chunk, 4 rows (1 KB) per load; lane L fills LDS slot
     // (row 4j + L/16, column L%16) of that 1 KB with global column (L%16) ^ (row & 15).  Rows past the end of
@@ -949,23 +932,23 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
         if (g.y_acc) rows.token = (uint32_t)g.row_token[row];
     }
 
-    float16_t acc[NA][2];
+    float16_t acc[NA][NJ];
 #pragma unroll
     for (int i = 0; i < NA; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
     // Weight words of DEPTH + 1 chunks live in registers: chunk c sits in set c % (DEPTH + 1).  The loop is unrolled
     // over the sets so that no set is ever copied into another (a register copy of loaded data waits for the load).
     constexpr int NSET = DEPTH + 1;
-    typename QF::Raw raw[NSET][2];
-    const TileCtx<QF, NA> ctx{w0, w1, wrow[0], wrow[1], h, a_glb, a_dst, lds_raw, frag0, n_chunks, mi, c0,
+    typename QF::Raw raw[NSET][NJ];
+    const TileCtx<QF, NA> ctx{w0, w1, wrow[0], wrow[1], h, a_glb, a_dst, lds_raw, frag0, n_chunks, c0,
                               (g.K % kBK) ? n_all - 1u : 0xFFFFFFFFu, (BM / 4u) * wave};
     a_rows_to_lds<QF, NA>(ctx, a_off, 0, a_dst);
-    raw[0][0] = QF::load(w0, wrow[0], c0, h);
-    raw[0][1] = QF::load(w1, wrow[1], c0, h);
+    __builtin_amdgcn_sched_barrier(0);   // the wait below counts the weight loads behind the A rows
+    load_weights<QF, NA, NJ>(ctx, c0, raw[0]);
     typename GemmWin<QF>::type win[2];
     if constexpr (GemmWin<QF>::on) {
         // The scale table behind the A buffers: thread t copies table row t = 64 wave' + 32 tile + r', the scales of the
@@ -1006,22 +989,34 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
         win[0].row = lds_base + ABUF2 + (wave * 64u + r) * pitch;
         win[1].row = lds_base + ABUF2 + (wave * 64u + 32u + r) * pitch;
     }
-    wait_vmcnt<0>();
-    __syncthreads();
+    if constexpr (KW == 2) {
+        // few chunks per wave: everything its first chunks need is requested in one go, and the wait is for the A rows only
+        constexpr int W_LOADS_MIN = DEPTH * NJ * (int)((sizeof(typename QF::Raw) + 15) / 16);
 #pragma unroll
-    for (int d = 1; d < DEPTH; ++d) {
-        const uint32_t cd = (uint32_t)d < n_chunks ? (uint32_t)d : n_chunks - 1;
-        raw[d][0] = QF::load(w0, wrow[0], c0 + cd, h);
-        raw[d][1] = QF::load(w1, wrow[1], c0 + cd, h);
+        for (int d = 1; d < DEPTH; ++d) {
+            const uint32_t cd = (uint32_t)d < n_chunks ? (uint32_t)d : n_chunks - 1;
+            load_weights<QF, NA, NJ>(ctx, c0 + cd, raw[d]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<W_LOADS_MIN>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    } else {
+        wait_vmcnt<0>();
+        __syncthreads();
+#pragma unroll
+        for (int d = 1; d < DEPTH; ++d) {
+            const uint32_t cd = (uint32_t)d < n_chunks ? (uint32_t)d : n_chunks - 1;
+            load_weights<QF, NA, NJ>(ctx, c0 + cd, raw[d]);
+        }
     }
 
-#define CHUNK(P, c, more, tail) gemm_chunk<QF, PIPE, PARTIAL, NA, DEPTH, P, tail>(ctx, a_off, raw, win, acc, c, more)
+#define CHUNK(P, c, more, tail) gemm_chunk<QF, NA, NJ, DEPTH, P, tail>(ctx, a_off, raw, win, acc, c, more)
     if constexpr (DEPTH == 1) {
         // two sets, and the set just loaded is copied into set 0 at the end of a chunk, where it has to have arrived anyway
         for (uint32_t c = 0; c + 1 < n_chunks; ++c) {
             CHUNK(0, c, true, false);
-            raw[0][0] = raw[1][0];
-            raw[0][1] = raw[1][1];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) raw[0][j] = raw[1][j];
         }
         CHUNK(0, n_chunks - 1, false, true);
     } else {
@@ -1046,26 +1041,27 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
         // halves are done with their A buffers behind the first barrier) and leaves; the first half adds them to its own.
         typedef float f32x4_t __attribute__((ext_vector_type(4)));
         const bool second = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)) != 0u;
-        f32x4_t* red = reinterpret_cast<f32x4_t*>(lds_red) + (size_t)wave * (NA * 2 * 4) * 64u + lane;
+        if (n_chunks < n_chunks_max) asm volatile("s_barrier" ::: "memory");   // one chunk, and so one barrier, fewer than the first half
+        f32x4_t* red = reinterpret_cast<f32x4_t*>(lds_red) + (size_t)wave * (NA * NJ * 4) * 64u + lane;
         __syncthreads();
         if (second) {
 #pragma unroll
             for (int i = 0; i < NA; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < NJ; ++j)
 #pragma unroll
                     for (int v4 = 0; v4 < 4; ++v4)
-                        red[((i * 2 + j) * 4 + v4) * 64] = f32x4_t{acc[i][j][4 * v4], acc[i][j][4 * v4 + 1], acc[i][j][4 * v4 + 2], acc[i][j][4 * v4 + 3]};
+                        red[((i * NJ + j) * 4 + v4) * 64] = f32x4_t{acc[i][j][4 * v4], acc[i][j][4 * v4 + 1], acc[i][j][4 * v4 + 2], acc[i][j][4 * v4 + 3]};
         }
         __syncthreads();
         if (second) return;
 #pragma unroll
         for (int i = 0; i < NA; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int v4 = 0; v4 < 4; ++v4) {
-                    const f32x4_t t = red[((i * 2 + j) * 4 + v4) * 64];
+                    const f32x4_t t = red[((i * NJ + j) * 4 + v4) * 64];
                     acc[i][j][4 * v4] += t.x;
                     acc[i][j][4 * v4 + 1] += t.y;
                     acc[i][j][4 * v4 + 2] += t.z;
@@ -1123,7 +1119,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
                     const uint32_t row = 32u * i + 8u * (v / 4) + (v % 4);
                     const float w = MODE == GEMM_MOE_DOWN ? row_w[row + lane_row] : 1.f;
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         float o = acc[i][j][v];
                         if constexpr (MODE == GEMM_MOE_DOWN) {
                             o *= w;
@@ -1268,14 +1264,18 @@ __device__ __forceinline__ bool find_grouped_tile(const uint32_t* expert_offsets
     return found;
 }
 
-// NI = 32-token tiles per workgroup tile: 4 (128 tokens, two workgroups per CU), or 2 (64 tokens,
-// three per CU) for dense launches whose 128-token tiles would leave CUs without work.
-template <class QF, int MODE, int NI, int KW = 1>
-__global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : NI == 2 ? 3 : 2) void gemm_kernel(typename QF::Bank bank0, typename QF::Bank bank1, GemmArgs g) {
+// Chunks of weight words in flight per wave of an eight-wave workgroup: as many as the registers beside 32 NA accumulators hold.
+template <int NA, int NJ>
+constexpr int gemm_k2_depth() { return NA * NJ <= 4 ? 2 : 1; }
+
+// NI = 32-token tiles per workgroup tile.  KW = 1: four waves, 128 tokens, two workgroups per CU.  KW = 2: eight waves, the two
+// halves of the K slice side by side, one workgroup per CU, 32 to 128 tokens.
+template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
+__global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kernel(typename QF::Bank bank0, typename QF::Bank bank1, GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
     constexpr uint32_t BM = 32u * NI;   // tokens per tile
     constexpr bool GATE_UP = MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI;
-    constexpr uint32_t BN = GATE_UP ? 4 * 32 : 4 * kWaveN;   // output columns per workgroup
+    constexpr uint32_t BN = GATE_UP ? 4 * 32 : 4 * 32 * NJ;   // output columns per workgroup
 
     // ---- which tile: XCD-aware order (workgroup i runs on XCD i % 8; each XCD walks a
     // contiguous range of tiles, 4 token tiles x consecutive column tiles at a time)
@@ -1325,7 +1325,7 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : NI == 2 ? 3 : 2) v
 
     const uint32_t tid = threadIdx.x, r = tid & 31u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((tid >> 6) & 3u));
-    const uint32_t n_base = tn * BN + wave * (GATE_UP ? 32 : kWaveN);
+    const uint32_t n_base = tn * BN + wave * (BN / 4u);
     // weight rows of the two MFMA column tiles of this wave (gate/up: same row in two matrices)
     uint32_t wrow[2];
     wrow[0] = n_base + r;
@@ -1334,14 +1334,16 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : NI == 2 ? 3 : 2) v
     if (wrow[1] >= g.N) wrow[1] = g.N - 1;
 
     if constexpr (MODE == GEMM_DENSE) {
-        const uint32_t n_all = (g.K + kBK - 1) / kBK, per = (n_all + ksplit - 1) / ksplit;
-        const uint32_t c0 = ks * per, c1 = (c0 + per < n_all) ? c0 + per : n_all;
+        // K slices differ by at most one chunk
+        const uint32_t n_all = (g.K + kBK - 1) / kBK, per = n_all / ksplit, longer = n_all % ksplit;
+        const uint32_t c0 = ks * per + (ks < longer ? ks : longer), n_slice = per + (ks < longer ? 1u : 0u);
         if constexpr (KW == 2) {
-            // the launcher takes this form for an even number of chunks and no K slices across workgroups
-            const uint32_t kw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)), half = n_all / 2u;
-            gemm_tile<QF, MODE, true, 4, 1, 2>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw + kw * (2u * BM * kBK * 2u), kw * half, half, 0, 0, lds_raw);
+            // the launcher takes this form for slices of at least two chunks
+            const uint32_t kw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)), first = (n_slice + 1u) / 2u;
+            gemm_tile<QF, MODE, NI, gemm_k2_depth<NI, NJ>(), 2, NJ>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw + kw * (2u * BM * kBK * 2u), c0 + kw * first,
+                                                                      kw ? n_slice - first : first, ks, 0, lds_raw, first);
         } else {
-            gemm_tile<QF, MODE, NI == 4, NI, 1>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw, c0, c1 - c0, ks);
+            gemm_tile<QF, MODE, NI, 1>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw, c0, n_slice, ks);
         }
     } else {
         (void)ks;
@@ -1358,7 +1360,7 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : NI == 2 ? 3 : 2) v
             table2 = need <= room - 2u * 64u * kBK * 2u;
             table1 = need <= room - 2u * 32u * kBK * 2u;
         }
-#define MX_TILE(Q, na, depth) gemm_tile<Q, MODE, true, na, depth>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw, 0, 0, 0, e)
+#define MX_TILE(Q, na, depth) gemm_tile<Q, MODE, na, depth>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw, 0, 0, 0, e)
         if (live > 64u) {
             if (table4) MX_TILE(QL, 4, 1);
             else MX_TILE(QF, 4, 1);
@@ -1374,9 +1376,9 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : NI == 2 ? 3 : 2) v
 }
 
 // ---------------------------------------------------------------- host side
-template <class QF, int MODE, int NI, int KW = 1>
+template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
 static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound) {
-    constexpr uint32_t BN = (MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI) ? 128 : 256, BM = 32u * NI;
+    constexpr uint32_t BN = (MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI) ? 128 : 128 * NJ, BM = 32u * NI;
     constexpr uint32_t lds = KW * 2u * BM * kBK * 2u + ((MODE != GEMM_DENSE && GemmLdsScales<QF>::on) ? kGemmLdsScaleBytes : 0u);
     g.tiles_n = (g.N + BN - 1) / BN;
     g.tiles_m = (MODE == GEMM_DENSE) ? (g.M + BM - 1) / BM : rows_bound / BM + g.E;   // grouped: an upper bound, workgroups past the real count leave at once
@@ -1386,9 +1388,9 @@ static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const type
     if (grid > 0x7FFFFFFFull) return MX_ERR_SHAPE;
     if constexpr (lds > kLdsDefaultLimit) {
         static LdsLimit limit;
-        if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&gemm_kernel<QF, MODE, NI, KW>), limit, lds)) return rc;
+        if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&gemm_kernel<QF, MODE, NI, KW, NJ>), limit, lds)) return rc;
     }
-    hipLaunchKernelGGL((gemm_kernel<QF, MODE, NI, KW>), dim3((uint32_t)grid), dim3(kGemmThreads * KW), lds, as_stream(s), b0, b1, g);
+    hipLaunchKernelGGL((gemm_kernel<QF, MODE, NI, KW, NJ>), dim3((uint32_t)grid), dim3(kGemmThreads * KW), lds, as_stream(s), b0, b1, g);
     return launch_status();
 }
 
@@ -1401,62 +1403,74 @@ static int gemm_cu_count() {
     return n;
 }
 
-// Dense launches whose 128-token tiles cover at most half of the CUs take 64-token tiles instead
-// (twice the workgroups; measured: 64 tiles -> +20 %, 224 tiles -> -9 %); everything else runs
-// 128-token tiles.
+// How a dense launch is cut.  Two forms: eight-wave workgroups that walk the two halves of their K slice, one per CU, over tiles
+// of 32 na tokens x 128 nj weight rows (na = 1 .. 4, nj = 1, 2; KW = 2 of the kernel), and four-wave workgroups, two per CU, over
+// tiles of 128 x 256.  The second is the better one where there are tiles enough to fill the chip several times; below that the
+// chip is filled by small tiles and by K slices, each of which has its price: a narrow tile reads the activation rows more often,
+// a short one dequantizes the same weights for fewer tokens, a slice writes fp32 partial sums that a second launch adds.  The
+// form with the least modelled time is taken.  The model is microseconds, fitted to 468 measured shapes (Q4_K, Q6_K, Q8_0 planes,
+// K and N 2048 .. 14336, M 17 .. 4096, cold weights) with one set of constants for all formats; the plans it takes are 0.4 % slower
+// than the best plan of each shape on average, 13 % at worst but for one shape.  Where it moves launches from the rule before
+// (128-token tiles, K slices of four-wave workgroups until the CUs are covered), us with the partial-sum launch:
+// Q4_K 4096 -> 14336: 20 tokens 31 -> 17.7, 77 tokens 32 -> 25.7, 200 tokens 58 -> 41; Q6_K 14336 -> 4096: 77 tokens 52 -> 34.5.
+struct GemmPlan {
+    uint32_t na;        // 32-token tiles per workgroup tile, 0: the four-wave form
+    uint32_t nj;        // 32-row column tiles per wave
+    uint32_t k_split;
+};
+static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus) {
+    const uint64_t n_chunks = (K + kBK - 1) / kBK;
+    auto up = [](uint64_t a, uint64_t b) { return (a + b - 1) / b; };
+    GemmPlan best{0, 2, 1};
+    const uint64_t tiles4 = up(M, 128) * up(N, 256), full = tiles4 / (2 * cus), rest = tiles4 % (2 * cus);
+    // a round of two workgroups per CU, and a last one that may have one per CU
+    double t_best = (double)(full + (rest > cus ? 1 : 0)) * (5.0 + 3.74 * (double)n_chunks) + (rest && rest <= cus ? 5.0 + 2.37 * (double)n_chunks : 0.0);
+    if (n_chunks < 2) return best;
+    for (uint64_t na = 1; na <= 4 && na <= up(M, 32); ++na)
+        for (uint64_t nj = 1; nj <= 2; ++nj) {
+            const uint64_t tiles = up(M, 32 * na) * up(N, 128 * nj);
+            for (uint64_t k = 1; k <= kGemmSplitMax && 2 * k <= n_chunks && (k == 1 || k * M * N <= cap); ++k) {
+                const double per_wave = (double)up(up(n_chunks, k), 2), chunk = (1.35 + 0.23 * (double)na) * (double)nj + 0.04 * (double)na;
+                const double slices = k > 1 ? 5.5 + 1.4e-6 * (double)(k * M * N) : 0.0;
+                const double t = (double)up(tiles * k, cus) * (2.2 + per_wave * chunk) + slices;
+                if (t < t_best) {
+                    t_best = t;
+                    best = GemmPlan{(uint32_t)na, (uint32_t)nj, (uint32_t)k};
+                }
+            }
+        }
+    return best;
+}
+
 template <class QF, int MODE>
 static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound,
                        const SplitWs* caller_ws = nullptr) {
     if constexpr (MODE == GEMM_DENSE) {
-        const uint64_t cus = (uint64_t)gemm_cu_count();
-        const uint64_t tiles128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 255) / 256);
-        const uint64_t tiles64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 255) / 256);
-        const uint64_t mn = (uint64_t)g.M * g.N, n_chunks = (g.K + kBK - 1) / kBK;
-        const uint64_t cap = caller_ws ? caller_ws->elems : kGemmSplitElems;   // partial sums the scratch holds
-        // K slices a tiling could take: until every CU has a workgroup, each slice at least 8 chunks deep, the partial
-        // sums within the scratch
-        auto slices = [&](uint64_t tiles) {
-            uint64_t k = tiles ? cus / tiles : 1;
-            if (k > kGemmSplitMax) k = kGemmSplitMax;
-            if (k > n_chunks / 8) k = n_chunks / 8;
-            if (k * mn > cap) k = cap / mn;
-            return k < 1 ? (uint64_t)1 : k;
-        };
-        bool ni2 = false;
-        uint64_t k_split = 1;
-        if (2 * tiles128 <= cus) {
-            // 128-token tiles would leave half the CUs idle.  They stay (they do twice the matrix work per dequantized
-            // weight) when K slices alone fill three quarters of the chip; otherwise 64-token tiles, sliced as well.
-            // Measured at K = 14336, N = 4096: T = 128 94 -> 39 us, T = 512 162 -> 111 us.
-            const uint64_t k4 = slices(tiles128);
-            if (4 * tiles128 * k4 >= 3 * cus || g.M <= 64) {
-                k_split = k4;
-            } else {
-                ni2 = true;
-                k_split = slices(tiles64);
-            }
-        }
-        if (2 * tiles128 > cus && tiles128 <= cus && n_chunks % 2 == 0 && n_chunks >= 16) {
-            // One workgroup per CU would leave every SIMD with a single wave: eight-wave workgroups instead, each half of
-            // the waves walking half of K (no scratch, no second launch).  T = 512, K = 4096, N = 14336: 224 tiles.
-            return launch_gemm_ni<QF, MODE, 4, 2>(s, b0, b1, g, rows_bound);
-        }
-        if (k_split >= 2) {
-            const uint32_t per = (uint32_t)((n_chunks + k_split - 1) / k_split);
-            g.k_split = (uint32_t)((n_chunks + per - 1) / per);   // no empty slice
+        const GemmPlan p = gemm_plan(g.M, g.K, g.N, caller_ws ? caller_ws->elems : kGemmSplitElems, (uint64_t)gemm_cu_count());
+        g.k_split = p.k_split;
+        if (p.k_split > 1) {
             if (caller_ws) {
                 g.split_acc = caller_ws->ptr;
             } else {
-                void* p = nullptr;
-                if (int rc = scratch_address(HIP_SYMBOL(g_gemm_splitk_acc), g_gemm_splitk_addr, &p)) return rc;
-                g.split_acc = static_cast<float*>(p);
+                void* q = nullptr;
+                if (int rc = scratch_address(HIP_SYMBOL(g_gemm_splitk_acc), g_gemm_splitk_addr, &q)) return rc;
+                g.split_acc = static_cast<float*>(q);
             }
-            const int rc = ni2 ? launch_gemm_ni<QF, MODE, 2>(s, b0, b1, g, rows_bound) : launch_gemm_ni<QF, MODE, 4>(s, b0, b1, g, rows_bound);
-            if (rc != MX_OK) return rc;
-            hipLaunchKernelGGL(gemm_splitk_store_kernel, dim3((uint32_t)((mn + 255) / 256)), dim3(256), 0, as_stream(s), g.Y, g.split_acc, (uint32_t)mn, g.k_split);
-            return launch_status();
         }
-        if (ni2) return launch_gemm_ni<QF, MODE, 2>(s, b0, b1, g, rows_bound);
+        int rc;
+        switch (p.na * 2 + p.nj - 1) {
+            case 2: rc = launch_gemm_ni<QF, MODE, 1, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 3: rc = launch_gemm_ni<QF, MODE, 1, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 4: rc = launch_gemm_ni<QF, MODE, 2, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 5: rc = launch_gemm_ni<QF, MODE, 2, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 6: rc = launch_gemm_ni<QF, MODE, 3, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 7: rc = launch_gemm_ni<QF, MODE, 3, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 8: rc = launch_gemm_ni<QF, MODE, 4, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 9: rc = launch_gemm_ni<QF, MODE, 4, 2, 2>(s, b0, b1, g, rows_bound); break;
+            default: rc = launch_gemm_ni<QF, MODE, 4>(s, b0, b1, g, rows_bound);
+        }
+        if (rc != MX_OK || p.k_split < 2) return rc;
+        return launch_splitk_store(s, g.Y, g.split_acc, (uint64_t)g.M * g.N, g.k_split);
     }
     return launch_gemm_ni<QF, MODE, 4>(s, b0, b1, g, rows_bound);
 }
@@ -1551,9 +1565,8 @@ int mx_gemm_q8_0_soa(mx_stream_t s, const uint16_t* A, const int8_t* qs_W, const
 int mx_gemm_ws_bytes(uint32_t M, uint32_t K, uint32_t N, uint64_t* bytes) {
     MX_REQUIRE_PTR(bytes);
     MX_REQUIRE_SHAPE(M > 0 && K > 0 && N > 0);
-    // K is sliced only when the 128-token tiles cover at most half of the CUs; then up to kGemmSplitMax planes of M x N floats
-    const uint64_t tiles128 = (uint64_t)((M + 127) / 128) * ((N + 255) / 256);
-    *bytes = (2 * tiles128 <= (uint64_t)gemm_cu_count() && K / kBK >= 16) ? (uint64_t)kGemmSplitMax * M * N * sizeof(float) : 0;
+    // kGemmSplitMax planes of M x N floats wherever an unlimited workspace would be used
+    *bytes = gemm_plan(M, K, N, ~0ull, (uint64_t)gemm_cu_count()).k_split > 1 ? (uint64_t)kGemmSplitMax * M * N * sizeof(float) : 0;
     return MX_OK;
 }
 int mx_gemm_q4_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {

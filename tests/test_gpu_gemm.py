@@ -48,6 +48,35 @@ def test_gemm_k_slices(mx, fmt, M, K, N):
         assert torch.equal(fn(a_d, w_d, M, K, N), got), "K-sliced GEMM differs from launch to launch"
 
 
+@pytest.mark.parametrize("fmt,M,K,N", [
+    ("q8_0", 1, 128, 33), ("q8_0", 1, 384, 200), ("q8_0", 17, 2176, 201), ("q8_0", 260, 384, 3899), ("q8_0", 199, 3712, 611),
+    ("q8_0", 257, 384, 6776), ("q8_0", 260, 2176, 1433), ("q8_0", 200, 384, 10886), ("q8_0", 193, 3712, 1844), ("q8_0", 260, 384, 10886),
+    ("q8_0", 257, 384, 13352), ("q8_0", 259, 3712, 3899), ("q8_0", 200, 3712, 5543), ("q4_K", 31, 7424, 257), ("q6_K", 95, 5376, 130),
+    ("mxfp4", 40, 2880, 160), ("mxfp4", 127, 320, 1100)])
+def test_gemm_plans(mx, fmt, M, K, N):
+    """One shape per form a dense launch can take (32 .. 128 tokens x 128 or 256 weight rows, with and without K slices, four-wave
+    workgroups), at odd numbers of chunks, so that slices and the two K halves of a workgroup differ in length, ragged M and N, one
+    row, one chunk and a row that ends half way through a chunk.  Against the fp32-weight product in fp64: the sum of K exact fp16
+    products in fp32, rounded to fp16, as every other case here."""
+    from machx_inference_engine_amd import synth
+
+    ofmt = {"q8_0": O.Q8_0, "q4_K": O.Q4_K, "q6_K": O.Q6_K, "mxfp4": O.MXFP4}[fmt]
+    w = synth.normal_weights(fmt, N, K, 77 + M, device="cuda")
+    A = f16(O.normal(2301 + M, (M, K)))
+    W16 = torch.from_numpy(O.dequant(ofmt, host(w).reshape(-1), N * K).reshape(N, K)).half().double()
+    ref = (torch.from_numpy(A).double() @ W16.t()).numpy()
+    a = dev(A).half()
+    if fmt == "q8_0":
+        run = lambda: mx.ops.gemm_q8_0_soa(a, *synth.split_q8_0(w), M, K, N)  # noqa: E731
+    elif fmt == "mxfp4":
+        run = lambda: mx.ops.gemm_mxfp4_soa(a, *synth.split_mxfp4(w), M, K, N)  # noqa: E731
+    else:
+        run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, w.reshape(-1), M, K, N)  # noqa: E731
+    got = run()
+    check(host(got).astype(np.float32), ref, "gemm %s M=%d K=%d N=%d" % (fmt, M, K, N))
+    assert torch.equal(run(), got), "differs from launch to launch"
+
+
 @pytest.mark.parametrize("M,K,N", [(128, 128, 256), (260, 768, 2048), (77, 2048, 768)])
 def test_gemm_q8_0_soa(mx, M, K, N):
     W = weights(O.Q8_0, 2100 + N, N, K)
