@@ -54,13 +54,15 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 // fp16 (v_cvt_pk_f16_f32).  The power-of-two rescale of `scale` is exact, so the value is
 // bit-identical to converting the code to float first.  Left to itself the compiler fuses
 // convert + fma + convert into v_fma_mixlo/mixhi_f16, which measures about half the rate of the
-// other VALU ops next to MFMA work on this chip; spelling the pack as an instruction keeps the two
-// halves apart.
+// other VALU ops next to MFMA work on this chip; the two fp32 values are made opaque to keep the
+// halves apart.  The pack itself stays the compiler's: a matrix instruction must not read a vector
+// result for two wait states, and only an instruction it knows gets them (the pack written as
+// inline asm gave wrong fragments wherever it came last before its matrix instruction and wrote
+// the first register of the operand).
 __device__ __forceinline__ uint32_t mix_pair(_Float16 x0, _Float16 x1, float scale, float off) {
-    const float f0 = __builtin_fmaf((float)x0, scale, off), f1 = __builtin_fmaf((float)x1, scale, off);
-    uint32_t r;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(f0), "v"(f1));
-    return r;
+    float f0 = __builtin_fmaf((float)x0, scale, off), f1 = __builtin_fmaf((float)x1, scale, off);
+    asm("" : "+v"(f0), "+v"(f1));
+    return pack_h2(f0, f1);
 }
 __device__ __forceinline__ half2_t as_h2(uint32_t u) { return __builtin_bit_cast(half2_t, u); }
 
