@@ -86,6 +86,63 @@ union Frag {
     uint4 q;
 };
 
+// ---------------------------------------------------------------- weight rows in whole lines
+// An MFMA operand wants one weight row per lane, and a load instruction whose 64 lanes read 64 rows takes the vector memory
+// pipeline (one cache line looked up at a time) about 64 cycles, four times what it takes for the same bytes as whole lines:
+// in launches of 4096 tokens the address unit was busy 64 % (Q4_K) to 79 % (Q8_0 planes) of the time, the matrix pipe 58 % and 51 %.
+// So two (Q4_K, MXFP4: 32 bytes of a row per lane half) or four neighbouring lanes (Q8_0 planes: 64 bytes) read 16-byte pieces
+// of ONE row per instruction, two or four instructions for two or four rows, and exchange the pieces in registers:
+//   exchange_pieces<1>(a, b): in the even lane of a pair (a, b) = its (piece 0, the neighbour's piece 0) -> its pieces 0 and 1
+// (four pieces: <1> on (0, 1), (2, 3), then <2> on (0, 2), (1, 3)).  Every dword is one v_cndmask with a DPP operand; the masks
+// are lane constants.  All 64 lanes are active wherever this is called.
+template <int X>
+__device__ __forceinline__ void exchange_pieces(uint4& a, uint4& b) {
+    static_assert(X == 1 || X == 2, "lane distance inside a quad");
+    uint4 m, n;
+    // two wait states between a vector write and a DPP read of it
+#define MX_EXCHANGE(lanes, perm)                                                                    \
+    asm("s_nop 1\n\ts_mov_b32 vcc_lo, " lanes "\n\ts_mov_b32 vcc_hi, " lanes "\n\t"                \
+        "v_cndmask_b32_dpp %0, %12, %8, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"      \
+        "v_cndmask_b32_dpp %1, %13, %9, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"      \
+        "v_cndmask_b32_dpp %2, %14, %10, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"     \
+        "v_cndmask_b32_dpp %3, %15, %11, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"     \
+        "s_not_b64 vcc, vcc\n\t"                                                                   \
+        "v_cndmask_b32_dpp %4, %8, %12, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"      \
+        "v_cndmask_b32_dpp %5, %9, %13, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"      \
+        "v_cndmask_b32_dpp %6, %10, %14, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf\n\t"     \
+        "v_cndmask_b32_dpp %7, %11, %15, vcc quad_perm:" perm " row_mask:0xf bank_mask:0xf"          \
+        : "=&v"(m.x), "=&v"(m.y), "=&v"(m.z), "=&v"(m.w), "=&v"(n.x), "=&v"(n.y), "=&v"(n.z), "=&v"(n.w) \
+        : "v"(a.x), "v"(a.y), "v"(a.z), "v"(a.w), "v"(b.x), "v"(b.y), "v"(b.z), "v"(b.w)              \
+        : "vcc", "scc")
+    if constexpr (X == 1) MX_EXCHANGE("0x55555555", "[1,0,3,2]");
+    else MX_EXCHANGE("0x33333333", "[2,3,0,1]");
+#undef MX_EXCHANGE
+    a = m;
+    b = n;
+}
+// (a, b) with lane halves (aL aU), (bL bU) -> (aL bL), (aU bU)
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+// one value per half -> the lower half's in every lane, the upper half's in every lane
+__device__ __forceinline__ void spread_halves(uint32_t v, uint32_t& lower, uint32_t& upper) {
+    lower = v;
+    upper = v;
+    swap_halves(lower, upper);
+}
+// Byte offset of row i (0 .. G - 1) of the lane's group of G rows, counted from row `first`: rows past N are row N - 1.
+template <uint32_t G>
+__device__ __forceinline__ uint32_t group_row_offset(uint32_t n_tile, uint32_t first, uint32_t i, uint32_t N, uint32_t row_bytes) {
+    const uint32_t n = n_tile + (threadIdx.x & 31u & ~(G - 1u)) + i;
+    return ((n < N ? n : N - 1u) - first) * row_bytes;
+}
+__device__ __forceinline__ uint32_t lane_row(uint32_t n_tile, uint32_t N) {
+    const uint32_t n = n_tile + (threadIdx.x & 31u);
+    return n < N ? n : N - 1u;
+}
+
 // ---------------------------------------------------------------- weight fragment producers
 // Q4_K: chunk kc of a row = half c = kc%2 of block kc/2; lane half h owns the 32 bytes
 // qs[32g, 32g+32), g = 2c + h: low nibbles = sub-block 2g, high = sub-block 2g+1.
@@ -148,6 +205,58 @@ struct GemmQ4K {
     __device__ static __forceinline__ void frag(const Raw& r, const Dec& dc, Frag& f) {
         frag_half<S, 0>(r, dc, f);
         frag_half<S, 1>(r, dc, f);
+    }
+};
+
+// The same blocks, two lanes to a row per load, and the block headers of a wave's two column tiles in one instruction, the
+// lower half those of the first tile (6 loads of 64 rows -> 4 of 32 row pieces and 1).  A wave with one column tile loads as
+// GemmQ4K does: there the exchange costs what it saves (prefill of 20 tokens, Q4_K_M 4096/14336: 62.5 us, 63.6 with it).
+// Block of 4096 tokens 1571 -> 1555 us, of 700 (3072/8192) 173.5 -> 171.3; expert block of 2048 tokens, 128 experts 380 -> 368.
+struct GemmQ4KPair : GemmQ4K {
+    struct Lane {
+        const uint8_t* base;   // uniform: row `first` of the tile
+        uint32_t off[2];
+        const uint8_t* hdr;
+    };
+    template <int NJ>
+    static constexpr int loads = NJ == 2 ? 5 : 3;
+    template <int NJ>
+    __device__ static __forceinline__ void lanes(const W& w0, const W& w1, const uint32_t (&n_tile)[2], uint32_t N, uint32_t h, Lane (&L)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const W& w = j ? w1 : w0;
+            const uint32_t first = n_tile[j] < N ? n_tile[j] : N - 1u;
+            L[j].base = w.base + (size_t)first * w.row_bytes;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                L[j].off[i] = (NJ == 2 ? group_row_offset<2>(n_tile[j], first, (uint32_t)i, N, w.row_bytes) + 16u * (threadIdx.x & 1u)
+                                       : (lane_row(n_tile[j], N) - first) * w.row_bytes + 16u * i) + 16u + 32u * h;
+        }
+        const bool second = NJ == 2 && h;
+        L[0].hdr = (second ? w1.base : w0.base) + (size_t)lane_row(second ? n_tile[1] : n_tile[0], N) * w0.row_bytes;
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void load(const Lane (&L)[NJ], uint32_t kc, uint32_t, Raw (&r)[NJ]) {
+        const size_t blk = (size_t)(kc >> 1) * kQ4KBytes;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint8_t* p = L[j].base + blk + 64u * (kc & 1u);
+            r[j].q0 = *reinterpret_cast<const uint4*>(p + L[j].off[0]);
+            r[j].q1 = *reinterpret_cast<const uint4*>(p + L[j].off[1]);
+        }
+        r[0].hdr = *reinterpret_cast<const uint4*>(L[0].hdr + blk);
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void settle(Raw (&r)[NJ]) {
+        if constexpr (NJ == 2) {
+            exchange_pieces<1>(r[0].q0, r[0].q1);
+            exchange_pieces<1>(r[1].q0, r[1].q1);
+            const uint4 v = r[0].hdr;
+            spread_halves(v.x, r[0].hdr.x, r[1].hdr.x);
+            spread_halves(v.y, r[0].hdr.y, r[1].hdr.y);
+            spread_halves(v.z, r[0].hdr.z, r[1].hdr.z);
+            spread_halves(v.w, r[0].hdr.w, r[1].hdr.w);
+        }
     }
 };
 
@@ -233,6 +342,61 @@ struct GemmQ8SoaLds : GemmQ8Soa {
     __device__ static __forceinline__ Dec prepare(const Raw&, const Win& wn, uint32_t kc, uint32_t h) {
         typedef __attribute__((address_space(3))) const uint32_t lds_u32_t;
         return dec_of(*reinterpret_cast<lds_u32_t*>((uintptr_t)(wn.row + kc * 8u + 4u * h)));
+    }
+};
+
+// The planes with four lanes to a row per load (whole 64-byte pieces), and the four scales of a chunk for both column tiles of
+// a wave in one instruction (10 loads of 64 rows -> 8 of 16 row pieces and 1).  Prefill, 4096/14336: 300 tokens 204 -> 188 us,
+// 512 tokens 244 -> 236 (251 -> 249 on another day).  Expert-grouped tiles do not gain (scale table in LDS, more registers: 356 -> 365 us
+// for 2048 tokens and 128 experts) and keep GemmQ8Soa.
+struct GemmQ8Quad : GemmQ8Soa {
+    struct Lane {
+        const uint8_t* base;   // uniform: row `first` of the tile
+        uint32_t off[4];
+        const uint8_t* d;
+    };
+    template <int NJ>
+    static constexpr int loads = 4 * NJ + 1;
+    template <int NJ>
+    __device__ static __forceinline__ void lanes(const W& w0, const W& w1, const uint32_t (&n_tile)[2], uint32_t N, uint32_t h, Lane (&L)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const W& w = j ? w1 : w0;
+            const uint32_t first = n_tile[j] < N ? n_tile[j] : N - 1u;
+            L[j].base = reinterpret_cast<const uint8_t*>(w.qs) + (size_t)first * w.K;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) L[j].off[i] = group_row_offset<4>(n_tile[j], first, (uint32_t)i, N, w.K) + 64u * h + 16u * (threadIdx.x & 3u);
+        }
+        const bool second = NJ == 2 && h;
+        L[0].d = reinterpret_cast<const uint8_t*>((second ? w1.d : w0.d) + (size_t)lane_row(second ? n_tile[1] : n_tile[0], N) * (w0.K >> 5)) + (NJ == 2 ? 0u : 4u * h);
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void load(const Lane (&L)[NJ], uint32_t kc, uint32_t, Raw (&r)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint8_t* p = L[j].base + (size_t)kc * 128u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[j].q[i] = *reinterpret_cast<const uint4*>(p + L[j].off[i]);
+        }
+        const uint8_t* d = L[0].d + (size_t)kc * 8u;
+        if constexpr (NJ == 2) {
+            const uint2 v = load_u2_a2(d);
+            r[0].d2 = v.x;
+            r[1].d2 = v.y;
+        } else {
+            r[0].d2 = *reinterpret_cast<const uint32_t*>(d);
+        }
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void settle(Raw (&r)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            exchange_pieces<1>(r[j].q[0], r[j].q[1]);
+            exchange_pieces<1>(r[j].q[2], r[j].q[3]);
+            exchange_pieces<2>(r[j].q[0], r[j].q[2]);
+            exchange_pieces<2>(r[j].q[1], r[j].q[3]);
+        }
+        if constexpr (NJ == 2) swap_halves(r[0].d2, r[1].d2);   // (d01 of tile 0 | of tile 1), (d23 | d23) -> a tile's (d01 | d23)
     }
 };
 
@@ -557,8 +721,8 @@ struct GemmMxfp4Soa {
         o.o[1] = -128.f * s1;
         return o;
     }
-    template <int S, int HF>
-    __device__ static __forceinline__ void frag_half(const Raw& r, const Dec& dc, Frag& f) {
+    template <int S, int HF, class RawT>
+    __device__ static __forceinline__ void frag_half(const RawT& r, const Dec& dc, Frag& f) {
         constexpr int blk = S / 4, j = 2 * (S % 2) + HF, hi = (S % 4) / 2;   // word j of the block, nibble half
         const uint32_t w = j == 0 ? r.q[blk].x : j == 1 ? r.q[blk].y : j == 2 ? r.q[blk].z : r.q[blk].w;
         const uint32_t nib = hi ? w >> 4 : w;
@@ -568,10 +732,60 @@ struct GemmMxfp4Soa {
         f.u[2 * HF] = mix_pair(w01.x, w01.y, d, o);
         f.u[2 * HF + 1] = mix_pair(w23.x, w23.y, d, o);
     }
-    template <int S>
-    __device__ static __forceinline__ void frag(const Raw& r, const Dec& dc, Frag& f) {
+    template <int S, class RawT>
+    __device__ static __forceinline__ void frag(const RawT& r, const Dec& dc, Frag& f) {
         frag_half<S, 0>(r, dc, f);
         frag_half<S, 1>(r, dc, f);
+    }
+};
+
+// The planes with two lanes to a row per load, and the two exponents of a lane in one.  Expert block of 64 tokens, 32 experts,
+// 2880: 225 -> 209 us, of 1000 tokens 440 -> 417.
+struct GemmMxfp4Pair : GemmMxfp4Soa {
+    struct Raw {
+        uint4 q[2];
+        uint32_t e01, live;
+    };
+    struct Lane {
+        const uint8_t* base;   // uniform: row `first` of the tile
+        uint32_t off[2], K;
+        const uint8_t* e;
+    };
+    template <int NJ>
+    static constexpr int loads = 3 * NJ;
+    template <int NJ>
+    __device__ static __forceinline__ void lanes(const W& w0, const W& w1, const uint32_t (&n_tile)[2], uint32_t N, uint32_t h, Lane (&L)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const W& w = j ? w1 : w0;
+            const uint32_t first = n_tile[j] < N ? n_tile[j] : N - 1u;
+            L[j].base = w.qs + (size_t)first * (w.K >> 1);
+            L[j].K = w.K;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) L[j].off[i] = group_row_offset<2>(n_tile[j], first, (uint32_t)i, N, w.K >> 1) + 32u * h + 16u * (threadIdx.x & 1u);
+            L[j].e = w.e + (size_t)lane_row(n_tile[j], N) * (w.K >> 5) + 2u * h;
+        }
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void load(const Lane (&L)[NJ], uint32_t kc, uint32_t h, Raw (&r)[NJ]) {
+        struct __attribute__((packed, aligned(1))) U16 { uint16_t v; };
+        const uint32_t dead = 128u * kc + 64u * h < L[0].K ? 0u : 1u;   // the upper half of a chunk that ends half way: the lower half's bytes, scale 0
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint8_t* p = L[j].base + (size_t)kc * 64u;
+            r[j].q[0] = *reinterpret_cast<const uint4*>(p + (L[j].off[0] - 32u * dead));
+            r[j].q[1] = *reinterpret_cast<const uint4*>(p + (L[j].off[1] - 32u * dead));
+            r[j].e01 = reinterpret_cast<const U16*>(L[j].e + (size_t)kc * 4u - 2u * dead)->v;
+            r[j].live = 1u - dead;
+        }
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void settle(Raw (&r)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) exchange_pieces<1>(r[j].q[0], r[j].q[1]);
+    }
+    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t kc, uint32_t h) {
+        return GemmMxfp4Soa::prepare(GemmMxfp4Soa::Raw{{}, r.e01 & 0xFFu, r.e01 >> 8, r.live}, kc, h);
     }
 };
 
@@ -799,10 +1013,40 @@ struct GemmLdsScales<QF, std::void_t<typename QF::LdsScales>> {
 };
 constexpr uint32_t kGemmLdsScaleBytes = 16u * 1024u;   // LDS beyond the A buffers of a full tile, for launches of such formats
 
-template <class QF, int NA>
+// What a lane needs to load the weight words of its column tiles: a row of each, or what a producer with loads of its own
+// (`Lane`: whole lines, exchanged by settle() once they have arrived) keeps.
+template <class QF, class = void>
+struct GemmLanes {
+    struct type {
+        typename QF::W w;
+        uint32_t n;
+    };
+    static constexpr bool own = false;
+    template <int NJ>
+    static constexpr int loads = NJ * (int)((sizeof(typename QF::Raw) + 15) / 16);
+    template <int NJ>
+    __device__ static __forceinline__ void lanes(const typename QF::W& w0, const typename QF::W& w1, const uint32_t (&n_tile)[2], uint32_t N, uint32_t, type (&L)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) L[j] = type{j ? w1 : w0, lane_row(n_tile[j], N)};
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void load(const type (&L)[NJ], uint32_t kc, uint32_t h, typename QF::Raw (&r)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) r[j] = QF::load(L[j].w, L[j].n, kc, h);
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void settle(typename QF::Raw (&)[NJ]) {}
+};
+template <class QF>
+struct GemmLanes<QF, std::void_t<typename QF::Lane>> : QF {
+    using type = typename QF::Lane;
+    static constexpr bool own = true;
+};
+
+template <class QF, int NA, int NJ>
 struct TileCtx {
-    typename QF::W w0, w1;
-    uint32_t wrow0, wrow1, h;
+    typename GemmLanes<QF>::type lanes[NJ];
+    uint32_t h;
     const uint8_t* a_glb;
     uint32_t a_dst;
     const uint8_t* lds_raw;
@@ -815,8 +1059,8 @@ struct TileCtx {
 // The A rows of chunk `c` (slice-local) into the LDS buffer at `dst`.  In a chunk that ends half way (K % 128 = 64) a lane
 // whose column lies past K reads the column 8 below instead (the same row, inside K): the weights of those columns are
 // zero, so any finite value will do, and nothing is read past the row.
-template <class QF, int NA>
-__device__ __forceinline__ void a_rows_to_lds(const TileCtx<QF, NA>& t, const uint32_t (&a_off)[2 * NA], uint32_t c, uint32_t dst) {
+template <class QF, int NA, int NJ>
+__device__ __forceinline__ void a_rows_to_lds(const TileCtx<QF, NA, NJ>& t, const uint32_t (&a_off)[2 * NA], uint32_t c, uint32_t dst) {
     const uint8_t* src = t.a_glb + (size_t)c * (kBK * 2u);
     if (QF::K_ALIGN == 64 && t.c0 + c == t.tail_chunk) {
         const uint32_t lane = threadIdx.x & 63u;
@@ -831,29 +1075,23 @@ __device__ __forceinline__ void a_rows_to_lds(const TileCtx<QF, NA>& t, const ui
     }
 }
 
-// The weight words of chunk `kc` of the lane's NJ weight rows.
-template <class QF, int NA, int NJ>
-__device__ __forceinline__ void load_weights(const TileCtx<QF, NA>& t, uint32_t kc, typename QF::Raw (&raw)[NJ]) {
-    raw[0] = QF::load(t.w0, t.wrow0, kc, t.h);
-    if constexpr (NJ == 2) raw[1] = QF::load(t.w1, t.wrow1, kc, t.h);
-}
-
 // Chunk c out of register set P; meanwhile (`more`) the A rows of chunk c+1 and the weights of chunk c+DEPTH are requested.
 // TAIL = one of the last chunks of the K loop, where chunk c+DEPTH may lie past the end: then no weight loads are issued
 // (loads nobody reads may be dropped by the compiler, and the wait below counts on them) and the A rows are waited for
 // with vmcnt(0).
 template <class QF, int NA, int NJ, int DEPTH, int P, bool TAIL>
-__device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA>& t, const uint32_t (&a_off)[2 * NA], typename QF::Raw (&raw)[DEPTH + 1][NJ],
+__device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA, NJ>& t, const uint32_t (&a_off)[2 * NA], typename QF::Raw (&raw)[DEPTH + 1][NJ],
                                            const typename GemmWin<QF>::type (&win)[2], float16_t (&acc)[NA][NJ], uint32_t c, bool more) {
     constexpr int NSET = DEPTH + 1, PN = (P + DEPTH) % NSET;
     constexpr uint32_t ABUF = 32u * NA * kBK * 2u;
-    constexpr int W_LOADS_MIN = NJ * (int)((sizeof(typename QF::Raw) + 15) / 16);
+    constexpr int W_LOADS_MIN = GemmLanes<QF>::template loads<NJ>;
     const bool w_next = !TAIL || c + DEPTH < t.n_chunks;   // the weights of chunk c+DEPTH exist
     if (more) {
-        a_rows_to_lds<QF, NA>(t, a_off, c + 1, t.a_dst + ((c + 1) & 1u) * ABUF);
-        if (w_next) load_weights<QF, NA, NJ>(t, t.c0 + c + DEPTH, raw[PN]);
+        a_rows_to_lds<QF, NA, NJ>(t, a_off, c + 1, t.a_dst + ((c + 1) & 1u) * ABUF);
+        if (w_next) GemmLanes<QF>::template load<NJ>(t.lanes, t.c0 + c + DEPTH, t.h, raw[PN]);
         __builtin_amdgcn_sched_barrier(0);   // the scheduler must not sink these loads towards their uses
     }
+    if constexpr (DEPTH > 1) GemmLanes<QF>::template settle<NJ>(raw[P]);
     typename QF::Dec dec[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) dec[j] = gemm_prepare<QF>(raw[P][j], win[j], t.c0 + c, t.h);
@@ -887,9 +1125,8 @@ __device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA>& t, const uint3
 // before the epilogue.  The first half runs `n_chunks_max` chunks, the second as many or one fewer; every chunk ends in one
 // barrier of the workgroup, and a half that is a chunk short adds one, so the barriers pair up.
 template <class QF, int MODE, int NA, int DEPTH, int KW = 1, int NJ = 2>
-__device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::W& w0, const typename QF::W& w1, const uint32_t (&wrow)[2],
-                                          uint32_t row_lo, uint32_t row_hi, uint32_t n_base, uint8_t* lds_raw, uint32_t c0 = 0,
-                                          uint32_t n_chunks_slice = 0, uint32_t ks = 0, uint32_t e = 0, uint8_t* lds_red = nullptr,
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::W& w0, const typename QF::W& w1, uint32_t row_lo, uint32_t row_hi,
+                                          uint32_t n_base, uint8_t* lds_raw, uint32_t c0 = 0, uint32_t n_chunks_slice = 0, uint32_t ks = 0, uint32_t e = 0, uint8_t* lds_red = nullptr,
                                           uint32_t n_chunks_max = 0) {
     static_assert(DEPTH == 1 || DEPTH == 2, "prefetch depth");
     static_assert(KW == 1 || (KW == 2 && MODE == GEMM_DENSE), "K halves inside a workgroup: dense launches only");
@@ -946,11 +1183,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
     // over the sets so that no set is ever copied into another (a register copy of loaded data waits for the load).
     constexpr int NSET = DEPTH + 1;
     typename QF::Raw raw[NSET][NJ];
-    const TileCtx<QF, NA> ctx{w0, w1, wrow[0], wrow[1], h, a_glb, a_dst, lds_raw, frag0, n_chunks, c0,
+    TileCtx<QF, NA, NJ> ctx{{}, h, a_glb, a_dst, lds_raw, frag0, n_chunks, c0,
                               (g.K % kBK) ? n_all - 1u : 0xFFFFFFFFu, (BM / 4u) * wave};
-    a_rows_to_lds<QF, NA>(ctx, a_off, 0, a_dst);
+    a_rows_to_lds<QF, NA, NJ>(ctx, a_off, 0, a_dst);
+    const uint32_t n_tile[2] = {n_base, GATE_UP ? n_base : n_base + 32u};
+    GemmLanes<QF>::template lanes<NJ>(w0, w1, n_tile, g.N, h, ctx.lanes);
     __builtin_amdgcn_sched_barrier(0);   // the wait below counts the weight loads behind the A rows
-    load_weights<QF, NA, NJ>(ctx, c0, raw[0]);
+    GemmLanes<QF>::template load<NJ>(ctx.lanes, c0, h, raw[0]);
     typename GemmWin<QF>::type win[2];
     if constexpr (GemmWin<QF>::on) {
         // The scale table behind the A buffers: thread t copies table row t = 64 wave' + 32 tile + r', the scales of the
@@ -993,11 +1232,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
     }
     if constexpr (KW == 2) {
         // few chunks per wave: everything its first chunks need is requested in one go, and the wait is for the A rows only
-        constexpr int W_LOADS_MIN = DEPTH * NJ * (int)((sizeof(typename QF::Raw) + 15) / 16);
+        constexpr int W_LOADS_MIN = DEPTH * GemmLanes<QF>::template loads<NJ>;
 #pragma unroll
         for (int d = 1; d < DEPTH; ++d) {
             const uint32_t cd = (uint32_t)d < n_chunks ? (uint32_t)d : n_chunks - 1;
-            load_weights<QF, NA, NJ>(ctx, c0 + cd, raw[d]);
+            GemmLanes<QF>::template load<NJ>(ctx.lanes, c0 + cd, h, raw[d]);
         }
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<W_LOADS_MIN>();
@@ -1008,17 +1247,19 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
 #pragma unroll
         for (int d = 1; d < DEPTH; ++d) {
             const uint32_t cd = (uint32_t)d < n_chunks ? (uint32_t)d : n_chunks - 1;
-            load_weights<QF, NA, NJ>(ctx, c0 + cd, raw[d]);
+            GemmLanes<QF>::template load<NJ>(ctx.lanes, c0 + cd, h, raw[d]);
         }
     }
 
 #define CHUNK(P, c, more, tail) gemm_chunk<QF, NA, NJ, DEPTH, P, tail>(ctx, a_off, raw, win, acc, c, more)
     if constexpr (DEPTH == 1) {
-        // two sets, and the set just loaded is copied into set 0 at the end of a chunk, where it has to have arrived anyway
+        // two sets, and the set just loaded is moved into set 0 at the end of a chunk, where it has to have arrived anyway
+        GemmLanes<QF>::template settle<NJ>(raw[0]);
         for (uint32_t c = 0; c + 1 < n_chunks; ++c) {
             CHUNK(0, c, true, false);
 #pragma unroll
             for (int j = 0; j < NJ; ++j) raw[0][j] = raw[1][j];
+            GemmLanes<QF>::template settle<NJ>(raw[0]);
         }
         CHUNK(0, n_chunks - 1, false, true);
     } else {
@@ -1325,15 +1566,9 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kerne
     }
     const typename QF::W w0 = QF::expert(bank0, e), w1 = QF::expert(GATE_UP ? bank1 : bank0, e);
 
-    const uint32_t tid = threadIdx.x, r = tid & 31u;
+    const uint32_t tid = threadIdx.x;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((tid >> 6) & 3u));
     const uint32_t n_base = tn * BN + wave * (BN / 4u);
-    // weight rows of the two MFMA column tiles of this wave (gate/up: same row in two matrices)
-    uint32_t wrow[2];
-    wrow[0] = n_base + r;
-    wrow[1] = GATE_UP ? n_base + r : n_base + 32 + r;
-    if (wrow[0] >= g.N) wrow[0] = g.N - 1;
-    if (wrow[1] >= g.N) wrow[1] = g.N - 1;
 
     if constexpr (MODE == GEMM_DENSE) {
         // K slices differ by at most one chunk
@@ -1342,10 +1577,10 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kerne
         if constexpr (KW == 2) {
             // the launcher takes this form for slices of at least two chunks
             const uint32_t kw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)), first = (n_slice + 1u) / 2u;
-            gemm_tile<QF, MODE, NI, gemm_k2_depth<NI, NJ>(), 2, NJ>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw + kw * (2u * BM * kBK * 2u), c0 + kw * first,
+            gemm_tile<QF, MODE, NI, gemm_k2_depth<NI, NJ>(), 2, NJ>(g, w0, w1, row_lo, row_hi, n_base, lds_raw + kw * (2u * BM * kBK * 2u), c0 + kw * first,
                                                                       kw ? n_slice - first : first, ks, 0, lds_raw, first);
         } else {
-            gemm_tile<QF, MODE, NI, 1>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw, c0, n_slice, ks);
+            gemm_tile<QF, MODE, NI, 1>(g, w0, w1, row_lo, row_hi, n_base, lds_raw, c0, n_slice, ks);
         }
     } else {
         (void)ks;
@@ -1362,7 +1597,7 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kerne
             table2 = need <= room - 2u * 64u * kBK * 2u;
             table1 = need <= room - 2u * 32u * kBK * 2u;
         }
-#define MX_TILE(Q, na, depth) gemm_tile<Q, MODE, na, depth>(g, w0, w1, wrow, row_lo, row_hi, n_base, lds_raw, 0, 0, 0, e)
+#define MX_TILE(Q, na, depth) gemm_tile<Q, MODE, na, depth>(g, w0, w1, row_lo, row_hi, n_base, lds_raw, 0, 0, 0, e)
         if (live > 64u) {
             if (table4) MX_TILE(QL, 4, 1);
             else MX_TILE(QF, 4, 1);
@@ -1528,8 +1763,8 @@ static int gemm_dense_q8_soa(mx_stream_t s, const uint16_t* A, const int8_t* qs_
     MX_REQUIRE_ALIGN(d_W, 4);
     GemmArgs g{};
     g.A = reinterpret_cast<const half_t*>(A); g.Y = reinterpret_cast<half_t*>(y); g.M = M; g.K = K; g.N = N; g.E = 1;
-    GemmQ8Soa::Bank b{qs_W, d_W, 0, 0, K};
-    return launch_gemm<GemmQ8Soa, GEMM_DENSE>(s, b, b, g, M, ws);
+    GemmQ8Quad::Bank b{qs_W, d_W, 0, 0, K};
+    return launch_gemm<GemmQ8Quad, GEMM_DENSE>(s, b, b, g, M, ws);
 }
 // A caller's workspace: any size is accepted, the number of K slices adapts to what it holds (none below 2 M N floats).
 static int gemm_ws(void* ws, uint64_t ws_bytes, SplitWs* out) {
@@ -1548,7 +1783,7 @@ using namespace mxq;
 extern "C" {
 
 int mx_gemm_q4_K(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N) {
-    return gemm_dense_aos<GemmQ4K>(s, A, W, y, M, K, N, 256, 16, K / 256 * (uint32_t)kQ4KBytes, nullptr);
+    return gemm_dense_aos<GemmQ4KPair>(s, A, W, y, M, K, N, 256, 16, K / 256 * (uint32_t)kQ4KBytes, nullptr);
 }
 int mx_gemm_q6_K(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N) {
     return gemm_dense_aos<GemmQ6K>(s, A, W, y, M, K, N, 256, 2, K / 256 * (uint32_t)kQ6KBytes, nullptr);
@@ -1574,7 +1809,7 @@ int mx_gemm_ws_bytes(uint32_t M, uint32_t K, uint32_t N, uint64_t* bytes) {
 int mx_gemm_q4_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {
     SplitWs w;
     if (int rc = gemm_ws(ws, ws_bytes, &w)) return rc;
-    return gemm_dense_aos<GemmQ4K>(s, A, W, y, M, K, N, 256, 16, K / 256 * (uint32_t)kQ4KBytes, &w);
+    return gemm_dense_aos<GemmQ4KPair>(s, A, W, y, M, K, N, 256, 16, K / 256 * (uint32_t)kQ4KBytes, &w);
 }
 int mx_gemm_q6_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {
     SplitWs w;
@@ -1647,7 +1882,7 @@ int mx_moe_gemm_gate_up_silu_q4k(mx_stream_t s, const uint16_t* x_packed, const 
     if (soa)
         return moe_gemm_aos<GemmQ4KStr, GEMM_MOE_GATE_UP_SILU>(s, x_packed, gate_W, up_W, expert_stride_bytes, expert_offsets, nullptr, h_packed, E, H, E_ffn,
                                                                total_rows, kQ4KBytes, 16);
-    return moe_gemm_aos<GemmQ4K, GEMM_MOE_GATE_UP_SILU>(s, x_packed, gate_W, up_W, expert_stride_bytes, expert_offsets, nullptr, h_packed, E, H, E_ffn,
+    return moe_gemm_aos<GemmQ4KPair, GEMM_MOE_GATE_UP_SILU>(s, x_packed, gate_W, up_W, expert_stride_bytes, expert_offsets, nullptr, h_packed, E, H, E_ffn,
                                                         total_rows, kQ4KBytes, 16);
 }
 
@@ -1659,7 +1894,7 @@ int mx_moe_gemm_gate_up_silu_q4k_gather(mx_stream_t s, const uint16_t* x, const 
     if (soa)
         return moe_gemm_aos<GemmQ4KStr, GEMM_MOE_GATE_UP_SILU>(s, x, gate_W, up_W, expert_stride_bytes, expert_offsets, nullptr, h_packed, E, H, E_ffn,
                                                                total_rows, kQ4KBytes, 16, nullptr, nullptr, sorted_idx);
-    return moe_gemm_aos<GemmQ4K, GEMM_MOE_GATE_UP_SILU>(s, x, gate_W, up_W, expert_stride_bytes, expert_offsets, nullptr, h_packed, E, H, E_ffn,
+    return moe_gemm_aos<GemmQ4KPair, GEMM_MOE_GATE_UP_SILU>(s, x, gate_W, up_W, expert_stride_bytes, expert_offsets, nullptr, h_packed, E, H, E_ffn,
                                                         total_rows, kQ4KBytes, 16, nullptr, nullptr, sorted_idx);
 }
 
@@ -1668,7 +1903,7 @@ int mx_moe_gemm_down_q4k(mx_stream_t s, const uint16_t* h_packed, const void* do
     if (soa)
         return moe_gemm_aos<GemmQ4KStr, GEMM_MOE_DOWN>(s, h_packed, down_W, down_W, expert_stride_bytes, expert_offsets, sorted_w, out_packed, E, E_ffn, H,
                                                        total_rows, kQ4KBytes, 16);
-    return moe_gemm_aos<GemmQ4K, GEMM_MOE_DOWN>(s, h_packed, down_W, down_W, expert_stride_bytes, expert_offsets, sorted_w, out_packed, E, E_ffn, H,
+    return moe_gemm_aos<GemmQ4KPair, GEMM_MOE_DOWN>(s, h_packed, down_W, down_W, expert_stride_bytes, expert_offsets, sorted_w, out_packed, E, E_ffn, H,
                                                 total_rows, kQ4KBytes, 16);
 }
 
@@ -1691,8 +1926,8 @@ int mx_gemm_mxfp4_soa(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, con
     MX_REQUIRE_PTR(e_W);
     GemmArgs g{};
     g.A = reinterpret_cast<const half_t*>(A); g.Y = reinterpret_cast<half_t*>(y); g.M = M; g.K = K; g.N = N; g.E = 1;
-    GemmMxfp4Soa::Bank b{qs_W, e_W, 0, 0, K};
-    return launch_gemm<GemmMxfp4Soa, GEMM_DENSE>(s, b, b, g, M, nullptr);
+    GemmMxfp4Pair::Bank b{qs_W, e_W, 0, 0, K};
+    return launch_gemm<GemmMxfp4Pair, GEMM_DENSE>(s, b, b, g, M, nullptr);
 }
 static int moe_gemm_gate_up_oai_mxfp4(mx_stream_t s, const uint16_t* x_packed, const int32_t* sorted_idx, uint32_t n_tokens, const uint8_t* g_qs,
                                       const uint8_t* g_e, const uint8_t* u_qs, const uint8_t* u_e, uint64_t qs_stride, uint64_t e_stride,
@@ -1725,8 +1960,8 @@ static int moe_gemm_gate_up_oai_mxfp4(mx_stream_t s, const uint16_t* x_packed, c
     g.A = reinterpret_cast<const half_t*>(x_packed); g.Y = reinterpret_cast<half_t*>(h_packed); g.expert_offsets = expert_offsets;
     g.a_row_index = sorted_idx;
     g.M = total_rows; g.K = H; g.N = E_ffn; g.E = E; g.bias0 = gate_bias; g.bias1 = up_bias; g.alpha = alpha; g.limit = limit;
-    GemmMxfp4Soa::Bank bg{g_qs, g_e, qs_stride, e_stride, H}, bu{u_qs, u_e, qs_stride, e_stride, H};
-    return launch_gemm<GemmMxfp4Soa, GEMM_MOE_GATE_UP_OAI>(s, bg, bu, g, total_rows);
+    GemmMxfp4Pair::Bank bg{g_qs, g_e, qs_stride, e_stride, H}, bu{u_qs, u_e, qs_stride, e_stride, H};
+    return launch_gemm<GemmMxfp4Pair, GEMM_MOE_GATE_UP_OAI>(s, bg, bu, g, total_rows);
 }
 int mx_moe_gemm_down_mxfp4(mx_stream_t s, const uint16_t* h_packed, const uint8_t* d_qs, const uint8_t* d_e, uint64_t qs_stride, uint64_t e_stride,
                            const float* down_bias, const uint32_t* expert_offsets, uint16_t* out_packed, uint32_t E, uint32_t H, uint32_t E_ffn,
@@ -1737,8 +1972,8 @@ int mx_moe_gemm_down_mxfp4(mx_stream_t s, const uint16_t* h_packed, const uint8_
     GemmArgs g{};
     g.A = reinterpret_cast<const half_t*>(h_packed); g.Y = reinterpret_cast<half_t*>(out_packed); g.expert_offsets = expert_offsets;
     g.M = total_rows; g.K = E_ffn; g.N = H; g.E = E; g.bias0 = down_bias;
-    GemmMxfp4Soa::Bank b{d_qs, d_e, qs_stride, e_stride, E_ffn};
-    return launch_gemm<GemmMxfp4Soa, GEMM_MOE_DOWN>(s, b, b, g, total_rows);
+    GemmMxfp4Pair::Bank b{d_qs, d_e, qs_stride, e_stride, E_ffn};
+    return launch_gemm<GemmMxfp4Pair, GEMM_MOE_DOWN>(s, b, b, g, total_rows);
 }
 
 // moe_prefill_proj_q4_0_xmx (include/ie/ops.hpp:192-204): plain projection of expert-sorted fp16 rows through Q4_0 experts.
@@ -1760,7 +1995,7 @@ int mx_moe_prefill_down_q4k(mx_stream_t s, const uint16_t* h_packed, const void*
                             const uint16_t* sorted_token_w, float* y_fp32, uint32_t E, uint32_t H, uint32_t E_ffn, uint64_t expert_stride_bytes,
                             uint32_t total_rows) {
     MX_REQUIRE_PTR(sorted_token_idx); MX_REQUIRE_PTR(sorted_token_w); MX_REQUIRE_PTR(y_fp32);
-    return moe_gemm_aos<GemmQ4K, GEMM_MOE_DOWN>(s, h_packed, down_W, down_W, expert_stride_bytes, expert_offsets, sorted_token_w, nullptr, E, E_ffn, H,
+    return moe_gemm_aos<GemmQ4KPair, GEMM_MOE_DOWN>(s, h_packed, down_W, down_W, expert_stride_bytes, expert_offsets, sorted_token_w, nullptr, E, E_ffn, H,
                                                 total_rows, kQ4KBytes, 16, sorted_token_idx, y_fp32);
 }
 int mx_moe_prefill_down_q6k(mx_stream_t s, const uint16_t* h_packed, const void* down_W, const uint32_t* expert_offsets, const int32_t* sorted_token_idx,

@@ -52,7 +52,8 @@ def test_gemm_k_slices(mx, fmt, M, K, N):
     ("q8_0", 1, 128, 33), ("q8_0", 1, 384, 200), ("q8_0", 17, 2176, 201), ("q8_0", 260, 384, 3899), ("q8_0", 199, 3712, 611),
     ("q8_0", 257, 384, 6776), ("q8_0", 260, 2176, 1433), ("q8_0", 200, 384, 10886), ("q8_0", 193, 3712, 1844), ("q8_0", 260, 384, 10886),
     ("q8_0", 257, 384, 13352), ("q8_0", 259, 3712, 3899), ("q8_0", 200, 3712, 5543), ("q4_K", 31, 7424, 257), ("q6_K", 95, 5376, 130),
-    ("mxfp4", 40, 2880, 160), ("mxfp4", 127, 320, 1100)])
+    ("mxfp4", 40, 2880, 160), ("mxfp4", 127, 320, 1100), ("q4_K", 260, 512, 13353), ("q4_K", 64, 2560, 6001), ("mxfp4", 260, 320, 13351),
+    ("q8_0", 130, 896, 14335), ("q4_K", 700, 256, 14333), ("mxfp4", 700, 192, 14335)])
 def test_gemm_plans(mx, fmt, M, K, N):
     """One shape per form a dense launch can take (32 .. 128 tokens x 128 or 256 weight rows, with and without K slices, four-wave
     workgroups), at odd numbers of chunks, so that slices and the two K halves of a workgroup differ in length, ragged M and N, one
