@@ -485,14 +485,19 @@ static int launch_mmq_grouped_cfg(hipStream_t st, const typename P::Bank& b0, co
         static LdsLimit limit;
         if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&mmq_kernel<P, TV, NW, WR, WK, EPI>), limit, kMmqMoeLdsBudgetBig)) return rc;
     }
-    // token tiles of an expert are dealt over gridDim.z workgroups: the expert sizes live on the device and are skewed (a few
-    // experts hold most rows), so the split is sized for experts several times the average; workgroups without a tile leave at once
-    uint32_t zt = 2;   // even with small experts a few hold more rows than one tile: their second tile gets a workgroup of its own
+    // Token tiles of an expert are dealt over gridDim.z workgroups: the expert sizes live on the device and are skewed (a few
+    // experts hold most rows), so the split is sized for an expert of eight times the average, and for four tiles at least: the
+    // launch lasts as long as its largest expert, and a workgroup without a tile leaves at once.  Whole expert block over q8 rows, two
+    // tiles and four times the average before / now, us: Q4_K + Q6_K, 128 experts, k = 8, hidden 2048: 64 tokens 171 / 158, 128 tokens 251 /
+    // 220, 333 tokens 331 / 271, 500 tokens 435 / 336.  Native MXFP4 images are dear to build, four times the average stays (32 experts,
+    // k = 4, hidden 2880: 32 tokens 178 / 161, 64 tokens 239 / 212 by the four tiles; 300 tokens 570, with eight times 574).
+    uint32_t zt;
     if (!m.expert_offsets) {
         zt = (m.n_rows + TT - 1u) / TT;   // every tile its own workgroup, up to the 32 that share a row block's weights through L2
         if (zt > 32u) zt = 32u;
-    } else if (avg == 0 || avg > TT) {
-        zt = avg ? (4u * avg + TT - 1u) / TT : 8u;
+    } else {
+        zt = avg ? (uint32_t)(((NATIVE ? 4ull : 8ull) * avg + TT - 1u) / TT) : 8u;
+        if (zt < 4u) zt = 4u;
         if (zt > 32u) zt = 32u;
     }
     // Workgroups per expert along the weight rows: when the staged image covers K, a workgroup streams several row blocks against
@@ -519,6 +524,17 @@ static int launch_mmq_grouped_cfg(hipStream_t st, const typename P::Bank& b0, co
 template <class P, int NW, int EPI>
 static int launch_mmq_grouped(mx_stream_t s, const typename P::Bank& b0, const typename P::Bank& b1, const MoeArgs& m, uint32_t E, uint32_t avg_rows) {
     hipStream_t st = as_stream(s);
+    if constexpr (P::K_ALIGN == 256 && EPI != MMQ_STORE) {
+        // K-quants, 4 to 16 rows per expert: passes of 16 tokens whose four waves take row blocks of their own instead of K ranges (a row
+        // is a few super-blocks long: a wave with a quarter of them neither fills its load pipeline nor pays for the exchange),
+        // as long as that leaves three workgroups per CU.  Expert block over q8 rows, K ranges / row blocks, us: 128 experts, k = 8, hidden
+        // 2048, 768: 64 tokens 158 / 145, 128 tokens 220 / 185, 200 tokens 266 / 225; 32 experts, k = 4, hidden 4096, 1536: 32 tokens 140 /
+        // 131, 100 tokens 223 / 187.  Below: 8 tokens there 84 / 96; with 512 workgroups (64 experts of 3072 -> 1024, 3 rows each) 121 / 133.
+        constexpr uint32_t WR = NW == 1 ? 4u : 2u;
+        if (m.expert_offsets && avg_rows >= 4 && avg_rows <= 16 &&
+            (uint64_t)((m.N + 32u * WR - 1u) / (32u * WR)) * E >= 3ull * (uint64_t)cu_count_moe())
+            return launch_mmq_grouped_cfg<P, 8, NW, (int)WR, 1, EPI>(st, b0, b1, m, E, avg_rows);
+    }
     if (avg_rows && avg_rows <= 8) return launch_mmq_grouped_cfg<P, 4, NW, 1, 4 / NW, EPI>(st, b0, b1, m, E, avg_rows);
     if (avg_rows && avg_rows <= 16) return launch_mmq_grouped_cfg<P, 8, NW, 1, 4 / NW, EPI>(st, b0, b1, m, E, avg_rows);
     if constexpr (mmq_native<P>::value) return launch_mmq_grouped_cfg<P, 8, NW, 1, 4 / NW, EPI>(st, b0, b1, m, E, avg_rows);   // passes of at most 16 tokens

@@ -544,3 +544,11 @@ def test_moe_scatter_add_bit_exact(mx, n_tok, hidden):
     ref = y0.copy()
     ref[idx] = (y0[idx].astype(np.float32) + xp.astype(np.float32) * w[:, None].astype(np.float32)).astype(np.float16).astype(np.float32)
     assert np.array_equal(host(y).astype(np.float32), ref)
+
+
+@pytest.mark.parametrize("avg,K,N_gate,N_down", [(4, 256, 384, 768), (16, 256, 383, 768), (4, 256, 320, 640), (17, 256, 384, 768)])
+def test_moe_grouped_int_dot_row_blocks_or_k_ranges(mx, avg, K, N_gate, N_down):
+    """Both sides of the rule that gives the four waves of a workgroup row blocks or K ranges: 4 and 16 rows per expert with exactly three
+    workgroups per CU, one workgroup per expert fewer, and one row per expert more.  A row is one super-block, so with K ranges three
+    of the four waves have none."""
+    test_moe_grouped_int_dot_streams_row_blocks(mx, avg, K, N_gate, N_down)
