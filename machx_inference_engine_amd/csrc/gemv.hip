@@ -842,7 +842,10 @@ static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, co
     hipLaunchKernelGGL((mmq_kernel<P, TV, 1, WR, WK, MMQ_STORE>), dim3(rgs, 1, Z), dim3(64 * WR * WK), lds, st, a);
     if (Z > 1) {
         const uint32_t mn = T * N;
-        hipLaunchKernelGGL(mmq_reduce_kernel, dim3((mn + 255u) / 256u), dim3(256), 0, st, y, ws.ptr, mn, Z);
+        if (mn % 4u == 0 && aligned(y, 8) && aligned(ws.ptr, 16))
+            hipLaunchKernelGGL(mmq_reduce_kernel<4>, dim3((mn / 4u + 255u) / 256u), dim3(256), 0, st, y, ws.ptr, mn, Z);
+        else
+            hipLaunchKernelGGL(mmq_reduce_kernel<1>, dim3((mn + 255u) / 256u), dim3(256), 0, st, y, ws.ptr, mn, Z);
     }
     return launch_status();
 }

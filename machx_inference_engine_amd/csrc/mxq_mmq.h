@@ -1105,13 +1105,18 @@ __global__ __launch_bounds__(64 * NW * WR * WK, (mmq_workgroups_per_cu<P, TV, NW
     }
 }
 
-// reduction of the K ranges of a dense launch, in range order
+// Reduction of the K ranges of a dense launch, in range order: V outputs per thread, four where n, the planes and y allow it (feed-forward
+// block of 16 tokens, Q6_K 4096/14336, three such launches: 83.1 -> 82.0 us; of 12 tokens, Q8_0 2048/6144: 41.5 -> 40.7).
+template <int V>
 static __global__ __launch_bounds__(256) void mmq_reduce_kernel(half_t* y, const float* part, uint32_t mn, uint32_t n_split) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    typedef float fv_t __attribute__((ext_vector_type(V)));
+    typedef half_t hv_t __attribute__((ext_vector_type(V)));
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (i >= mn) return;
-    float v = 0.f;
-    for (uint32_t k = 0; k < n_split; ++k) v += part[(size_t)k * mn + i];
-    y[i] = (half_t)v;
+    fv_t v = {};
+#pragma unroll 4
+    for (uint32_t k = 0; k < n_split; ++k) v += *reinterpret_cast<const fv_t*>(part + (size_t)k * mn + i);
+    *reinterpret_cast<hv_t*>(y + i) = __builtin_convertvector(v, hv_t);
 }
 
 }  // namespace mxq
