@@ -81,7 +81,7 @@ def _config3_weights(K, N):
 @pytest.mark.parametrize("T", [2048, 512, 4096])
 @pytest.mark.parametrize("K,N", [(H, FF), (FF, H)])
 def test_config3_gemm_full_size(mx, K, N, T):
-    """T = 512 on N = 4096 runs 64-token tiles in K slices (another launch than 2048 / 4096)."""
+    """T = 512 runs eight-wave workgroups (another launch than 2048 / 4096)."""
     ops = mx.ops
     W = _config3_weights(K, N)
     A = f16(O.normal(4100 + N, (T, K), 0.0, 1.0))

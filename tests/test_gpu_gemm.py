@@ -35,8 +35,7 @@ def test_gemm_q4_K(mx, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(8, 4096, 512), (64, 2048, 260), (200, 3072, 768), (512, 7168, 256)])
 def test_gemm_k_slices(mx, fmt, M, K, N):
     """Launches with too few output tiles for the chip run as K slices plus a launch that adds the slices in order:
-    4 slices of 128-token tiles (M <= 64), 2..8 slices of 64-token tiles, a last slice shorter than the others
-    (K = 3072: 24 chunks in 3 slices; K = 7168: 56 chunks in 7).  Against the oracle, and the same bits from launch to launch."""
+    6 to 8 slices of 32-token tiles here.  Against the oracle, and the same bits from launch to launch."""
     W = weights(fmt, 2100 + N, N, K)
     A = f16(O.normal(2101 + M, (M, K)))
     ref = O.gemv_f64(fmt, W, A, K, N, round_w_fp16=True)
@@ -495,9 +494,9 @@ def test_moe_grouped_gemm_q8_random_shapes(mx):
 
 @pytest.mark.parametrize("fmt", (O.Q4_K, O.Q6_K, O.Q8_0))
 def test_gemm_eight_wave_workgroups(mx, fmt):
-    """Dense launches whose 128-token tiles cover between half and all of the CUs (here 2 x 70 = 140 tiles) run
-    eight-wave workgroups: waves 4 - 7 walk the second half of K and hand their sums over through LDS.  A ragged second
-    token tile, and output columns sampled across every column tile, against the oracle."""
+    """Dense launches of one 128-token tile or less per CU (here 2 x 70 tiles) run eight-wave workgroups: waves 4 - 7
+    walk the second half of K and hand their sums over through LDS.  A ragged last token tile, and output columns sampled
+    across every column tile, against the oracle."""
     M, K, N = 160, 2048, 256 * 70
     W = weights(fmt, 2300, N, K)
     A = f16(O.normal(2301, (M, K)))
