@@ -94,20 +94,22 @@ __global__ __launch_bounds__(kGemvThreads, (TT == 1 && NW == 1 && F::SUM_GRAN ==
                 for (int t = 0; t < TT; ++t) acc[r][t] = 0.f;
             for (uint32_t tile = 0; tile < n_tiles; ++tile) {
                 const uint32_t k0 = tile * KT, kt = (K - k0 < KT) ? K - k0 : KT;
+                const uint32_t n_units = (kt + 63) / 64;
+                const bool half_tail = (kt & 63u) != 0;
+                // a row may have fewer units than the group has lanes: the lanes left over start at its first unit
+                const uint32_t first = kMoeWholeRow<F, TT, NW> && gl >= n_units ? 0u : gl;
                 typename F::Cursor cu[NW * R];
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const uint32_t n = (n0 + r < N) ? n0 + r : N - 1;
-                    cu[NW * r] = F::cursor(w0, n, k0 / 64 + gl);
-                    if (NW == 2) cu[NW * r + 1] = F::cursor(w1, n, k0 / 64 + gl);
+                    cu[NW * r] = F::cursor(w0, n, k0 / 64 + first);
+                    if (NW == 2) cu[NW * r + 1] = F::cursor(w1, n, k0 / 64 + first);
                 }
-                const uint32_t n_units = (kt + 63) / 64;
-                const bool half_tail = (kt & 63u) != 0;
                 if (kMoeWholeRow<F, TT, NW> && n_tiles == 1 && !staged && !half_tail && n_units <= 3u * G) {
                     // A workgroup of a decode launch lives for one row group.  The whole of its rows (up to three rounds
                     // of units) is requested right behind the activation loads and in front of the barrier, so the launch
                     // is one round trip to memory and the first round is summed while the later ones arrive.  Lanes
-                    // past the end of the row read their first unit again and drop the product.
+                    // past the end of the row read the unit of their cursor (again) and drop the product.
                     constexpr int AHEAD = 3;
                     typename F::Raw pre[3][NW * R];
                     auto request = [&]() {
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(kGemvThreads, (TT == 1 && NW == 1 && F::SUM_GRAN ==
                         for (int r = 0; r < NW * R; ++r)
 #pragma unroll
                             for (int t = 0; t < TT; ++t) part[r][t] = 0.f;
-                        gemv_step<F, TT, NW * R>(pre[u], cu, lv ? gl + u * G : gl, act, part);
+                        gemv_step<F, TT, NW * R>(pre[u], cu, lv ? gl + u * G : first, act, part);
 #pragma unroll
                         for (int r = 0; r < NW * R; ++r)
 #pragma unroll

@@ -552,3 +552,17 @@ def test_moe_grouped_int_dot_row_blocks_or_k_ranges(mx, avg, K, N_gate, N_down):
     workgroups per CU, one workgroup per expert fewer, and one row per expert more.  A row is one super-block, so with K ranges three
     of the four waves have none."""
     test_moe_grouped_int_dot_streams_row_blocks(mx, avg, K, N_gate, N_down)
+
+
+@pytest.mark.parametrize("EF", [64, 512, 768, 1152, 1920, 3200])
+def test_moe_mxfp4_down_rows_shorter_than_a_lane_group(mx, EF):
+    """One-token down launch with fewer 64-element units in a row than lanes that share it (8 of 16, 18 of 32, 50 of 64, ..), every
+    expert routed, the last one and its last row included: the lanes left over must add nothing.  Where they read is checked in
+    test_host_weight_reads.py."""
+    ops, E, H = mx.ops, 3, 130
+    Wd, dq, de, dqs_st, de_st = make_experts(O.MXFP4, 300, E, H, EF)
+    bd = O.normal(3, (E, H))
+    ids = np.arange(E, dtype=np.int32)
+    hq = O.quantize_q8_1(f16(O.normal(4, (E, EF))))
+    out = ops.moe_down_mxfp4(dev(hq), dev(dq), dev(de), dqs_st, de_st, dev(bd), dev(ids), 1, E, EF, H, E)
+    check_down_bias_rows(host(out).astype(np.float32), Wd, bd, ids, hq, EF, H, "moe down + bias, rows of %d" % EF)
