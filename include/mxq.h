@@ -315,13 +315,14 @@ int mx_gemv_q8_0_f32(mx_stream_t s, const float* A, const void* W, float* y, uin
  * K % 256 == 0 (Q4_K), K % 128 == 0 (Q8_0 planes); A and W 16-byte aligned.
  * mx_gemm_q8_0_soa takes the SoA planes of gemv_q8_0_soa_q8 (the reference runs Q8_0 prefill
  * as dequant_q8_0_soa_to_Bt + gemm_fp16, src/model/qwen35_dense.cpp:811-831).
- * A launch whose tiles would not fill the chip (a short batch against a narrow matrix) is cut into
- * 2..8 K slices; their fp32 partial sums go through a
+ * Shared scratch.  A launch with K >= 2048 whose 128 x 256 output tiles cover at most half of the CUs,
+ * ceil(M / 128) * ceil(N / 256) <= 128 on MI355X, may be cut into 2..8 K slices (every mx_gemm_* of a quantized
+ * weight, Q4_0, Q5_K and MXFP4 included; mx_gemm_plan tells).  Their fp32 partial sums go through a
  * 32 MB per-device scratch array owned by the library (a file-scope device array resolved with hipGetSymbolAddress,
  * never allocated; slices * M * N <= 8 Mi floats, fewer slices beyond that) and are added in slice
  * order by a second small launch: two such calls that overlap on one device race on it, as the
- * reference's static per-device scratch buffers would (src/model/dense_dispatch.hpp:547-560).  The *_ws forms
- * below keep the partial sums in the caller's workspace instead.  */
+ * reference's static per-device scratch buffers would (src/model/dense_dispatch.hpp:547-560).  No other shape uses it.
+ * The *_ws forms below keep the partial sums in the caller's workspace instead and slice wherever it pays.  */
 int mx_gemm_q4_K(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N);
 int mx_gemm_q8_0_soa(mx_stream_t s, const uint16_t* A, const int8_t* qs_W, const uint16_t* d_W, uint16_t* y, uint32_t M,
                      uint32_t K, uint32_t N);
@@ -331,10 +332,11 @@ int mx_gemm_q8_0_soa(mx_stream_t s, const uint16_t* A, const int8_t* qs_W, const
  * K % 256 == 0 (Q6_K), K % 128 == 0 (Q8_0); W is the GGUF block stream, 2-byte aligned.  */
 int mx_gemm_q6_K(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N);
 int mx_gemm_q8_0(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N);
-/* Caller-workspace forms (no counterpart in the reference): same results; K-sliced launches keep their partial sums
+/* Caller-workspace forms (no counterpart in the reference): the same product; K-sliced launches keep their partial sums
  * in `ws` (16-byte aligned device memory), so launches on different streams can overlap.  mx_gemm_ws_bytes gives the
  * size that allows every slice the launch would like (0: the shape is never sliced); a smaller workspace, NULL / 0
- * included, is legal and means fewer slices or none.  */
+ * included, is legal and means fewer slices or none.  Equal slices give equal bits; another number of slices adds the
+ * same fp32 products in another order.  */
 int mx_gemm_ws_bytes(uint32_t M, uint32_t K, uint32_t N, uint64_t* bytes);
 int mx_gemm_q4_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws,
                     uint64_t ws_bytes);
@@ -342,8 +344,19 @@ int mx_gemm_q6_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y
                     uint64_t ws_bytes);
 int mx_gemm_q8_0_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws,
                     uint64_t ws_bytes);
+int mx_gemm_q4_0_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws,
+                    uint64_t ws_bytes);
 int mx_gemm_q8_0_soa_ws(mx_stream_t s, const uint16_t* A, const int8_t* qs_W, const uint16_t* d_W, uint16_t* y, uint32_t M,
                         uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes);
+int mx_gemm_q5_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws,
+                    uint64_t ws_bytes);
+int mx_gemm_mxfp4_soa_ws(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, const uint8_t* e_W, uint16_t* y, uint32_t M,
+                         uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes);
+/* How a dense quant-GEMM of this shape is cut on the current device (host only, nothing is launched): plan[0] = 32-token
+ * tiles per workgroup tile of an eight-wave workgroup (1..4; 0: four-wave workgroups over 128 x 256), plan[1] = 32-row
+ * column tiles per wave (1 or 2), plan[2] = K slices (1: no scratch is used).  own_ws = 0: the forms without a workspace;
+ * else the *_ws forms with a workspace of ws_bytes.  */
+int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* plan);
 /* Q4_0 weights through the same kernel: gemm_q4_0 / gemm_q4_0_xmx  include/ie/ops.hpp:530-534, src/ops/gemv_q4_0.cpp,
  * src/ops/gemm_q4k_xmx.cpp:418-522; K % 128 == 0, W 2-byte aligned.  */
 int mx_gemm_q4_0(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N);

@@ -1682,11 +1682,19 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint
     return best;
 }
 
+// Floats of the library's scratch that a launch without a caller's workspace may use.  Calls that overlap on one device race on it, so
+// the shapes that use it are those the header names, in terms a caller can evaluate, and no others: a plan that would slice elsewhere
+// runs unsliced there.
+static uint64_t gemm_library_scratch(uint64_t M, uint64_t K, uint64_t N, uint64_t cus) {
+    return K >= 2048 && 2 * ((M + 127) / 128) * ((N + 255) / 256) <= cus ? kGemmSplitElems : 0;
+}
+
 template <class QF, int MODE>
 static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound,
                        const SplitWs* caller_ws = nullptr) {
     if constexpr (MODE == GEMM_DENSE) {
-        const GemmPlan p = gemm_plan(g.M, g.K, g.N, caller_ws ? caller_ws->elems : kGemmSplitElems, (uint64_t)gemm_cu_count());
+        const uint64_t cus = (uint64_t)gemm_cu_count();
+        const GemmPlan p = gemm_plan(g.M, g.K, g.N, caller_ws ? caller_ws->elems : gemm_library_scratch(g.M, g.K, g.N, cus), cus);
         g.k_split = p.k_split;
         if (p.k_split > 1) {
             if (caller_ws) {
@@ -1749,7 +1757,7 @@ static int moe_gemm_aos(mx_stream_t s, const uint16_t* rows, const void* W0, con
     }
 }
 
-// Dense entry points.  ws = NULL: K-sliced launches keep their partial sums in the library's per-device scratch.
+// Dense entry points.  ws = NULL: K-sliced launches keep their partial sums in the library's per-device scratch (gemm_library_scratch).
 template <class QF>
 static int gemm_dense_aos(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, uint32_t k_align,
                           uint32_t w_align, uint32_t row_bytes, const SplitWs* ws) {
@@ -1768,6 +1776,15 @@ static int gemm_dense_q8_soa(mx_stream_t s, const uint16_t* A, const int8_t* qs_
     g.A = reinterpret_cast<const half_t*>(A); g.Y = reinterpret_cast<half_t*>(y); g.M = M; g.K = K; g.N = N; g.E = 1;
     GemmQ8Quad::Bank b{qs_W, d_W, 0, 0, K};
     return launch_gemm<GemmQ8Quad, GEMM_DENSE>(s, b, b, g, M, ws);
+}
+static int gemm_dense_mxfp4_soa(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, const uint8_t* e_W, uint16_t* y, uint32_t M, uint32_t K,
+                                uint32_t N, const SplitWs* ws) {
+    if (int rc = check_gemm(A, qs_W, y, M, K, N, 64)) return rc;
+    MX_REQUIRE_PTR(e_W);
+    GemmArgs g{};
+    g.A = reinterpret_cast<const half_t*>(A); g.Y = reinterpret_cast<half_t*>(y); g.M = M; g.K = K; g.N = N; g.E = 1;
+    GemmMxfp4Pair::Bank b{qs_W, e_W, 0, 0, K};
+    return launch_gemm<GemmMxfp4Pair, GEMM_DENSE>(s, b, b, g, M, ws);
 }
 // A caller's workspace: any size is accepted, the number of K slices adapts to what it holds (none below 2 M N floats).
 static int gemm_ws(void* ws, uint64_t ws_bytes, SplitWs* out) {
@@ -1809,6 +1826,14 @@ int mx_gemm_ws_bytes(uint32_t M, uint32_t K, uint32_t N, uint64_t* bytes) {
     *bytes = gemm_plan(M, K, N, ~0ull, (uint64_t)gemm_cu_count()).k_split > 1 ? (uint64_t)kGemmSplitMax * M * N * sizeof(float) : 0;
     return MX_OK;
 }
+int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* plan) {
+    MX_REQUIRE_PTR(plan);
+    MX_REQUIRE_SHAPE(M > 0 && K > 0 && N > 0);
+    const uint64_t cus = (uint64_t)gemm_cu_count();
+    const GemmPlan p = gemm_plan(M, K, N, own_ws ? ws_bytes / 4 : gemm_library_scratch(M, K, N, cus), cus);
+    plan[0] = p.na; plan[1] = p.nj; plan[2] = p.k_split;
+    return MX_OK;
+}
 int mx_gemm_q4_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {
     SplitWs w;
     if (int rc = gemm_ws(ws, ws_bytes, &w)) return rc;
@@ -1823,6 +1848,11 @@ int mx_gemm_q8_0_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y
     SplitWs w;
     if (int rc = gemm_ws(ws, ws_bytes, &w)) return rc;
     return gemm_dense_aos<GemmQ8Aos>(s, A, W, y, M, K, N, 128, 2, K / 32 * (uint32_t)kQ8_0Bytes, &w);
+}
+int mx_gemm_q4_0_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {
+    SplitWs w;
+    if (int rc = gemm_ws(ws, ws_bytes, &w)) return rc;
+    return gemm_dense_aos<GemmQ40>(s, A, W, y, M, K, N, 128, 2, K / 32 * 18u, &w);
 }
 int mx_gemm_q8_0_soa_ws(mx_stream_t s, const uint16_t* A, const int8_t* qs_W, const uint16_t* d_W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N,
                         void* ws, uint64_t ws_bytes) {
@@ -1925,12 +1955,18 @@ int mx_gemm_q5_K(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, u
     return gemm_dense_aos<GemmQ5K>(s, A, W, y, M, K, N, 256, 16, K / 256 * 176u, nullptr);
 }
 int mx_gemm_mxfp4_soa(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, const uint8_t* e_W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N) {
-    if (int rc = check_gemm(A, qs_W, y, M, K, N, 64)) return rc;
-    MX_REQUIRE_PTR(e_W);
-    GemmArgs g{};
-    g.A = reinterpret_cast<const half_t*>(A); g.Y = reinterpret_cast<half_t*>(y); g.M = M; g.K = K; g.N = N; g.E = 1;
-    GemmMxfp4Pair::Bank b{qs_W, e_W, 0, 0, K};
-    return launch_gemm<GemmMxfp4Pair, GEMM_DENSE>(s, b, b, g, M, nullptr);
+    return gemm_dense_mxfp4_soa(s, A, qs_W, e_W, y, M, K, N, nullptr);
+}
+int mx_gemm_q5_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {
+    SplitWs w;
+    if (int rc = gemm_ws(ws, ws_bytes, &w)) return rc;
+    return gemm_dense_aos<GemmQ5K>(s, A, W, y, M, K, N, 256, 16, K / 256 * 176u, &w);
+}
+int mx_gemm_mxfp4_soa_ws(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, const uint8_t* e_W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N,
+                         void* ws, uint64_t ws_bytes) {
+    SplitWs w;
+    if (int rc = gemm_ws(ws, ws_bytes, &w)) return rc;
+    return gemm_dense_mxfp4_soa(s, A, qs_W, e_W, y, M, K, N, &w);
 }
 static int moe_gemm_gate_up_oai_mxfp4(mx_stream_t s, const uint16_t* x_packed, const int32_t* sorted_idx, uint32_t n_tokens, const uint8_t* g_qs,
                                       const uint8_t* g_e, const uint8_t* u_qs, const uint8_t* u_e, uint64_t qs_stride, uint64_t e_stride,

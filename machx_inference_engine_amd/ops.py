@@ -6,6 +6,9 @@ the queue becomes torch's current stream, and a violated precondition raises
 MxError instead of silently doing nothing.  Outputs are allocated here when the
 caller does not pass them (the reference's callers own all buffers).
 """
+import ctypes
+import functools
+
 import numpy as np
 import torch
 
@@ -180,7 +183,6 @@ def init():
 
 
 def gemv_batched_ws_bytes(K, N, T):
-    import ctypes
     n = ctypes.c_uint64(0)
     rc = lib.mx_gemv_batched_ws_bytes(K, N, T, ctypes.addressof(n))
     if rc != 0:
@@ -189,7 +191,6 @@ def gemv_batched_ws_bytes(K, N, T):
 
 
 def gemm_ws_bytes(M, K, N):
-    import ctypes
     n = ctypes.c_uint64(0)
     rc = lib.mx_gemm_ws_bytes(M, K, N, ctypes.addressof(n))
     if rc != 0:
@@ -206,11 +207,49 @@ def gemv_q8_batched_ws(fmt, x_q8, wargs, K, N, T, ws, y=None):
     return y
 
 
+def gemm_plan(M, K, N, ws_bytes=None):
+    """(32-token tiles, 32-row column tiles, K slices) of a dense quant-GEMM; ws_bytes None: the forms without a workspace."""
+    plan = (ctypes.c_uint32 * 3)()
+    rc = lib.mx_gemm_plan(M, K, N, ws_bytes is not None, ws_bytes or 0, ctypes.addressof(plan))
+    if rc != 0:
+        raise MxError("mx_gemm_plan", rc)
+    return tuple(plan)
+
+
 def gemm_ws(fmt, A, wargs, M, K, N, ws, y=None):
-    """Caller-workspace dense quant-GEMM: fmt in ('q4_K', 'q6_K', 'q8_0', 'q8_0_soa')."""
+    """Caller-workspace dense quant-GEMM: fmt in ('q4_K', 'q6_K', 'q8_0', 'q8_0_soa', 'q4_0', 'q5_K', 'mxfp4_soa')."""
     y = _out(y, (M, N), torch.float16, A)
     _call("mx_gemm_%s_ws" % fmt, _f16(A), *[_ptr(w) for w in wargs], _ptr(y), M, K, N, _ptr(ws) if ws is not None else None,
           ws.numel() * ws.element_size() if ws is not None else 0)
+    return y
+
+
+_GEMM_OWN_BYTES = 32 << 20
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_own_bytes(M, K, N):
+    """Bytes for the partial sums of a shape that is faster in K slices but does not use the library's shared scratch (at most
+    32 MB, fewer slices beyond that); 0: not sliced, or the shared scratch holds them."""
+    try:
+        if gemm_plan(M, K, N)[2] > 1:
+            return 0
+        k = gemm_plan(M, K, N, _GEMM_OWN_BYTES)[2]
+    except MxError:
+        return 0   # the call itself names what is wrong
+    return 4 * k * M * N if k > 1 else 0
+
+
+def _gemm(fmt, A, wargs, M, K, N, y):
+    """Dense quant-GEMM; the partial sums of a K-sliced launch are in memory of this call's own (stream-ordered, as y is) except where
+    the header promises the shared scratch."""
+    y = _out(y, (M, N), torch.float16, A)
+    own = _gemm_own_bytes(M, K, N)
+    if own:
+        ws = torch.empty(own, dtype=torch.uint8, device=A.device)
+        _call("mx_gemm_%s_ws" % fmt, _f16(A), *wargs, _ptr(y), M, K, N, _ptr(ws), own)
+    else:
+        _call("mx_gemm_" + fmt, _f16(A), *wargs, _ptr(y), M, K, N)
     return y
 
 
@@ -528,9 +567,7 @@ def gemv_q5_K_q8(x_q8, W, K, N, T=1, y=None):
 
 
 def gemm_q4_0(A, W, M, K, N, y=None):
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_q4_0", _f16(A), _u8(W), _ptr(y), M, K, N)
-    return y
+    return _gemm("q4_0", A, (_u8(W),), M, K, N, y)
 
 
 def moe_prefill_proj_q4_0(kind, rows, W, expert_offsets, TK, E, K, N, stride, out_packed=None):
@@ -720,21 +757,15 @@ def gated_rms_norm_q8(x, z, weight, eps):
 
 # ---------------------------------------------------------------- prefill GEMM (MFMA)
 def gemm_q4_K(A, W, M, K, N, y=None):
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_q4_K", _f16(A), _u8(W), _ptr(y), M, K, N)
-    return y
+    return _gemm("q4_K", A, (_u8(W),), M, K, N, y)
 
 
 def gemm_q6_K(A, W, M, K, N, y=None):
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_q6_K", _f16(A), _u8(W), _ptr(y), M, K, N)
-    return y
+    return _gemm("q6_K", A, (_u8(W),), M, K, N, y)
 
 
 def gemm_q8_0(A, W, M, K, N, y=None):
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_q8_0", _f16(A), _u8(W), _ptr(y), M, K, N)
-    return y
+    return _gemm("q8_0", A, (_u8(W),), M, K, N, y)
 
 
 def moe_gemm_gate_up_silu_q4k(x_packed, gate_W, up_W, expert_offsets, TK, E, H, E_ffn, expert_stride_bytes, h_packed=None, soa=False, sorted_idx=None):
@@ -759,16 +790,12 @@ def moe_gemm_down_kquant(fmt, h_packed, down_W, expert_offsets, sorted_w, TK, E,
 
 
 def gemm_q5_K(A, W, M, K, N, y=None):
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_q5_K", _f16(A), _u8(W), _ptr(y), M, K, N)
-    return y
+    return _gemm("q5_K", A, (_u8(W),), M, K, N, y)
 
 
 def gemm_mxfp4_soa(A, qs_plane, e_plane, M, K, N, y=None):
     """y[M,N] = A . half(deq(W))^T for MXFP4 planes, K % 64 == 0 (fused: no [K,N] fp16 matrix is written)."""
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_mxfp4_soa", _f16(A), _u8(qs_plane), _u8(e_plane), _ptr(y), M, K, N)
-    return y
+    return _gemm("mxfp4_soa", A, (_u8(qs_plane), _u8(e_plane)), M, K, N, y)
 
 
 def moe_gemm_gate_up_oai_mxfp4(x_packed, g_qs, g_e, u_qs, u_e, qs_stride, e_stride, gate_bias, up_bias, expert_offsets, TK, E, H, E_ffn,
@@ -794,9 +821,7 @@ def moe_gemm_down_mxfp4(h_packed, d_qs, d_e, qs_stride, e_stride, down_bias, exp
 
 
 def gemm_q8_0_soa(A, qs_W, d_W, M, K, N, y=None):
-    y = _out(y, (M, N), torch.float16, A)
-    _call("mx_gemm_q8_0_soa", _f16(A), _u8(qs_W), _ptr(d_W), _ptr(y), M, K, N)
-    return y
+    return _gemm("q8_0_soa", A, (_u8(qs_W), _ptr(d_W)), M, K, N, y)
 
 
 def moe_gemm_gate_up_silu_q8(x_packed, g_qs, g_d, u_qs, u_d, qs_stride, d_stride, expert_offsets, TK, E, H, E_ffn, h_packed=None, sorted_idx=None):

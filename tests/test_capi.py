@@ -104,3 +104,32 @@ def test_query_sized_workspace_is_never_refused(lib):
                        l.mx_gemv_q6_K_q8_batched_ws(None, p16, p16, p16, K, N, T, ws, n.value),
                        l.mx_gemv_q8_0_q8_batched_ws(None, p16, p16, p16, K, N, T, ws, n.value)):
                 assert rc != WORKSPACE, (K, N, T, n.value)
+
+
+def test_dense_gemm_uses_the_shared_scratch_only_where_the_header_says(lib):
+    """Without a workspace a dense quant-GEMM is K-sliced, and so uses the scratch that overlapping calls race on, only for K >= 2048
+    and 128 x 256 tiles on at most half of the CUs (256 without a GPU), within its 8 Mi floats.  A workspace lifts the first two
+    conditions; the Python entry points bring one of their own for exactly those shapes."""
+    l, _ = lib
+    from machx_inference_engine_amd import ops
+    sliced = own = 0
+    for M in (1, 17, 64, 77, 137, 200, 256, 337, 512, 700, 1024, 2048):
+        for K in (128, 1024, 1280, 1792, 1984, 2048, 2880, 5888, 8448, 14336):
+            for N in (33, 512, 896, 1024, 4096, 11712, 14336, 16640):
+                k = ops.gemm_plan(M, K, N)[2]
+                documented = K >= 2048 and 2 * (-(-M // 128) * -(-N // 256)) <= 256
+                assert 1 <= k <= 8 and (k == 1 or (documented and k * M * N <= 8 << 20)), (M, K, N, k)
+                with_ws = ops.gemm_plan(M, K, N, 32 << 20)[2]
+                assert k in (1, with_ws), (M, K, N, k, with_ws)
+                assert ops._gemm_own_bytes(M, K, N) == (4 * with_ws * M * N if with_ws > k else 0), (M, K, N)
+                assert ops.gemm_plan(M, K, N, 4 * with_ws * M * N) == ops.gemm_plan(M, K, N, 32 << 20)
+                sliced += k > 1
+                own += with_ws > k
+    assert sliced > 50 and own > 20
+    assert ops.gemm_plan(64, 1280, 896)[2] == ops.gemm_plan(256, 1792, 1024)[2] == ops.gemm_plan(137, 5888, 16640)[2] == 1
+    plan = (C.c_uint32 * 3)()
+    assert l.mx_gemm_plan(64, 1280, 896, 0, 0, None) == 1 and l.mx_gemm_plan(64, 0, 896, 0, 0, C.addressof(plan)) == 2
+    p16 = 0x1000
+    for name, w in (("q4_0", (p16,)), ("q5_K", (p16,)), ("mxfp4_soa", (p16, p16))):
+        fn = getattr(l, "mx_gemm_%s_ws" % name)
+        assert fn(None, p16, *w, p16, 64, 1280, 896, None, 64) == 1 and fn(None, p16, *w, p16, 64, 1280, 896, 0x1004, 64) == 3

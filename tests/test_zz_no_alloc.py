@@ -74,3 +74,43 @@ def test_k_sliced_gemm_static_scratch_equals_workspace_form(mx):
     rows = np.arange(0, N, 131)
     check(host(y0).astype(np.float32)[:, rows], O.gemv_f64(O.Q4_K, host(W[torch.from_numpy(rows).cuda()]), A[:100], K, len(rows), round_w_fp16=True),
           "unsliced GEMM (no workspace)")
+
+
+@pytest.mark.parametrize("fmt,M,K,N", [("q8_0_soa", 64, 1280, 896), ("q8_0", 64, 1280, 896), ("q6_K", 256, 1792, 1024), ("q4_K", 137, 5888, 16640),
+                                       ("q4_0", 64, 1280, 896), ("q5_K", 256, 1792, 1024), ("mxfp4_soa", 40, 1344, 896)])
+def test_gemms_outside_the_shared_scratch_overlap(mx, fmt, M, K, N):
+    """Shapes that a workspace would cut in K slices but that the header does not name as users of the shared scratch: calls on two
+    streams give each stream's own bits, through the Python entry points (partial sums of their own) and through the C entry points
+    without a workspace (unsliced)."""
+    ops = mx.ops
+    assert ops.gemm_plan(M, K, N)[2] == 1 and ops.gemm_plan(M, K, N, 32 << 20)[2] > 1
+    if fmt in ("q4_0", "q5_K"):
+        w = O.normal(64, (N, K), 0.0, 0.02)
+        wargs = (dev((O.quantize(O.Q4_0, w) if fmt == "q4_0" else O.synth_q5_K(w, 65)).reshape(-1)),)
+    else:
+        W = synth.normal_weights(fmt.replace("_soa", ""), N, K, seed=64)
+        wargs = synth.split_q8_0(W) if fmt == "q8_0_soa" else synth.split_mxfp4(W) if fmt == "mxfp4_soa" else (W.reshape(-1),)
+    A = [dev(f16(O.normal(6400 + i, (M, K)))).half() for i in range(2)]
+
+    def by_ops(a):
+        return getattr(ops, "gemm_" + fmt)(a, *wargs, M, K, N)
+
+    def by_capi(a):
+        y = torch.empty((M, N), dtype=torch.float16, device="cuda")
+        ops._call("mx_gemm_" + fmt, a.data_ptr(), *[w.data_ptr() for w in wargs], y.data_ptr(), M, K, N)
+        return y
+
+    streams = [torch.cuda.Stream() for _ in A]
+    for call in (by_ops, by_capi):
+        want = []
+        for a in A:
+            want.append(call(a))
+            torch.cuda.synchronize()
+        got = [[], []]
+        for _ in range(20):
+            for i, s in enumerate(streams):
+                with torch.cuda.stream(s):
+                    got[i].append(call(A[i]))
+        torch.cuda.synchronize()
+        for i in range(2):
+            assert all(torch.equal(y, want[i]) for y in got[i]), (call.__name__, i)
