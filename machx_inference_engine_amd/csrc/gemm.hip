@@ -1822,8 +1822,10 @@ int mx_gemm_q8_0_soa(mx_stream_t s, const uint16_t* A, const int8_t* qs_W, const
 int mx_gemm_ws_bytes(uint32_t M, uint32_t K, uint32_t N, uint64_t* bytes) {
     MX_REQUIRE_PTR(bytes);
     MX_REQUIRE_SHAPE(M > 0 && K > 0 && N > 0);
-    // kGemmSplitMax planes of M x N floats wherever an unlimited workspace would be used
-    *bytes = gemm_plan(M, K, N, ~0ull, (uint64_t)gemm_cu_count()).k_split > 1 ? (uint64_t)kGemmSplitMax * M * N * sizeof(float) : 0;
+    // one plane of M x N floats per slice that an unlimited workspace would take; kGemmSplitMax of them, as always, for the shapes that
+    // the library's own scratch serves
+    const uint64_t cus = (uint64_t)gemm_cu_count(), k = gemm_plan(M, K, N, ~0ull, cus).k_split;
+    *bytes = k < 2 ? 0 : (gemm_library_scratch(M, K, N, cus) ? (uint64_t)kGemmSplitMax : k) * M * N * sizeof(float);
     return MX_OK;
 }
 int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* plan) {

@@ -133,3 +133,16 @@ def test_dense_gemm_uses_the_shared_scratch_only_where_the_header_says(lib):
     for name, w in (("q4_0", (p16,)), ("q5_K", (p16,)), ("mxfp4_soa", (p16, p16))):
         fn = getattr(l, "mx_gemm_%s_ws" % name)
         assert fn(None, p16, *w, p16, 64, 1280, 896, None, 64) == 1 and fn(None, p16, *w, p16, 64, 1280, 896, 0x1004, 64) == 3
+
+
+def test_gemm_workspace_query_names_what_the_plan_uses(lib):
+    """A workspace of the queried size gives the plan of an unlimited one, and outside the shapes that the library's own scratch
+    serves it is no larger than that plan's partial sums."""
+    l, _ = lib
+    from machx_inference_engine_amd import ops
+    for M, K, N in [(572, 12800, 27584), (64, 1280, 896), (256, 1792, 1024), (137, 5888, 16640), (77, 14336, 4096), (256, 14336, 4096),
+                    (512, 4096, 14336), (4096, 4096, 14336), (1, 128, 33), (337, 8448, 11712)]:
+        need, k = ops.gemm_ws_bytes(M, K, N), ops.gemm_plan(M, K, N, 1 << 62)[2]
+        assert ops.gemm_plan(M, K, N, need) == ops.gemm_plan(M, K, N, 1 << 62), (M, K, N)
+        served = K >= 2048 and 2 * (-(-M // 128) * -(-N // 256)) <= 256
+        assert need == (0 if k == 1 else (8 if served else k) * M * N * 4), (M, K, N, k, need)
