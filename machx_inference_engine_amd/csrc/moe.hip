@@ -487,19 +487,23 @@ static int launch_mmq_grouped_cfg(hipStream_t st, const typename P::Bank& b0, co
         static LdsLimit limit;
         if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&mmq_kernel<P, TV, NW, WR, WK, EPI>), limit, kMmqMoeLdsBudgetBig)) return rc;
     }
-    // Token tiles of an expert are dealt over gridDim.z workgroups: the expert sizes live on the device and are skewed (a few
-    // experts hold most rows), so the split is sized for an expert of eight times the average, and for four tiles at least: the
-    // launch lasts as long as its largest expert, and a workgroup without a tile leaves at once.  Whole expert block over q8 rows, two
-    // tiles and four times the average before / now, us: Q4_K + Q6_K, 128 experts, k = 8, hidden 2048: 64 tokens 171 / 158, 128 tokens 251 /
-    // 220, 333 tokens 331 / 271, 500 tokens 435 / 336.  Native MXFP4 images are dear to build, four times the average stays (32 experts,
-    // k = 4, hidden 2880: 32 tokens 178 / 161, 64 tokens 239 / 212 by the four tiles; 300 tokens 570, with eight times 574).
+    // Token tiles of an expert are dealt over gridDim.z workgroups.  The expert sizes live on the device: the launch lasts as long as its
+    // largest expert, so the split is sized for one of five times the average (popularity by rank^-0.5 makes it 3.3 times the average
+    // with 32 experts, 5.9 with 128), but a workgroup without a tile still has to be scheduled.  Native MXFP4 images are dear to build:
+    // four times the average.  Two tiles at least; four for native MXFP4 from four rows an expert on, whose passes hold 8.
+    // gate + up and down launch, us, two tiles or four times the average / four tiles or eight times / this, for experts by rank^-0.5 and
+    // (even): Q4_K + Q6_K, 128 experts, k = 8, 2048/768: 8 tokens 55 / 55 / 55 (62 / 63 / 62), 64 tokens 131 / 110 / 110 (116 / 102 / 103),
+    // 200 tokens 189 / 151 / 150 (153 / 116 / 115), 500 tokens 267 / 238 / 235 (161 / 167 / 162); MXFP4, 32 experts, k = 4, 2880/2880, 64
+    // tokens 189 / 162 / 162 (122 / 122 / 122); 64 experts, k = 6, 2048/1408, 16 tokens 74 / 74 / 74 (90 / 92 / 90).  Many experts with short
+    // rows lose by it: 128 experts, k = 8, 2048/768, MXFP4, 128 tokens 187 / 192 / 192 (132 / 138 / 138).
     uint32_t zt;
     if (!m.expert_offsets) {
         zt = (m.n_rows + TT - 1u) / TT;   // every tile its own workgroup, up to the 32 that share a row block's weights through L2
         if (zt > 32u) zt = 32u;
     } else {
-        zt = avg ? (uint32_t)(((NATIVE ? 4ull : 8ull) * avg + TT - 1u) / TT) : 8u;
-        if (zt < 4u) zt = 4u;
+        zt = avg ? (uint32_t)(((NATIVE ? 4ull : 5ull) * avg + TT - 1u) / TT) : 8u;
+        const uint32_t least = NATIVE && avg >= 4u ? 4u : 2u;
+        if (zt < least) zt = least;
         if (zt > 32u) zt = 32u;
     }
     // Workgroups per expert along the weight rows: when the staged image covers K, a workgroup streams several row blocks against
@@ -531,7 +535,7 @@ static int launch_mmq_grouped(mx_stream_t s, const typename P::Bank& b0, const t
         // is a few super-blocks long: a wave with a quarter of them neither fills its load pipeline nor pays for the exchange),
         // as long as that leaves three workgroups per CU.  Expert block over q8 rows, K ranges / row blocks, us: 128 experts, k = 8, hidden
         // 2048, 768: 64 tokens 158 / 145, 128 tokens 220 / 185, 200 tokens 266 / 225; 32 experts, k = 4, hidden 4096, 1536: 32 tokens 140 /
-        // 131, 100 tokens 223 / 187.  Below: 8 tokens there 84 / 96; with 512 workgroups (64 experts of 3072 -> 1024, 3 rows each) 121 / 133.
+        // 131 (experts of equal size 90 / 90), 100 tokens 223 / 187.  Below: 8 tokens there 84 / 96; with 512 workgroups (64 experts of 3072 -> 1024, 3 rows each) 121 / 133.
         constexpr uint32_t WR = NW == 1 ? 4u : 2u;
         if (m.expert_offsets && avg_rows >= 4 && avg_rows <= 16 &&
             (uint64_t)((m.N + 32u * WR - 1u) / (32u * WR)) * E >= 3ull * (uint64_t)cu_count_moe())
