@@ -54,9 +54,9 @@ def test_gemm_k_slices(mx, fmt, M, K, N):
     ("mxfp4", 40, 2880, 160), ("mxfp4", 127, 320, 1100), ("q4_K", 260, 512, 13353), ("q4_K", 64, 2560, 6001), ("mxfp4", 260, 320, 13351),
     ("q8_0", 130, 896, 14335), ("q4_K", 700, 256, 14333), ("mxfp4", 700, 192, 14335)])
 def test_gemm_plans(mx, fmt, M, K, N):
-    """One shape per form a dense launch can take (32 .. 128 tokens x 128 or 256 weight rows, with and without K slices, four-wave
-    workgroups), at odd numbers of chunks, so that slices and the two K halves of a workgroup differ in length, ragged M and N, one
-    row, one chunk and a row that ends half way through a chunk.  Against the fp32-weight product in fp64: the sum of K exact fp16
+    """Forms a dense launch can take, mostly for Q8_0 planes (every form with every loader: test_gemm_every_form_and_loader), at odd
+    numbers of chunks, so that slices and the two K halves of a workgroup differ in length, ragged M and N, one row, one chunk and a
+    row that ends half way through a chunk.  Against the fp32-weight product in fp64: the sum of K exact fp16
     products in fp32, rounded to fp16, as every other case here."""
     from machx_inference_engine_amd import synth
 
@@ -74,6 +74,52 @@ def test_gemm_plans(mx, fmt, M, K, N):
         run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, w.reshape(-1), M, K, N)  # noqa: E731
     got = run()
     check(host(got).astype(np.float32), ref, "gemm %s M=%d K=%d N=%d" % (fmt, M, K, N))
+    assert torch.equal(run(), got), "differs from launch to launch"
+
+
+def any_weights(fmt, N, K, seed):
+    """Random blocks of any dense format with small scales -> (arguments of its GEMM, fp16 values [N, K]).  MXFP4 and "q8_0_soa" as planes."""
+    base = fmt.replace("_soa", "")
+    ofmt = {"q8_0": O.Q8_0, "q4_K": O.Q4_K, "q6_K": O.Q6_K, "mxfp4": O.MXFP4, "q5_K": O.Q5_K, "q4_0": O.Q4_0}[base]
+    elems, size = O.BLOCK_ELEMS[ofmt], O.BLOCK_BYTES[ofmt]
+    rng = np.random.default_rng(seed)
+    b = rng.integers(0, 256, (N * K // elems, size), dtype=np.uint8)
+    if base == "mxfp4":
+        b[:, 0] = rng.integers(118, 124, len(b))                               # E8M0 exponents
+    else:
+        scales = rng.uniform(0.002, 0.01, (len(b), 2)).astype(np.float16).view(np.uint8)
+        at = {"q6_K": slice(208, 210), "q4_K": slice(0, 4), "q5_K": slice(0, 4)}.get(base, slice(0, 2))
+        b[:, at] = scales[:, :at.stop - at.start]
+    values = torch.from_numpy(O.dequant(ofmt, b.reshape(-1), N * K).reshape(N, K)).cuda().half()
+    if base == "mxfp4":
+        return tuple(dev(p) for p in O.repack_mxfp4_to_soa(b.reshape(N, -1))), values
+    if fmt == "q8_0_soa":
+        return tuple(dev(p) for p in O.repack_q8_0_to_soa(b.reshape(N, -1))), values
+    return (dev(b.reshape(-1)),), values
+
+
+# (32-token tiles, 32-row column tiles, K slices or not) -> a shape of whole super-blocks that takes this form and one with K % 128 = 64
+FORMS = [((0, 2, False), (773, 256, 10057), (1, 64, 33)), ((1, 1, False), (4, 256, 33), (1, 192, 33)), ((1, 1, True), (1, 1280, 33), (3, 1216, 35)),
+         ((1, 2, False), (3, 256, 33094), (1, 192, 33098)), ((1, 2, True), (1, 1792, 4623), (1, 1984, 5661)), ((2, 1, False), (747, 256, 1337), (755, 192, 1303)),
+         ((2, 1, True), (693, 1536, 129), (607, 1728, 131)), ((2, 2, False), (777, 256, 4671), (774, 192, 4691)), ((2, 2, True), (33, 3328, 8253), (38, 2368, 11217)),
+         ((3, 1, False), (775, 256, 2443), (773, 192, 2529)), ((3, 1, True), (685, 2048, 257), (653, 1984, 259)), ((3, 2, False), (777, 256, 4881), (785, 192, 4867)),
+         ((3, 2, True), (263, 3840, 3621), (267, 3648, 3689)), ((4, 1, False), (793, 256, 3587), (789, 192, 3823)), ((4, 1, True), (193, 1792, 1581), (201, 1728, 1555)),
+         ((4, 2, False), (685, 256, 8353), (791, 192, 7225)), ((4, 2, True), (709, 7168, 1285), (797, 6976, 1157))]
+
+
+@pytest.mark.parametrize("fmt", ["q4_K", "q6_K", "q8_0_soa", "q8_0", "q4_0", "q5_K", "mxfp4_soa"])
+@pytest.mark.parametrize("form,whole,half", FORMS, ids=["%d-%d%s" % (f[0], f[1], "-slices" * f[2]) for f, _, _ in FORMS])
+def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
+    """Every form of a dense launch with every weight loader, MXFP4 with a row that ends half way through a chunk; the form a shape takes
+    is asked of the library, so that a change of the rule shows.  Against the exact products of the fp16 weights in fp64."""
+    M, K, N = half if fmt == "mxfp4_soa" else whole
+    na, nj, k = mx.ops.gemm_plan(M, K, N, 32 << 20)
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or (na, nj, k > 1) == form, (na, nj, k)
+    wargs, values = any_weights(fmt, N, K, 2500 + M)
+    a = dev(f16(O.normal(2501 + M, (M, K)))).half()
+    run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, *wargs, M, K, N)  # noqa: E731
+    got = run()
+    check(host(got).astype(np.float32), host(a.double() @ values.double().t()), "gemm %s M=%d K=%d N=%d" % (fmt, M, K, N))
     assert torch.equal(run(), got), "differs from launch to launch"
 
 
