@@ -117,7 +117,8 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or (na, nj, k > 1) == form, (na, nj, k)
     wargs, values = any_weights(fmt, N, K, 2500 + M)
     a = dev(f16(O.normal(2501 + M, (M, K)))).half()
-    run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, *wargs, M, K, N)  # noqa: E731
+    ws = torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
+    run = lambda: mx.ops.gemm_ws(fmt, a, wargs, M, K, N, ws)  # noqa: E731
     got = run()
     check(host(got).astype(np.float32), host(a.double() @ values.double().t()), "gemm %s M=%d K=%d N=%d" % (fmt, M, K, N))
     assert torch.equal(run(), got), "differs from launch to launch"

@@ -80,8 +80,8 @@ def test_k_sliced_gemm_static_scratch_equals_workspace_form(mx):
                                        ("q4_0", 64, 1280, 896), ("q5_K", 256, 1792, 1024), ("mxfp4_soa", 40, 1344, 896)])
 def test_gemms_outside_the_shared_scratch_overlap(mx, fmt, M, K, N):
     """Shapes that a workspace would cut in K slices but that the header does not name as users of the shared scratch: calls on two
-    streams give each stream's own bits, through the Python entry points (partial sums of their own) and through the C entry points
-    without a workspace (unsliced)."""
+    streams give each stream's own bits, through the Python entry points (unsliced, or partial sums of their own where the tiles are too
+    many) and through the C entry points without a workspace (unsliced)."""
     ops = mx.ops
     assert ops.gemm_plan(M, K, N)[2] == 1 and ops.gemm_plan(M, K, N, 32 << 20)[2] > 1
     if fmt in ("q4_0", "q5_K"):
