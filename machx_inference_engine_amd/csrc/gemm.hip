@@ -5,16 +5,16 @@
 // i.e. the arithmetic of the reference's XMX route (weights dequantized to fp16,
 // src/ops/gemm_q4k_xmx.cpp:71-111,183-231) and of its dequant + dense-GEMM route
 // (src/model/dense_dispatch.hpp:658-693) without ever materialising the fp16
-// weight matrix: every weight byte is read once per 128-token tile and
-// dequantized in registers straight into MFMA operand fragments.
+// weight matrix: every weight byte is read once per token tile (32 to 128 tokens)
+// and dequantized in registers straight into MFMA operand fragments.
 //
 // Tiling (wave64, v_mfma_f32_32x32x16_f16), K walked in chunks of 128:
 //   workgroup = 4 waves, 128 tokens x (4 x 64) weight rows, two per CU; wave = 128 tokens x 64 rows = 4 x 2 MFMA tiles
 //               (128 accumulator VGPRs).  Dense launches that would not fill the chip so: 8 waves, one workgroup per CU, the
 //               two halves of K (or of a K slice) side by side, 32 .. 128 tokens x 128 or 256 weight rows (gemm_plan);
-//   tokens    : the fp16 A chunk [128 x 128] is staged in LDS (double buffered, unpadded
+//   tokens    : the fp16 A chunk [tokens x 128] is staged in LDS (double buffered, unpadded
 //               256-byte rows whose 16-byte columns are XOR-swizzled by the row number, so a
-//               fragment read is bank-conflict free) and shared by the four waves;
+//               fragment read is bank-conflict free) and shared by four waves;
 //   weights   : lane (r = lane%32, h = lane/32) of a wave owns weight row r of a tile
 //               and the 64 consecutive elements [64h, 64h+64) of the chunk: it loads
 //               them from global as 128-bit words (32 B of Q4_K nibbles or 64 B of
@@ -1117,9 +1117,10 @@ __device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA, NJ>& t, const u
 // which covers the latency when a chunk carries 64 MFMAs per wave; a tile with one or two live token tiles
 // finishes a chunk in a fraction of the memory latency, so it keeps two chunks of weights in flight.  At the
 // end of chunk c the A rows of chunk c+1 must be in LDS: they are older than the weight loads issued after
-// them in the same iteration, of which there are at least 2 ceil(sizeof(Raw) / 16) (a load instruction
-// brings at most 16 bytes per lane), so waiting until at most that many loads are outstanding is enough
-// whatever the compiler made of QF::load.
+// them in the same iteration (load_to_lds16 is volatile asm that clobbers memory, so no load moves in front of
+// it), of which there are at least GemmLanes::loads (NJ ceil(sizeof(Raw) / 16) where the producer does not say:
+// a load instruction brings at most 16 bytes per lane), so waiting until at most that many loads are outstanding
+// is enough whatever the compiler made of the producer's loads.
 // KW = 2: a workgroup of eight waves, waves 4 - 7 walking the second half of K over A buffers of their own (`lds_raw` is
 // then this half's buffer pair, `lds_red` the start of the workgroup's LDS); their sums meet the first half's in LDS
 // before the epilogue.  The first half runs `n_chunks_max` chunks, the second as many or one fewer; every chunk ends in one
@@ -1280,8 +1281,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
 
 #undef CHUNK
     if constexpr (KW == 2) {
-        // The second K half hands its sums over through LDS (32 KB per wave, the whole allocation for four waves: both
-        // halves are done with their A buffers behind the first barrier) and leaves; the first half adds them to its own.
+        // The second K half hands its sums over through LDS (4 NA NJ KB per wave, over the A buffers: both halves are done
+        // with theirs behind the first barrier) and leaves; the first half adds them to its own.
         typedef float f32x4_t __attribute__((ext_vector_type(4)));
         const bool second = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)) != 0u;
         if (n_chunks < n_chunks_max) asm volatile("s_barrier" ::: "memory");   // one chunk, and so one barrier, fewer than the first half
@@ -1353,7 +1354,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
             }
             __syncthreads();
         }
-        // `put(i, v, row, j, o)` for every live output of the lane, o already times the row's weight
+        // `put(row, j, o)` for every live output of the lane (row without the lane's share), o already times the row's weight
         auto each = [&](auto put) {
 #pragma unroll
             for (int i = 0; i < NA; ++i)
@@ -1507,7 +1508,7 @@ __device__ __forceinline__ bool find_grouped_tile(const uint32_t* expert_offsets
     return found;
 }
 
-// Chunks of weight words in flight per wave of an eight-wave workgroup: as many as the registers beside 32 NA accumulators hold.
+// Chunks of weight words in flight per wave of an eight-wave workgroup: as many as the registers beside its 16 NA NJ accumulators hold.
 template <int NA, int NJ>
 constexpr int gemm_k2_depth() { return NA * NJ <= 4 ? 2 : 1; }
 
@@ -1648,11 +1649,13 @@ static int gemm_cu_count() {
 // tiles of 128 x 256.  The second is the better one where there are tiles enough to fill the chip several times; below that the
 // chip is filled by small tiles and by K slices, each of which has its price: a narrow tile reads the activation rows more often,
 // a short one dequantizes the same weights for fewer tokens, a slice writes fp32 partial sums that a second launch adds.  The
-// form with the least modelled time is taken.  The model is microseconds, fitted to 468 measured shapes (Q4_K, Q6_K, Q8_0 planes,
-// K and N 2048 .. 14336, M 17 .. 4096, cold weights) with one set of constants for all formats; the plans it takes are 0.4 % slower
-// than the best plan of each shape on average, 13 % at worst but for one shape.  Where it moves launches from the rule before
-// (128-token tiles, K slices of four-wave workgroups until the CUs are covered), us with the partial-sum launch:
-// Q4_K 4096 -> 14336: 20 tokens 31 -> 17.7, 77 tokens 32 -> 25.7, 200 tokens 58 -> 41; Q6_K 14336 -> 4096: 77 tokens 52 -> 34.5.
+// form with the least modelled time is taken.  The model is microseconds, fitted to launches of Q4_K, Q6_K and Q8_0 planes (K and N
+// 2048 .. 14336, M 17 .. 4096), with one set of constants for all formats.  Against every other plan, 896 shapes of the seven formats,
+// M 1 .. 4096: 2.8 % slower than the best one on average, 22 to 38 % at worst by format (launches of 10 to 27 us; Q6_K 2048 -> 6144, one
+// row: 15.2, best 11.0).  Against the rule before it (128-token tiles, K slices of four-wave workgroups until the CUs are covered), us
+// with the partial-sum launch: Q4_K 4096 -> 14336: 17 tokens 26.9 -> 18.5, 77 tokens 34.4 -> 25.0, 200 tokens 53 -> 40; Q6_K 14336 -> 4096:
+// 77 tokens 54.9 -> 34.3; of 1000 shapes one is slower by more than 1.5 %: Q5_K 14336 -> 4096, 2048 tokens, 313 -> 327, where the
+// eight-wave form spills.
 struct GemmPlan {
     uint32_t na;        // 32-token tiles per workgroup tile, 0: the four-wave form
     uint32_t nj;        // 32-row column tiles per wave
