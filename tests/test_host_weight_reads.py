@@ -173,9 +173,10 @@ def kernels(name, before):
     ("moe.hip", "// ---------------------------------------------------------------- fp16-activation decode", MOE),
     ("gemv.hip", "// true if the launch was made: one matrix, one token", DENSE)], ids=["experts", "dense"])
 def test_reads_stay_inside_the_weights(tmp_path, name, before, program):
+    # -O0: a load whose value the stand-ins drop is made all the same
     src, exe = tmp_path / "t.cpp", tmp_path / "t"
     src.write_text(SHIM + kernels(name, before) + CHECK + program)
-    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "-x", "c++", "-D__HIP_PLATFORM_AMD__", "-std=c++17", "-O1", "-w", "-I", CSRC,
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "-x", "c++", "-D__HIP_PLATFORM_AMD__", "-std=c++17", "-O0", "-w", "-I", CSRC,
                     "-I", "/opt/rocm/include", str(src), "-o", str(exe)], check=True)
     p = subprocess.run([str(exe)], capture_output=True, text=True)
     assert p.returncode == 0, p.stdout + p.stderr
