@@ -355,7 +355,8 @@ int mx_gemm_mxfp4_soa_ws(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, 
 /* How a dense quant-GEMM of this shape is cut on the current device (host only, nothing is launched): plan[0] = 32-token
  * tiles per workgroup tile of an eight-wave workgroup (1..4; 0: four-wave workgroups over 128 x 256), plan[1] = 32-row
  * column tiles per wave (1 or 2), plan[2] = K slices (1: no scratch is used).  own_ws = 0: the forms without a workspace;
- * else the *_ws forms with a workspace of ws_bytes.  */
+ * else the *_ws forms with a workspace of ws_bytes.  Launches of more than 256 tokens may run over 256 x 256 tiles, unsliced
+ * and without scratch, in place of this plan, by format.  */
 int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* plan);
 /* Q4_0 weights through the same kernel: gemm_q4_0 / gemm_q4_0_xmx  include/ie/ops.hpp:530-534, src/ops/gemv_q4_0.cpp,
  * src/ops/gemm_q4k_xmx.cpp:418-522; K % 128 == 0, W 2-byte aligned.  */

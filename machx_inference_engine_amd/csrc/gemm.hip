@@ -11,7 +11,8 @@
 // Tiling (wave64, v_mfma_f32_32x32x16_f16), K walked in chunks of 128:
 //   workgroup = 4 waves, 128 tokens x (4 x 64) weight rows, two per CU; wave = 128 tokens x 64 rows = 4 x 2 MFMA tiles
 //               (128 accumulator VGPRs).  Dense launches that would not fill the chip so: 8 waves, one workgroup per CU, the
-//               two halves of K (or of a K slice) side by side, 32 .. 128 tokens x 128 or 256 weight rows (gemm_plan);
+//               two halves of K (or of a K slice) side by side, 32 .. 128 tokens x 128 or 256 weight rows (gemm_plan).  Large
+//               ones may run 256 tokens x 256 rows in four waves, one workgroup per CU (gemm_tall);
 //   tokens    : the fp16 A chunk [tokens x 128] is staged in LDS (double buffered, unpadded
 //               256-byte rows whose 16-byte columns are XOR-swizzled by the row number, so a
 //               fragment read is bank-conflict free) and shared by four waves;
@@ -54,12 +55,20 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 // fp16 (v_cvt_pk_f16_f32).  The power-of-two rescale of `scale` is exact, so the value is
 // bit-identical to converting the code to float first.  Left to itself the compiler fuses
 // convert + fma + convert into v_fma_mixlo/mixhi_f16, which measures about half the rate of the
-// other VALU ops next to MFMA work on this chip; the two fp32 values are made opaque to keep the
-// halves apart.  The pack itself stays the compiler's: a matrix instruction must not read a vector
-// result for two wait states, and only an instruction it knows gets them (the pack written as
-// inline asm gave wrong fragments wherever it came last before its matrix instruction and wrote
-// the first register of the operand).
+// other VALU ops next to MFMA work on this chip; the canonicalisation of the two fp32 values (no
+// instruction: the multiply-add's result is canonical) keeps the halves apart.  An empty asm on them
+// does so too, but the compiler then guards every value against hazards it cannot see (4096 tokens,
+// 14336 -> 4096, Q6_K, 128-token tiles: 589 us with it, 567 without).  The pack itself stays the
+// compiler's: a matrix instruction must not read a vector result for two wait states, and only an
+// instruction it knows gets them (the pack written as inline asm gave wrong fragments wherever it
+// came last before its matrix instruction and wrote the first register of the operand).
 __device__ __forceinline__ uint32_t mix_pair(_Float16 x0, _Float16 x1, float scale, float off) {
+    const float f0 = __builtin_canonicalizef(__builtin_fmaf((float)x0, scale, off)), f1 = __builtin_canonicalizef(__builtin_fmaf((float)x1, scale, off));
+    return pack_h2(f0, f1);
+}
+// The same with the empty asm, for Q5_K: its 128-token forms are short of registers and spill more with the looser schedule that the
+// canonicalisation allows (4096 -> 14336, 1024 tokens: 167 us with the asm, 176 without).
+__device__ __forceinline__ uint32_t mix_pair_tight(_Float16 x0, _Float16 x1, float scale, float off) {
     float f0 = __builtin_fmaf((float)x0, scale, off), f1 = __builtin_fmaf((float)x1, scale, off);
     asm("" : "+v"(f0), "+v"(f1));
     return pack_h2(f0, f1);
@@ -658,8 +667,8 @@ struct GemmQ5K {
         const uint32_t code = ((sub ? w >> 4 : w) & 0x0F0F0F0Fu) | (((qh >> (dc.bit + sub)) & 0x01010101u) << 4);
         const half2_t ev = as_h2(code & 0x00FF00FFu), od = as_h2((code >> 8) & 0x00FF00FFu);   // bytes (0,2), (1,3)
         const float d1 = dc.d1[sub], c1 = dc.c1[sub];
-        f.u[2 * HF] = mix_pair(ev.x, od.x, d1, c1);
-        f.u[2 * HF + 1] = mix_pair(ev.y, od.y, d1, c1);
+        f.u[2 * HF] = mix_pair_tight(ev.x, od.x, d1, c1);
+        f.u[2 * HF + 1] = mix_pair_tight(ev.y, od.y, d1, c1);
     }
     template <int S>
     __device__ static __forceinline__ void frag(const Raw& r, const Dec& dc, Frag& f) {
@@ -867,6 +876,7 @@ struct GemmArgs {
     uint32_t M, K, N, E;
     uint32_t tiles_m, tiles_n;        // dense tile grid; grouped: tiles_m is an upper bound
     uint32_t k_split;                 // dense only: K slices per output tile (above 1: fp32 partial sums go to split_acc)
+    uint32_t whole;                   // 256-token tiles: tiles that run whole, those behind them as two column halves
     float* split_acc;                 // [k_split][M][N] partial sums of a K-sliced launch
     const float* bias0;               // [E][N] fp32 or NULL: gate bias (GEMM_MOE_GATE_UP_OAI), down bias (GEMM_MOE_DOWN)
     const float* bias1;               // [E][N] up bias
@@ -1515,7 +1525,7 @@ constexpr int gemm_k2_depth() { return NA * NJ <= 4 ? 2 : 1; }
 // NI = 32-token tiles per workgroup tile.  KW = 1: four waves, 128 tokens, two workgroups per CU.  KW = 2: eight waves, the two
 // halves of the K slice side by side, one workgroup per CU, 32 to 128 tokens.
 template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
-__global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kernel(typename QF::Bank bank0, typename QF::Bank bank1, GemmArgs g) {
+__global__ __launch_bounds__(kGemmThreads * KW, (KW == 2 || NI == 8) ? 1 : 2) void gemm_kernel(typename QF::Bank bank0, typename QF::Bank bank1, GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
     constexpr uint32_t BM = 32u * NI;   // tokens per tile
     constexpr bool GATE_UP = MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI;
@@ -1528,8 +1538,19 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kerne
     const uint32_t ksplit = (MODE == GEMM_DENSE) ? g.k_split : 1u;   // workgroups per output tile (K slices)
     const uint32_t total = g.tiles_m * g.tiles_n * ksplit;
     const uint32_t per_xcd = (total + 7) / 8;
-    const uint32_t lin_ks = (MODE == GEMM_DENSE) ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
-    if ((MODE == GEMM_DENSE && (blockIdx.x >> 3) >= per_xcd) || lin_ks >= total) return;
+    uint32_t lin_ks = (MODE == GEMM_DENSE) ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x, half = 0;
+    bool halves = false;
+    if constexpr (NI == 8) {
+        // the whole tiles, and behind them the column halves of the rest, each dealt to the XCDs in contiguous ranges
+        const uint32_t whole8 = (g.whole + 7u) / 8u * 8u, per_w = whole8 / 8u, per_h = (2u * (total - g.whole) + 7u) / 8u;
+        halves = blockIdx.x >= whole8;
+        const uint32_t b = blockIdx.x - (halves ? whole8 : 0u), in = (b & 7u) * (halves ? per_h : per_w) + (b >> 3);
+        if (in >= (halves ? 2u * (total - g.whole) : g.whole)) return;
+        lin_ks = halves ? g.whole + in / 2u : in;
+        half = halves ? in % 2u : 0u;
+    } else {
+        if ((MODE == GEMM_DENSE && (blockIdx.x >> 3) >= per_xcd) || lin_ks >= total) return;
+    }
     const uint32_t linear = lin_ks / ksplit, ks = lin_ks - linear * ksplit;
     uint32_t tm, tn;
     {
@@ -1580,6 +1601,9 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kerne
             const uint32_t kw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)), first = (n_slice + 1u) / 2u;
             gemm_tile<QF, MODE, NI, gemm_k2_depth<NI, NJ>(), 2, NJ>(g, w0, w1, row_lo, row_hi, n_base, lds_raw + kw * (2u * BM * kBK * 2u), c0 + kw * first,
                                                                       kw ? n_slice - first : first, ks, 0, lds_raw, first);
+        } else if (NI == 8 && halves) {
+            const uint32_t n_half = tn * BN + half * (BN / 2u) + wave * (BN / 8u);
+            if (tn * BN + half * (BN / 2u) < g.N) gemm_tile<QF, MODE, NI, 1, 1, 1>(g, w0, w1, row_lo, row_hi, n_half, lds_raw, c0, n_slice, ks);
         } else {
             gemm_tile<QF, MODE, NI, 1>(g, w0, w1, row_lo, row_hi, n_base, lds_raw, c0, n_slice, ks);
         }
@@ -1617,6 +1641,15 @@ __global__ __launch_bounds__(kGemmThreads * KW, KW == 2 ? 1 : 2) void gemm_kerne
 }
 
 // ---------------------------------------------------------------- host side
+static int gemm_cu_count() {
+    static int n = 0;
+    if (!n) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    }
+    return n;
+}
+
 template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
 static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound) {
     constexpr uint32_t BN = (MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI) ? 128 : 128 * NJ, BM = 32u * NI;
@@ -1625,7 +1658,13 @@ static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const type
     g.tiles_m = (MODE == GEMM_DENSE) ? (g.M + BM - 1) / BM : rows_bound / BM + g.E;   // grouped: an upper bound, workgroups past the real count leave at once
     if (MODE != GEMM_DENSE || g.k_split == 0) g.k_split = 1;
     const uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.k_split;
-    const uint64_t grid = (total + 7) / 8 * 8;
+    uint64_t grid = (total + 7) / 8 * 8;
+    if constexpr (NI == 8) {
+        // a last round that covers at most half of the CUs runs as twice as many halves
+        const uint64_t cus = (uint64_t)gemm_cu_count(), rest = total % cus;
+        g.whole = (uint32_t)(2 * rest <= cus ? total - rest : total);
+        grid = ((uint64_t)g.whole + 7) / 8 * 8 + (2 * (total - g.whole) + 7) / 8 * 8;
+    }
     if (grid > 0x7FFFFFFFull) return MX_ERR_SHAPE;
     if constexpr (lds > kLdsDefaultLimit) {
         static LdsLimit limit;
@@ -1633,15 +1672,6 @@ static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const type
     }
     hipLaunchKernelGGL((gemm_kernel<QF, MODE, NI, KW, NJ>), dim3((uint32_t)grid), dim3(kGemmThreads * KW), lds, as_stream(s), b0, b1, g);
     return launch_status();
-}
-
-static int gemm_cu_count() {
-    static int n = 0;
-    if (!n) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    }
-    return n;
 }
 
 // How a dense launch is cut.  Two forms: eight-wave workgroups that walk the two halves of their K slice, one per CU, over tiles
@@ -1661,13 +1691,14 @@ struct GemmPlan {
     uint32_t nj;        // 32-row column tiles per wave
     uint32_t k_split;
 };
-static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus) {
+static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus, double* modelled = nullptr) {
     const uint64_t n_chunks = (K + kBK - 1) / kBK;
     auto up = [](uint64_t a, uint64_t b) { return (a + b - 1) / b; };
     GemmPlan best{0, 2, 1};
     const uint64_t tiles4 = up(M, 128) * up(N, 256), full = tiles4 / (2 * cus), rest = tiles4 % (2 * cus);
     // a round of two workgroups per CU, and a last one that may have one per CU
     double t_best = (double)(full + (rest > cus ? 1 : 0)) * (5.0 + 3.74 * (double)n_chunks) + (rest && rest <= cus ? 5.0 + 2.37 * (double)n_chunks : 0.0);
+    if (modelled) *modelled = t_best;
     if (n_chunks < 2) return best;
     for (uint64_t na = 1; na <= 4 && na <= up(M, 32); ++na)
         for (uint64_t nj = 1; nj <= 2; ++nj) {
@@ -1682,7 +1713,24 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint
                 }
             }
         }
+    if (modelled) *modelled = t_best;
     return best;
+}
+
+// Tiles of 256 tokens x 256 weight rows, four waves, one workgroup per CU with the accumulators in the other half of the registers:
+// a weight is dequantized for twice as many tokens, which matters most where that is most work (4096 tokens, 14336 -> 4096, us: Q6_K
+// 567 -> 480, Q4_K 449 -> 420, Q8_0 planes 449 -> 421).  But the rounds are coarse, and one workgroup alone on a CU shows the start and
+// end of a tile (K = 1024, 4096 tokens, 4096 rows, Q4_K: 43 us in four-wave workgroups, 50 so; 4096 -> 14336, 3.5 rounds: 451 and 473);
+// a last round that would leave more than half of the CUs idle runs as column halves.  Taken in place of the plan above where its
+// modelled time (microseconds, fitted like the plan's, K from 2048 on) is less; `cost` = the format's time so against its time in the
+// plan's forms, 1 for Q4_K and Q8_0 (Q6_K 4096 -> 14336: 1024 tokens 185 -> 164, 2048 tokens 348 -> 318, 4096 tokens 608 -> 558).
+template <class QF> constexpr double gemm_tall_cost = 1.0;
+template <> constexpr double gemm_tall_cost<GemmQ6K> = 0.83;
+static bool gemm_tall(uint64_t M, uint64_t K, uint64_t N, uint64_t cus, double cost, double t_plan) {
+    const uint64_t n_chunks = (K + kBK - 1) / kBK, tiles = ((M + 255) / 256) * ((N + 255) / 256), full = tiles / cus, rest = tiles % cus;
+    if (M <= 256 || n_chunks < 16) return false;
+    const double whole = 14.0 + 3.62 * (double)n_chunks, halves = 14.0 + 2.6 * (double)n_chunks;
+    return cost * ((double)full * whole + (rest == 0 ? 0.0 : 2 * rest <= cus ? halves : whole)) < t_plan;
 }
 
 // Floats of the library's scratch that a launch without a caller's workspace may use.  Calls that overlap on one device race on it, so
@@ -1697,7 +1745,12 @@ static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typenam
                        const SplitWs* caller_ws = nullptr) {
     if constexpr (MODE == GEMM_DENSE) {
         const uint64_t cus = (uint64_t)gemm_cu_count();
-        const GemmPlan p = gemm_plan(g.M, g.K, g.N, caller_ws ? caller_ws->elems : gemm_library_scratch(g.M, g.K, g.N, cus), cus);
+        double t_plan = 0.0;
+        const GemmPlan p = gemm_plan(g.M, g.K, g.N, caller_ws ? caller_ws->elems : gemm_library_scratch(g.M, g.K, g.N, cus), cus, &t_plan);
+        if (gemm_tall(g.M, g.K, g.N, cus, gemm_tall_cost<QF>, t_plan)) {
+            g.k_split = 1;
+            return launch_gemm_ni<QF, MODE, 8>(s, b0, b1, g, rows_bound);
+        }
         g.k_split = p.k_split;
         if (p.k_split > 1) {
             if (caller_ws) {

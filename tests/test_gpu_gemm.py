@@ -124,6 +124,20 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     assert torch.equal(run(), got), "differs from launch to launch"
 
 
+@pytest.mark.parametrize("fmt,M,K,N", [("q6_K", 1100, 2048, 13000), ("q6_K", 1600, 2048, 12900), ("q4_K", 1100, 12288, 13000), ("q8_0_soa", 1100, 12288, 13000),
+                                       ("q8_0", 1100, 12288, 13000), ("q4_0", 1100, 12288, 13000), ("q5_K", 1100, 12288, 13000), ("mxfp4_soa", 1100, 12224, 13000)])
+def test_gemm_256_token_tiles(mx, fmt, M, K, N):
+    """The tiles of 256 tokens (gemm_tall in csrc/gemm.hip; 256 CUs) with every weight loader, ragged in tokens and columns; the second shape
+    ends in column halves, one of them past N; MXFP4 in a row that ends half way through a chunk.  The sums run over K in one piece: against the
+    exact products of the fp16 weights in fp64, as every other form."""
+    wargs, values = any_weights(fmt, N, K, 2600 + M)
+    a = dev(f16(O.normal(2601 + M, (M, K)))).half()
+    run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, *wargs, M, K, N)  # noqa: E731
+    got = run()
+    check(host(got).astype(np.float32), host(a.double() @ values.double().t()), "gemm %s M=%d K=%d N=%d" % (fmt, M, K, N))
+    assert torch.equal(run(), got), "differs from launch to launch"
+
+
 @pytest.mark.parametrize("M,K,N", [(128, 128, 256), (260, 768, 2048), (77, 2048, 768)])
 def test_gemm_q8_0_soa(mx, M, K, N):
     W = weights(O.Q8_0, 2100 + N, N, K)
