@@ -48,7 +48,7 @@ const char* mx_status_string(int status);
 int mx_last_hip_error(void);  /* hipError_t of the last MX_ERR_LAUNCH on this thread */
 int mx_version(void);
 /* Optional set-up for the current device: resolves the addresses of the library's per-device scratch arrays (see the
- * batched GEMVs and mx_gemm_* below) and raises the packing kernel's LDS limit, so that no first launch does it.  Callers that record HIP
+ * batched GEMVs and mx_gemm_* below), so that no first launch does it.  Callers that record HIP
  * graphs call it once per device before capturing; everyone else may leave it to the first launch.  */
 int mx_init(void);
 

@@ -29,8 +29,7 @@ int mx_version(void) { return 110; }
 
 int mx_init(void) {
     if (int rc = mxq::gemv_init_device()) return rc;
-    if (int rc = mxq::gemm_init_device()) return rc;
-    return mxq::routing_init_device();
+    return mxq::gemm_init_device();
 }
 
 }  // extern "C"

@@ -86,10 +86,9 @@ inline int raise_lds_limit(const void* kernel, LdsLimit& slot, uint32_t limit) {
 int launch_gemv_q6_planes(hipStream_t st, int nseg, const void* x_q8, const uint8_t* const* lo, const uint8_t* const* hi, const int8_t* const* sc,
                           const uint16_t* const* d, uint16_t* const* y, uint32_t K, uint32_t N);
 
-// per-device set-up of the translation units that own scratch arrays or raise an LDS limit (mx_init)
+// per-device set-up of the translation units that own scratch arrays (mx_init)
 int gemv_init_device();
 int gemm_init_device();
-int routing_init_device();
 
 }  // namespace mxq
 

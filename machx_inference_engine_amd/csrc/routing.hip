@@ -250,188 +250,105 @@ __global__ void pack_decode_kernel(const int32_t* topk_idx, const half_t* topk_w
     }
 }
 
-// T tokens, up to kPackMaxExperts experts: stable counting sort of the T*K slots by expert id in one workgroup.  Wave w owns a
-// contiguous range of the slots.  Count: 64 slots at a time, the lanes of one expert are found with one ballot per id bit, a
-// slot's rank among its wave's slots of that expert is kept in tk_to_packed.  Scan: per expert over the waves, then over the
-// experts.  Place: every slot knows its position; the inverse (position -> slot) is built in LDS when it fits (`staged`: u16
-// slot and the weight of every position), so that every global store is coalesced, and scattered straight to memory else.
-// One CU does it because the work is small and serial in the experts' totals: 16384 slots, 128 experts 16.5 us (three
-// launches, in which every expert's workgroup read all slots, took 41), 128 slots of 32 experts 3.7 us (5.7).
-constexpr uint32_t kPackMaxExperts = 1024;
-constexpr uint32_t kPackLdsMax = 152u * 1024u;
+// T tokens: stable counting sort of the T*K slots by expert id, in one launch.  Workgroup g sorts the slots of the Q experts
+// from e0 = Q g on: it reads all ids, its waves a contiguous range each, counts the slots of every one of its experts (a
+// ballot each) and those of all experts below e0, which is where its own begin; the counts of the waves meet in LDS, and in a
+// second round over its ids a lane whose slot is one of the workgroup's knows its place.  So nothing passes between workgroups, at the
+// price of reading the ids E / Q times, from L2.  With at most R = 4 or 16 slots a lane the ids stay in registers
+// between the rounds (R = 0: read again).  One expert a workgroup up to 128 experts (128 experts, 16384 slots 10.5 us on cold caches,
+// four experts a workgroup 14.6), four beyond, where the ids would be read too often.  Bound by the vector instructions per 64 slots.  us, one
+// workgroup that ranks the slots of all experts with a ballot per id bit (bound by the pipes of its one CU) / this: 32 experts, 128
+// slots 4.7 / 4.0; 128 experts, 2664 slots 6.9 / 4.7, 16384 slots 17.4 / 7.4, 65536 slots 101 / 21; 256 experts, 16384 slots 18.7 / 10.9;
+// 1024 experts, 256 slots 10.2 / 3.7, 36000 slots 72 / 16.
+template <int R, uint32_t Q>
 __global__ __launch_bounds__(1024) void pack_kernel(const int32_t* __restrict__ topk_idx, const uint16_t* __restrict__ topk_w, uint32_t n, uint32_t K, uint32_t E,
-                                                    uint32_t id_bits, uint32_t staged, uint32_t* __restrict__ expert_offsets, int32_t* __restrict__ sorted_idx,
-                                                    uint16_t* __restrict__ weights_packed, uint32_t* tk_to_packed) {
-    extern __shared__ __align__(16) uint32_t pack_lds[];
+                                                    uint32_t* __restrict__ expert_offsets, int32_t* __restrict__ sorted_idx,
+                                                    uint16_t* __restrict__ weights_packed, int32_t* __restrict__ tk_to_packed) {
+    __shared__ uint32_t counts[16][Q + 1];   // [wave]: slots of the Q experts, slots of experts below
     const uint32_t tid = threadIdx.x, lane = tid & 63u, n_waves = blockDim.x / 64u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    uint32_t* hist = pack_lds;                       // [n_waves][E]: counts, then positions of the wave's first slot of an expert
-    uint32_t* base = hist + n_waves * E;             // [E + 1]
-    uint16_t* slot_s = reinterpret_cast<uint16_t*>(base + E + 1);   // staged: [n] slot and [n] weight of every position
-    uint16_t* w_s = slot_s + n;
-    for (uint32_t i = tid; i < n_waves * E; i += blockDim.x) hist[i] = 0u;
-    __syncthreads();
-    const uint32_t seg = (n + n_waves * 64u - 1u) / (n_waves * 64u) * 64u, lo = wave * seg < n ? wave * seg : n, hi = lo + seg < n ? lo + seg : n;
-    uint32_t* own = hist + wave * E;
-    constexpr int U = 4;
-    for (uint32_t c = lo; c < hi; c += 64u * U) {
-        uint32_t id[U];
+    const uint32_t e0 = blockIdx.x * Q, n_own = E - e0 < Q ? E - e0 : Q;
+    const uint32_t batches = (n + 63u) / 64u, per = (batches + n_waves - 1u) / n_waves;   // of 64 slots; a wave's
+    const uint64_t lo64 = (uint64_t)wave * per * 64u, hi64 = lo64 + (uint64_t)per * 64u;
+    const uint32_t lo = lo64 < n ? (uint32_t)lo64 : n, hi = hi64 < n ? (uint32_t)hi64 : n;
+    constexpr int U = R ? R : 4;
+    uint32_t id[U];
+    auto load = [&](uint32_t c) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t i = c + 64u * u + lane;
-            id[u] = i < hi ? (uint32_t)topk_idx[i] : 0xFFFFFFFFu;
+            id[u] = i < hi ? (uint32_t)topk_idx[i] : 0xFFFFFFFFu;   // no expert's: slots without an expert of the bank are left out
         }
+    };
+    uint32_t cnt[Q] = {}, below = 0;
+    auto count = [&]() {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint32_t i = c + 64u * u + lane;
-            const bool valid = id[u] < E;                                  // slots without an expert of the bank are left out
-            const unsigned long long ok = __ballot(valid);
-            uint32_t s_lo = (uint32_t)ok, s_hi = (uint32_t)(ok >> 32);     // lanes whose id agrees with this lane's in the bits seen so far
-            for (uint32_t b = 0; b < id_bits; ++b) {
-                const uint32_t t = (uint32_t)((int)(id[u] << (31u - b)) >> 31);   // all ones where the bit is set
-                const unsigned long long m = __ballot(t != 0u);
-                s_lo &= ~((uint32_t)m ^ t);
-                s_hi &= ~((uint32_t)(m >> 32) ^ t);
-            }
-            const uint32_t before = (uint32_t)__builtin_amdgcn_mbcnt_hi(s_hi, __builtin_amdgcn_mbcnt_lo(s_lo, 0u));
-            if (valid) {
-                const uint32_t first = own[id[u]];
-                __builtin_amdgcn_wave_barrier();   // every lane has read its count before one of them moves it
-                if (before == 0u) own[id[u]] = first + (uint32_t)(__builtin_popcount(s_lo) + __builtin_popcount(s_hi));
-                tk_to_packed[i] = first + before;
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-    __syncthreads();
-    for (uint32_t e = tid; e < E; e += blockDim.x) {
-        uint32_t s = 0;
-#pragma unroll 4
-        for (uint32_t w = 0; w < n_waves; ++w) {
-            const uint32_t c = hist[w * E + e];
-            hist[w * E + e] = s;
-            s += c;
-        }
-        base[e + 1] = s;
-    }
-    if (tid == 0) base[0] = 0u;
-    __syncthreads();
-    if (wave == 0) {
-        uint32_t run = 0;
-        for (uint32_t e0 = 0; e0 < E; e0 += 64u) {
-            uint32_t v = e0 + lane < E ? base[e0 + lane + 1u] : 0u;
+            below += (uint32_t)__popcll(__ballot(id[u] < e0));
 #pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const uint32_t o = (uint32_t)__shfl_up((int)v, d);
-                if (lane >= (uint32_t)d) v += o;
-            }
-            if (e0 + lane < E) base[e0 + lane + 1u] = run + v;
-            run += (uint32_t)__shfl((int)v, 63);
+            for (uint32_t q = 0; q < Q; ++q) cnt[q] += (uint32_t)__popcll(__ballot(id[u] == e0 + q));
+        }
+    };
+    if constexpr (R > 0) {
+        load(lo);
+        count();
+    } else {
+        for (uint32_t c = lo; c < hi; c += 64u * U) {
+            load(c);
+            count();
         }
     }
+    if (lane <= Q) {
+        uint32_t v = below;
+#pragma unroll
+        for (uint32_t q = 0; q < Q; ++q) v = lane == q ? cnt[q] : v;
+        counts[wave][lane] = v;
+    }
     __syncthreads();
-    for (uint32_t e = tid; e <= E; e += blockDim.x) expert_offsets[e] = base[e];
-    for (uint32_t c = lo; c < hi; c += 64u * U) {
-        uint32_t id[U], rank[U];
-        uint16_t wt[U];
+    // lane q <= Q: the sum over all waves and the one over the waves before this one
+    uint32_t all = 0, before = 0;
+    for (uint32_t w = 0; w < n_waves; ++w) {
+        const uint32_t v = lane <= Q ? counts[w][lane] : 0u;
+        all += v;
+        before += w < wave ? v : 0u;
+    }
+    uint32_t at[Q], first = (uint32_t)__builtin_amdgcn_readlane((int)all, (int)Q);
+#pragma unroll
+    for (uint32_t q = 0; q < Q; ++q) {
+        if (tid == 0 && q < n_own) expert_offsets[e0 + q] = first;
+        at[q] = first + (uint32_t)__builtin_amdgcn_readlane((int)before, (int)q);
+        if (q < n_own) first += (uint32_t)__builtin_amdgcn_readlane((int)all, (int)q);
+    }
+    if (tid == 0 && e0 + n_own == E) expert_offsets[E] = first;
+    const bool small = n <= 65536u;
+    const uint32_t inv = K > 1u ? 0xFFFFFFFFu / K + 1u : 0u;   // slot / K by a multiplication: exact below 2^16
+    auto place = [&](uint32_t c) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint32_t i = c + 64u * u + lane;
-            id[u] = i < hi ? (uint32_t)topk_idx[i] : 0xFFFFFFFFu;
-            rank[u] = i < hi ? tk_to_packed[i] : 0u;
-            wt[u] = i < hi ? topk_w[i] : (uint16_t)0;
-        }
+            const uint32_t i = c + 64u * u + lane, rel = id[u] - e0;
+            if (__ballot(rel < n_own) == 0ull) continue;
+            uint32_t p = 0;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t i = c + 64u * u + lane;
-            if (id[u] < E) {
-                const uint32_t p = base[id[u]] + own[id[u]] + rank[u];
-                tk_to_packed[i] = p;
-                if (staged) {
-                    slot_s[p] = (uint16_t)i;
-                    w_s[p] = wt[u];
-                } else {
-                    sorted_idx[p] = (int32_t)(i / K);
-                    weights_packed[p] = wt[u];
-                }
+            for (uint32_t q = 0; q < Q; ++q) {
+                const unsigned long long m = __ballot(rel == q);
+                const uint32_t r = at[q] + (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                p = rel == q ? r : p;
+                at[q] += (uint32_t)__popcll(m);
+            }
+            if (rel < n_own) {
+                sorted_idx[p] = (int32_t)(K == 1u ? i : small ? __umulhi(i, inv) : i / K);
+                weights_packed[p] = topk_w[i];
+                tk_to_packed[i] = (int32_t)p;
             }
         }
-    }
-    if (!staged) return;
-    __syncthreads();
-    for (uint32_t p = tid; p < base[E]; p += blockDim.x) {
-        sorted_idx[p] = (int32_t)((uint32_t)slot_s[p] / K);
-        weights_packed[p] = w_s[p];
-    }
-}
-
-static int raise_pack_lds() {
-    static LdsLimit limit;
-    return raise_lds_limit(reinterpret_cast<const void*>(&pack_kernel), limit, kPackLdsMax);
-}
-int routing_init_device() {
-    (void)raise_pack_lds();   // refused: the launches take the form that needs no more than the default
-    return MX_OK;
-}
-
-// More experts than that: the same sort, in three launches.
-//   count : workgroup e counts its slots                      -> expert_offsets[e + 1]
-//   scan  : one workgroup turns the counts into offsets        (inclusive scan in place)
-//   place : workgroup e walks the slots in order and writes its own, keeping slot order
-__global__ __launch_bounds__(256) void pack_count_kernel(const int32_t* topk_idx, uint32_t n_slots, uint32_t* expert_offsets) {
-    __shared__ uint32_t red[4];
-    const uint32_t e = blockIdx.x;
-    uint32_t c = 0;
-    for (uint32_t i = threadIdx.x; i < n_slots; i += 256) c += ((uint32_t)topk_idx[i] == e) ? 1u : 0u;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) c += (uint32_t)__shfl_xor((int)c, d);
-    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = c;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        expert_offsets[e + 1] = red[0] + red[1] + red[2] + red[3];
-        if (e == 0) expert_offsets[0] = 0;
-    }
-}
-__global__ __launch_bounds__(64) void pack_scan_kernel(uint32_t* expert_offsets, uint32_t E) {
-    // one wave: running inclusive scan over chunks of 64 counts
-    const uint32_t lane = threadIdx.x;
-    uint32_t base = 0;
-    for (uint32_t e0 = 0; e0 < E; e0 += 64) {
-        const uint32_t e = e0 + lane;
-        uint32_t v = e < E ? expert_offsets[e + 1] : 0u;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t o = (uint32_t)__shfl_up((int)v, d);
-            if (lane >= (uint32_t)d) v += o;
+    };
+    if constexpr (R > 0) {
+        place(lo);
+    } else {
+        for (uint32_t c = lo; c < hi; c += 64u * U) {
+            load(c);
+            place(c);
         }
-        if (e < E) expert_offsets[e + 1] = base + v;
-        base += (uint32_t)__shfl((int)v, 63);
-    }
-}
-__global__ __launch_bounds__(256) void pack_place_kernel(const int32_t* topk_idx, const half_t* topk_w, uint32_t n_slots, uint32_t K,
-                                                         const uint32_t* expert_offsets, int32_t* sorted_idx, half_t* weights_packed,
-                                                         int32_t* tk_to_packed) {
-    __shared__ uint32_t wave_cnt[4];
-    const uint32_t e = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t base = expert_offsets[e];
-    if (expert_offsets[e + 1] == base) return;
-    for (uint32_t i0 = 0; i0 < n_slots; i0 += 256) {
-        const uint32_t i = i0 + threadIdx.x;
-        const bool mine = i < n_slots && (uint32_t)topk_idx[i] == e;
-        const unsigned long long mask = __ballot(mine);
-        const uint32_t before = (uint32_t)__builtin_popcountll(mask & ((1ull << lane) - 1ull));
-        __syncthreads();
-        if (lane == 0) wave_cnt[wave] = (uint32_t)__builtin_popcountll(mask);
-        __syncthreads();
-        uint32_t wave_base = 0;
-        for (uint32_t w = 0; w < wave; ++w) wave_base += wave_cnt[w];
-        if (mine) {
-            const uint32_t p = base + wave_base + before;
-            sorted_idx[p] = (int32_t)(i / K);
-            weights_packed[p] = topk_w[i];
-            tk_to_packed[i] = (int32_t)p;
-        }
-        base += wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
     }
 }
 
@@ -473,29 +390,20 @@ int mx_moe_build_packing_device(mx_stream_t s, const int32_t* topk_idx, const ui
     MX_REQUIRE_PTR(topk_idx); MX_REQUIRE_PTR(topk_w); MX_REQUIRE_PTR(expert_offsets); MX_REQUIRE_PTR(sorted_idx); MX_REQUIRE_PTR(tk_to_packed);
     MX_REQUIRE_PTR(weights_packed);
     MX_REQUIRE_SHAPE(E > 0 && E <= 65535 && K > 0 && T > 0 && (uint64_t)T * K <= 0x7FFFFFFFull);
-    const uint32_t n = T * K;
+    const uint32_t n = T * K, waves = n <= 256 ? 4u : n <= 2048 ? 8u : 16u, slots = (n + 64u * waves - 1u) / (64u * waves);   // a lane's
     hipStream_t st = as_stream(s);
-    if (E <= kPackMaxExperts) {
-        uint32_t waves = n <= 256 ? 4u : n <= 2048 ? 8u : 16u;
-        auto hist_bytes = [&] { return (waves * E + E + 1) * 4u; };
-        uint32_t staged = n <= 65536u && hist_bytes() + 4u * n <= kPackLdsMax ? 1u : 0u;
-        if (hist_bytes() + (staged ? 4u * n : 0u) > kLdsDefaultLimit && raise_pack_lds() != MX_OK) {   // the form that needs no more
-            staged = 0u;
-            while (hist_bytes() > kLdsDefaultLimit) waves /= 2u;
-        }
-        const uint32_t lds = hist_bytes() + (staged ? 4u * n : 0u);
-        uint32_t id_bits = 0;
-        while ((1u << id_bits) < E) ++id_bits;
-        hipLaunchKernelGGL(pack_kernel, dim3(1), dim3(64 * waves), lds, st, topk_idx, topk_w, n, K, E, id_bits, staged, expert_offsets, sorted_idx, weights_packed,
-                           reinterpret_cast<uint32_t*>(tk_to_packed));
-        return launch_status();
+#define MX_PACK(R, Q) \
+    hipLaunchKernelGGL((pack_kernel<R, Q>), dim3((E + Q - 1u) / Q), dim3(64u * waves), 0, st, topk_idx, topk_w, n, K, E, expert_offsets, sorted_idx, weights_packed, tk_to_packed)
+    if (E <= 128u) {
+        if (slots <= 4u) MX_PACK(4, 1);
+        else if (slots <= 16u) MX_PACK(16, 1);
+        else MX_PACK(0, 1);
+    } else {
+        if (slots <= 4u) MX_PACK(4, 4);
+        else if (slots <= 16u) MX_PACK(16, 4);
+        else MX_PACK(0, 4);
     }
-    hipLaunchKernelGGL(pack_count_kernel, dim3(E), dim3(256), 0, st, topk_idx, n, expert_offsets);
-    if (int rc = launch_status()) return rc;
-    hipLaunchKernelGGL(pack_scan_kernel, dim3(1), dim3(64), 0, st, expert_offsets, E);
-    if (int rc = launch_status()) return rc;
-    hipLaunchKernelGGL(pack_place_kernel, dim3(E), dim3(256), 0, st, topk_idx, reinterpret_cast<const half_t*>(topk_w), n, K, (const uint32_t*)expert_offsets,
-                       sorted_idx, reinterpret_cast<half_t*>(weights_packed), tk_to_packed);
+#undef MX_PACK
     return launch_status();
 }
 

@@ -180,10 +180,11 @@ def test_moe_topk_expert_counts(mx, T, E, k):
     check(host(w).astype(np.float32)[same], w_ref[same], "topk weights", max_rel=2e-3)
 
 
-@pytest.mark.parametrize("T,E,K", [(1, 1, 1), (7, 3, 9), (64, 1024, 1), (65, 1000, 4), (513, 7, 4), (1025, 128, 2), (9000, 1024, 4), (20001, 60, 4), (300, 1100, 3)])
+@pytest.mark.parametrize("T,E,K", [(1, 1, 1), (7, 3, 9), (64, 1024, 1), (65, 1000, 4), (513, 7, 4), (1025, 128, 2), (9000, 1024, 4), (20001, 60, 4), (300, 1100, 3),
+                                   (129, 129, 2), (1024, 131, 16), (4096, 128, 4), (4097, 128, 4), (66000, 130, 1)])
 def test_moe_packing_device_sizes(mx, T, E, K):
-    """Slot counts around the waves' 64-slot pieces, one expert, the most experts of the one-workgroup form and one more, positions
-    that fit in LDS and that do not; every id drawn freely (a token may name an expert twice)."""
+    """Slot counts around the waves' 64-slot pieces and around 4 and 16 slots a lane, one expert, 128 experts and one more, a last
+    workgroup with fewer than four, more slots than 2^16; every id drawn freely (a token may name an expert twice)."""
     rng = np.random.default_rng(T * E)
     ids = np.minimum(rng.integers(0, E, (T, K)), rng.integers(0, E, (T, K))).astype(np.int32)
     w = f16(rng.random((T, K)).astype(np.float32))
