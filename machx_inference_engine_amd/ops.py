@@ -27,8 +27,17 @@ class MxError(RuntimeError):
         super().__init__("%s: %s" % (fn, msg))
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+# The current device's current stream as an address.  torch.cuda.current_stream() builds a Stream object for it, 2.7 of the 9 us that a
+# small call costs the host; the raw handle of the same stream takes 0.2 (one token, Q4_K 4096 -> 4096, quantizer and product, called one after
+# the other: 13.4 us, 18.9 before).
+def _stream_handle():
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+    if raw is None or device is None:   # a torch built without a device
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw(device())
+
+
+_stream = _stream_handle()
 
 
 def _ptr(t):
@@ -59,7 +68,7 @@ def _u8(t):
 
 def _out(y, shape, dtype, like):
     if y is None:
-        y = torch.empty(shape, dtype=dtype, device=like.device)
+        return torch.empty(shape, dtype=dtype, device=like.device)
     assert y.dtype == dtype and y.numel() == int(torch.Size(shape).numel())
     return y
 
