@@ -795,13 +795,13 @@ static MmqQ8Aos::Bank mmq_bank(const FmtQ8Aos::W& w) { return {w.base, 0, w.row_
 static typename FmtQ6K::Bank mmq_bank(const FmtQ6K::W& w) { return {w.base, 0, w.row_bytes}; }
 static typename FmtMxfp4Soa::Bank mmq_bank(const FmtMxfp4Soa::W& w) { return {w.qs, w.e, 0, 0, w.K}; }
 
-constexpr uint32_t kMmqLdsBudget = 48 * 1024;
+constexpr uint32_t kMmqLdsBudget = 48 * 1024, kMmqLdsWide = 150 * 1024;   // of a workgroup of four waves, of eight
 constexpr uint32_t kMmqMaxRanges = 16;   // K ranges across workgroups of one dense launch
 
 // staged k range per pass: the largest multiple of `gran` elements whose LDS image fits the budget
-static uint32_t mmq_pass_range(uint32_t T, int TV, bool has_min, uint32_t gran) {
+static uint32_t mmq_pass_range(uint32_t budget, uint32_t T, int TV, bool has_min, uint32_t gran) {
     const uint32_t per256 = T * 256u + 8u * (uint32_t)(2 * TV) * 4u * (has_min ? 2u : 1u);
-    const uint32_t n256 = (kMmqLdsBudget - 32u * T) / per256;
+    const uint32_t n256 = (budget - 32u * T) / per256;
     const uint32_t kr = n256 * 256u / gran * gran;
     return kr ? kr : gran;
 }
@@ -818,27 +818,33 @@ static uint32_t mmq_dense_ranges(uint32_t K, uint32_t N, uint32_t WR, uint32_t W
     return Z < 1 ? 1 : Z;
 }
 
+// ranges = 0: mmq_dense_ranges
 template <class P, int TV, int WR, int WK>
 static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, const uint8_t* xq8, half_t* y, uint32_t K, uint32_t N, uint32_t T,
-                                bool split, const SplitWs& ws) {
+                                bool split, const SplitWs& ws, uint32_t ranges = 0) {
+    constexpr bool WIDE = WR * WK == 8;   // one workgroup of eight waves per CU: its LDS is the CU's
+    constexpr uint32_t red = (uint32_t)(WR * WK) * TV * 64u * 4u;
     const uint32_t nb = K / 32u, n_groups = (nb + 7u) / 8u;
     const uint32_t rgs = (N + 32u * WR - 1u) / (32u * WR);
-    uint32_t Z = mmq_dense_ranges(K, N, WR, WK);   // the partial sums have to fit the scratch
+    uint32_t Z = ranges ? ranges : mmq_dense_ranges(K, N, WR, WK);   // the partial sums have to fit the scratch
     if (Z > 1 && (!ws.ptr || (uint64_t)Z * T * N > ws.elems)) {
-        if (ws.caller) return MX_ERR_WORKSPACE;
-        while (Z > 1 && (uint64_t)Z * T * N > ws.elems) --Z;
+        if (ws.caller && !ranges) return MX_ERR_WORKSPACE;
+        while (Z > 1 && (!ws.ptr || (uint64_t)Z * T * N > ws.elems)) --Z;
     }
     const uint32_t gz = (n_groups + Z - 1u) / Z;
     Z = (n_groups + gz - 1u) / gz;
-    uint32_t kr = mmq_pass_range(T, TV, P::HAS_MIN, 256u * WK);
+    uint32_t kr = mmq_pass_range(WIDE ? kMmqLdsWide - red : kMmqLdsBudget, T, TV, P::HAS_MIN, 256u * WK);
     const uint32_t need = (gz + WK - 1u) / WK * WK * 256u;
     if (kr > need) kr = need;
     MmqArgs<P> a{};
     a.bank0 = bank; a.bank1 = bank; a.xq8 = xq8; a.out = y; a.part = Z > 1 ? ws.ptr : nullptr;
     a.M = T; a.K = K; a.N = N; a.E = 1; a.q8_split = split ? 1u : 0u; a.kr = kr;
-    const uint32_t red = (uint32_t)(WR * WK) * TV * 64u * 4u;
     a.red_off = (mmq_lds_bytes(T, kr, TV, P::HAS_MIN) + 15u) & ~15u;
     const uint32_t lds = a.red_off + red;
+    if (lds > kLdsDefaultLimit) {
+        static LdsLimit limit;
+        if (int rc = raise_lds_limit(reinterpret_cast<const void*>(&mmq_kernel<P, TV, 1, WR, WK, MMQ_STORE>), limit, kMmqLdsWide)) return rc;
+    }
     hipLaunchKernelGGL((mmq_kernel<P, TV, 1, WR, WK, MMQ_STORE>), dim3(rgs, 1, Z), dim3(64 * WR * WK), lds, st, a);
     if (Z > 1) {
         const uint32_t mn = T * N;
@@ -850,10 +856,27 @@ static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, co
     return launch_status();
 }
 
+// Workgroups of four waves, two or three per CU, K ranges across them where the row blocks are too few; or of eight waves, one per CU, whose
+// waves share K among themselves: no partial sums in memory and no second launch where the row blocks alone come close to the number
+// of CUs (fewer than three fifths leave more idle than that saves, more than one each run a second round).  Four waves / eight, us with
+// the partial-sum launch: 9 to 16 tokens, blocks of 64 rows, K from 2048 on (1024: equal): 4096 -> 14336, 16 tokens, Q6_K 24.3 / 22.0,
+// Q4_K 17.1 / 15.1, Q8_0 planes 22.8 / 19.1; 3072 -> 12288 18.7 / 16.9, 14.3 / 12.4, 15.3 / 13.1; 6144 -> 16000 35.0 / 31.1, 23.9 / 22.8, 31.4 / 28.7;
+// blocks of 32 rows, K up to 4096: 2048 -> 8192 12.0 / 9.9, 10.9 / 9.4, 11.0 / 9.8, 4096 -> 8192 16.6 / 15.4, 13.4 / 12.9, 14.3 / 13.4 (6144 -> 5120 17.2 / 18.8).
+// Up to 8 tokens the waves take 16 to 24 groups (shorter rows leave waves without one: 3072 -> 7936, Q6_K, 10.2 / 11.2; longer ones stream
+// better in ranges: 8192 -> 4096 15.2 / 18.7), with K ranges up to one workgroup per CU: 4096 -> 8192, 8 tokens 15.0 / 12.9, 11.6 / 9.6, 13.3 / 11.4;
+// 4096 -> 2048 10.4 / 8.4, 9.1 / 8.2, 9.2 / 8.1; 6144 -> 3072 14.6 / 12.9, 11.1 / 10.3, 12.6 / 11.4.  Not between seven sixteenths and three
+// fifths of the CUs, where both fill them in two ranges: 5120 -> 4096 11.9 / 12.6, 10.1 / 10.2, 11.5 / 11.6.
 template <class P>
 static int launch_mmq_dense(hipStream_t st, const typename P::Bank& bank, const uint8_t* xq8, half_t* y, uint32_t K, uint32_t N, uint32_t T, bool split,
                             const SplitWs& ws) {
-    if (T <= 8) return launch_mmq_dense_cfg<P, 4, 1, 4>(st, bank, xq8, y, K, N, T, split, ws);
+    const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u, r64 = (N + 63u) / 64u;
+    if (T <= 8) {
+        if (n_groups >= 16u && n_groups <= 24u && (16u * r32 <= 7u * cus || (5u * r32 >= 3u * cus && r32 <= cus)))
+            return launch_mmq_dense_cfg<P, 4, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, 8u * r32 <= cus ? 8u : cus / r32);
+        return launch_mmq_dense_cfg<P, 4, 1, 4>(st, bank, xq8, y, K, N, T, split, ws);
+    }
+    if (5u * r64 >= 3u * cus && r64 <= cus && n_groups >= 8u && n_groups <= 32u) return launch_mmq_dense_cfg<P, 8, 2, 4>(st, bank, xq8, y, K, N, T, split, ws, 1);
+    if (5u * r32 >= 3u * cus && r32 <= cus && n_groups <= 16u) return launch_mmq_dense_cfg<P, 8, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, 1);
     return launch_mmq_dense_cfg<P, 8, 2, 2>(st, bank, xq8, y, K, N, T, split, ws);
 }
 

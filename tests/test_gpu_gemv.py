@@ -416,3 +416,31 @@ def test_probe_stream_read(mx):
         mx.ops.probe_stream_read(buf, 24)          # not a multiple of 16
     with pytest.raises(mx.ops.MxError):
         mx.ops.probe_stream_read(buf[8:], 16)      # misaligned
+
+
+@pytest.mark.parametrize("fmt", [O.Q4_K, O.Q6_K, O.Q8_0, O.MXFP4], ids=lambda f: O.FMT_NAMES[f])
+@pytest.mark.parametrize("K,N,T", [(2048, 9825, 9), (8192, 9826, 16), (4096, 16383, 13), (8448, 9856, 12), (2304, 9999, 10), (4096, 4897, 16), (256, 8192, 9),
+                                   (2816, 8190, 11), (4352, 5000, 12), (4096, 33, 5), (6144, 300, 8), (5120, 2047, 6), (4096, 8191, 7), (4096, 4100, 8), (4608, 3000, 5)])
+def test_gemv_q8_batched_eight_waves(mx, fmt, K, N, T):
+    """Workgroups of eight waves (launch_mmq_dense in csrc/gemv.hip; 256 CUs) at the edges of their rules: row blocks around three fifths of the CUs
+    and around all of them, the shortest and the longest rows and one group more, groups that do not divide over the waves, K ranges
+    with ragged columns.  Twice: the same bits."""
+    from machx_inference_engine_amd import synth
+
+    w = synth.normal_weights(O.FMT_NAMES[fmt], N, K, 91 + N, device="cuda")
+    xq = O.quantize_q8_1(f16(O.normal(9100 + K, (T, K))))
+    b = dev(xq).reshape(-1, 40)
+    x = (b[:, :4].contiguous().view(torch.float32).double() * b[:, 8:].contiguous().view(torch.int8).double()).reshape(T, K)
+    ref = host(x @ mx.ops.dequant(O.FMT_NAMES[fmt], w.reshape(-1), N * K, dtype=torch.float32).reshape(N, K).double().t())   # the q8 chain in 64 bits
+    if fmt == O.MXFP4:
+        run = lambda: mx.ops.gemv_mxfp4_soa_q8_batched(dev(xq), *synth.split_mxfp4(w), K, N, T)  # noqa: E731
+    elif fmt == O.Q8_0:
+        run = lambda: mx.ops.gemv_q8_0_soa_q8_batched(dev(xq), *synth.split_q8_0(w), K, N, T)  # noqa: E731
+    else:
+        run = lambda: getattr(mx.ops, "gemv_%s_q8_batched" % O.FMT_NAMES[fmt])(dev(xq), w.reshape(-1), K, N, T)  # noqa: E731
+    got = run()
+    check(host(got).astype(np.float32), ref, "%s K=%d N=%d T=%d" % (O.FMT_NAMES[fmt], K, N, T))
+    assert torch.equal(run(), got), "differs from launch to launch"
+    if fmt == O.Q8_0 and T >= 9:
+        got = mx.ops.gemv_q8_0_q8_batched(dev(xq), w.reshape(-1), K, N, T)   # GGUF blocks
+        check(host(got).astype(np.float32), ref, "blocks K=%d N=%d T=%d" % (K, N, T))
