@@ -444,3 +444,16 @@ def test_gemv_q8_batched_eight_waves(mx, fmt, K, N, T):
     if fmt == O.Q8_0 and T >= 9:
         got = mx.ops.gemv_q8_0_q8_batched(dev(xq), w.reshape(-1), K, N, T)   # GGUF blocks
         check(host(got).astype(np.float32), ref, "blocks K=%d N=%d T=%d" % (K, N, T))
+
+
+@pytest.mark.parametrize("K,N,T", [(256, 40, 5), (768, 100, 16), (1024, 64, 8), (2304, 257, 9), (4096, 96, 12)])
+def test_gemv_q6_K_q8_batched_two_bytes_off(mx, K, N, T):
+    """Q6_K blocks are 210 bytes and need two-byte alignment only; the int-dot kernels of the matrix cores load whole dwords and shift (MmqQ6K).  Rows of
+    an odd and of an even number of blocks, from an address that is a multiple of four and from one two bytes on: the same bits, and the oracle's."""
+    W = weights(O.Q6_K, 9200 + N, N, K)
+    xq = O.quantize_q8_1(acts(9201 + K, T, K))
+    got = mx.ops.gemv_q6_K_q8_batched(dev(xq), dev(W).reshape(-1), K, N, T)
+    check(host(got).astype(np.float32), O.gemv_q8chain(O.Q6_K, W, xq, K, N), "q6_K K=%d N=%d T=%d" % (K, N, T))
+    room = torch.full((W.size + 4,), 255, dtype=torch.uint8, device="cuda")
+    room[2:-2] = dev(W).reshape(-1)
+    assert torch.equal(mx.ops.gemv_q6_K_q8_batched(dev(xq), room[2:-2], K, N, T), got)
