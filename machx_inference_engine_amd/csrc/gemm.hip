@@ -256,7 +256,7 @@ struct GemmQ4KPair : GemmQ4K {
         r[0].hdr = *reinterpret_cast<const uint4*>(L[0].hdr + blk);
     }
     template <int NJ>
-    __device__ static __forceinline__ void settle(Raw (&r)[NJ]) {
+    __device__ static __forceinline__ void settle(const Lane (&)[NJ], uint32_t, Raw (&r)[NJ]) {
         if constexpr (NJ == 2) {
             exchange_pieces<1>(r[0].q0, r[0].q1);
             exchange_pieces<1>(r[1].q0, r[1].q1);
@@ -397,7 +397,7 @@ struct GemmQ8Quad : GemmQ8Soa {
         }
     }
     template <int NJ>
-    __device__ static __forceinline__ void settle(Raw (&r)[NJ]) {
+    __device__ static __forceinline__ void settle(const Lane (&)[NJ], uint32_t, Raw (&r)[NJ]) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             exchange_pieces<1>(r[j].q[0], r[j].q[1]);
@@ -610,6 +610,99 @@ struct GemmQ6K {
     }
 };
 
+// The same blocks loaded as whole dwords and shifted.  Every other block lies two bytes off a dword, and lanes that read 16 such bytes of a row
+// each take the load pipeline three times as long (MmqQ6K).  A lane half reads 32 consecutive bytes of the half block's ql and 16 of its qh from
+// the dword the block's first byte lies in; `ext` is the dword behind the 64 bytes of ql (lower half) or the 32 of qh (upper half), `tail`
+// the last two scales and d.  For the forms whose launches wait for weights: us, pieces from where they lie / so: 4096 -> 14336, 30 tokens
+// (32 x 128) 21.7 / 20.7, 200 tokens (128 x 128) 52.4 / 49.9; 1024 -> 3072, 64 tokens 12.0 / 11.0; 2304 -> 6144, 128 tokens 31.5 / 28.3; 96 x 256,
+// 77 tokens 46.0 / 42.3; through the library 2048 -> 6144, 30 tokens 15.7 / 12.5, 3072 -> 8192, 47 tokens 18.5 / 17.1.  Tiles of 128 x 256 and 256 x 256 are bound by their vector instructions, of which this adds a tenth, and have no
+// registers left: 512 tokens 93.9 / 95.2, 4096 tokens 521 / 532.
+struct GemmQ6KDw : GemmQ6K {
+    struct Raw {
+        uint4 qla, qlb, qh;
+        uint32_t sc0, sc1, sc2, ext, tail;
+        uint2 sc;      // settled
+    };
+    struct Lane {
+        const uint8_t* row;
+        uint32_t odd;   // bit 1: the row's block 0 lies two bytes off; bit 2: its block 0 is read where it lies (nothing in front of the matrix is read)
+    };
+    template <int NJ>
+    static constexpr int loads = 6 * NJ;
+    __device__ static __forceinline__ uint32_t offset(const Lane& l, uint32_t kc) { return kc < 2u && (l.odd & 4u) ? 0u : (l.odd + (kc & ~1u)) & 2u; }   // 210 b = 2 b mod 4
+    template <int NJ>
+    __device__ static __forceinline__ void lanes(const W& w0, const W& w1, const uint32_t (&n_tile)[2], uint32_t N, uint32_t, Lane (&L)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const W& w = j ? w1 : w0;
+            const uint32_t n = lane_row(n_tile[j], N);
+            L[j].row = w.base + (size_t)n * w.row_bytes;
+            L[j].odd = ((uint32_t)(uintptr_t)L[j].row & 2u) | (n == 0 ? 4u : 0u);
+        }
+    }
+    template <int NJ>
+    __device__ static __forceinline__ void load(const Lane (&L)[NJ], uint32_t kc, uint32_t j2, Raw (&r)[NJ]) {
+        const uint32_t c = kc & 1u;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint8_t *blk = L[j].row + (size_t)(kc >> 1) * kQ6KBytes, *p = blk - offset(L[j], kc);
+            r[j].qla = load_u4_a2(p + 64u * c + 32u * j2);
+            r[j].qlb = load_u4_a2(p + 64u * c + 32u * j2 + 16u);
+            r[j].qh = load_u4_a2(p + 128u + 32u * c + 16u * j2);
+            r[j].ext = load_u1_a2(p + (j2 ? 160u + 32u * c : 64u + 64u * c));
+            const U3 s = *reinterpret_cast<const U3*>(p + 192u + 4u * c);   // bytes 192 .. 203, 196 .. 207 from the dword on
+            r[j].sc0 = s.x;
+            r[j].sc1 = s.y;
+            r[j].sc2 = s.z;
+            r[j].tail = load_u1_a2(blk + 206);
+        }
+    }
+    struct __attribute__((packed, aligned(2))) U3 { uint32_t x, y, z; };
+    template <int NJ>
+    __device__ static __forceinline__ void settle(const Lane (&L)[NJ], uint32_t kc, Raw (&r)[NJ]) {
+        const uint32_t h = (threadIdx.x >> 5) & 1u, c = kc & 1u;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint32_t shift = 8u * offset(L[j], kc);
+            auto sh = [&](uint32_t lo, uint32_t hi) { return __builtin_amdgcn_alignbit(hi, lo, shift); };
+            auto run = [&](uint4& v, uint32_t next) { v = make_uint4(sh(v.x, v.y), sh(v.y, v.z), sh(v.z, v.w), sh(v.w, next)); };
+            // behind a half's ql: the other half's first dword or the lower half's ext; behind its qh: the other half's first or ext
+            uint32_t a = r[j].qla.x, b = r[j].ext, lower, upper;
+            swap_halves(a, b);
+            spread_halves(r[j].qh.x, lower, upper);
+            const uint32_t ql_next = h ? a : b, qh_next = h ? r[j].ext : upper;
+            run(r[j].qla, r[j].qlb.x);
+            run(r[j].qlb, ql_next);
+            run(r[j].qh, qh_next);
+            r[j].sc.x = c ? sh(r[j].sc1, r[j].sc2) : sh(r[j].sc0, r[j].sc1);
+            r[j].sc.y = c ? sh(r[j].sc2, r[j].tail) : sh(r[j].sc1, r[j].sc2);
+            swap_halves(r[j].qla.x, r[j].qlb.x);   // pieces (0 | 2), (1 | 3) -> (0 | 1), (2 | 3)
+            swap_halves(r[j].qla.y, r[j].qlb.y);
+            swap_halves(r[j].qla.z, r[j].qlb.z);
+            swap_halves(r[j].qla.w, r[j].qlb.w);
+        }
+    }
+    __device__ static __forceinline__ Dec prepare(const Raw& r, uint32_t kc, uint32_t j) {
+        GemmQ6K::Raw t;
+        t.sc = r.sc;
+        t.d = r.tail >> 16;
+        return GemmQ6K::prepare(t, kc, j);
+    }
+    template <int S, int HF>
+    __device__ static __forceinline__ void frag_half(const Raw& r, const Dec& dc, Frag& f) {
+        GemmQ6K::Raw t;
+        t.qla = r.qla;
+        t.qlb = r.qlb;
+        t.qh = r.qh;
+        GemmQ6K::frag_half<S, HF>(t, dc, f);
+    }
+    template <int S>
+    __device__ static __forceinline__ void frag(const Raw& r, const Dec& dc, Frag& f) {
+        frag_half<S, 0>(r, dc, f);
+        frag_half<S, 1>(r, dc, f);
+    }
+};
+
 // Q5_K (176-byte blocks: d, dmin, scales[12], qh[32], qs[128]; include/ie/quant_blocks.hpp): Q4_K's nibbles plus one
 // high bit per element, bit j of qh[l] for sub-block j and position l.  Same chunk / lane-half split as Q4_K (lane half h
 // owns qs[32 g, 32 g + 32), g = 2 (kc % 2) + h: sub-blocks 2 g in the low and 2 g + 1 in the high nibbles); the lane also
@@ -789,7 +882,7 @@ struct GemmMxfp4Pair : GemmMxfp4Soa {
         }
     }
     template <int NJ>
-    __device__ static __forceinline__ void settle(Raw (&r)[NJ]) {
+    __device__ static __forceinline__ void settle(const Lane (&)[NJ], uint32_t, Raw (&r)[NJ]) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) exchange_pieces<1>(r[j].q[0], r[j].q[1]);
     }
@@ -1045,7 +1138,7 @@ struct GemmLanes {
         for (int j = 0; j < NJ; ++j) r[j] = QF::load(L[j].w, L[j].n, kc, h);
     }
     template <int NJ>
-    __device__ static __forceinline__ void settle(typename QF::Raw (&)[NJ]) {}
+    __device__ static __forceinline__ void settle(const type (&)[NJ], uint32_t, typename QF::Raw (&)[NJ]) {}
 };
 template <class QF>
 struct GemmLanes<QF, std::void_t<typename QF::Lane>> : QF {
@@ -1101,7 +1194,7 @@ __device__ __forceinline__ void gemm_chunk(const TileCtx<QF, NA, NJ>& t, const u
         if (w_next) GemmLanes<QF>::template load<NJ>(t.lanes, t.c0 + c + DEPTH, t.h, raw[PN]);
         __builtin_amdgcn_sched_barrier(0);   // the scheduler must not sink these loads towards their uses
     }
-    if constexpr (DEPTH > 1) GemmLanes<QF>::template settle<NJ>(raw[P]);
+    if constexpr (DEPTH > 1) GemmLanes<QF>::template settle<NJ>(t.lanes, t.c0 + c, raw[P]);
     typename QF::Dec dec[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) dec[j] = gemm_prepare<QF>(raw[P][j], win[j], t.c0 + c, t.h);
@@ -1265,12 +1358,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, const typename QF::
 #define CHUNK(P, c, more, tail) gemm_chunk<QF, NA, NJ, DEPTH, P, tail>(ctx, a_off, raw, win, acc, c, more)
     if constexpr (DEPTH == 1) {
         // two sets, and the set just loaded is moved into set 0 at the end of a chunk, where it has to have arrived anyway
-        GemmLanes<QF>::template settle<NJ>(raw[0]);
+        GemmLanes<QF>::template settle<NJ>(ctx.lanes, c0, raw[0]);
         for (uint32_t c = 0; c + 1 < n_chunks; ++c) {
             CHUNK(0, c, true, false);
 #pragma unroll
             for (int j = 0; j < NJ; ++j) raw[0][j] = raw[1][j];
-            GemmLanes<QF>::template settle<NJ>(raw[0]);
+            GemmLanes<QF>::template settle<NJ>(ctx.lanes, c0 + c + 1u, raw[0]);
         }
         CHUNK(0, n_chunks - 1, false, true);
     } else {
@@ -1740,6 +1833,10 @@ static uint64_t gemm_library_scratch(uint64_t M, uint64_t K, uint64_t N, uint64_
     return K >= 2048 && 2 * ((M + 127) / 128) * ((N + 255) / 256) <= cus ? kGemmSplitElems : 0;
 }
 
+// the producer a format uses in eight-wave workgroups over less than 128 x 256
+template <class QF> struct GemmSmall { using type = QF; };
+template <> struct GemmSmall<GemmQ6K> { using type = GemmQ6KDw; };
+
 template <class QF, int MODE>
 static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound,
                        const SplitWs* caller_ws = nullptr) {
@@ -1761,15 +1858,16 @@ static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typenam
                 g.split_acc = static_cast<float*>(q);
             }
         }
+        using QS = typename GemmSmall<QF>::type;
         int rc;
         switch (p.na * 2 + p.nj - 1) {
-            case 2: rc = launch_gemm_ni<QF, MODE, 1, 2, 1>(s, b0, b1, g, rows_bound); break;
-            case 3: rc = launch_gemm_ni<QF, MODE, 1, 2, 2>(s, b0, b1, g, rows_bound); break;
-            case 4: rc = launch_gemm_ni<QF, MODE, 2, 2, 1>(s, b0, b1, g, rows_bound); break;
-            case 5: rc = launch_gemm_ni<QF, MODE, 2, 2, 2>(s, b0, b1, g, rows_bound); break;
-            case 6: rc = launch_gemm_ni<QF, MODE, 3, 2, 1>(s, b0, b1, g, rows_bound); break;
-            case 7: rc = launch_gemm_ni<QF, MODE, 3, 2, 2>(s, b0, b1, g, rows_bound); break;
-            case 8: rc = launch_gemm_ni<QF, MODE, 4, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 2: rc = launch_gemm_ni<QS, MODE, 1, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 3: rc = launch_gemm_ni<QS, MODE, 1, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 4: rc = launch_gemm_ni<QS, MODE, 2, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 5: rc = launch_gemm_ni<QS, MODE, 2, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 6: rc = launch_gemm_ni<QS, MODE, 3, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 7: rc = launch_gemm_ni<QS, MODE, 3, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 8: rc = launch_gemm_ni<QS, MODE, 4, 2, 1>(s, b0, b1, g, rows_bound); break;
             case 9: rc = launch_gemm_ni<QF, MODE, 4, 2, 2>(s, b0, b1, g, rows_bound); break;
             default: rc = launch_gemm_ni<QF, MODE, 4>(s, b0, b1, g, rows_bound);
         }
