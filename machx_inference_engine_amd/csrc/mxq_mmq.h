@@ -955,6 +955,17 @@ constexpr int mmq_workgroups_per_cu() {
     return TV == 8 && NW == 1 && (std::is_same<P, MmqQ8Soa>::value || (EPI == MMQ_STORE && std::is_same<P, MmqQ4K>::value)) ? 3 : 2;
 }
 
+// Grouped K-quant passes of 32 rows: a remainder of at most 16 rows runs as a tile of 16, which folds half as many sums per block (the fold,
+// 78 vector instructions of a 32x32x32 block for Q4_K and 97 for Q6_K, is what the launches spend their time on; experts differ in size, so
+// that near every second one ends in such a remainder).  Whole expert block over q8 rows, Q4_K + Q6_K, 128 experts, k = 8, 2048/768, 333 / 600 /
+// 1000 / 2000 tokens: 258 / 361 / 495 / 866 -> 248 / 346 / 479 / 840 us; 32 experts, k = 4, 4096/1536, 140 / 300 tokens 204 / 297 -> 202 /
+// 290.  Not the other formats: Q8_0 planes, 128 experts, 333 / 900 tokens 247 / 415 -> 249 / 424 (its fold is half as long, and the two paths
+// cost it more than they save); native MXFP4 has tiles of 16 at most.
+template <class P, int TV, int EPI>
+constexpr bool mmq_short_tiles() {
+    return TV == 16 && EPI != MMQ_STORE && P::K_ALIGN == 256;
+}
+
 template <class P>
 struct MmqArgs {
     typename P::Bank bank0, bank1;    // NW = 2: gate and up
@@ -983,6 +994,24 @@ __device__ __forceinline__ float mmq_swiglu_oai(float g, float u, float alpha, f
     return (x / (1.f + __expf(alpha * -x))) * (z + 1.f);
 }
 
+// One tile of a kernel with tiles of two sizes.  A function of its own, simplified before it becomes part of the kernel: with the text twice
+// in the kernel the registers spill (27 to 106); and the kernels with one size of tile keep the text in their loop: as a function
+// native MXFP4 is 3 % slower.
+template <class P, int TR, int NW, int WR, int WK, int EPI>
+__device__ __forceinline__ void mmq_tile(const MmqArgs<P>& a, uint8_t* lds, uint32_t e, uint32_t t0, uint32_t r_end, uint32_t kzi, uint32_t G0, uint32_t G1) {
+    constexpr bool NATIVE = mmq_native<P>::value;
+    const uint32_t lane = threadIdx.x & 63u, j = lane & 31u, h = lane >> 5;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t wk = wave % WK, wr = (wave / WK) % WR, wm = wave / (WK * WR);
+    const typename P::W w = P::expert((NW == 2 && wm) ? a.bank1 : a.bank0, e);
+    const uint32_t nb = a.K / 32u, n_rb = (a.N + 32u * WR - 1u) / (32u * WR);
+    const uint32_t gp = a.kr / 256u;
+    const bool single = G1 - G0 <= gp && a.red_off != 0;
+    const size_t q8_row_bytes = (size_t)nb * (a.q8_split ? kQ81sBytes : kQ81xBytes);
+    float* red = reinterpret_cast<float*>(lds + a.red_off);
+#include "mxq_mmq_tile.h"
+}
+
 // Grid: x = workgroups per expert (each takes the blocks of 32 WR weight rows x, x + gridDim.x, ...), y = expert (grouped)
 // or 1, z = K range (dense, with `part`) or token tile dealing (grouped).  Workgroup = NW x WR x WK waves.  A pass covers
 // up to 2 TV token rows: T <= 8 (TV = 4), 16 (TV = 8), 32 (TV = 16); an expert with more rows runs several passes over
@@ -993,8 +1022,7 @@ __device__ __forceinline__ float mmq_swiglu_oai(float g, float u, float alpha, f
 template <class P, int TV, int NW, int WR, int WK, int EPI>
 __global__ __launch_bounds__(64 * NW * WR * WK, (mmq_workgroups_per_cu<P, TV, NW, EPI>())) void mmq_kernel(MmqArgs<P> a) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr uint32_t TT = 2 * TV;   // token rows per pass
-    constexpr bool NATIVE = mmq_native<P>::value;
+    constexpr bool NATIVE = mmq_native<P>::value, SHORT_TILES = mmq_short_tiles<P, TV, EPI>();
     const uint32_t lane = threadIdx.x & 63u, j = lane & 31u, h = lane >> 5;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t wk = wave % WK, wr = (wave / WK) % WR, wm = wave / (WK * WR);
@@ -1021,131 +1049,12 @@ __global__ __launch_bounds__(64 * NW * WR * WK, (mmq_workgroups_per_cu<P, TV, NW
     float* red = reinterpret_cast<float*>(lds + a.red_off);
 
     for (uint32_t t0 = r_begin + t_first; t0 < r_end; t0 += t_step) {
-        const uint32_t nt = r_end - t0 < TT ? r_end - t0 : TT;
-        auto xrow = [&](uint32_t t) { return a.xq8 + (size_t)(t0 + t) * q8_row_bytes; };
-        auto hrow = [&](uint32_t t) { return a.act_f16 + (size_t)(t0 + t) * a.K; };
-        // token rows past the tile re-read its last row (their results are dropped)
-        const uint32_t jt = NATIVE ? (j & 15u) : j, row_a = jt < nt ? jt : nt - 1u;
-        typename std::conditional<NATIVE, MmqWalkNative<P, TV>, MmqWalk<P, TV, mmq_two_tails<P, TV, EPI>()>>::type walk;
-        MmqAct act{};
-        bool staged = false, requested = false;
-        // what the epilogue reads from global memory is requested ahead of the weight walk: a load issued in the epilogue
-        // would have to wait for the whole queue of weight words requested for the next row block before it
-        float rw[EPI == MMQ_DOWN_WEIGHTED ? TV : 1];
-        if constexpr (EPI == MMQ_DOWN_WEIGHTED) {
-#pragma unroll
-            for (int v = 0; v < TV; ++v) {
-                const uint32_t t = mmq_row(v) + 4u * h;
-                rw[v] = (float)a.route_w[t0 + (t < nt ? t : nt - 1u)];
-            }
-        }
-        for (uint32_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x) {
-            const uint32_t n0 = (rb * WR + wr) * 32u;
-            const uint32_t n = n0 + j < a.N ? n0 + j : a.N - 1u;
-            // MMQ_OAI: the bias of this wave's matrix joins its partial sum before the exchange (wave wk = 0 of each matrix);
-            // MMQ_DOWN_BIAS: added after the fp16 rounding of the sum, in the epilogue
-            float bias_a = 0.f;
-            if (EPI == MMQ_OAI || EPI == MMQ_DOWN_BIAS) {
-                const float* bp = (NW == 2 && wm) ? a.bias1 : a.bias0;
-                if (bp) bias_a = bp[(size_t)e * a.N + n];
-            }
-            float acc[TV];
-#pragma unroll
-            for (int v = 0; v < TV; ++v) acc[v] = 0.f;
-            for (uint32_t gb = G0; gb < G1; gb += gp) {
-                const uint32_t ge = gb + gp < G1 ? gb + gp : G1;          // groups [gb, ge) of this pass
-                const uint32_t per = (ge - gb + WK - 1u) / WK;
-                const uint32_t g_lo = gb + wk * per < ge ? gb + wk * per : ge, g_hi = g_lo + per < ge ? g_lo + per : ge;
-                // the pipeline takes whole groups and a partial last group follows it, except where the producer loads both alike
-                const uint32_t g_full = (NATIVE || g_hi < nb / 8u) ? g_hi : nb / 8u;
-                if (!requested && g_lo < g_full) walk.prefetch(w, n, g_lo, g_full, h, nb);
-                requested = false;
-                if (!staged) {
-                    mmq_lds_barrier();                                        // the image of the previous pass is no longer read
-                    act = a.act_f16 ? mmq_stage_f16<TV, P::HAS_MIN, NATIVE>(lds, hrow, nt, gb * 256u, (ge - gb) * 256u, a.K)
-                                    : mmq_stage<TV, P::HAS_MIN, NATIVE>(lds, xrow, nt, gb * 256u, (ge - gb) * 256u, a.K, a.q8_split != 0);
-                    mmq_lds_barrier();
-                    staged = single;
-                }
-                const uint32_t a_off = row_a * act.stride + 16u * h + (NATIVE ? 64u * (j >> 4) : 0u);
-                if (g_lo < g_full) walk.run(w, n, g_lo, g_full, gb, h, nb, act, a_off, acc);
-                if (g_hi > g_full && g_lo <= g_full) walk.tail(w, n, g_full, gb, h, nb, act, a_off, acc);
-                // the epilogue's operands are made to arrive here, while nothing else is outstanding: otherwise the wait for
-                // them would sit in the epilogue, behind the weight words requested just below
-                asm volatile("" : "+v"(bias_a));
-                if constexpr (EPI == MMQ_DOWN_WEIGHTED) {
-#pragma unroll
-                    for (int v = 0; v < TV; ++v) asm volatile("" : "+v"(rw[v]));
-                }
-                if (EPI == MMQ_OAI && ge == G1 && wk == 0) {
-#pragma unroll
-                    for (int v = 0; v < TV; ++v) acc[v] += bias_a;
-                }
-                if (single && rb + gridDim.x < n_rb && g_lo < g_full) {
-                    // the next row block's first weight words, requested before the partial sums of this one meet
-                    const uint32_t nn0 = ((rb + gridDim.x) * WR + wr) * 32u;
-                    walk.prefetch(w, nn0 + j < a.N ? nn0 + j : a.N - 1u, g_lo, g_full, h, nb);
-                    requested = true;
-                }
-            }
-            // ---- partial sums of the WK waves (and the NW matrices) meet in LDS; a workgroup of row blocks only has none to meet
-            if constexpr (NW * WK > 1) {
-                mmq_lds_barrier();
-#pragma unroll
-                for (int v = 0; v < TV; ++v) red[((size_t)wave * TV + v) * 64u + lane] = acc[v];
-                mmq_lds_barrier();
-            }
-            if (wk == 0 && wm == 0) {
-                // Row v of a lane is t0 + 4 h + mmq_row(v): the lane's share of an address is one 32-bit offset and the rest is
-                // uniform.  The offset is made opaque here, once per row block: 2 TV addresses kept in registers across the
-                // weight walk were what made the walk spill (Q6_K, TV = 16: 256 registers and 46 more in scratch).
-                uint32_t lane_at = 4u * h * a.N + j;
-                asm volatile("" : "+v"(lane_at));
-                const bool col_ok = n0 + j < a.N;
-                if (a.part) {
-                    float* base = a.part + ((size_t)kzi * a.M + t0) * a.N + n0;
-#pragma unroll
-                    for (int v = 0; v < TV; ++v) {
-                        float s0 = acc[v];
-                        if constexpr (NW * WK > 1) {
-                            s0 = 0.f;
-#pragma unroll
-                            for (int k = 0; k < WK; ++k) s0 += red[((size_t)(wr * WK + k) * TV + v) * 64u + lane];
-                        }
-                        if (mmq_row(v) + 4u * h < nt && col_ok) (base + (size_t)mmq_row(v) * a.N)[lane_at] = s0;
-                    }
-                } else {
-                    half_t* base = a.out + (size_t)t0 * a.N + n0;
-#pragma unroll
-                    for (int v = 0; v < TV; ++v) {
-                        float s0 = acc[v], s1 = 0.f;
-                        if constexpr (NW * WK > 1) {
-                            s0 = 0.f;
-#pragma unroll
-                            for (int k = 0; k < WK; ++k) {
-                                s0 += red[((size_t)((0 * WR + wr) * WK + k) * TV + v) * 64u + lane];
-                                if (NW == 2) s1 += red[((size_t)((1 * WR + wr) * WK + k) * TV + v) * 64u + lane];
-                            }
-                        }
-                        float o;
-                        if constexpr (EPI == MMQ_SILU) {
-                            o = mmq_silu_mul(s0, s1);                                          // src/ops/moe_q8.cpp:94-97
-                        } else if constexpr (EPI == MMQ_OAI) {
-                            // rounding points of the reference chain: half(acc + bias) per projection, then the fp16 activation
-                            const float g = (float)(half_t)s0, u = (float)(half_t)s1;   // sums with their biases
-                            o = mmq_swiglu_oai(g, u, a.alpha, a.limit);
-                        } else if constexpr (EPI == MMQ_DOWN_WEIGHTED) {
-                            o = rw[v] * s0;                                                   // src/ops/moe_q8.cpp:143-144
-                        } else if constexpr (EPI == MMQ_DOWN_BIAS) {
-                            o = (float)(half_t)s0;                                            // gemv out, then add_bias (elementwise.cpp:782-793)
-                            if (a.bias0) o += bias_a;
-                        } else {
-                            o = s0;
-                        }
-                        if (mmq_row(v) + 4u * h < nt && col_ok) (base + (size_t)mmq_row(v) * a.N)[lane_at] = (half_t)o;
-                    }
-                }
-            }
+        if constexpr (SHORT_TILES) {
+            if (r_end - t0 <= TV) mmq_tile<P, TV / 2, NW, WR, WK, EPI>(a, lds, e, t0, r_end, kzi, G0, G1);
+            else mmq_tile<P, TV, NW, WR, WK, EPI>(a, lds, e, t0, r_end, kzi, G0, G1);
+        } else {
+            constexpr int TR = TV;
+#include "mxq_mmq_tile.h"
         }
     }
 }

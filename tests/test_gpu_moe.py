@@ -554,6 +554,35 @@ def test_moe_grouped_int_dot_row_blocks_or_k_ranges(mx, avg, K, N_gate, N_down):
     test_moe_grouped_int_dot_streams_row_blocks(mx, avg, K, N_gate, N_down)
 
 
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+@pytest.mark.parametrize("K", [768, 4096])
+def test_moe_grouped_int_dot_short_tiles(mx, fmt, K):
+    """Tiles of 32 rows whose remainder of at most 16 runs as a tile of 16: experts of 0 to 64 rows at every edge, all with the same
+    weights and the same first rows, so that a row has the same bits in a tile of either size; the longest expert against the oracle.
+    K = 768 is staged at once, with an odd number of groups; 4096 in several ranges under the exchange area."""
+    ops, N = mx.ops, 112
+    F = {"q4k": O.Q4_K, "q6k": O.Q6_K}[fmt]
+    counts = [64, 0, 1, 15, 16, 17, 31, 32, 33, 48, 49]
+    E, off = len(counts), np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    TK = int(off[-1])
+    assert (TK + E - 1) // E > 16
+    x = f16(O.normal(8700, (64, K)))
+    xq = ops.quantize_q8_1s(dev(np.concatenate([x[:c] for c in counts])).half())
+    rows = host(xq).reshape(TK, -1)[:64]
+    W = [O.quantize(F, O.normal(8701 + i, (N, K), 0.0, 0.02)) for i in range(2)]
+    stride = W[0].size
+    ref = [O.gemv_q8schain(F, w, rows, K, N) for w in W]
+    bank = [np.concatenate([w.ravel()] * E) for w in W]
+    for soa in (False, True):
+        a, b = (dev(ops.repack_moe_kquant_soa(fmt, w, E, stride // O.BLOCK_BYTES[F])) if soa else dev(w) for w in bank)
+        h = ops.moe_prefill_gate_up_silu_kquant_q8(fmt, xq, a, b, dev(off), TK, E, K, N, stride, soa=soa)
+        y = ops.moe_prefill_down_packed_kquant_q8(fmt, xq, b, dev(off), TK, E, N, K, stride, soa=soa)
+        check(host(h)[:64].astype(np.float32), O.swiglu_np(ref[0].astype(np.float32), ref[1].astype(np.float32)), "gate_up %s" % fmt)
+        check(host(y)[:64].astype(np.float32), ref[1], "down %s" % fmt)
+        for e, c in enumerate(counts):
+            assert torch.equal(h[off[e]:off[e] + c], h[:c]) and torch.equal(y[off[e]:off[e] + c], y[:c]), (soa, c)
+
+
 @pytest.mark.parametrize("EF", [64, 512, 768, 1152, 1920, 3200])
 def test_moe_mxfp4_down_rows_shorter_than_a_lane_group(mx, EF):
     """One-token down launch with fewer 64-element units in a row than lanes that share it (8 of 16, 18 of 32, 50 of 64, ..), every
