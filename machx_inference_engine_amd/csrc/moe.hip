@@ -317,9 +317,13 @@ __global__ __launch_bounds__(256) void merge_f32_kernel(const float* y32, half_t
 // moe_reduce_q8 (src/ops/moe_q8.cpp:149-158): y[t] = sum_k y_packed[t*K+k]
 // moe_prefill_reduce_sum (:368-384): y[t] = sum_k out_packed[tk_to_packed[t*K+k]]
 // moe_prefill_reduce (src/ops/moe_fused.cpp:1927-1954): y[t] += sum_k w[row] * out_packed[row]
-// A thread owns 8 consecutive columns (16-byte loads) and requests four packed rows before it adds the first, in slot order:
-// 2048 tokens of hidden 2048, k = 8 (75 MB) take 12.5 us (6 TB/s); one column per thread, row after row, took 44.
-template <bool WEIGHTED, bool ACCUMULATE>
+// A thread owns 8 consecutive columns (16-byte loads), requests the rows' numbers of G slots and then the G rows, and adds them in slot
+// order.  Bound by two trips to memory for few tokens and by the bytes for many (2048 tokens of hidden 2048, k = 8, 75 MB: 15.8 us on cold
+// caches).  With every slot under a test of its own, a row's number waited for the row before it, and few outputs of more than four rows
+// were better off with a column a thread.  us so / now: k = 8, hidden 2048, routing weights, 1 token 2.8 / 2.3, 64 tokens 3.2 / 2.5, 333
+// tokens 5.8 / 4.3, 2048 tokens 17.6 / 16.7, without weights 333 tokens 5.3 / 4.4, 2048 tokens 15.5 / 15.8; k = 4, hidden 2880, 1 token
+// 2.3 / 2.1, 2048 tokens 15.2 / 12.7.
+template <bool WEIGHTED, bool ACCUMULATE, int G>
 __global__ __launch_bounds__(256) void moe_reduce8_kernel(const half_t* __restrict__ packed, const uint32_t* __restrict__ tk_to_packed, const half_t* __restrict__ w,
                                                           half_t* __restrict__ y, uint32_t T, uint32_t Ktop, uint32_t H8) {
     typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -333,20 +337,27 @@ __global__ __launch_bounds__(256) void moe_reduce8_kernel(const half_t* __restri
     if (ACCUMULATE) y0 = *out;
 #pragma unroll
     for (int c = 0; c < 8; ++c) s[c] = ACCUMULATE ? (float)y0[c] : 0.f;
-    for (uint32_t k0 = 0; k0 < Ktop; k0 += 4) {
-        h8_t v[4];
-        float wt[4];
+    for (uint32_t k0 = 0; k0 < Ktop; k0 += G) {
+        const size_t first = (size_t)t * Ktop;
+        uint32_t row[G];   // of slots past the last one: the last one's again, not added
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (k0 + u < Ktop) {
-                const size_t slot = (size_t)t * Ktop + k0 + u;
-                const uint32_t row = tk_to_packed ? tk_to_packed[slot] : (uint32_t)slot;
-                v[u] = rows[(size_t)row * H8];
-                wt[u] = WEIGHTED ? (float)w[row] : 1.f;
-            }
+        for (int u = 0; u < G; ++u) row[u] = k0 + u < Ktop ? k0 + u : Ktop - 1u;
+        if (tk_to_packed) {
+#pragma unroll
+            for (int u = 0; u < G; ++u) row[u] = tk_to_packed[first + row[u]];
+        } else {
+#pragma unroll
+            for (int u = 0; u < G; ++u) row[u] += (uint32_t)first;
+        }
+        h8_t v[G];
+        float wt[G];
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+            v[u] = rows[(size_t)row[u] * H8];
+            wt[u] = WEIGHTED ? (float)w[row[u]] : 1.f;
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < G; ++u) {
             if (k0 + u < Ktop) {
 #pragma unroll
                 for (int c = 0; c < 8; ++c) s[c] += WEIGHTED ? wt[u] * (float)v[u][c] : (float)v[u][c];
@@ -358,7 +369,7 @@ __global__ __launch_bounds__(256) void moe_reduce8_kernel(const half_t* __restri
     for (int c = 0; c < 8; ++c) o[c] = (half_t)s[c];
     *out = o;
 }
-// any H, any alignment, and few outputs
+// any H, any alignment
 template <bool WEIGHTED, bool ACCUMULATE>
 __global__ __launch_bounds__(256) void moe_reduce_kernel(const half_t* packed, const uint32_t* tk_to_packed, const half_t* w, half_t* y,
                                                          uint32_t T, uint32_t Ktop, uint32_t H) {
@@ -378,12 +389,15 @@ template <bool WEIGHTED, bool ACCUMULATE>
 static int launch_reduce(hipStream_t st, const uint16_t* packed, const uint32_t* tk_to_packed, const uint16_t* w, uint16_t* y, uint32_t T, uint32_t K, uint32_t H) {
     const half_t *p = reinterpret_cast<const half_t*>(packed), *wh = reinterpret_cast<const half_t*>(w);
     half_t* yh = reinterpret_cast<half_t*>(y);
-    // More than four rows a sum take the wide form two trips to memory; with too few threads to hide them one column per thread is
-    // faster: k = 8, hidden 2048, us, wide / narrow: 4 tokens 3.1 / 2.9, 32 tokens 3.1 / 2.95, 64 tokens 3.2 / 3.3, 128 tokens 3.25 / 3.5.
-    const bool few = K > 4 && (uint64_t)T * H < 131072u;
-    if (!few && H % 8 == 0 && aligned(packed, 16) && aligned(y, 16)) {
+    if (H % 8 == 0 && aligned(packed, 16) && aligned(y, 16)) {
         const uint64_t n = (uint64_t)T * (H / 8);
-        hipLaunchKernelGGL((moe_reduce8_kernel<WEIGHTED, ACCUMULATE>), dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, p, tk_to_packed, wh, yh, T, K, H / 8);
+        const dim3 grid((uint32_t)((n + 255) / 256)), block(256);
+        // rows requested at once: all of a token's up to eight, with few to spare (a spare one costs its cached load: k = 2, 2048 tokens
+        // of 4096 columns 9.0 us in a group of two, 9.4 of four; k = 8, 333 tokens 4.4 of eight, 5.7 of two)
+        if (K <= 2) hipLaunchKernelGGL((moe_reduce8_kernel<WEIGHTED, ACCUMULATE, 2>), grid, block, 0, st, p, tk_to_packed, wh, yh, T, K, H / 8);
+        else if (K <= 4) hipLaunchKernelGGL((moe_reduce8_kernel<WEIGHTED, ACCUMULATE, 4>), grid, block, 0, st, p, tk_to_packed, wh, yh, T, K, H / 8);
+        else if (K <= 6) hipLaunchKernelGGL((moe_reduce8_kernel<WEIGHTED, ACCUMULATE, 6>), grid, block, 0, st, p, tk_to_packed, wh, yh, T, K, H / 8);
+        else hipLaunchKernelGGL((moe_reduce8_kernel<WEIGHTED, ACCUMULATE, 8>), grid, block, 0, st, p, tk_to_packed, wh, yh, T, K, H / 8);
     } else {
         hipLaunchKernelGGL((moe_reduce_kernel<WEIGHTED, ACCUMULATE>), dim3((uint32_t)(((uint64_t)T * H + 255) / 256)), dim3(256), 0, st, p, tk_to_packed, wh, yh,
                            T, K, H);

@@ -196,10 +196,11 @@ def test_moe_packing_device_sizes(mx, T, E, K):
     assert np.array_equal(host(wp).astype(np.float32), wp_r)
 
 
-@pytest.mark.parametrize("T,K,H", [(1, 4, 2880), (3, 5, 8), (2, 9, 20), (33, 8, 1032), (64, 8, 2048), (130, 9, 1032), (127, 5, 1032)])
+@pytest.mark.parametrize("T,K,H", [(1, 4, 2880), (3, 5, 8), (2, 9, 20), (33, 8, 1032), (64, 8, 2048), (130, 9, 1032), (127, 5, 1032),
+                                   (5, 1, 16), (9, 2, 40), (9, 3, 40), (4, 6, 64), (4, 7, 64), (4, 16, 64), (3, 17, 64)])
 def test_moe_reduce_columns(mx, T, K, H):
-    """Rows of whole 8-column pieces and not, slot counts around the four rows in flight, both sides of the 131072 outputs from which
-    longer sums take the wide form: fp32 sums of the fp16 rows in slot order."""
+    """Rows of whole 8-column pieces and not, slot counts at and around the two, four, six and eight rows requested at once, in one group and
+    several: fp32 sums of the fp16 rows in slot order."""
     rng = np.random.default_rng(H)
     packed = f16(O.normal(9600, (T * K, H)))
     rows = rng.permutation(T * K).astype(np.int32)
