@@ -161,7 +161,8 @@ int mx_gemv_mxfp4_soa_q8_x2(mx_stream_t s, const void* x_q8, const uint8_t* gate
  *
  * Library-owned scratch (no counterpart in the reference's signatures; it is what lets callers that cannot
  * allocate -- code under HIP graph capture, serving loops, harnesses that forbid hipMalloc -- use these entry
- * points as they are): batched launches with T >= 2 and K >= 8192 whose row groups alone would leave CUs idle
+ * points as they are): batched launches whose row groups alone would leave CUs idle (at most those for which
+ * mx_gemv_batched_ws_bytes is not 0: T >= 2 with K >= 8192, T >= 4 with K > 3840, T >= 9 with K > 1792)
  * split K over workgroups and keep slices x T x N fp32 partial sums in a 2 MB file-scope device array (one copy
  * per device, resolved with hipGetSymbolAddress on first use or by mx_init, never allocated or freed).  Limit:
  * slices * min(T, 8) * N <= 524288 floats (e.g. T = 8, N = 16384); a launch beyond it runs unsplit.  Every call

@@ -828,7 +828,7 @@ static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, co
     const uint32_t rgs = (N + 32u * WR - 1u) / (32u * WR);
     uint32_t Z = ranges ? ranges : mmq_dense_ranges(K, N, WR, WK);   // the partial sums have to fit the scratch
     if (Z > 1 && (!ws.ptr || (uint64_t)Z * T * N > ws.elems)) {
-        if (ws.caller && !ranges) return MX_ERR_WORKSPACE;
+        if (ws.caller) return MX_ERR_WORKSPACE;
         while (Z > 1 && (!ws.ptr || (uint64_t)Z * T * N > ws.elems)) --Z;
     }
     const uint32_t gz = (n_groups + Z - 1u) / Z;
@@ -856,6 +856,13 @@ static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, co
     return launch_status();
 }
 
+// K ranges of the form of eight waves for up to 8 tokens (launch_mmq_dense), 0 for the shapes that do not take it; also what a workspace is sized for
+static uint32_t mmq_wide_ranges(uint32_t K, uint32_t N) {
+    const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u;
+    if (n_groups < 16u || n_groups > 24u || !(16u * r32 <= 7u * cus || (5u * r32 >= 3u * cus && r32 <= cus))) return 0;
+    return 8u * r32 <= cus ? 8u : cus / r32;
+}
+
 // Workgroups of four waves, two or three per CU, K ranges across them where the row blocks are too few; or of eight waves, one per CU, whose
 // waves share K among themselves: no partial sums in memory and no second launch where the row blocks alone come close to the number
 // of CUs (fewer than three fifths leave more idle than that saves, more than one each run a second round).  Four waves / eight, us with
@@ -871,8 +878,7 @@ static int launch_mmq_dense(hipStream_t st, const typename P::Bank& bank, const 
                             const SplitWs& ws) {
     const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u, r64 = (N + 63u) / 64u;
     if (T <= 8) {
-        if (n_groups >= 16u && n_groups <= 24u && (16u * r32 <= 7u * cus || (5u * r32 >= 3u * cus && r32 <= cus)))
-            return launch_mmq_dense_cfg<P, 4, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, 8u * r32 <= cus ? 8u : cus / r32);
+        if (const uint32_t ranges = mmq_wide_ranges(K, N)) return launch_mmq_dense_cfg<P, 4, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, ranges);
         return launch_mmq_dense_cfg<P, 4, 1, 4>(st, bank, xq8, y, K, N, T, split, ws);
     }
     if (5u * r64 >= 3u * cus && r64 <= cus && n_groups >= 8u && n_groups <= 32u) return launch_mmq_dense_cfg<P, 8, 2, 4>(st, bank, xq8, y, K, N, T, split, ws, 1);
@@ -1190,7 +1196,8 @@ int mx_gemv_batched_ws_bytes(uint32_t K, uint32_t N, uint32_t T, uint64_t* bytes
     uint32_t Z = 1;
     if (T >= 2 && T <= 8 && K >= 8192) Z = kSplitMaxSlices;
     if (T >= 4) {
-        const uint32_t zm = T <= 8 ? mmq_dense_ranges(K, N, 1, 4) : mmq_dense_ranges(K, N, 2, 2);
+        uint32_t zm = T <= 8 ? mmq_dense_ranges(K, N, 1, 4) : mmq_dense_ranges(K, N, 2, 2);
+        if (T <= 8 && mmq_wide_ranges(K, N) > zm) zm = mmq_wide_ranges(K, N);
         if (zm > Z) Z = zm;
     }
     *bytes = Z > 1 ? (uint64_t)Z * T * N * sizeof(float) : 0;

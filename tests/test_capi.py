@@ -106,6 +106,18 @@ def test_query_sized_workspace_is_never_refused(lib):
                 assert rc != WORKSPACE, (K, N, T, n.value)
 
 
+@pytest.mark.parametrize("K,N,T,ranges", [(4096, 2048, 8, 4), (4096, 1024, 5, 8), (6144, 2048, 7, 4), (6144, 3584, 7, 3), (6400, 2048, 8, 3), (4096, 8192, 8, 2)])
+def test_workspace_covers_the_k_ranges_of_eight_wave_workgroups(lib, K, N, T, ranges):
+    """Without a GPU: 256 CUs.  The form of eight waves takes more K ranges than the one of four; a workspace for fewer would be answered with
+    other fp32 sums than the form without a workspace gives, so less than that is refused."""
+    l, _ = lib
+    n = C.c_uint64(7)
+    assert l.mx_gemv_batched_ws_bytes(K, N, T, C.addressof(n)) == 0 and n.value == 4 * ranges * T * N
+    for fmt in ("q4_K", "q6_K"):
+        run = lambda size: getattr(l, "mx_gemv_%s_q8_batched_ws" % fmt)(None, 0x1000, 0x1000, 0x1000, K, N, T, 0x1000, size)  # noqa: E731,B023
+        assert run(n.value) != 9 and run(n.value - 4) == 9
+
+
 def test_dense_gemm_uses_the_shared_scratch_only_where_the_header_says(lib):
     """Without a workspace a dense quant-GEMM is K-sliced, and so uses the scratch that overlapping calls race on, only for K >= 2048
     and 128 x 256 tiles on at most half of the CUs (256 without a GPU), within its 8 Mi floats.  A workspace lifts the first two

@@ -48,6 +48,20 @@ def test_split_k_gemv_static_scratch_equals_workspace_form(mx):
         ops.gemv_q8_batched_ws("q8_0_soa", xq, (qs, d), K, N1, T1, torch.empty(1024, dtype=torch.float32, device="cuda"))
 
 
+@pytest.mark.parametrize("K,N,T", [(4096, 2048, 8), (4096, 33, 5), (6144, 3000, 6), (5888, 1000, 7)])
+def test_eight_wave_int_dot_scratch_equals_workspace_form(mx, K, N, T):
+    """K ranges of the eight-wave workgroups (16 to 24 groups of K, up to 8 tokens): the same cut, hence the same bits, either way."""
+    ops = mx.ops
+    xq = ops.quantize_q8_1(dev(f16(O.normal(6200 + N, (T, K)))).half())
+    for fmt in ("q4_K", "q6_K", "q8_0_soa"):
+        W = synth.normal_weights("q8_0" if fmt == "q8_0_soa" else fmt, N, K, seed=64)
+        w = synth.split_q8_0(W) if fmt == "q8_0_soa" else (W,)
+        ws = torch.full((ops.gemv_batched_ws_bytes(K, N, T) // 4,), float("nan"), dtype=torch.float32, device="cuda")
+        y = getattr(ops, "gemv_%s_q8_batched" % fmt)(xq, *w, K, N, T)
+        assert torch.equal(y, ops.gemv_q8_batched_ws(fmt, xq, w, K, N, T, ws)), fmt
+        assert torch.isfinite(y.float()).all()
+
+
 def test_k_sliced_gemm_static_scratch_equals_workspace_form(mx):
     ops = mx.ops
     K, N = 14336, 4096
