@@ -186,6 +186,10 @@ int mx_gemv_q8_0_soa_q8_batched(mx_stream_t s, const void* x_q8, const int8_t* q
  * is 0 for shapes that never split), so launches on different streams can overlap.  A workspace that is too small
  * is MX_ERR_WORKSPACE; nothing is launched.  */
 int mx_gemv_batched_ws_bytes(uint32_t K, uint32_t N, uint32_t T, uint64_t* bytes);
+/* How a batch of this shape is cut on the current device (host only, nothing is launched), by the weight format of the entry point: "q4_K", "q6_K",
+ * "q8_0", "q8_0_soa" or "mxfp4_soa".  plan[0] = waves of a matrix-core workgroup (0: the vector kernels take the batch), plan[1] = blocks of 32
+ * weight rows of a workgroup, plan[2] = K ranges, fewer where the scratch does not hold their partial sums.  */
+int mx_gemv_batched_plan(const char* format, uint32_t K, uint32_t N, uint32_t T, uint32_t* plan);
 int mx_gemv_q4_K_q8_batched_ws(mx_stream_t s, const void* x_q8, const void* W, uint16_t* y, uint32_t K, uint32_t N, uint32_t T,
                                void* ws, uint64_t ws_bytes);
 int mx_gemv_q6_K_q8_batched_ws(mx_stream_t s, const void* x_q8, const void* W, uint16_t* y, uint32_t K, uint32_t N, uint32_t T,

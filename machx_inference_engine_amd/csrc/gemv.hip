@@ -4,6 +4,7 @@
 #include "mxq_gemv_core.h"
 #include "mxq_mmq.h"
 #include <stdlib.h>
+#include <string.h>
 
 #include <type_traits>
 
@@ -818,15 +819,14 @@ static uint32_t mmq_dense_ranges(uint32_t K, uint32_t N, uint32_t WR, uint32_t W
     return Z < 1 ? 1 : Z;
 }
 
-// ranges = 0: mmq_dense_ranges
 template <class P, int TV, int WR, int WK>
 static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, const uint8_t* xq8, half_t* y, uint32_t K, uint32_t N, uint32_t T,
-                                bool split, const SplitWs& ws, uint32_t ranges = 0) {
+                                bool split, const SplitWs& ws, uint32_t ranges) {
     constexpr bool WIDE = WR * WK == 8;   // one workgroup of eight waves per CU: its LDS is the CU's
     constexpr uint32_t red = (uint32_t)(WR * WK) * TV * 64u * 4u;
     const uint32_t nb = K / 32u, n_groups = (nb + 7u) / 8u;
     const uint32_t rgs = (N + 32u * WR - 1u) / (32u * WR);
-    uint32_t Z = ranges ? ranges : mmq_dense_ranges(K, N, WR, WK);   // the partial sums have to fit the scratch
+    uint32_t Z = ranges;   // the partial sums have to fit the scratch
     if (Z > 1 && (!ws.ptr || (uint64_t)Z * T * N > ws.elems)) {
         if (ws.caller) return MX_ERR_WORKSPACE;
         while (Z > 1 && (!ws.ptr || (uint64_t)Z * T * N > ws.elems)) --Z;
@@ -867,23 +867,47 @@ static uint32_t mmq_wide_ranges(uint32_t K, uint32_t N) {
 // waves share K among themselves: no partial sums in memory and no second launch where the row blocks alone come close to the number
 // of CUs (fewer than three fifths leave more idle than that saves, more than one each run a second round).  Four waves / eight, us with
 // the partial-sum launch: 9 to 16 tokens, blocks of 64 rows, K from 2048 on (1024: equal): 4096 -> 14336, 16 tokens, Q6_K 24.3 / 22.0,
-// Q4_K 17.1 / 15.1, Q8_0 planes 22.8 / 19.1; 3072 -> 12288 18.7 / 16.9, 14.3 / 12.4, 15.3 / 13.1; 6144 -> 16000 35.0 / 31.1, 23.9 / 22.8, 31.4 / 28.7;
+// Q4_K 17.1 / 15.1, Q8_0 planes 22.8 / 19.1, MXFP4 19.8 / 18.2, Q8_0 blocks 35.7 / 33.1; 3072 -> 12288 18.7 / 16.9, 14.3 / 12.4, 15.3 / 13.1; 6144 -> 16000 35.0 / 31.1, 23.9 / 22.8, 31.4 / 28.7.
+// Up to two thirds of the CUs four waves have a fourth K range where the rows are long enough for it, and beyond kFew groups they are faster so:
+// 8192 -> 10240, 16 tokens, Q8_0 blocks 47.3 / 61.1, Q4_K 22.2 / 24.7, Q8_0 planes 27.0 / 29.0, MXFP4 25.6 / 28.3; 3072 -> 9888 Q8_0 blocks
+// +6 %, Q6_K +5 %, Q4_K -8 %; 4096 -> 9888 MXFP4 +6 %, Q4_K -4 %, Q8_0 planes -5 % (from 171 blocks on, 8192 -> 11264: -3 to -12 %, every format);
 // blocks of 32 rows, K up to 4096: 2048 -> 8192 12.0 / 9.9, 10.9 / 9.4, 11.0 / 9.8, 4096 -> 8192 16.6 / 15.4, 13.4 / 12.9, 14.3 / 13.4 (6144 -> 5120 17.2 / 18.8).
 // Up to 8 tokens the waves take 16 to 24 groups (shorter rows leave waves without one: 3072 -> 7936, Q6_K, 10.2 / 11.2; longer ones stream
 // better in ranges: 8192 -> 4096 15.2 / 18.7), with K ranges up to one workgroup per CU: 4096 -> 8192, 8 tokens 15.0 / 12.9, 11.6 / 9.6, 13.3 / 11.4;
 // 4096 -> 2048 10.4 / 8.4, 9.1 / 8.2, 9.2 / 8.1; 6144 -> 3072 14.6 / 12.9, 11.1 / 10.3, 12.6 / 11.4.  Not between seven sixteenths and three
 // fifths of the CUs, where both fill them in two ranges: 5120 -> 4096 11.9 / 12.6, 10.1 / 10.2, 11.5 / 11.6.
+struct MmqPlan {
+    uint32_t wr, wk, ranges;   // blocks of 32 rows and K parts of a workgroup of wr x wk waves; K ranges across workgroups
+};
+template <class P>
+static MmqPlan mmq_plan(uint32_t K, uint32_t N, uint32_t T) {
+    const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u, r64 = (N + 63u) / 64u;
+    if (T <= 8) {
+        if (const uint32_t ranges = mmq_wide_ranges(K, N)) return {1, 8, ranges};
+        return {1, 4, mmq_dense_ranges(K, N, 1, 4)};
+    }
+    constexpr uint32_t kFew = std::is_same<P, MmqQ4K>::value || std::is_same<P, MmqQ8Soa>::value ? 16u : std::is_same<P, MmqMxfp4Soa>::value ? 12u : 11u;
+    if (5u * r64 >= 3u * cus && r64 <= cus && n_groups >= 8u && n_groups <= (3u * r64 < 2u * cus ? kFew : 32u)) return {2, 4, 1};
+    if (5u * r32 >= 3u * cus && r32 <= cus && n_groups <= 16u) return {1, 8, 1};
+    return {2, 2, mmq_dense_ranges(K, N, 2, 2)};
+}
+
 template <class P>
 static int launch_mmq_dense(hipStream_t st, const typename P::Bank& bank, const uint8_t* xq8, half_t* y, uint32_t K, uint32_t N, uint32_t T, bool split,
                             const SplitWs& ws) {
-    const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u, r64 = (N + 63u) / 64u;
-    if (T <= 8) {
-        if (const uint32_t ranges = mmq_wide_ranges(K, N)) return launch_mmq_dense_cfg<P, 4, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, ranges);
-        return launch_mmq_dense_cfg<P, 4, 1, 4>(st, bank, xq8, y, K, N, T, split, ws);
-    }
-    if (5u * r64 >= 3u * cus && r64 <= cus && n_groups >= 8u && n_groups <= 32u) return launch_mmq_dense_cfg<P, 8, 2, 4>(st, bank, xq8, y, K, N, T, split, ws, 1);
-    if (5u * r32 >= 3u * cus && r32 <= cus && n_groups <= 16u) return launch_mmq_dense_cfg<P, 8, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, 1);
-    return launch_mmq_dense_cfg<P, 8, 2, 2>(st, bank, xq8, y, K, N, T, split, ws);
+    const MmqPlan p = mmq_plan<P>(K, N, T);
+    if (T <= 8 && p.wk == 8) return launch_mmq_dense_cfg<P, 4, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, p.ranges);
+    if (T <= 8) return launch_mmq_dense_cfg<P, 4, 1, 4>(st, bank, xq8, y, K, N, T, split, ws, p.ranges);
+    if (p.wk == 4) return launch_mmq_dense_cfg<P, 8, 2, 4>(st, bank, xq8, y, K, N, T, split, ws, p.ranges);
+    if (p.wk == 8) return launch_mmq_dense_cfg<P, 8, 1, 8>(st, bank, xq8, y, K, N, T, split, ws, p.ranges);
+    return launch_mmq_dense_cfg<P, 8, 2, 2>(st, bank, xq8, y, K, N, T, split, ws, p.ranges);
+}
+// the smallest batch a format takes there (measured at launch_q8)
+template <class F>
+static constexpr uint32_t mmq_from(uint32_t K) {
+    constexpr uint32_t kFromT = std::is_same<F, FmtQ8Aos>::value ? 9u : 5u;
+    constexpr bool kEarlier = std::is_same<F, FmtQ8Soa>::value || std::is_same<F, FmtQ6K>::value;
+    return kEarlier && K >= 8192u ? kFromT - 1u : kFromT;
 }
 
 // T up to 16: passes of at most 8 tokens.
@@ -901,12 +925,9 @@ static int launch_q8(mx_stream_t s, GemvSeg<F, OutT> s0, GemvSeg<F, OutT> s1, in
         // measured crossover against the vector-ALU batch kernels (4096 -> 14336, us): Q8_0 planes T = 4: 15.4 vs 16.1,
         // T = 8: 20.4 vs 17.6; Q6_K T = 8: 26.2 vs 22.0; batches of 9 .. 16 take one pass here instead of two there
         // (GGUF Q8_0 blocks: the 2-byte aligned block walk loses below a full second pass, 24.4 vs 30.9 us at T = 8)
-        constexpr uint32_t kMmqFromT = std::is_same<F, FmtQ8Aos>::value ? 9u : 5u;
         // long rows (14336 -> 4096): batches of four cross over one row earlier for Q8_0 planes (19.6 vs 18.9 us) and Q6_K
         // (24.1 vs 22.7 us); Q4_K does not (15.4 vs 15.5 us)
-        constexpr bool kEarlier = std::is_same<F, FmtQ8Soa>::value || std::is_same<F, FmtQ6K>::value;
-        const uint32_t from = (kEarlier && K >= 8192u) ? kMmqFromT - 1u : kMmqFromT;
-        if (T >= from && nseg == 1 && !s0.bias) return launch_mmq_dense<P>(as_stream(s), mmq_bank(s0.w), x, s0.y, K, N, T, split, ws);
+        if (T >= mmq_from<F>(K) && nseg == 1 && !s0.bias) return launch_mmq_dense<P>(as_stream(s), mmq_bank(s0.w), x, s0.y, K, N, T, split, ws);
     }
     for (uint32_t t0 = 0; t0 < T; t0 += 8) {
         const uint32_t tn = (T - t0 < 8) ? T - t0 : 8;
@@ -1202,6 +1223,23 @@ int mx_gemv_batched_ws_bytes(uint32_t K, uint32_t N, uint32_t T, uint64_t* bytes
     }
     *bytes = Z > 1 ? (uint64_t)Z * T * N * sizeof(float) : 0;
     return MX_OK;
+}
+int mx_gemv_batched_plan(const char* format, uint32_t K, uint32_t N, uint32_t T, uint32_t* plan) {
+    MX_REQUIRE_PTR(format); MX_REQUIRE_PTR(plan);
+    MX_REQUIRE_SHAPE(K > 0 && N > 0 && T >= 1 && T <= 16);
+    auto is = [&](const char* name) { return strcmp(format, name) == 0; };
+    auto of = [&](auto fmt) {
+        using F = decltype(fmt);
+        const MmqPlan p = T >= mmq_from<F>(K) ? mmq_plan<typename MmqOf<F>::type>(K, N, T) : MmqPlan{0, 0, 0};
+        plan[0] = p.wr * p.wk; plan[1] = p.wr; plan[2] = p.ranges;
+        return (int)MX_OK;
+    };
+    if (is("q4_K")) return of(FmtQ4K{});
+    if (is("q6_K")) return of(FmtQ6K{});
+    if (is("q8_0")) return of(FmtQ8Aos{});
+    if (is("q8_0_soa")) return of(FmtQ8Soa{});
+    if (is("mxfp4_soa")) return of(FmtMxfp4Soa{});
+    return MX_ERR_UNSUPPORTED;
 }
 int mx_gemv_q8_0_soa_q8_batched_ws(mx_stream_t s, const void* x, const int8_t* qs_W, const uint16_t* d_W, uint16_t* y, uint32_t K, uint32_t N,
                                    uint32_t T, void* ws, uint64_t ws_bytes) {

@@ -216,6 +216,15 @@ def gemv_q8_batched_ws(fmt, x_q8, wargs, K, N, T, ws, y=None):
     return y
 
 
+def gemv_batched_plan(fmt, K, N, T):
+    """(waves of a matrix-core workgroup or 0, its blocks of 32 weight rows, K ranges) of a batch over q8 rows."""
+    plan = (ctypes.c_uint32 * 3)()
+    rc = lib.mx_gemv_batched_plan(fmt.encode(), K, N, T, ctypes.addressof(plan))
+    if rc != 0:
+        raise MxError("mx_gemv_batched_plan", rc)
+    return tuple(plan)
+
+
 def gemm_plan(M, K, N, ws_bytes=None):
     """(32-token tiles, 32-row column tiles, K slices) of a dense quant-GEMM; ws_bytes None: the forms without a workspace."""
     plan = (ctypes.c_uint32 * 3)()

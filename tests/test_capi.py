@@ -118,6 +118,33 @@ def test_workspace_covers_the_k_ranges_of_eight_wave_workgroups(lib, K, N, T, ra
         assert run(n.value) != 9 and run(n.value - 4) == 9
 
 
+FOUR, EIGHT = (4, 2), (8, 2)   # waves and blocks of 32 rows of a workgroup
+
+
+@pytest.mark.parametrize("K,N,forms", [(2816, 9888, dict.fromkeys(("q4_K", "q6_K", "q8_0", "q8_0_soa", "mxfp4_soa"), EIGHT)),
+                                       (3072, 10880, {"q4_K": EIGHT, "q6_K": FOUR, "q8_0": FOUR, "q8_0_soa": EIGHT, "mxfp4_soa": EIGHT}),
+                                       (4096, 9888, {"q4_K": EIGHT, "q6_K": FOUR, "q8_0": FOUR, "q8_0_soa": EIGHT, "mxfp4_soa": FOUR}),
+                                       (8192, 10240, dict.fromkeys(("q4_K", "q6_K", "q8_0", "q8_0_soa", "mxfp4_soa"), FOUR)),
+                                       (8192, 10944, dict.fromkeys(("q4_K", "q6_K", "q8_0", "q8_0_soa", "mxfp4_soa"), EIGHT))])
+@pytest.mark.parametrize("T", [9, 16])
+def test_int_dot_blocks_of_64_rows_where_eight_waves_are_faster(lib, T, K, N, forms):
+    """Without a GPU: 256 CUs.  Up to two thirds of them in row blocks, four waves have a fourth K range and are faster over long rows."""
+    from machx_inference_engine_amd import ops
+    assert {f: ops.gemv_batched_plan(f, K, N, T)[:2] for f in forms} == forms
+    assert all(ops.gemv_batched_plan(f, K, N, T)[2] == 1 or forms[f] == FOUR for f in forms)
+
+
+def test_int_dot_plan_query(lib):
+    l, _ = lib
+    from machx_inference_engine_amd import ops
+    plan = (C.c_uint32 * 3)()
+    p = C.addressof(plan)
+    assert l.mx_gemv_batched_plan(None, 4096, 4096, 8, p) == 1 and l.mx_gemv_batched_plan(b"q4_K", 4096, 4096, 8, None) == 1
+    assert l.mx_gemv_batched_plan(b"q4_K", 4096, 4096, 17, p) == 2 and l.mx_gemv_batched_plan(b"q5_K", 4096, 4096, 8, p) == 5
+    assert ops.gemv_batched_plan("q4_K", 4096, 4096, 4) == (0, 0, 0) and ops.gemv_batched_plan("q8_0", 4096, 14336, 8) == (0, 0, 0)
+    assert ops.gemv_batched_plan("q6_K", 8192, 4096, 4)[0] == 4 and ops.gemv_batched_plan("q4_K", 4096, 14336, 5) == (4, 1, 1)
+
+
 def test_dense_gemm_uses_the_shared_scratch_only_where_the_header_says(lib):
     """Without a workspace a dense quant-GEMM is K-sliced, and so uses the scratch that overlapping calls race on, only for K >= 2048
     and 128 x 256 tiles on at most half of the CUs (256 without a GPU), within its 8 Mi floats.  A workspace lifts the first two
