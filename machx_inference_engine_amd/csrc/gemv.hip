@@ -871,7 +871,9 @@ static uint32_t mmq_wide_ranges(uint32_t K, uint32_t N) {
 // Up to two thirds of the CUs four waves have a fourth K range where the rows are long enough for it, and beyond kFew groups they are faster so:
 // 8192 -> 10240, 16 tokens, Q8_0 blocks 47.3 / 61.1, Q4_K 22.2 / 24.7, Q8_0 planes 27.0 / 29.0, MXFP4 25.6 / 28.3; 3072 -> 9888 Q8_0 blocks
 // +6 %, Q6_K +5 %, Q4_K -8 %; 4096 -> 9888 MXFP4 +6 %, Q4_K -4 %, Q8_0 planes -5 % (from 171 blocks on, 8192 -> 11264: -3 to -12 %, every format);
-// blocks of 32 rows, K up to 4096: 2048 -> 8192 12.0 / 9.9, 10.9 / 9.4, 11.0 / 9.8, 4096 -> 8192 16.6 / 15.4, 13.4 / 12.9, 14.3 / 13.4 (6144 -> 5120 17.2 / 18.8).
+// blocks of 32 rows, K up to 4096: 2048 -> 8192 12.0 / 9.9, 10.9 / 9.4, 11.0 / 9.8, 4096 -> 8192 16.6 / 15.4, 13.4 / 12.9, 14.3 / 13.4 (6144 -> 5120 17.2 / 18.8),
+// and from three groups on, Q8_0 planes from 1024 elements (of two groups six waves have nothing to do: 512 -> 6144, 16 tokens, Q4_K 5.8 / 6.8, Q6_K 6.2 / 6.4
+// +11 %, MXFP4 6.4 / 6.7; 768 -> 6144 Q4_K -4 %, Q6_K -9 %, MXFP4 -14 %, Q8_0 blocks -14 %; Q8_0 planes 736 -> 8192 +10 %, 768 +3 %, 1024 -1 to -4 %).
 // Up to 8 tokens the waves take 16 to 24 groups (shorter rows leave waves without one: 3072 -> 7936, Q6_K, 10.2 / 11.2; longer ones stream
 // better in ranges: 8192 -> 4096 15.2 / 18.7), with K ranges up to one workgroup per CU: 4096 -> 8192, 8 tokens 15.0 / 12.9, 11.6 / 9.6, 13.3 / 11.4;
 // 4096 -> 2048 10.4 / 8.4, 9.1 / 8.2, 9.2 / 8.1; 6144 -> 3072 14.6 / 12.9, 11.1 / 10.3, 12.6 / 11.4.  Not between seven sixteenths and three
@@ -888,7 +890,8 @@ static MmqPlan mmq_plan(uint32_t K, uint32_t N, uint32_t T) {
     }
     constexpr uint32_t kFew = std::is_same<P, MmqQ4K>::value || std::is_same<P, MmqQ8Soa>::value ? 16u : std::is_same<P, MmqMxfp4Soa>::value ? 12u : 11u;
     if (5u * r64 >= 3u * cus && r64 <= cus && n_groups >= 8u && n_groups <= (3u * r64 < 2u * cus ? kFew : 32u)) return {2, 4, 1};
-    if (5u * r32 >= 3u * cus && r32 <= cus && n_groups <= 16u) return {1, 8, 1};
+    constexpr uint32_t kShort = std::is_same<P, MmqQ8Soa>::value ? 1024u : 513u;
+    if (5u * r32 >= 3u * cus && r32 <= cus && K >= kShort && n_groups <= 16u) return {1, 8, 1};
     return {2, 2, mmq_dense_ranges(K, N, 2, 2)};
 }
 

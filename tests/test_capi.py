@@ -134,6 +134,16 @@ def test_int_dot_blocks_of_64_rows_where_eight_waves_are_faster(lib, T, K, N, fo
     assert all(ops.gemv_batched_plan(f, K, N, T)[2] == 1 or forms[f] == FOUR for f in forms)
 
 
+@pytest.mark.parametrize("K,N,formats", [(256, 8192, ()), (512, 6144, ()), (544, 6144, ("q8_0", "mxfp4_soa")), (768, 4928, ("q4_K", "q6_K", "q8_0", "mxfp4_soa")),
+                                         (1024, 8192, ("q4_K", "q6_K", "q8_0", "q8_0_soa", "mxfp4_soa"))])
+def test_int_dot_blocks_of_32_rows_have_work_for_eight_waves(lib, K, N, formats):
+    """Without a GPU: 256 CUs.  Rows of one or two groups leave six of eight waves without one."""
+    from machx_inference_engine_amd import ops
+    all_formats = ("q4_K", "q6_K", "q8_0", "q8_0_soa", "mxfp4_soa") if K % 256 == 0 else ("q8_0", "q8_0_soa", "mxfp4_soa")
+    for f in all_formats:
+        assert ops.gemv_batched_plan(f, K, N, 12)[:2] == ((8, 1) if f in formats else (4, 2)), f
+
+
 def test_int_dot_plan_query(lib):
     l, _ = lib
     from machx_inference_engine_amd import ops
