@@ -860,7 +860,8 @@ static int launch_mmq_dense_cfg(hipStream_t st, const typename P::Bank& bank, co
 static uint32_t mmq_wide_ranges(uint32_t K, uint32_t N) {
     const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u;
     if (n_groups < 16u || n_groups > 24u || !(16u * r32 <= 7u * cus || (5u * r32 >= 3u * cus && r32 <= cus))) return 0;
-    return 8u * r32 <= cus ? 8u : cus / r32;
+    const uint32_t ranges = 8u * r32 <= cus ? 8u : cus / r32;
+    return ranges == 2u && n_groups >= 19u && n_groups <= 23u ? 0u : ranges;
 }
 
 // Workgroups of four waves, two or three per CU, K ranges across them where the row blocks are too few; or of eight waves, one per CU, whose
@@ -877,7 +878,10 @@ static uint32_t mmq_wide_ranges(uint32_t K, uint32_t N) {
 // Up to 8 tokens the waves take 16 to 24 groups (shorter rows leave waves without one: 3072 -> 7936, Q6_K, 10.2 / 11.2; longer ones stream
 // better in ranges: 8192 -> 4096 15.2 / 18.7), with K ranges up to one workgroup per CU: 4096 -> 8192, 8 tokens 15.0 / 12.9, 11.6 / 9.6, 13.3 / 11.4;
 // 4096 -> 2048 10.4 / 8.4, 9.1 / 8.2, 9.2 / 8.1; 6144 -> 3072 14.6 / 12.9, 11.1 / 10.3, 12.6 / 11.4.  Not between seven sixteenths and three
-// fifths of the CUs, where both fill them in two ranges: 5120 -> 4096 11.9 / 12.6, 10.1 / 10.2, 11.5 / 11.6.
+// fifths of the CUs, where both fill them in two ranges: 5120 -> 4096 11.9 / 12.6, 10.1 / 10.2, 11.5 / 11.6; and not with two ranges of 10 to
+// 12 groups, a second round that eight waves do not fill: 5120 -> 3072 Q6_K 11.1 / 11.9, MXFP4 +3 to +5 %, Q4_K and Q8_0 planes +-1 % (4608 -> 3072 -4
+// to 0 %, 6144 -> 3072, against three ranges of four waves, -2 to -12 %).  By format: 6144 -> 4928, one range against three, Q6_K +3 %, MXFP4 +1 %
+// (Q4_K -6 %, Q8_0 planes -3 %); MXFP4 4096 -> 3072 +3 %, 6144 -> 2560 +2 %.
 struct MmqPlan {
     uint32_t wr, wk, ranges;   // blocks of 32 rows and K parts of a workgroup of wr x wk waves; K ranges across workgroups
 };
@@ -885,7 +889,11 @@ template <class P>
 static MmqPlan mmq_plan(uint32_t K, uint32_t N, uint32_t T) {
     const uint32_t cus = (uint32_t)cu_count(), n_groups = (K / 32u + 7u) / 8u, r32 = (N + 31u) / 32u, r64 = (N + 63u) / 64u;
     if (T <= 8) {
-        if (const uint32_t ranges = mmq_wide_ranges(K, N)) return {1, 8, ranges};
+        constexpr bool Q6 = std::is_same<P, MmqQ6K>::value, FP4 = std::is_same<P, MmqMxfp4Soa>::value;
+        const uint32_t ranges = mmq_wide_ranges(K, N);
+        const bool four = ((Q6 || FP4) && ranges == 1u && n_groups == 24u && 3u * r32 < 2u * cus) ||
+                          (FP4 && ((ranges == 2u && n_groups == 16u) || (ranges == 3u && n_groups == 24u)));
+        if (ranges && !four) return {1, 8, ranges};
         return {1, 4, mmq_dense_ranges(K, N, 1, 4)};
     }
     constexpr uint32_t kFew = std::is_same<P, MmqQ4K>::value || std::is_same<P, MmqQ8Soa>::value ? 16u : std::is_same<P, MmqMxfp4Soa>::value ? 12u : 11u;

@@ -144,6 +144,17 @@ def test_int_dot_blocks_of_32_rows_have_work_for_eight_waves(lib, K, N, formats)
         assert ops.gemv_batched_plan(f, K, N, 12)[:2] == ((8, 1) if f in formats else (4, 2)), f
 
 
+@pytest.mark.parametrize("K,N,formats", [(4096, 3072, ("q4_K", "q6_K", "q8_0_soa")), (4608, 3072, ("q4_K", "q6_K", "q8_0_soa", "mxfp4_soa")), (5120, 3072, ()),
+                                         (5888, 2816, ()), (5120, 2560, ("q4_K", "q6_K", "q8_0_soa", "mxfp4_soa")), (6144, 2560, ("q4_K", "q6_K", "q8_0_soa")),
+                                         (6144, 3072, ("q4_K", "q6_K", "q8_0_soa", "mxfp4_soa")), (6144, 5440, ("q4_K", "q8_0_soa")),
+                                         (6144, 5472, ("q4_K", "q6_K", "q8_0_soa", "mxfp4_soa"))])
+def test_int_dot_k_ranges_of_eight_waves_where_they_are_faster(lib, K, N, formats):
+    """Without a GPU: 256 CUs.  Up to 8 tokens: two K ranges of 10 to 12 groups and, by format, the shapes where four waves have a third range run in those."""
+    from machx_inference_engine_amd import ops
+    for f in ("q4_K", "q6_K", "q8_0_soa", "mxfp4_soa"):
+        assert ops.gemv_batched_plan(f, K, N, 6)[0] == (8 if f in formats else 4), f
+
+
 def test_int_dot_plan_query(lib):
     l, _ = lib
     from machx_inference_engine_amd import ops
