@@ -322,7 +322,7 @@ int mx_gemv_q8_0_f32(mx_stream_t s, const float* A, const void* W, float* y, uin
  * as dequant_q8_0_soa_to_Bt + gemm_fp16, src/model/qwen35_dense.cpp:811-831).
  * Shared scratch.  A launch with K >= 2048 whose 128 x 256 output tiles cover at most half of the CUs,
  * ceil(M / 128) * ceil(N / 256) <= 128 on MI355X, may be cut into 2..8 K slices (every mx_gemm_* of a quantized
- * weight, Q4_0, Q5_K and MXFP4 included; mx_gemm_plan tells).  Their fp32 partial sums go through a
+ * weight, Q4_0, Q5_K and MXFP4 included; mx_gemm_form tells).  Their fp32 partial sums go through a
  * 32 MB per-device scratch array owned by the library (a file-scope device array resolved with hipGetSymbolAddress,
  * never allocated; slices * M * N <= 8 Mi floats, fewer slices beyond that) and are added in slice
  * order by a second small launch: two such calls that overlap on one device race on it, as the
@@ -360,9 +360,12 @@ int mx_gemm_mxfp4_soa_ws(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, 
 /* How a dense quant-GEMM of this shape is cut on the current device (host only, nothing is launched): plan[0] = 32-token
  * tiles per workgroup tile of an eight-wave workgroup (1..4; 0: four-wave workgroups over 128 x 256), plan[1] = 32-row
  * column tiles per wave (1 or 2), plan[2] = K slices (1: no scratch is used).  own_ws = 0: the forms without a workspace;
- * else the *_ws forms with a workspace of ws_bytes.  Launches of more than 256 tokens may run over 256 x 256 tiles, unsliced
- * and without scratch, in place of this plan, by format.  */
+ * else the *_ws forms with a workspace of ws_bytes.  This is the plan every format shares; by format, launches of more than 256 tokens
+ * run over 256 x 256 tiles in its place, unsliced and without scratch.  mx_gemm_form tells what a launch does: format = "q4_K", "q6_K", "q8_0",
+ * "q8_0_soa", "q4_0", "q5_K" or "mxfp4_soa", form[0..2] = the plan, form[0] = 8 for 256 x 256 tiles, form[3] = how many of
+ * those run as two column halves.  */
 int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* plan);
+int mx_gemm_form(const char* format, uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* form);
 /* Q4_0 weights through the same kernel: gemm_q4_0 / gemm_q4_0_xmx  include/ie/ops.hpp:530-534, src/ops/gemv_q4_0.cpp,
  * src/ops/gemm_q4k_xmx.cpp:418-522; K % 128 == 0, W 2-byte aligned.  */
 int mx_gemm_q4_0(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N);

@@ -25,6 +25,7 @@
 //               trip and no redundant dequantisation inside a workgroup.
 // The k order inside a chunk is (lanes 0-31: 8s.., lanes 32-63: 64+8s..); the
 // A fragments are read from LDS with the same order, so the products pair up.
+#include <string.h>
 #include <type_traits>
 
 #include "mxq_formats.h"
@@ -1743,6 +1744,9 @@ static int gemm_cu_count() {
     return n;
 }
 
+// 256-token tiles: a last round that covers at most half of the CUs runs as twice as many column halves
+static uint64_t gemm_whole_tiles(uint64_t tiles, uint64_t cus) { return 2 * (tiles % cus) <= cus ? tiles - tiles % cus : tiles; }
+
 template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
 static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound) {
     constexpr uint32_t BN = (MODE == GEMM_MOE_GATE_UP_SILU || MODE == GEMM_MOE_GATE_UP_OAI) ? 128 : 128 * NJ, BM = 32u * NI;
@@ -1753,9 +1757,7 @@ static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const type
     const uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.k_split;
     uint64_t grid = (total + 7) / 8 * 8;
     if constexpr (NI == 8) {
-        // a last round that covers at most half of the CUs runs as twice as many halves
-        const uint64_t cus = (uint64_t)gemm_cu_count(), rest = total % cus;
-        g.whole = (uint32_t)(2 * rest <= cus ? total - rest : total);
+        g.whole = (uint32_t)gemm_whole_tiles(total, (uint64_t)gemm_cu_count());
         grid = ((uint64_t)g.whole + 7) / 8 * 8 + (2 * (total - g.whole) + 7) / 8 * 8;
     }
     if (grid > 0x7FFFFFFFull) return MX_ERR_SHAPE;
@@ -1837,14 +1839,21 @@ static uint64_t gemm_library_scratch(uint64_t M, uint64_t K, uint64_t N, uint64_
 template <class QF> struct GemmSmall { using type = QF; };
 template <> struct GemmSmall<GemmQ6K> { using type = GemmQ6KDw; };
 
+// The form of a dense launch of a format: the plan, na = 8 where the 256-token tiles take its place.
+template <class QF>
+static GemmPlan gemm_form(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus) {
+    double t_plan = 0.0;
+    const GemmPlan p = gemm_plan(M, K, N, cap, cus, &t_plan);
+    return gemm_tall(M, K, N, cus, gemm_tall_cost<QF>, t_plan) ? GemmPlan{8, 2, 1} : p;
+}
+
 template <class QF, int MODE>
 static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound,
                        const SplitWs* caller_ws = nullptr) {
     if constexpr (MODE == GEMM_DENSE) {
         const uint64_t cus = (uint64_t)gemm_cu_count();
-        double t_plan = 0.0;
-        const GemmPlan p = gemm_plan(g.M, g.K, g.N, caller_ws ? caller_ws->elems : gemm_library_scratch(g.M, g.K, g.N, cus), cus, &t_plan);
-        if (gemm_tall(g.M, g.K, g.N, cus, gemm_tall_cost<QF>, t_plan)) {
+        const GemmPlan p = gemm_form<QF>(g.M, g.K, g.N, caller_ws ? caller_ws->elems : gemm_library_scratch(g.M, g.K, g.N, cus), cus);
+        if (p.na == 8) {
             g.k_split = 1;
             return launch_gemm_ni<QF, MODE, 8>(s, b0, b1, g, rows_bound);
         }
@@ -1988,6 +1997,25 @@ int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_byt
     const uint64_t cus = (uint64_t)gemm_cu_count();
     const GemmPlan p = gemm_plan(M, K, N, own_ws ? ws_bytes / 4 : gemm_library_scratch(M, K, N, cus), cus);
     plan[0] = p.na; plan[1] = p.nj; plan[2] = p.k_split;
+    return MX_OK;
+}
+int mx_gemm_form(const char* format, uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* form) {
+    MX_REQUIRE_PTR(format); MX_REQUIRE_PTR(form);
+    MX_REQUIRE_SHAPE(M > 0 && K > 0 && N > 0);
+    const uint64_t cus = (uint64_t)gemm_cu_count(), cap = own_ws ? ws_bytes / 4 : gemm_library_scratch(M, K, N, cus);
+    auto is = [&](const char* name) { return strcmp(format, name) == 0; };
+    GemmPlan p{0, 0, 0};
+    if (is("q4_K")) p = gemm_form<GemmQ4KPair>(M, K, N, cap, cus);
+    else if (is("q6_K")) p = gemm_form<GemmQ6K>(M, K, N, cap, cus);
+    else if (is("q8_0")) p = gemm_form<GemmQ8Aos>(M, K, N, cap, cus);
+    else if (is("q8_0_soa")) p = gemm_form<GemmQ8Quad>(M, K, N, cap, cus);
+    else if (is("q4_0")) p = gemm_form<GemmQ40>(M, K, N, cap, cus);
+    else if (is("q5_K")) p = gemm_form<GemmQ5K>(M, K, N, cap, cus);
+    else if (is("mxfp4_soa")) p = gemm_form<GemmMxfp4Pair>(M, K, N, cap, cus);
+    else return MX_ERR_UNSUPPORTED;
+    const uint64_t tiles = ((uint64_t)M + 255) / 256 * (((uint64_t)N + 255) / 256);
+    form[0] = p.na; form[1] = p.nj; form[2] = p.k_split;
+    form[3] = p.na == 8 ? (uint32_t)(tiles - gemm_whole_tiles(tiles, cus)) : 0u;
     return MX_OK;
 }
 int mx_gemm_q4_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {

@@ -234,6 +234,15 @@ def gemm_plan(M, K, N, ws_bytes=None):
     return tuple(plan)
 
 
+def gemm_form(fmt, M, K, N, ws_bytes=None):
+    """gemm_plan as a launch of this format has it, 8 as the first for tiles of 256 tokens, and how many of those run as column halves."""
+    form = (ctypes.c_uint32 * 4)()
+    rc = lib.mx_gemm_form(fmt.encode(), M, K, N, ws_bytes is not None, ws_bytes or 0, ctypes.addressof(form))
+    if rc != 0:
+        raise MxError("mx_gemm_form", rc)
+    return tuple(form)
+
+
 def gemm_ws(fmt, A, wargs, M, K, N, ws, y=None):
     """Caller-workspace dense quant-GEMM: fmt in ('q4_K', 'q6_K', 'q8_0', 'q8_0_soa', 'q4_0', 'q5_K', 'mxfp4_soa')."""
     y = _out(y, (M, N), torch.float16, A)

@@ -195,6 +195,24 @@ def test_dense_gemm_uses_the_shared_scratch_only_where_the_header_says(lib):
         assert fn(None, p16, *w, p16, 64, 1280, 896, None, 64) == 1 and fn(None, p16, *w, p16, 64, 1280, 896, 0x1004, 64) == 3
 
 
+DENSE = ("q4_K", "q6_K", "q8_0", "q8_0_soa", "q4_0", "q5_K", "mxfp4_soa")
+
+
+def test_gemm_form_query(lib):
+    """mx_gemm_plan is the plan the formats share; what a launch does depends on the format too, and mx_gemm_form says it."""
+    l, _ = lib
+    from machx_inference_engine_amd import ops
+    for M, K, N in [(1, 64, 33), (77, 14336, 4096), (256, 14336, 4096), (512, 4096, 14336), (700, 1792, 9000)]:
+        for f in DENSE:
+            for ws in (None, 32 << 20):
+                assert ops.gemm_form(f, M, K, N, ws) == ops.gemm_plan(M, K, N, ws) + (0,), (f, M, K, N)
+    assert all(ops.gemm_form(f, 4096, 14336, 4096) == (8, 2, 1, 0) for f in DENSE) and ops.gemm_plan(4096, 14336, 4096)[0] == 0
+    form = (C.c_uint32 * 4)()
+    p = C.addressof(form)
+    assert l.mx_gemm_form(None, 64, 1280, 896, 0, 0, p) == 1 and l.mx_gemm_form(b"q4_K", 64, 1280, 896, 0, 0, None) == 1
+    assert l.mx_gemm_form(b"q4_K", 64, 0, 896, 0, 0, p) == 2 and l.mx_gemm_form(b"q3_K", 64, 1280, 896, 0, 0, p) == 5
+
+
 def test_gemm_workspace_query_names_what_the_plan_uses(lib):
     """A workspace of the queried size gives the plan of an unlimited one, and outside the shapes that the library's own scratch
     serves it is no larger than that plan's partial sums."""

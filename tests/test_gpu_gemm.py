@@ -113,7 +113,7 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     """Every form of a dense launch with every weight loader, MXFP4 with a row that ends half way through a chunk; the form a shape takes
     is asked of the library, so that a change of the rule shows.  Against the exact products of the fp16 weights in fp64."""
     M, K, N = half if fmt == "mxfp4_soa" else whole
-    na, nj, k = mx.ops.gemm_plan(M, K, N, 32 << 20)
+    na, nj, k, _ = mx.ops.gemm_form(fmt, M, K, N, 32 << 20)
     assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or (na, nj, k > 1) == form, (na, nj, k)
     wargs, values = any_weights(fmt, N, K, 2500 + M)
     a = dev(f16(O.normal(2501 + M, (M, K)))).half()
@@ -130,6 +130,7 @@ def test_gemm_256_token_tiles(mx, fmt, M, K, N):
     """The tiles of 256 tokens (gemm_tall in csrc/gemm.hip; 256 CUs) with every weight loader, ragged in tokens and columns; the second shape
     ends in column halves, one of them past N; MXFP4 in a row that ends half way through a chunk.  The sums run over K in one piece: against the
     exact products of the fp16 weights in fp64, as every other form."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or mx.ops.gemm_form(fmt, M, K, N) == (8, 2, 1, 101 if M == 1600 else 0)
     wargs, values = any_weights(fmt, N, K, 2600 + M)
     a = dev(f16(O.normal(2601 + M, (M, K)))).half()
     run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, *wargs, M, K, N)  # noqa: E731
