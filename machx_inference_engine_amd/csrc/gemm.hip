@@ -1616,8 +1616,12 @@ __device__ __forceinline__ bool find_grouped_tile(const uint32_t* expert_offsets
 template <int NA, int NJ>
 constexpr int gemm_k2_depth() { return NA * NJ <= 4 ? 2 : 1; }
 
-// NI = 32-token tiles per workgroup tile.  KW = 1: four waves, 128 tokens, two workgroups per CU.  KW = 2: eight waves, the two
-// halves of the K slice side by side, one workgroup per CU, 32 to 128 tokens.
+// Whether 256-token tiles of the last round may run as column halves: for Q6_K, whose tiles are taken with a margin (gemm_tall).  For the
+// other formats the modelled gain is below 0.2 % wherever halves would be taken (6400 tokens, 24576 -> 10496: 3349 of 3352 us).
+template <class QF> constexpr bool gemm_tall_halves = std::is_same<QF, GemmQ6K>::value;
+
+// NI = 32-token tiles per workgroup tile.  KW = 1: four waves, 128 tokens (NI = 8: 256), two workgroups per CU (one).  KW = 2: eight waves,
+// the two halves of the K slice side by side, one workgroup per CU, 32 to 128 tokens.
 template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
 __global__ __launch_bounds__(kGemmThreads * KW, (KW == 2 || NI == 8) ? 1 : 2) void gemm_kernel(typename QF::Bank bank0, typename QF::Bank bank1, GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
@@ -1634,7 +1638,7 @@ __global__ __launch_bounds__(kGemmThreads * KW, (KW == 2 || NI == 8) ? 1 : 2) vo
     const uint32_t per_xcd = (total + 7) / 8;
     uint32_t lin_ks = (MODE == GEMM_DENSE) ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x, half = 0;
     bool halves = false;
-    if constexpr (NI == 8) {
+    if constexpr (NI == 8 && gemm_tall_halves<QF>) {
         // the whole tiles, and behind them the column halves of the rest, each dealt to the XCDs in contiguous ranges
         const uint32_t whole8 = (g.whole + 7u) / 8u * 8u, per_w = whole8 / 8u, per_h = (2u * (total - g.whole) + 7u) / 8u;
         halves = blockIdx.x >= whole8;
@@ -1695,9 +1699,13 @@ __global__ __launch_bounds__(kGemmThreads * KW, (KW == 2 || NI == 8) ? 1 : 2) vo
             const uint32_t kw = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8)), first = (n_slice + 1u) / 2u;
             gemm_tile<QF, MODE, NI, gemm_k2_depth<NI, NJ>(), 2, NJ>(g, w0, w1, row_lo, row_hi, n_base, lds_raw + kw * (2u * BM * kBK * 2u), c0 + kw * first,
                                                                       kw ? n_slice - first : first, ks, 0, lds_raw, first);
-        } else if (NI == 8 && halves) {
-            const uint32_t n_half = tn * BN + half * (BN / 2u) + wave * (BN / 8u);
-            if (tn * BN + half * (BN / 2u) < g.N) gemm_tile<QF, MODE, NI, 1, 1, 1>(g, w0, w1, row_lo, row_hi, n_half, lds_raw, c0, n_slice, ks);
+        } else if constexpr (NI == 8 && gemm_tall_halves<QF>) {
+            if (halves) {
+                const uint32_t n_half = tn * BN + half * (BN / 2u) + wave * (BN / 8u);
+                if (tn * BN + half * (BN / 2u) < g.N) gemm_tile<QF, MODE, NI, 1, 1, 1>(g, w0, w1, row_lo, row_hi, n_half, lds_raw, c0, n_slice, ks);
+            } else {
+                gemm_tile<QF, MODE, NI, 1>(g, w0, w1, row_lo, row_hi, n_base, lds_raw, c0, n_slice, ks);
+            }
         } else {
             gemm_tile<QF, MODE, NI, 1>(g, w0, w1, row_lo, row_hi, n_base, lds_raw, c0, n_slice, ks);
         }
@@ -1744,8 +1752,11 @@ static int gemm_cu_count() {
     return n;
 }
 
-// 256-token tiles: a last round that covers at most half of the CUs runs as twice as many column halves
-static uint64_t gemm_whole_tiles(uint64_t tiles, uint64_t cus) { return 2 * (tiles % cus) <= cus ? tiles - tiles % cus : tiles; }
+// how many of the 256-token tiles of a launch run whole
+template <class QF>
+static uint64_t gemm_whole_tiles(uint64_t tiles, uint64_t cus) {
+    return gemm_tall_halves<QF> && 2 * (tiles % cus) <= cus ? tiles - tiles % cus : tiles;
+}
 
 template <class QF, int MODE, int NI, int KW = 1, int NJ = 2>
 static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const typename QF::Bank& b1, GemmArgs g, uint32_t rows_bound) {
@@ -1757,7 +1768,7 @@ static int launch_gemm_ni(mx_stream_t s, const typename QF::Bank& b0, const type
     const uint64_t total = (uint64_t)g.tiles_m * g.tiles_n * g.k_split;
     uint64_t grid = (total + 7) / 8 * 8;
     if constexpr (NI == 8) {
-        g.whole = (uint32_t)gemm_whole_tiles(total, (uint64_t)gemm_cu_count());
+        g.whole = (uint32_t)gemm_whole_tiles<QF>(total, (uint64_t)gemm_cu_count());
         grid = ((uint64_t)g.whole + 7) / 8 * 8 + (2 * (total - g.whole) + 7) / 8 * 8;
     }
     if (grid > 0x7FFFFFFFull) return MX_ERR_SHAPE;
@@ -1816,16 +1827,16 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint
 // a weight is dequantized for twice as many tokens, which matters most where that is most work (4096 tokens, 14336 -> 4096, us: Q6_K
 // 567 -> 480, Q4_K 449 -> 420, Q8_0 planes 449 -> 421).  But the rounds are coarse, and one workgroup alone on a CU shows the start and
 // end of a tile (K = 1024, 4096 tokens, 4096 rows, Q4_K: 43 us in four-wave workgroups, 50 so; 4096 -> 14336, 3.5 rounds: 451 and 473);
-// a last round that would leave more than half of the CUs idle runs as column halves.  Taken in place of the plan above where its
+// a last round that would leave more than half of the CUs idle runs as column halves (gemm_tall_halves).  Taken in place of the plan above where its
 // modelled time (microseconds, fitted like the plan's, K from 2048 on) is less; `cost` = the format's time so against its time in the
 // plan's forms, 1 for Q4_K and Q8_0 (Q6_K 4096 -> 14336: 1024 tokens 185 -> 164, 2048 tokens 348 -> 318, 4096 tokens 608 -> 558).
 template <class QF> constexpr double gemm_tall_cost = 1.0;
 template <> constexpr double gemm_tall_cost<GemmQ6K> = 0.83;
-static bool gemm_tall(uint64_t M, uint64_t K, uint64_t N, uint64_t cus, double cost, double t_plan) {
+static bool gemm_tall(uint64_t M, uint64_t K, uint64_t N, uint64_t cus, double cost, bool with_halves, double t_plan) {
     const uint64_t n_chunks = (K + kBK - 1) / kBK, tiles = ((M + 255) / 256) * ((N + 255) / 256), full = tiles / cus, rest = tiles % cus;
     if (M <= 256 || n_chunks < 16) return false;
     const double whole = 14.0 + 3.62 * (double)n_chunks, halves = 14.0 + 2.6 * (double)n_chunks;
-    return cost * ((double)full * whole + (rest == 0 ? 0.0 : 2 * rest <= cus ? halves : whole)) < t_plan;
+    return cost * ((double)full * whole + (rest == 0 ? 0.0 : with_halves && 2 * rest <= cus ? halves : whole)) < t_plan;
 }
 
 // Floats of the library's scratch that a launch without a caller's workspace may use.  Calls that overlap on one device race on it, so
@@ -1844,7 +1855,7 @@ template <class QF>
 static GemmPlan gemm_form(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus) {
     double t_plan = 0.0;
     const GemmPlan p = gemm_plan(M, K, N, cap, cus, &t_plan);
-    return gemm_tall(M, K, N, cus, gemm_tall_cost<QF>, t_plan) ? GemmPlan{8, 2, 1} : p;
+    return gemm_tall(M, K, N, cus, gemm_tall_cost<QF>, gemm_tall_halves<QF>, t_plan) ? GemmPlan{8, 2, 1} : p;
 }
 
 template <class QF, int MODE>
@@ -2004,19 +2015,22 @@ int mx_gemm_form(const char* format, uint32_t M, uint32_t K, uint32_t N, int own
     MX_REQUIRE_SHAPE(M > 0 && K > 0 && N > 0);
     const uint64_t cus = (uint64_t)gemm_cu_count(), cap = own_ws ? ws_bytes / 4 : gemm_library_scratch(M, K, N, cus);
     auto is = [&](const char* name) { return strcmp(format, name) == 0; };
-    GemmPlan p{0, 0, 0};
-    if (is("q4_K")) p = gemm_form<GemmQ4KPair>(M, K, N, cap, cus);
-    else if (is("q6_K")) p = gemm_form<GemmQ6K>(M, K, N, cap, cus);
-    else if (is("q8_0")) p = gemm_form<GemmQ8Aos>(M, K, N, cap, cus);
-    else if (is("q8_0_soa")) p = gemm_form<GemmQ8Quad>(M, K, N, cap, cus);
-    else if (is("q4_0")) p = gemm_form<GemmQ40>(M, K, N, cap, cus);
-    else if (is("q5_K")) p = gemm_form<GemmQ5K>(M, K, N, cap, cus);
-    else if (is("mxfp4_soa")) p = gemm_form<GemmMxfp4Pair>(M, K, N, cap, cus);
-    else return MX_ERR_UNSUPPORTED;
-    const uint64_t tiles = ((uint64_t)M + 255) / 256 * (((uint64_t)N + 255) / 256);
-    form[0] = p.na; form[1] = p.nj; form[2] = p.k_split;
-    form[3] = p.na == 8 ? (uint32_t)(tiles - gemm_whole_tiles(tiles, cus)) : 0u;
-    return MX_OK;
+    auto of = [&](auto fmt) {
+        using QF = decltype(fmt);
+        const GemmPlan p = gemm_form<QF>(M, K, N, cap, cus);
+        const uint64_t tiles = ((uint64_t)M + 255) / 256 * (((uint64_t)N + 255) / 256);
+        form[0] = p.na; form[1] = p.nj; form[2] = p.k_split;
+        form[3] = p.na == 8 ? (uint32_t)(tiles - gemm_whole_tiles<QF>(tiles, cus)) : 0u;
+        return (int)MX_OK;
+    };
+    if (is("q4_K")) return of(GemmQ4KPair{});
+    if (is("q6_K")) return of(GemmQ6K{});
+    if (is("q8_0")) return of(GemmQ8Aos{});
+    if (is("q8_0_soa")) return of(GemmQ8Quad{});
+    if (is("q4_0")) return of(GemmQ40{});
+    if (is("q5_K")) return of(GemmQ5K{});
+    if (is("mxfp4_soa")) return of(GemmMxfp4Pair{});
+    return MX_ERR_UNSUPPORTED;
 }
 int mx_gemm_q4_K_ws(mx_stream_t s, const uint16_t* A, const void* W, uint16_t* y, uint32_t M, uint32_t K, uint32_t N, void* ws, uint64_t ws_bytes) {
     SplitWs w;

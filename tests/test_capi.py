@@ -213,6 +213,14 @@ def test_gemm_form_query(lib):
     assert l.mx_gemm_form(b"q4_K", 64, 0, 896, 0, 0, p) == 2 and l.mx_gemm_form(b"q3_K", 64, 1280, 896, 0, 0, p) == 5
 
 
+def test_gemm_column_halves_are_q6_K_s(lib):
+    """Column halves of 256-token tiles: the formats whose tiles the model takes without a margin run them whole."""
+    from machx_inference_engine_amd import ops
+    for M, K, N in [(33000, 14336, 4096), (6400, 24576, 10496), (1644, 13056, 4608), (4096, 14336, 5000)]:
+        assert ops.gemm_form("q6_K", M, K, N)[0] == 8 and all(ops.gemm_form(f, M, K, N)[3] == 0 for f in DENSE if f != "q6_K")
+    assert ops.gemm_form("q6_K", 1644, 13056, 4500)[3] == 126 and ops.gemm_form("q6_K", 1600, 2048, 12900)[3] == 101
+
+
 def test_gemm_workspace_query_names_what_the_plan_uses(lib):
     """A workspace of the queried size gives the plan of an unlimited one, and outside the shapes that the library's own scratch
     serves it is no larger than that plan's partial sums."""

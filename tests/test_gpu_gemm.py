@@ -124,13 +124,13 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     assert torch.equal(run(), got), "differs from launch to launch"
 
 
-@pytest.mark.parametrize("fmt,M,K,N", [("q6_K", 1100, 2048, 13000), ("q6_K", 1600, 2048, 12900), ("q4_K", 1100, 12288, 13000), ("q8_0_soa", 1100, 12288, 13000),
+@pytest.mark.parametrize("fmt,M,K,N", [("q6_K", 1100, 2048, 13000), ("q6_K", 1600, 2048, 12900), ("q6_K", 1644, 13056, 4500), ("q4_K", 1100, 12288, 13000), ("q8_0_soa", 1100, 12288, 13000),
                                        ("q8_0", 1100, 12288, 13000), ("q4_0", 1100, 12288, 13000), ("q5_K", 1100, 12288, 13000), ("mxfp4_soa", 1100, 12224, 13000)])
 def test_gemm_256_token_tiles(mx, fmt, M, K, N):
     """The tiles of 256 tokens (gemm_tall in csrc/gemm.hip; 256 CUs) with every weight loader, ragged in tokens and columns; the second shape
-    ends in column halves, one of them past N; MXFP4 in a row that ends half way through a chunk.  The sums run over K in one piece: against the
+    ends in column halves, one of them past N, the third has nothing else; MXFP4 in a row that ends half way through a chunk.  The sums run over K in one piece: against the
     exact products of the fp16 weights in fp64, as every other form."""
-    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or mx.ops.gemm_form(fmt, M, K, N) == (8, 2, 1, 101 if M == 1600 else 0)
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or mx.ops.gemm_form(fmt, M, K, N) == (8, 2, 1, {1600: 101, 1644: 126}.get(M, 0))
     wargs, values = any_weights(fmt, N, K, 2600 + M)
     a = dev(f16(O.normal(2601 + M, (M, K)))).half()
     run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, *wargs, M, K, N)  # noqa: E731
