@@ -25,6 +25,7 @@
 //               trip and no redundant dequantisation inside a workgroup.
 // The k order inside a chunk is (lanes 0-31: 8s.., lanes 32-63: 64+8s..); the
 // A fragments are read from LDS with the same order, so the products pair up.
+#include <math.h>
 #include <string.h>
 #include <type_traits>
 
@@ -1829,9 +1830,17 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint
 // end of a tile (K = 1024, 4096 tokens, 4096 rows, Q4_K: 43 us in four-wave workgroups, 50 so; 4096 -> 14336, 3.5 rounds: 451 and 473);
 // a last round that would leave more than half of the CUs idle runs as column halves (gemm_tall_halves).  Taken in place of the plan above where its
 // modelled time (microseconds, fitted like the plan's, K from 2048 on) is less; `cost` = the format's time so against its time in the
-// plan's forms, 1 for Q4_K and Q8_0 (Q6_K 4096 -> 14336: 1024 tokens 185 -> 164, 2048 tokens 348 -> 318, 4096 tokens 608 -> 558).
-template <class QF> constexpr double gemm_tall_cost = 1.0;
-template <> constexpr double gemm_tall_cost<GemmQ6K> = 0.83;
+// plan's form, 1 but for Q6_K.  Q6_K loses most time in the plan's four-wave and 128 x 256 forms (0.83; 4096 -> 14336: 1024 tokens 185 ->
+// 164 us, 2048 tokens 348 -> 318, 4096 tokens 608 -> 558; 76 such shapes: 0.74 to 0.96, one 1.0).  The smaller eight-wave forms
+// load whole dwords (GemmQ6KDw); against them the tiles gain 3 to 10 % in rows of an even number of blocks, which start on a dword, or from the second
+// round on (0.90: not against 96 x 128, 8704 -> 25344, 266 tokens +4 %), and lose in the others: 12032 -> 7936, 1292 tokens, 209 -> 215 us,
+// 4352 -> 5056, 1589 tokens, 114 -> 131, 5376 -> 26944, 284 tokens, 176 -> 200.
+template <class QF>
+static double gemm_tall_cost(const GemmPlan& p, uint64_t K, uint64_t tiles, uint64_t cus) {
+    if (!std::is_same<QF, GemmQ6K>::value) return 1.0;
+    if (p.na == 0 || (p.na == 4 && p.nj == 2)) return 0.83;
+    return K % 512 == 0 || tiles > cus ? 0.90 : HUGE_VAL;
+}
 static bool gemm_tall(uint64_t M, uint64_t K, uint64_t N, uint64_t cus, double cost, bool with_halves, double t_plan) {
     const uint64_t n_chunks = (K + kBK - 1) / kBK, tiles = ((M + 255) / 256) * ((N + 255) / 256), full = tiles / cus, rest = tiles % cus;
     if (M <= 256 || n_chunks < 16) return false;
@@ -1855,7 +1864,8 @@ template <class QF>
 static GemmPlan gemm_form(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus) {
     double t_plan = 0.0;
     const GemmPlan p = gemm_plan(M, K, N, cap, cus, &t_plan);
-    return gemm_tall(M, K, N, cus, gemm_tall_cost<QF>, gemm_tall_halves<QF>, t_plan) ? GemmPlan{8, 2, 1} : p;
+    const double cost = gemm_tall_cost<QF>(p, K, (M + 255) / 256 * ((N + 255) / 256), cus);
+    return gemm_tall(M, K, N, cus, cost, gemm_tall_halves<QF>, t_plan) ? GemmPlan{8, 2, 1} : p;
 }
 
 template <class QF, int MODE>
