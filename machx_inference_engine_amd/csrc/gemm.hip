@@ -1841,6 +1841,14 @@ static double gemm_tall_cost(const GemmPlan& p, uint64_t K, uint64_t tiles, uint
     if (p.na == 0 || (p.na == 4 && p.nj == 2)) return 0.83;
     return K % 512 == 0 || tiles > cus ? 0.90 : HUGE_VAL;
 }
+// Formats that cost little to dequantize lose what a last token tile of at most 128 rows computes for nothing, where it is one of few: 600 tokens,
+// 11008 -> 21208, one round, Q4_K +5 %, Q4_0 +6 %, Q8_0 planes +4 % (MXFP4 0, Q8_0 blocks -3 %, Q5_K -7 %); 780 tokens +2, +3, 0 %; 1300 tokens 0,
+// +1, 0 %; from the seventh on (1540, 4621 tokens) 0 to -5 %.
+template <class QF>
+static bool gemm_tall_padding(uint64_t M) {
+    constexpr bool light = std::is_same<QF, GemmQ4KPair>::value || std::is_same<QF, GemmQ40>::value || std::is_same<QF, GemmQ8Quad>::value;
+    return light && M <= 6 * 256 && (M - 1) % 256 < 128;
+}
 static bool gemm_tall(uint64_t M, uint64_t K, uint64_t N, uint64_t cus, double cost, bool with_halves, double t_plan) {
     const uint64_t n_chunks = (K + kBK - 1) / kBK, tiles = ((M + 255) / 256) * ((N + 255) / 256), full = tiles / cus, rest = tiles % cus;
     if (M <= 256 || n_chunks < 16) return false;
@@ -1864,6 +1872,7 @@ template <class QF>
 static GemmPlan gemm_form(uint64_t M, uint64_t K, uint64_t N, uint64_t cap, uint64_t cus) {
     double t_plan = 0.0;
     const GemmPlan p = gemm_plan(M, K, N, cap, cus, &t_plan);
+    if (gemm_tall_padding<QF>(M)) return p;
     const double cost = gemm_tall_cost<QF>(p, K, (M + 255) / 256 * ((N + 255) / 256), cus);
     return gemm_tall(M, K, N, cus, cost, gemm_tall_halves<QF>, t_plan) ? GemmPlan{8, 2, 1} : p;
 }

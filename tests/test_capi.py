@@ -231,6 +231,17 @@ def test_gemm_q6_K_takes_256_token_tiles_where_they_are_faster(lib, M, K, N, tal
     assert (form[0] == 8) == tall and (tall or form[:3] == ops.gemm_plan(M, K, N))
 
 
+@pytest.mark.parametrize("M,K,N,light", [(520, 11008, 21208, False), (600, 14336, 21208, False), (640, 14336, 21208, False), (641, 14336, 21208, True), (780, 12032, 15232, False),
+                                         (1100, 12288, 13000, False), (1300, 11008, 10456, False), (1540, 14336, 8920, True), (4621, 14336, 3288, True)])
+def test_gemm_256_token_tiles_with_a_half_empty_one(lib, M, K, N, light):
+    """Without a GPU: 256 CUs.  Formats that cost little to dequantize keep the plan where a last token tile of at most 128 rows is one of few."""
+    from machx_inference_engine_amd import ops
+    for f in DENSE[2:3] + DENSE[5:]:
+        assert ops.gemm_form(f, M, K, N)[0] == 8, f
+    for f in ("q4_K", "q4_0", "q8_0_soa"):
+        assert (ops.gemm_form(f, M, K, N)[0] == 8) == light, f
+
+
 def test_gemm_workspace_query_names_what_the_plan_uses(lib):
     """A workspace of the queried size gives the plan of an unlimited one, and outside the shapes that the library's own scratch
     serves it is no larger than that plan's partial sums."""
