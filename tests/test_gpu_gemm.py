@@ -124,6 +124,30 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     assert torch.equal(run(), got), "differs from launch to launch"
 
 
+# every eight-wave form below 128 x 256, rows of an odd and of an even number of Q6_K blocks, with K slices and without
+Q6K_SMALL = [(2, 256, 142, 1, 1), (10, 512, 38, 1, 1), (3, 1280, 57, 1, 1), (2, 1536, 36, 1, 1), (1, 1792, 4618, 1, 2), (1, 1536, 7854, 1, 2), (2, 5632, 8001, 1, 2),
+             (33, 256, 17035, 2, 1), (33, 512, 17355, 2, 1), (33, 1792, 2308, 2, 1), (34, 1536, 2772, 2, 1), (131, 256, 16946, 2, 2), (130, 512, 16681, 2, 2),
+             (35, 3328, 8224, 2, 2), (34, 2560, 11757, 2, 2), (66, 256, 16725, 3, 1), (66, 512, 16982, 3, 1), (67, 1792, 2306, 3, 1), (66, 1536, 2732, 3, 1),
+             (195, 256, 16518, 3, 2), (197, 512, 16429, 3, 2), (129, 3840, 5511, 3, 2), (130, 5120, 5498, 3, 2), (98, 256, 16570, 4, 1), (98, 512, 16391, 4, 1),
+             (97, 1792, 2396, 4, 1), (100, 2048, 2062, 4, 1)]
+
+
+@pytest.mark.parametrize("M,K,N,na,nj", Q6K_SMALL)
+def test_gemm_q6_K_two_bytes_off(mx, M, K, N, na, nj):
+    """Q6_K weights need two-byte alignment only, and the forms that load whole dwords (GemmQ6KDw) shift what lies two bytes off: from an address that is a
+    multiple of four and from one two bytes on, where even blocks are the ones that lie off and the matrix starts behind a dword's first byte, the same
+    bits, and the exact products."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or mx.ops.gemm_form("q6_K", M, K, N, 32 << 20)[:2] == (na, nj)
+    (w,), values = any_weights("q6_K", N, K, 2700 + M)
+    a = dev(f16(O.normal(2701 + M, (M, K)))).half()
+    ws = torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
+    got = mx.ops.gemm_ws("q6_K", a, (w,), M, K, N, ws)
+    check(host(got).astype(np.float32), host(a.double() @ values.double().t()), "gemm q6_K M=%d K=%d N=%d" % (M, K, N))
+    room = torch.full((w.numel() + 4,), 255, dtype=torch.uint8, device="cuda")
+    room[2:-2] = w
+    assert torch.equal(mx.ops.gemm_ws("q6_K", a, (room[2:-2],), M, K, N, ws), got)
+
+
 @pytest.mark.parametrize("fmt,M,K,N", [("q6_K", 1100, 2048, 13000), ("q6_K", 1600, 2048, 12900), ("q6_K", 1644, 13056, 4500), ("q4_K", 1450, 12288, 10700), ("q8_0_soa", 1450, 12288, 10700),
                                        ("q8_0", 1100, 12288, 13000), ("q4_0", 1450, 12288, 10700), ("q5_K", 1100, 12288, 13000), ("mxfp4_soa", 1100, 12224, 13000)])
 def test_gemm_256_token_tiles(mx, fmt, M, K, N):

@@ -446,6 +446,18 @@ def test_gemv_q8_batched_eight_waves(mx, fmt, K, N, T):
         check(host(got).astype(np.float32), ref, "blocks K=%d N=%d T=%d" % (K, N, T))
 
 
+@pytest.mark.parametrize("fmt", [O.Q8_0, O.MXFP4], ids=lambda f: O.FMT_NAMES[f])
+@pytest.mark.parametrize("K,N,T,wr", [(2880, 12000, 9, 2), (2080, 9999, 16, 2), (7968, 12001, 12, 2), (2880, 5120, 13, 1), (1056, 8190, 9, 1),
+                                      (4000, 8191, 7, 1), (6112, 2000, 5, 1), (4128, 33, 8, 1), (4768, 1500, 6, 1)])
+def test_gemv_q8_batched_eight_waves_partial_group(mx, fmt, K, N, T, wr):
+    """The same workgroups over rows whose last group of 256 elements is a partial one, alone in its wave or behind others, with and without K
+    ranges; that they run is asked of the library."""
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        names = ["mxfp4_soa"] if fmt == O.MXFP4 else ["q8_0_soa"] + ["q8_0"] * (T >= 9)
+        assert all(mx.ops.gemv_batched_plan(f, K, N, T)[:2] == (8, wr) for f in names)
+    test_gemv_q8_batched_eight_waves(mx, fmt, K, N, T)
+
+
 @pytest.mark.parametrize("K,N,T", [(256, 40, 5), (768, 100, 16), (1024, 64, 8), (2304, 257, 9), (4096, 96, 12)])
 def test_gemv_q6_K_q8_batched_two_bytes_off(mx, K, N, T):
     """Q6_K blocks are 210 bytes and need two-byte alignment only; the int-dot kernels of the matrix cores load whole dwords and shift (MmqQ6K).  Rows of

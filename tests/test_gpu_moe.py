@@ -583,6 +583,38 @@ def test_moe_grouped_int_dot_short_tiles(mx, fmt, K):
             assert torch.equal(h[off[e]:off[e] + c], h[:c]) and torch.equal(y[off[e]:off[e] + c], y[:c]), (soa, c)
 
 
+@pytest.mark.parametrize("K,N", [(768, 33), (256, 65), (512, 40)])
+@pytest.mark.parametrize("rows", [3, 12, 40])
+def test_moe_grouped_int_dot_q6_K_two_bytes_off(mx, K, N, rows):
+    """Expert banks of Q6_K blocks whose experts lie an odd number of blocks apart (every other one starts two bytes off a dword) and banks that start two
+    bytes off: the matrix-core int-dot loads whole dwords and shifts.  Against the oracle per expert, and the same bits from either address; few rows
+    per expert, a tile of 16 and more."""
+    ops, E = mx.ops, 5
+    counts = [rows, 0, rows + 1, rows, 1]
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    TK = int(off[-1])
+    xq = ops.quantize_q8_1s(dev(f16(O.normal(8800 + K, (TK, K)))).half())
+    host_rows = host(xq).reshape(TK, -1)
+    W = [[O.quantize(O.Q6_K, O.normal(8801 + 7 * m + e, (N, K), 0.0, 0.02)) for e in range(E)] for m in range(2)]
+    stride = W[0][0].size
+    assert stride % 4 == (2 if N * K // 256 % 2 else 0)
+    bank = [dev(np.concatenate([w.ravel() for w in m])) for m in W]
+    room = [torch.full((b.numel() + 4,), 255, dtype=torch.uint8, device="cuda") for b in bank]
+    for r, b in zip(room, bank):
+        r[2:-2] = b
+    out = []
+    for g, u in (bank, [r[2:-2] for r in room]):
+        out.append((ops.moe_prefill_gate_up_silu_kquant_q8("q6k", xq, g, u, dev(off), TK, E, K, N, stride),
+                    ops.moe_prefill_down_packed_kquant_q8("q6k", xq, u, dev(off), TK, E, N, K, stride)))
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        if lo < hi:
+            ref = [O.gemv_q8schain(O.Q6_K, m[e], host_rows[lo:hi], K, N) for m in W]
+            check(host(out[0][0])[lo:hi].astype(np.float32), O.swiglu_np(ref[0].astype(np.float32), ref[1].astype(np.float32)), "gate_up expert %d" % e)
+            check(host(out[0][1])[lo:hi].astype(np.float32), ref[1], "down expert %d" % e)
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("EF", [64, 512, 768, 1152, 1920, 3200])
 def test_moe_mxfp4_down_rows_shorter_than_a_lane_group(mx, EF):
     """One-token down launch with fewer 64-element units in a row than lanes that share it (8 of 16, 18 of 32, 50 of 64, ..), every
