@@ -196,6 +196,33 @@ def test_moe_packing_device_sizes(mx, T, E, K):
     assert np.array_equal(host(wp).astype(np.float32), wp_r)
 
 
+@pytest.mark.parametrize("E", [7, 128, 129, 131, 1000])
+@pytest.mark.parametrize("T,K", [(32, 2), (1000, 4), (1900, 8), (2500, 8)])
+def test_moe_packing_leaves_out_slots_without_an_expert(mx, T, K, E):
+    """Ids below 0 and from E on, among them those that a last workgroup of fewer than four experts counts next to its own (E to E + 2), with 4, 16
+    and more slots a lane: such slots reach no expert's rows, and nothing is written for them or behind the last row."""
+    rng = np.random.default_rng(T + E)
+    ids = rng.integers(0, E, (T, K)).astype(np.int32)
+    odd = rng.random((T, K)) < 0.3
+    ids[odd] = rng.choice(np.array([-1, -(2 ** 31), E, E + 1, E + 2, E + 3, 65536 + E - 1, 2 ** 31 - 1], np.int32), int(odd.sum()))
+    w = f16(rng.random((T, K)).astype(np.float32))
+    flat = ids.ravel()
+    kept = np.flatnonzero((flat >= 0) & (flat < E))
+    order = kept[np.argsort(flat[kept], kind="stable")]
+    n = len(order)
+    off = torch.full((E + 2,), 77, dtype=torch.int32, device="cuda")
+    si, t2p = (torch.full((T * K,), -77, dtype=torch.int32, device="cuda") for _ in range(2))
+    wp = torch.full((T * K,), -7.0, dtype=torch.float16, device="cuda")
+    ids_d, w_d = dev(ids), dev(w).half()
+    mx.ops._call("mx_moe_build_packing_device", ids_d.data_ptr(), w_d.data_ptr(), T, K, E, off.data_ptr(), si.data_ptr(), wp.data_ptr(), t2p.data_ptr())
+    assert np.array_equal(host(off), np.append(np.concatenate([[0], np.cumsum(np.bincount(flat[kept], minlength=E))]), 77))
+    assert np.array_equal(host(si)[:n], order // K) and np.array_equal(host(wp).astype(np.float32)[:n], w.ravel()[order])
+    place = np.full(T * K, -77)
+    place[order] = np.arange(n)
+    assert np.array_equal(host(t2p), place)
+    assert (host(si)[n:] == -77).all() and (host(wp)[n:] == -7.0).all()
+
+
 @pytest.mark.parametrize("T,K,H", [(1, 4, 2880), (3, 5, 8), (2, 9, 20), (33, 8, 1032), (64, 8, 2048), (130, 9, 1032), (127, 5, 1032),
                                    (5, 1, 16), (9, 2, 40), (9, 3, 40), (4, 6, 64), (4, 7, 64), (4, 16, 64), (3, 17, 64)])
 def test_moe_reduce_columns(mx, T, K, H):
