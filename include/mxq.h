@@ -363,7 +363,7 @@ int mx_gemm_mxfp4_soa_ws(mx_stream_t s, const uint16_t* A, const uint8_t* qs_W, 
  * else the *_ws forms with a workspace of ws_bytes.  This is the plan every format shares; by format, launches of more than 256 tokens
  * run over 256 x 256 tiles in its place, unsliced and without scratch.  mx_gemm_form tells what a launch does: format = "q4_K", "q6_K", "q8_0",
  * "q8_0_soa", "q4_0", "q5_K" or "mxfp4_soa", form[0..2] = the plan, form[0] = 8 for 256 x 256 tiles, form[3] = how many of
- * those run as two column halves.  */
+ * those run as two column halves, form[4] = 1 where Q6_K blocks are loaded as whole dwords.  */
 int mx_gemm_plan(uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* plan);
 int mx_gemm_form(const char* format, uint32_t M, uint32_t K, uint32_t N, int own_ws, uint64_t ws_bytes, uint32_t* form);
 /* Q4_0 weights through the same kernel: gemm_q4_0 / gemm_q4_0_xmx  include/ie/ops.hpp:530-534, src/ops/gemv_q4_0.cpp,

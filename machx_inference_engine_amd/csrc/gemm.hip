@@ -615,9 +615,9 @@ struct GemmQ6K {
 // The same blocks loaded as whole dwords and shifted.  Every other block lies two bytes off a dword, and lanes that read 16 such bytes of a row
 // each take the load pipeline three times as long (MmqQ6K).  A lane half reads 32 consecutive bytes of the half block's ql and 16 of its qh from
 // the dword the block's first byte lies in; `ext` is the dword behind the 64 bytes of ql (lower half) or the 32 of qh (upper half), `tail`
-// the last two scales and d.  For the forms whose launches wait for weights: us, pieces from where they lie / so: 4096 -> 14336, 30 tokens
-// (32 x 128) 21.7 / 20.7, 200 tokens (128 x 128) 52.4 / 49.9; 1024 -> 3072, 64 tokens 12.0 / 11.0; 2304 -> 6144, 128 tokens 31.5 / 28.3; 96 x 256,
-// 77 tokens 46.0 / 42.3; through the library 2048 -> 6144, 30 tokens 15.7 / 12.5, 3072 -> 8192, 47 tokens 18.5 / 17.1.  Tiles of 128 x 256 and 256 x 256 are bound by their vector instructions, of which this adds a tenth, and have no
+// the last two scales and d.  For the forms whose launches wait for weights (gemm_small): us, pieces from where they lie / so: 4096 -> 14336, 30 tokens
+// (32 x 128) 21.7 / 20.7; 1024 -> 3072, 64 tokens 12.0 / 11.0; 2304 -> 6144, 128 tokens 31.5 / 28.3; 96 x 256, 77 tokens 46.0 / 42.3; through the library
+// 2048 -> 6144, 30 tokens 15.7 / 12.5, 3072 -> 8192, 47 tokens 18.5 / 17.1.  Tiles of 128 x 256 and 256 x 256 are bound by their vector instructions, of which this adds a tenth, and have no
 // registers left: 512 tokens 93.9 / 95.2, 4096 tokens 521 / 532.
 struct GemmQ6KDw : GemmQ6K {
     struct Raw {
@@ -1863,9 +1863,23 @@ static uint64_t gemm_library_scratch(uint64_t M, uint64_t K, uint64_t N, uint64_
     return K >= 2048 && 2 * ((M + 127) / 128) * ((N + 255) / 256) <= cus ? kGemmSplitElems : 0;
 }
 
-// the producer a format uses in eight-wave workgroups over less than 128 x 256
+// The producer a format uses in eight-wave workgroups over less than 128 x 256.  Q6_K: the one that loads whole dwords, in rows of an odd number of
+// blocks in every form (every other row starts two bytes off, and each load of a wave meets lanes that do; us, pieces from where they lie / so:
+// 6400 -> 17152, 4 tokens 65.1 / 53.8, 6400 -> 8896, 38 tokens 40.4 / 35.3, 6400 -> 1984, 542 tokens 43.8 / 37.0).  In rows of an even number only
+// every other block lies off, for all lanes at once, and the shifts cost what the loads save in the forms that load most per chunk (64 x 256: 7168
+// -> 18752, 42 tokens 65.7 / 68.6; 128 x 128: 11776 -> 6528, 114 tokens 44.7 / 47.3; 32 x 256 over a large matrix: 4096 -> 19008, 5 tokens 37.3 / 39.1,
+// 11264 -> 14720, 7 tokens 67.7 / 72.0, but 4608 -> 11136, 11 tokens 30.1 / 29.2) and where 96 rows of tokens are all there are for a large matrix
+// (96 x 128: 4096 -> 14336, 77 tokens 33.1 / 34.0, 7168 -> 13696, 94 tokens 51.8 / 53.5; 96 x 256: 7680 -> 17408, 96 tokens 73.3 / 78.2); the others gain 3 % in the mean.
 template <class QF> struct GemmSmall { using type = QF; };
 template <> struct GemmSmall<GemmQ6K> { using type = GemmQ6KDw; };
+template <class QF>
+static bool gemm_small(const GemmPlan& p, uint64_t M, uint64_t K, uint64_t N) {
+    if (std::is_same<QF, typename GemmSmall<QF>::type>::value || p.na == 0 || p.na == 8 || (p.na == 4 && p.nj == 2)) return false;
+    if (K % 512) return true;
+    if (p.na == 1) return p.nj == 1 || K * N < 64u << 20;
+    if (p.na == 2) return p.nj == 1;
+    return p.na == 3 && (M > 96 || K * N < 48u << 20);
+}
 
 // The form of a dense launch of a format: the plan, na = 8 where the 256-token tiles take its place.
 template <class QF>
@@ -1898,15 +1912,16 @@ static int launch_gemm(mx_stream_t s, const typename QF::Bank& b0, const typenam
             }
         }
         using QS = typename GemmSmall<QF>::type;
+        const bool small = gemm_small<QF>(p, g.M, g.K, g.N);
         int rc;
         switch (p.na * 2 + p.nj - 1) {
             case 2: rc = launch_gemm_ni<QS, MODE, 1, 2, 1>(s, b0, b1, g, rows_bound); break;
-            case 3: rc = launch_gemm_ni<QS, MODE, 1, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 3: rc = small ? launch_gemm_ni<QS, MODE, 1, 2, 2>(s, b0, b1, g, rows_bound) : launch_gemm_ni<QF, MODE, 1, 2, 2>(s, b0, b1, g, rows_bound); break;
             case 4: rc = launch_gemm_ni<QS, MODE, 2, 2, 1>(s, b0, b1, g, rows_bound); break;
-            case 5: rc = launch_gemm_ni<QS, MODE, 2, 2, 2>(s, b0, b1, g, rows_bound); break;
-            case 6: rc = launch_gemm_ni<QS, MODE, 3, 2, 1>(s, b0, b1, g, rows_bound); break;
-            case 7: rc = launch_gemm_ni<QS, MODE, 3, 2, 2>(s, b0, b1, g, rows_bound); break;
-            case 8: rc = launch_gemm_ni<QS, MODE, 4, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 5: rc = small ? launch_gemm_ni<QS, MODE, 2, 2, 2>(s, b0, b1, g, rows_bound) : launch_gemm_ni<QF, MODE, 2, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 6: rc = small ? launch_gemm_ni<QS, MODE, 3, 2, 1>(s, b0, b1, g, rows_bound) : launch_gemm_ni<QF, MODE, 3, 2, 1>(s, b0, b1, g, rows_bound); break;
+            case 7: rc = small ? launch_gemm_ni<QS, MODE, 3, 2, 2>(s, b0, b1, g, rows_bound) : launch_gemm_ni<QF, MODE, 3, 2, 2>(s, b0, b1, g, rows_bound); break;
+            case 8: rc = small ? launch_gemm_ni<QS, MODE, 4, 2, 1>(s, b0, b1, g, rows_bound) : launch_gemm_ni<QF, MODE, 4, 2, 1>(s, b0, b1, g, rows_bound); break;
             case 9: rc = launch_gemm_ni<QF, MODE, 4, 2, 2>(s, b0, b1, g, rows_bound); break;
             default: rc = launch_gemm_ni<QF, MODE, 4>(s, b0, b1, g, rows_bound);
         }
@@ -2040,6 +2055,7 @@ int mx_gemm_form(const char* format, uint32_t M, uint32_t K, uint32_t N, int own
         const uint64_t tiles = ((uint64_t)M + 255) / 256 * (((uint64_t)N + 255) / 256);
         form[0] = p.na; form[1] = p.nj; form[2] = p.k_split;
         form[3] = p.na == 8 ? (uint32_t)(tiles - gemm_whole_tiles<QF>(tiles, cus)) : 0u;
+        form[4] = gemm_small<QF>(p, M, K, N) ? 1u : 0u;
         return (int)MX_OK;
     };
     if (is("q4_K")) return of(GemmQ4KPair{});

@@ -235,8 +235,9 @@ def gemm_plan(M, K, N, ws_bytes=None):
 
 
 def gemm_form(fmt, M, K, N, ws_bytes=None):
-    """gemm_plan as a launch of this format has it, 8 as the first for tiles of 256 tokens, and how many of those run as column halves."""
-    form = (ctypes.c_uint32 * 4)()
+    """gemm_plan as a launch of this format has it, 8 as the first for tiles of 256 tokens; how many of those run as column halves; 1 where Q6_K
+    blocks are loaded as whole dwords."""
+    form = (ctypes.c_uint32 * 5)()
     rc = lib.mx_gemm_form(fmt.encode(), M, K, N, ws_bytes is not None, ws_bytes or 0, ctypes.addressof(form))
     if rc != 0:
         raise MxError("mx_gemm_form", rc)

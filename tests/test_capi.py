@@ -205,9 +205,9 @@ def test_gemm_form_query(lib):
     for M, K, N in [(1, 64, 33), (77, 14336, 4096), (256, 14336, 4096), (512, 4096, 14336), (700, 1792, 9000)]:
         for f in DENSE:
             for ws in (None, 32 << 20):
-                assert ops.gemm_form(f, M, K, N, ws) == ops.gemm_plan(M, K, N, ws) + (0,), (f, M, K, N)
-    assert all(ops.gemm_form(f, 4096, 14336, 4096) == (8, 2, 1, 0) for f in DENSE) and ops.gemm_plan(4096, 14336, 4096)[0] == 0
-    form = (C.c_uint32 * 4)()
+                assert ops.gemm_form(f, M, K, N, ws)[:4] == ops.gemm_plan(M, K, N, ws) + (0,), (f, M, K, N)
+    assert all(ops.gemm_form(f, 4096, 14336, 4096) == (8, 2, 1, 0, 0) for f in DENSE) and ops.gemm_plan(4096, 14336, 4096)[0] == 0
+    form = (C.c_uint32 * 5)()
     p = C.addressof(form)
     assert l.mx_gemm_form(None, 64, 1280, 896, 0, 0, p) == 1 and l.mx_gemm_form(b"q4_K", 64, 1280, 896, 0, 0, None) == 1
     assert l.mx_gemm_form(b"q4_K", 64, 0, 896, 0, 0, p) == 2 and l.mx_gemm_form(b"q3_K", 64, 1280, 896, 0, 0, p) == 5
@@ -240,6 +240,18 @@ def test_gemm_256_token_tiles_with_a_half_empty_one(lib, M, K, N, light):
         assert ops.gemm_form(f, M, K, N)[0] == 8, f
     for f in ("q4_K", "q4_0", "q8_0_soa"):
         assert (ops.gemm_form(f, M, K, N)[0] == 8) == light, f
+
+
+@pytest.mark.parametrize("M,K,N,form,dwords", [(30, 2048, 6144, (1, 1), 1), (4, 6400, 17152, (1, 2), 1), (7, 11264, 14720, (1, 2), 0), (18, 12288, 10944, (1, 2), 0),
+                                               (16, 5120, 20352, (1, 2), 0), (5, 4096, 19008, (1, 2), 0), (11, 4608, 11136, (1, 2), 1), (30, 3584, 12288, (1, 2), 1), (38, 6400, 8896, (2, 2), 1), (42, 7168, 18752, (2, 2), 0), (542, 6400, 1984, (4, 1), 1),
+                                               (114, 11776, 6528, (4, 1), 0), (77, 14336, 4096, (3, 1), 0), (94, 7168, 13696, (3, 1), 0), (96, 7680, 17408, (3, 2), 0), (65, 3072, 9152, (3, 1), 1), (159, 5120, 3456, (3, 1), 1), (156, 2304, 10880, (2, 1), 1),
+                                               (527, 3072, 10688, (3, 2), 1), (512, 4096, 14336, (4, 2), 0)])
+def test_gemm_q6_K_loads_dwords_where_that_is_faster(lib, M, K, N, form, dwords):
+    """Without a GPU: 256 CUs.  Rows of an odd number of blocks in every eight-wave form below 128 x 256; of an even number not in those that lose 1 to 7 %."""
+    from machx_inference_engine_amd import ops
+    f = ops.gemm_form("q6_K", M, K, N)
+    assert f[:2] == form and f[4] == dwords
+    assert all(ops.gemm_form(o, M, K, N)[4] == 0 for o in DENSE if o != "q6_K")
 
 
 def test_gemm_workspace_query_names_what_the_plan_uses(lib):

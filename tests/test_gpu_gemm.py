@@ -113,7 +113,7 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     """Every form of a dense launch with every weight loader, MXFP4 with a row that ends half way through a chunk; the form a shape takes
     is asked of the library, so that a change of the rule shows.  Against the exact products of the fp16 weights in fp64."""
     M, K, N = half if fmt == "mxfp4_soa" else whole
-    na, nj, k, _ = mx.ops.gemm_form(fmt, M, K, N, 32 << 20)
+    na, nj, k = mx.ops.gemm_form(fmt, M, K, N, 32 << 20)[:3]
     assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or (na, nj, k > 1) == form, (na, nj, k)
     wargs, values = any_weights(fmt, N, K, 2500 + M)
     a = dev(f16(O.normal(2501 + M, (M, K)))).half()
@@ -124,12 +124,12 @@ def test_gemm_every_form_and_loader(mx, form, whole, half, fmt):
     assert torch.equal(run(), got), "differs from launch to launch"
 
 
-# every eight-wave form below 128 x 256, rows of an odd and of an even number of Q6_K blocks, with K slices and without
+# every eight-wave form below 128 x 256, rows of an odd and of an even number of Q6_K blocks, with K slices and without, both producers
 Q6K_SMALL = [(2, 256, 142, 1, 1), (10, 512, 38, 1, 1), (3, 1280, 57, 1, 1), (2, 1536, 36, 1, 1), (1, 1792, 4618, 1, 2), (1, 1536, 7854, 1, 2), (2, 5632, 8001, 1, 2),
              (33, 256, 17035, 2, 1), (33, 512, 17355, 2, 1), (33, 1792, 2308, 2, 1), (34, 1536, 2772, 2, 1), (131, 256, 16946, 2, 2), (130, 512, 16681, 2, 2),
              (35, 3328, 8224, 2, 2), (34, 2560, 11757, 2, 2), (66, 256, 16725, 3, 1), (66, 512, 16982, 3, 1), (67, 1792, 2306, 3, 1), (66, 1536, 2732, 3, 1),
              (195, 256, 16518, 3, 2), (197, 512, 16429, 3, 2), (129, 3840, 5511, 3, 2), (130, 5120, 5498, 3, 2), (98, 256, 16570, 4, 1), (98, 512, 16391, 4, 1),
-             (97, 1792, 2396, 4, 1), (100, 2048, 2062, 4, 1)]
+             (97, 1792, 2396, 4, 1), (100, 2048, 2062, 4, 1), (66, 4608, 11008, 3, 1), (70, 7680, 17408, 3, 2)]
 
 
 @pytest.mark.parametrize("M,K,N,na,nj", Q6K_SMALL)
@@ -154,7 +154,7 @@ def test_gemm_256_token_tiles(mx, fmt, M, K, N):
     """The tiles of 256 tokens (gemm_tall in csrc/gemm.hip; 256 CUs) with every weight loader, ragged in tokens and columns; the second shape
     ends in column halves, one of them past N, the third has nothing else; MXFP4 in a row that ends half way through a chunk.  The sums run over K in one piece: against the
     exact products of the fp16 weights in fp64, as every other form."""
-    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or mx.ops.gemm_form(fmt, M, K, N) == (8, 2, 1, {1600: 101, 1644: 126}.get(M, 0))
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or mx.ops.gemm_form(fmt, M, K, N)[:4] == (8, 2, 1, {1600: 101, 1644: 126}.get(M, 0))
     wargs, values = any_weights(fmt, N, K, 2600 + M)
     a = dev(f16(O.normal(2601 + M, (M, K)))).half()
     run = lambda: getattr(mx.ops, "gemm_" + fmt)(a, *wargs, M, K, N)  # noqa: E731
