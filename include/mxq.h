@@ -164,8 +164,10 @@ int mx_gemv_mxfp4_soa_q8_x2(mx_stream_t s, const void* x_q8, const uint8_t* gate
  * points as they are): batched launches whose row groups alone would leave CUs idle (at most those for which
  * mx_gemv_batched_ws_bytes is not 0: T >= 2 with K >= 8192, T >= 4 with K > 3840, T >= 9 with K > 1792)
  * split K over workgroups and keep slices x T x N fp32 partial sums in a 2 MB file-scope device array (one copy
- * per device, resolved with hipGetSymbolAddress on first use or by mx_init, never allocated or freed).  Limit:
- * slices * min(T, 8) * N <= 524288 floats (e.g. T = 8, N = 16384); a launch beyond it runs unsplit.  Every call
+ * per device, resolved with hipGetSymbolAddress on first use or by mx_init, never allocated or freed) of 524288
+ * floats.  The vector kernels (plan[0] = 0 of mx_gemv_batched_plan) need slices * min(T, 8) * N of
+ * them (e.g. T = 8, N = 16384) and run unsplit beyond that; the matrix-core kernels need slices * T * N and take fewer
+ * slices beyond it.  Every call
  * on a device shares that device's array: two such calls that overlap on one device (different streams, graph
  * branches) race on it, exactly as calls sharing the reference's static per-device scratch buffers would
  * (src/model/dense_dispatch.hpp:547-560).  Callers that overlap launches use the *_ws forms below.  */

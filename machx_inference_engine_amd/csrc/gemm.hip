@@ -12,7 +12,7 @@
 //   workgroup = 4 waves, 128 tokens x (4 x 64) weight rows, two per CU; wave = 128 tokens x 64 rows = 4 x 2 MFMA tiles
 //               (128 accumulator VGPRs).  Dense launches that would not fill the chip so: 8 waves, one workgroup per CU, the
 //               two halves of K (or of a K slice) side by side, 32 .. 128 tokens x 128 or 256 weight rows (gemm_plan).  Large
-//               ones may run 256 tokens x 256 rows in four waves, one workgroup per CU (gemm_tall);
+//               ones may run 256 tokens x 256 rows in four waves, one workgroup per CU (gemm_tall), by format;
 //   tokens    : the fp16 A chunk [tokens x 128] is staged in LDS (double buffered, unpadded
 //               256-byte rows whose 16-byte columns are XOR-swizzled by the row number, so a
 //               fragment read is bank-conflict free) and shared by four waves;
@@ -1935,7 +1935,7 @@ static int check_gemm(const void* A, const void* W, const void* y, uint32_t M, u
     MX_REQUIRE_PTR(A);
     MX_REQUIRE_PTR(W);
     MX_REQUIRE_PTR(y);
-    MX_REQUIRE_SHAPE(M > 0 && N > 0 && K > 0 && K % k_align == 0 && K <= (1u << 22));   // a 128-row A tile is addressed with 32-bit byte offsets
+    MX_REQUIRE_SHAPE(M > 0 && N > 0 && K > 0 && K % k_align == 0 && K <= (1u << 22));   // an A tile, up to 256 rows, is addressed with unsigned 32-bit byte offsets
     MX_REQUIRE_ALIGN(A, 16);
     MX_REQUIRE_ALIGN(W, w_align);
     return MX_OK;

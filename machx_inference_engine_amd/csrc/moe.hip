@@ -321,8 +321,8 @@ __global__ __launch_bounds__(256) void merge_f32_kernel(const float* y32, half_t
 // order.  Bound by two trips to memory for few tokens and by the bytes for many (2048 tokens of hidden 2048, k = 8, 75 MB: 15.8 us on cold
 // caches).  With every slot under a test of its own, a row's number waited for the row before it, and few outputs of more than four rows
 // were better off with a column a thread.  us so / now: k = 8, hidden 2048, routing weights, 1 token 2.8 / 2.3, 64 tokens 3.2 / 2.5, 333
-// tokens 5.8 / 4.3, 2048 tokens 17.6 / 16.7, without weights 333 tokens 5.3 / 4.4, 2048 tokens 15.5 / 15.8; k = 4, hidden 2880, 1 token
-// 2.3 / 2.1, 2048 tokens 15.2 / 12.7.
+// tokens 5.8 / 4.3, 2048 tokens 17.4 / 16.6, without weights 333 tokens 5.3 / 4.4, 2048 tokens 15.8 / 16.1 (1024 tokens 11.0 / 9.2, 4096 tokens 30.7 /
+// 30.2); k = 4, hidden 2880, 1 token 2.3 / 2.1, 2048 tokens 15.2 / 12.7.
 template <bool WEIGHTED, bool ACCUMULATE, int G>
 __global__ __launch_bounds__(256) void moe_reduce8_kernel(const half_t* __restrict__ packed, const uint32_t* __restrict__ tk_to_packed, const half_t* __restrict__ w,
                                                           half_t* __restrict__ y, uint32_t T, uint32_t Ktop, uint32_t H8) {

@@ -949,7 +949,8 @@ constexpr bool mmq_two_tails() {
     return std::is_same<P, MmqQ8Soa>::value || (EPI == MMQ_STORE && (TV == 4 || (TV == 8 && P::K_ALIGN == 256)));
 }
 // Three workgroups of four waves per CU instead of two where that costs no scratch: a dense launch of 512 to 768 workgroups is then one
-// round (4096 -> 14336, 12 tokens: Q4_K 19.6 -> 16.4 us, Q8_0 planes 23.4 -> 21.6).  Q6_K and MXFP4 would spill.
+// round (4096 -> 14336, 12 tokens: Q4_K 19.6 -> 16.4 us, Q8_0 planes 23.4 -> 21.6).  Q6_K and MXFP4 would spill.  The bound is waves per SIMD,
+// and workgroups of eight waves, which leave two there, are compiled under it too; they were timed so, not without it.
 template <class P, int TV, int NW, int EPI>
 constexpr int mmq_workgroups_per_cu() {
     return TV == 8 && NW == 1 && (std::is_same<P, MmqQ8Soa>::value || (EPI == MMQ_STORE && std::is_same<P, MmqQ4K>::value)) ? 3 : 2;

@@ -1,5 +1,7 @@
-// Body of the loop over token tiles of mmq_kernel (mxq_mmq.h), for a tile of at most 2 TR rows from row t0 on; included there once per
-// tile size of the kernel.
+// Body of the loop over token tiles of mmq_kernel (mxq_mmq.h), for a tile of at most 2 TR rows from row t0 on; included there twice, as text (mmq_tile
+// says why), so without a guard.  What it takes from around it: the template parameters P, TR, NW, WR, WK, EPI and NATIVE; the arguments a, lds, e
+// (expert), t0, r_end (end of the expert's rows), kzi, G0, G1 (the workgroup's K range and its groups); lane, j, h, wave, wk, wr, wm; w (the wave's
+// matrix), nb, n_rb (blocks of 32 elements, row blocks), gp (groups staged at once), single (all at once), q8_row_bytes, red (the exchange area).
 const uint32_t nt = r_end - t0 < 2 * TR ? r_end - t0 : 2 * TR;
 auto xrow = [&](uint32_t t) { return a.xq8 + (size_t)(t0 + t) * q8_row_bytes; };
 auto hrow = [&](uint32_t t) { return a.act_f16 + (size_t)(t0 + t) * a.K; };
